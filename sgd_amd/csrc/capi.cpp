@@ -15,13 +15,14 @@
 #include "../../include/sgdct.h"
 #include "footprint.hpp"
 #include "projector.hpp"
+#include "symmetry.hpp"
 
 namespace sgdct {
-hipError_t launch_forward(int basis, const Proj2DArgs& g, const float* img, float* sino, int batch, int nseg,
-                          double* part, hipStream_t s);
-hipError_t launch_backward(int basis, const Proj2DArgs& g, bool use_lds, const float* sino, float* img, int batch,
-                           int ngroup, double* part, hipStream_t s);
-int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host);
+hipError_t launch_forward(int basis, const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino,
+                          hipStream_t s);
+hipError_t launch_backward(int basis, const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img,
+                           hipStream_t s);
+int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough);
 hipError_t launch_count(const Proj2DArgs& g, unsigned long long* out, hipStream_t s);
 hipError_t launch_sf_forward(const Proj2DArgs& g, const float* img, float* sino, int batch, int nseg, double* part,
                              hipStream_t s);
@@ -165,7 +166,12 @@ struct sgdct_projector {
   float* h_sino = nullptr;  // pinned
   unsigned long long* d_count = nullptr;
   long long evals = -1;
-  bool bwd_lds = false;  // A^T stages bin windows in LDS (B0 / B1)
+  bool bwd_lds = false;  // the batched A^T stages bin windows in LDS (B0 / B1)
+  // B0 / B1: the scan's symmetries (group2d.hpp) and A^T's LDS bin window
+  // (0: too wide, records are read from global memory)
+  SymPlan sym{};
+  int* d_sym = nullptr;
+  int win = 0;
   // B0 / B1 / SF: A splits each bin's walk into line segments and A^T the views
   // into groups; fwd_auto / bwd_auto are chosen at creation from one image's
   // launch size, fwd_split / bwd_split (0 = automatic) override them.  The
@@ -213,6 +219,7 @@ struct sgdct_projector {
   ~sgdct_projector() {
     if (d_views) (void)hipFree(d_views);
     if (d_bins) (void)hipFree(d_bins);
+    if (d_sym) (void)hipFree(d_sym);
     if (d_img) (void)hipFree(d_img);
     if (d_sino) (void)hipFree(d_sino);
     if (d_count) (void)hipFree(d_count);
@@ -263,6 +270,14 @@ struct sgdct_batch {
 
 namespace {
 
+bool grouped(int basis) { return basis == BASIS_B0 || basis == BASIS_B1; }
+int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views);
+constexpr size_t kLdsBytes = (size_t)64 << 10;
+size_t bwd_lds_bytes(int win, int views, int g) { return (size_t)win * views * (32 + 4 * g); }
+size_t work_doubles(const sgdct_projector* h);
+SymPlan plain_plan(const sgdct_projector* h);
+int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
+int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
 int auto_fwd_split(const sgdct_projector* h);
 int auto_bwd_split(const sgdct_projector* h);
 int ensure_part(sgdct_projector* h, size_t doubles);
@@ -400,7 +415,15 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
   a.h = h->h;
   a.nchunk = (nu + 63) / 64;
   // 2 bins of slack for FP64 contraction differences between host and device
-  if (basis == BASIS_B0 || basis == BASIS_B1) h->bwd_lds = max_tile_window(a, views.data()) <= kMaxWindow - 2;
+  if (grouped(basis)) {
+    const int w = max_tile_window(a, views.data(), kMaxWindow - 2) + 2;
+    h->bwd_lds = w <= kMaxWindow;
+    if (setup_symmetry(h, views) != SGDCT_OK) {
+      delete h;
+      return nullptr;
+    }
+    if (bwd_lds_bytes(w, 1, h->sym.nh) <= kLdsBytes) h->win = w;
+  }
   if (splits(basis)) {
     // hexagonal A runs unsplit unless asked: at 296 x 256 points, 1024 views
     // and 1024 bins, 2..16 row segments took one image from 1.11 to 1.20..1.40
@@ -408,7 +431,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     // lattice rows only, before steep waves walked the vertical lines)
     h->fwd_auto = is_hex(basis) ? 1 : auto_fwd_split(h);
     h->bwd_auto = auto_bwd_split(h);
-    if (ensure_part(h, part_images(h) * part_need(h)) != SGDCT_OK) {
+    if (ensure_part(h, work_doubles(h)) != SGDCT_OK) {
       delete h;
       return nullptr;
     }
@@ -542,20 +565,146 @@ int cone_backward(sgdct_projector* h, const float* proj, float* vol, int batch, 
 // times in A (its per-wave work is uneven) and 12 times in A^T.  B1 at
 // 512 x 512, 720 views, 768 bins thus runs 24 segments and 24 view groups:
 // A 0.942 ms, A^T 0.922 ms, against 0.960 / 0.932 ms at 16 / 16.
-constexpr long long kFwdWaveTarget = 200000, kBwdWaveTarget = 98304;
+constexpr long long kFwdWaveTarget = 200000, kBwdWaveTarget = 98304, kBwdBlockTarget = 4600, kBwdSmallBlocks = 1024;
+// A^T stages as many views at a time as fill 16 KB of LDS (16, 24, 32 KB: 200
+// us at 512 x 512, 720 views; 48 KB, which costs a workgroup per CU, 210 us).
+constexpr size_t kBwdStageBytes = (size_t)16 << 10;
+constexpr int kBwdMaxViews = 8;
 constexpr int kAutoMaxSplit = 24;  // automatic splits stop here
 constexpr int kMaxSplit = 32;      // sgdct_split_config accepts 1..kMaxSplit
 
 int auto_fwd_split(const sgdct_projector* h) {
+  if (grouped(h->basis)) return kAutoMaxSplit;
   const long long waves = (long long)h->np * h->args.nchunk;
   return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, (kFwdWaveTarget + waves - 1) / waves));
 }
 
 int auto_bwd_split(const sgdct_projector* h) {
+  if (grouped(h->basis)) {
+    const long long tiles = h->win ? h->sym.ntile : plain_plan(h).ntile;
+    // groups of >= 16 views while they add blocks up to kBwdBlockTarget; a
+    // small image, which leaves the GPU idle, takes groups of >= 4 views up
+    // to kBwdSmallBlocks (64 x 64, 60 views: 29.2 us at 16 views per group,
+    // 14.4 us at 4; 512 x 512, 90 views, batch 8: 205 us at 16, 257 us at 4)
+    const long long target = h->sym.nh > 1 ? kBwdBlockTarget / tiles : (kBwdWaveTarget / 4 + tiles - 1) / tiles;
+    const long long many = std::min<long long>(h->np / 16, target);
+    const long long few = std::min<long long>(h->np / 4, kBwdSmallBlocks / tiles);
+    return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, std::max(many, few)));
+  }
   const long long waves = 4LL * ((h->nx + kTile - 1) / kTile) * ((h->ny + kTile - 1) / kTile);
   const long long by_views = std::max(1, h->np / (4 * kViewChunk));  // groups of >= 16 views
   return (int)std::max(1LL, std::min<long long>(std::min<long long>(kAutoMaxSplit, by_views),
                                                 (kBwdWaveTarget + waves - 1) / waves));
+}
+
+// The identity only.
+SymPlan plain_plan(const sgdct_projector* h) {
+  SymPlan p{};
+  p.nh = 1;
+  p.nrep = h->np;
+  p.ntile = ((h->nx + kTile - 1) / kTile) * ((h->ny + kTile - 1) / kTile);
+  return p;
+}
+
+// Largest number of values per footprint whose interleaved image keeps
+// 32-bit byte offsets.
+int max_group(const sgdct_projector* h) {
+  int g = kMaxGroup;
+  while (g > 1 && (unsigned long long)h->nx * h->ny * 4 * g >= (1ull << 32)) g >>= 1;
+  return g;
+}
+
+// Symmetries are used as far as they leave A this many workgroups per image
+// (one per CU).  B1 with the limit at 256 / 512 workgroups, A + A^T: 128 x
+// 128, 180 views 47 / 72 us, 256 x 256, 90 views 72 / 104 us; at 64 the
+// smallest launches run out of workgroups (96 x 96, 90 views 50 / 44 us).
+constexpr long long kSymBlocks = 256;
+
+int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views) {
+  h->sym = plain_plan(h);
+  // B0's footprint is cut off at the corner range where it is not small, so
+  // that a pixel corner that falls on a bin edge (every axis-aligned view of
+  // an even image has such) belongs to either bin by rounding alone; a
+  // symmetric view would take the representative's choice (6e-7 of a 256 x
+  // 256, 360-view sinogram).  B0 shares footprints between images only.
+  int most = h->basis == BASIS_B0 ? 1 : max_group(h);
+  while (most > 1 && (long long)(h->np / most) * h->args.nchunk < kSymBlocks) most >>= 1;
+  // mirrors and half turns for any grid, axis swaps for square ones
+  unsigned allowed = 1u | 1u << SymOp::kFlipX | 1u << SymOp::kFlipY | 1u << (SymOp::kFlipX | SymOp::kFlipY);
+  if (h->nx == h->ny && h->dx == h->dy) allowed = 0xff;
+  const SymTables t = find_symmetries(views, h->nx, h->ny, h->nu, allowed, most, 4e-12 * (h->lsd + h->lso));
+  if (t.nh() == 1) return SGDCT_OK;
+  const size_t nr = t.rep.size(), nv = t.rep_view.size(), np = t.view.size(), nt = t.tile.size();
+  std::vector<int> all(nr + nv + np + nt + (t.owner.size() + 3) / 4);
+  std::copy(t.rep.begin(), t.rep.end(), all.begin());
+  std::copy(t.rep_view.begin(), t.rep_view.end(), all.begin() + nr);
+  std::copy(t.view.begin(), t.view.end(), all.begin() + nr + nv);
+  std::copy(t.tile.begin(), t.tile.end(), all.begin() + nr + nv + np);
+  std::memcpy(all.data() + nr + nv + np + nt, t.owner.data(), t.owner.size());
+  hipError_t e = hipMalloc(&h->d_sym, all.size() * sizeof(int));
+  if (e == hipSuccess) e = hipMemcpy(h->d_sym, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice);
+  if (e != hipSuccess) return hip_fail(e, "symmetry tables");
+  SymPlan& p = h->sym;
+  p.nh = t.nh();
+  p.lg = p.nh == 8 ? 3 : (p.nh == 4 ? 2 : 1);
+  for (int k = 0; k < p.nh; ++k) p.op[k] = t.op[k];
+  p.nrep = (int)nr;
+  p.rep = h->d_sym;
+  p.rep_view = h->d_sym + nr;
+  p.view = h->d_sym + nr + nv;
+  p.ntile = (int)nt;
+  p.tile = h->d_sym + nr + nv + np;
+  p.owner = reinterpret_cast<const unsigned char*>(h->d_sym + nr + nv + np + nt);
+  return SGDCT_OK;
+}
+
+// Values per footprint of a launch on m images: a power of two.
+int group_size(int nh, int m) {
+  int g = nh;
+  while (g < nh * m) g <<= 1;
+  return g;
+}
+
+// Of n line segments, kFwdWaves are the waves of a workgroup (interleaved
+// lines, summed in LDS) and the rest are grid segments with FP64 partial sums.
+// Grid segments pay where a workgroup per (view, chunk) leaves the launch
+// short of waves, and where the image outgrows the L2 caches and the segments
+// walk it band by band: A at 24 / 8 segments, B1: 256 x 256, 360 views 43 / 65
+// us; 2048 x 2048, 1440 views 4.70 / 5.05 ms.  Otherwise their partial sums
+// only cost, and the launch keeps one: 512 x 512, 721 views (two symmetries,
+// 4332 workgroups) 453 / 422 us; 64 x 64, 60 views 11.9 / 9.7 us (a launch
+// more).
+int grid_segments(const sgdct_projector* h, int n) {
+  const long long blocks = (long long)h->sym.nrep * h->args.nchunk;
+  const size_t bytes = (size_t)h->nx * h->ny * h->sym.nh * sizeof(float);
+  const bool more = std::max(h->nx, h->ny) > 96 && (blocks < 2048 || bytes > ((size_t)16 << 20));
+  return more ? (n + kFwdWaves - 1) / kFwdWaves : 1;
+}
+
+// Workspace of a grouped A: [partial sums | interleaved images | transposes],
+// in doubles, for image groups of m images.
+size_t fwd_group_doubles(const sgdct_projector* h, int nh, int nseg, int m) {
+  const size_t n = (((size_t)h->nx * h->ny * group_size(nh, m) + 3) / 4 * 4) / 2;
+  return (nseg > 1 ? ((size_t)nseg * m * h->np * h->nu + 1) / 2 * 2 : 0) + 2 * n;
+}
+
+// One image of at most this edge without symmetries is read in place: its
+// transpose is a launch that the column walks do not earn back.
+constexpr int kDirectEdge = 96;
+
+constexpr size_t kGroupBytes = (size_t)64 << 20;  // several image groups per launch up to this much workspace
+
+// Workspace of a handle: for B0 / B1 one image group of A with as many images
+// as fit kMaxGroup values, more while it stays within kGroupBytes; the FP64
+// partial images of A^T.
+size_t work_doubles(const sgdct_projector* h) {
+  const size_t part = part_images(h) * part_need(h);
+  if (!grouped(h->basis)) return part;
+  const int m = std::max(1, max_group(h) / h->sym.nh);
+  size_t need = fwd_group_doubles(h, h->sym.nh, grid_segments(h, fwd_segments(h)), m);
+  need *= std::max<size_t>(1, std::min<size_t>(16, kGroupBytes / sizeof(double) / need));
+  const int bs = bwd_groups(h);
+  return std::max(need, bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0);
 }
 
 // Room for `doubles` partial sums.
@@ -601,15 +750,80 @@ int part_images(const sgdct_projector* h) {
 hipError_t launch_fwd2d(const sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* part,
                         hipStream_t s) {
   if (h->basis == BASIS_SF) return launch_sf_forward(h->args, img, sino, batch, nseg, part, s);
-  if (is_hex(h->basis)) return launch_hex_forward(h->basis, h->args, h->dt, img, sino, batch, nseg, part, s);
-  return launch_forward(h->basis, h->args, img, sino, batch, nseg, part, s);
+  return launch_hex_forward(h->basis, h->args, h->dt, img, sino, batch, nseg, part, s);
 }
 
 hipError_t launch_bwd2d(const sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* part,
                         hipStream_t s) {
   if (h->basis == BASIS_SF) return launch_sf_backward(h->args, sino, img, batch, ngroup, part, s);
-  if (is_hex(h->basis)) return launch_hex_backward(h->basis, h->args, h->dt, sino, img, batch, ngroup, part, s);
-  return launch_backward(h->basis, h->args, h->bwd_lds, sino, img, batch, ngroup, part, s);
+  return launch_hex_backward(h->basis, h->args, h->dt, sino, img, batch, ngroup, part, s);
+}
+
+// B0 / B1 A: images in groups of m, as many groups per launch as the
+// workspace buf[0, cap) holds.  Every image's values are formed the same way
+// whatever the batch.  A workspace too small for one group of one image
+// runs without symmetries, reading the image in place (partial sums, which a
+// fixed split needs, must fit).
+int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* buf, size_t cap,
+                  bool plain, hipStream_t s) {
+  const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
+  nseg = grid_segments(h, nseg);
+  if (nseg > 1 && (!buf || cap < nseg * ns)) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
+  GroupRun r;
+  r.sym = plain ? plain_plan(h) : h->sym;
+  r.split = nseg;
+  r.m = plain ? 1 : std::max(1, std::min(batch, max_group(h) / r.sym.nh));
+  while (r.m > 1 && fwd_group_doubles(h, r.sym.nh, nseg, r.m) > cap) --r.m;
+  const size_t per = fwd_group_doubles(h, r.sym.nh, nseg, r.m);
+  const bool interleave = buf && per <= cap && (r.sym.nh * r.m > 1 || std::max(h->nx, h->ny) > kDirectEdge);
+  if (!interleave) r.sym = plain_plan(h), r.m = 1;
+  r.g = group_size(r.sym.nh, r.m);
+  const size_t groups = interleave ? cap / per : (nseg > 1 ? cap / (nseg * ns) : (size_t)batch);
+  const int step = (int)std::min<size_t>(batch, groups * r.m);
+  hipError_t e = hipSuccess;
+  for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += step) {
+    r.batch = std::min(step, batch - b0);
+    if (r.batch < r.m) r.m = r.batch, r.g = group_size(r.sym.nh, r.m);
+    double* at = buf;
+    if (nseg > 1) {
+      r.part = at;
+      at += (size_t)nseg * r.batch * ns;
+    }
+    if (interleave) {
+      if ((at - buf) & 1) ++at;  // 16-byte alignment
+      const size_t n = (ni * r.g + 3) / 4 * 4 * r.groups();
+      r.rows = r.g > 1 ? reinterpret_cast<float*>(at) : nullptr;
+      r.cols = reinterpret_cast<float*>(at) + n;
+    }
+    e = launch_forward(h->basis, h->args, r, img + b0 * ni, sino + b0 * ns, s);
+  }
+  return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
+}
+
+// B0 / B1 A^T, view groups' FP64 partial images in buf[0, cap).
+int group_backward(sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* buf, size_t cap,
+                   bool plain, hipStream_t s) {
+  const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
+  if (ngroup > 1 && (!buf || cap < ngroup * ni)) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
+  GroupRun r;
+  r.sym = h->win && !plain ? h->sym : plain_plan(h);
+  r.split = ngroup;
+  r.part = ngroup > 1 ? buf : nullptr;
+  r.win = h->win;
+  r.vpg = (h->np + ngroup - 1) / ngroup;
+  const size_t fit = ngroup > 1 ? cap / (ngroup * ni) : (size_t)batch;
+  r.m = h->win ? (int)std::min<size_t>({(size_t)batch, (size_t)(kMaxGroup / r.sym.nh), fit}) : 1;
+  while (r.m > 1 && bwd_lds_bytes(r.win, 1, group_size(r.sym.nh, r.m)) > kLdsBytes) --r.m;
+  const int step = (int)std::min<size_t>(batch, fit / r.m * r.m);
+  hipError_t e = hipSuccess;
+  for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += step) {
+    r.batch = std::min(step, batch - b0);
+    r.m = std::min(r.m, r.batch);
+    r.g = group_size(r.sym.nh, r.m);
+    if (r.win) r.nvc = (int)std::max<size_t>(1, std::min<size_t>(kBwdMaxViews, kBwdStageBytes / bwd_lds_bytes(r.win, 1, r.g)));
+    e = launch_backward(h->basis, h->args, r, sino + b0 * ns, img + b0 * ni, s);
+  }
+  return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
 }
 
 // Fan-beam A of `batch` images with each bin's walk in `nseg` line segments,
@@ -617,7 +831,8 @@ hipError_t launch_bwd2d(const sgdct_projector* h, const float* sino, float* img,
 // as the buffer holds, so every image is computed the same way whatever the
 // batch size or the buffer.
 int fan_forward(sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* part, size_t cap,
-                hipStream_t s) {
+                bool plain, hipStream_t s) {
+  if (grouped(h->basis)) return group_forward(h, img, sino, batch, nseg, part, cap, plain, s);
   hipError_t e = hipSuccess;
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu, per = (size_t)nseg * ns;
   if (nseg == 1) {
@@ -633,7 +848,8 @@ int fan_forward(sgdct_projector* h, const float* img, float* sino, int batch, in
 
 // Fan-beam A^T with the views in `ngroup` groups, partial sums as above.
 int fan_backward(sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* part, size_t cap,
-                 hipStream_t s) {
+                 bool plain, hipStream_t s) {
+  if (grouped(h->basis)) return group_backward(h, sino, img, batch, ngroup, part, cap, plain, s);
   hipError_t e = hipSuccess;
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu, per = (size_t)ngroup * ni;
   if (ngroup == 1) {
@@ -647,17 +863,24 @@ int fan_backward(sgdct_projector* h, const float* sino, float* img, int batch, i
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
 }
 
-int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
-int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
+// plain: every view's footprints by themselves, without the scan's
+// symmetries, so that a view's values do not depend (in the last FP32 bit) on
+// which other views the handle holds.  The FP64 host-array entry points run
+// this way while the conversions and copies of their arrays are most of the
+// call (256 x 256, 360 views: the kernels are 0.18 of 0.46 ms per pair); from
+// kHostPairs (pixel, view) pairs on the kernels are, and they take the
+// symmetries.
+constexpr double kHostPairs = 1.5e8;
+bool host_plain(const sgdct_projector* h) { return (double)h->nx * h->ny * h->np < kHostPairs; }
 
-int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s) {
+int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s, bool plain = false) {
   if (is_cone(h->basis)) return cone_forward(h, img, sino, batch, s);
-  return fan_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, s);
+  return fan_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, plain, s);
 }
 
-int run_backward(sgdct_projector* h, const float* sino, float* img, int batch, hipStream_t s) {
+int run_backward(sgdct_projector* h, const float* sino, float* img, int batch, hipStream_t s, bool plain = false) {
   if (is_cone(h->basis)) return cone_backward(h, sino, img, batch, s);
-  return fan_backward(h, sino, img, batch, bwd_groups(h), h->d_part, h->part_cap, s);
+  return fan_backward(h, sino, img, batch, bwd_groups(h), h->d_part, h->part_cap, plain, s);
 }
 
 // Footprint evaluations of the reference's cone-beam forward
@@ -754,7 +977,7 @@ int host_forward(double* b, double* x, sgdct_projector* h) {
     const size_t ni = (size_t)nx * ny, ns = (size_t)h->np * h->nu;
     e = hipMemcpy(h->d_img, h->h_img, ni * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "upload image");
-    rc = run_forward(h, h->d_img, h->d_sino, 1, nullptr);
+    rc = run_forward(h, h->d_img, h->d_sino, 1, nullptr, host_plain(h));
     if (rc) return rc;
     e = hipMemcpy(h->h_sino, h->d_sino, ns * sizeof(float), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "download sinogram");
@@ -781,7 +1004,7 @@ int host_backward(double* b, double* x, sgdct_projector* h) {
     for (size_t i = 0; i < ns; ++i) h->h_sino[i] = (float)b[i];
     e = hipMemcpy(h->d_sino, h->h_sino, ns * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "upload sinogram");
-    rc = run_backward(h, h->d_sino, h->d_img, 1, nullptr);
+    rc = run_backward(h, h->d_sino, h->d_img, 1, nullptr, host_plain(h));
     if (rc) return rc;
     e = hipMemcpy(h->h_img, h->d_img, ni * sizeof(float), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "download image");
@@ -1251,7 +1474,7 @@ int sgdct_split_config(sgdct_projector* h, int fwd_split, int bwd_split) {
   const int fs = h->fwd_split, bs = h->bwd_split;
   h->fwd_split = fwd_split;
   h->bwd_split = bwd_split;
-  if (int rc = ensure_part(h, part_images(h) * part_need(h))) {
+  if (int rc = ensure_part(h, work_doubles(h))) {
     h->fwd_split = fs;
     h->bwd_split = bs;
     return rc;
@@ -1297,8 +1520,8 @@ int sgdct_project_dev_noalloc(sgdct_projector* h, int direction, const float* in
     n = (int)std::max<size_t>(1, kScratchDoubles / unit);
   }
   hipStream_t s = (hipStream_t)stream;
-  return direction == 0 ? fan_forward(h, in, out, batch, n, part, kScratchDoubles, s)
-                        : fan_backward(h, in, out, batch, n, part, kScratchDoubles, s);
+  return direction == 0 ? fan_forward(h, in, out, batch, n, part, kScratchDoubles, false, s)
+                        : fan_backward(h, in, out, batch, n, part, kScratchDoubles, false, s);
 }
 
 int sgdct_shape(const sgdct_projector* h, int* out) {

@@ -1,18 +1,20 @@
 // proj2d.hip -- gfx950 kernels of the 2-D fan-beam footprint projectors.
 //
-//   fwd_bin_kernel   A   (image -> sinogram).  One lane per (view, bin): the
+//   fwd_group_kernel A   (image -> sinogram).  One lane per (view, bin): the
 //                    lane walks the pixels of its bin's strip line by line and
-//                    gathers sum_pixel conv * x.  No atomics, deterministic.
-//   bwd_pix_kernel   A^T (sinogram -> image).  One lane per pixel, 16x16
+//                    gathers sum_pixel conv * x for the G values (symmetric
+//                    views x images, group2d.hpp) that share the footprint.
+//                    No atomics, deterministic.
+//   bwd_group_kernel A^T (sinogram -> image).  One lane per pixel, 16x16
 //                    pixel tiles per workgroup; per-bin constants and the
 //                    sinogram values of the bins the tile sees are staged in
-//                    LDS, kViewChunk views at a time.  Deterministic gather.
+//                    LDS, a few views at a time.  Deterministic gather.
 //   sum_parts_kernel adds the FP64 partial results of split launches in a
-//                    fixed order: A may split every bin's walk into line
-//                    segments and A^T the views into groups (grid z), so that
-//                    a single image fills the GPU; each segment / group
-//                    writes its partial sums, and the split is chosen per
-//                    projector from one image's launch size.
+//                    fixed order: A may split every bin's walk into grid
+//                    segments and A^T the views into groups, so that a single
+//                    image fills the GPU; the split is chosen per projector
+//                    from one image's launch size.
+//   interleave_kernel  the G-fold image A reads, and its transpose.
 //   count_kernel     number of footprint evaluations under the reference's
 //                    corner rule (the value layers/A_B1.cu:50,643 returns).
 //
@@ -28,20 +30,95 @@
 
 namespace sgdct {
 
-// grid (waves, batch, nseg), one wave per workgroup: waves of a view differ
-// in length, and single-wave workgroups let the dispatcher refill each wave
-// slot as soon as it frees (four-wave workgroups waited for their slowest
-// wave: B1 A 1.058 -> 0.959 ms at 512 x 512, 720 views, 768 bins).  With
-// nseg > 1 every (segment, image) writes FP64 partial sums to
-// part[(seg * batch + image) * np * nu + ...], which sum_parts_kernel adds in
-// segment order.
-template <int BASIS>
-__global__ __launch_bounds__(64) void fwd_bin_kernel(Proj2DArgs g, const float* __restrict__ img,
-                                                     float* __restrict__ sino, double* __restrict__ part) {
-  const int b = blockIdx.y, seg = blockIdx.z, nseg = gridDim.z;
-  const size_t nsino = (size_t)g.np * g.nu;
-  fwd_bin_wave<BASIS>(g, img + (size_t)b * g.nx * g.ny, sino + b * nsino, blockIdx.x, seg, nseg,
-                      nseg > 1 ? part + ((size_t)seg * gridDim.y + b) * nsino : nullptr);
+hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts, hipStream_t s);
+
+// A for G = nh * m values per footprint (group2d.hpp).  grid (nrep * nchunk,
+// image groups, nseg): a workgroup of kFwdWaves waves takes one
+// representative view and 64-bin chunk; its waves walk interleaved lines, so
+// they stay level, and their FP64 sums are added in wave order through LDS
+// (no partial sums in HBM).  With nseg > 1 every segment writes FP64 partial
+// sums for sum_parts_kernel.
+// Bound by VALU issue (62 % of it at the size below) and the vector L1, which
+// feeds 4 G bytes per lane and footprint.  B1 at 512 x 512, 720 views, 768
+// bins, per call: 960 us with one value per footprint and 24 partial sums,
+// 178 us with the scan's 8 symmetries; 2048 x 2048, 1440 views, 3072 bins
+// 44.6 -> 4.7 ms.  Eight waves: four 214 us (too few waves per view), sixteen
+// 202 us (one workgroup per CU).  Column walks read the transposed copy, so
+// that both walks read consecutive pixels (512 x 512, 721 views without
+// symmetries, read in place 947 us, with the copy 782 us).
+template <int BASIS, int G>
+__global__ __launch_bounds__(64 * kFwdWaves) void fwd_group_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                                   const float* __restrict__ rows_img,
+                                                                   const float* __restrict__ cols_img,
+                                                                   float* __restrict__ sino,
+                                                                   double* __restrict__ part) {
+  __shared__ double red[kFwdWaves][G][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
+  const int chunk = centre_out(rank, g.nchunk);
+  const int v = sp.rep ? sp.rep[rep] : rep;
+  const size_t nsino = (size_t)g.np * g.nu, gpix = (size_t)G * g.nx * g.ny;
+  const int seg = blockIdx.z, nseg = gridDim.z;
+  double acc[G];
+#pragma unroll
+  for (int s = 0; s < G; ++s) acc[s] = 0.0;
+  fwd_bin_lines<BASIS, G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr,
+                          wv, kFwdWaves, seg, nseg, acc);
+#pragma unroll
+  for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
+  __syncthreads();
+  const int u = chunk * 64 + lane;
+  if (u >= g.nu) return;
+  const typename Traits<BASIS>::Bin* bins = reinterpret_cast<const typename Traits<BASIS>::Bin*>(g.bins);
+  const float scale = Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]);
+  const int img0 = blockIdx.y * m, nimg = min(m, batch - img0);
+  for (int s = wv; s < sp.nh * nimg; s += kFwdWaves) {
+    const int k = s >> sp.lg, h = s & (sp.nh - 1);
+    const int vh = sp.rep_view ? sp.rep_view[rep * sp.nh + h] : v;
+    if (vh < 0) continue;
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < kFwdWaves; ++w) t += red[w][s][lane];
+    t = t * g.dx * g.dy * scale;
+    const int uh = SymOp::reverses(sp.op[h]) ? g.nu - 1 - u : u;
+    const size_t o = (img0 + k) * nsino + (size_t)vh * g.nu + uh;
+    if (nseg > 1) part[(size_t)seg * batch * nsino + o] = t;
+    else sino[o] = (float)t;
+  }
+}
+
+// Interleaved copies of the images of one launch: slot s = image * nh + h of
+// pixel p holds the image at h p, rows[(iy nx + ix) G + s], and transposed,
+// cols[(ix ny + iy) G + s] (either null: not wanted).  grid (tiles x, tiles y, image
+// groups), 16 x 16 pixels per block; slots past the last image hold zeros.
+template <int G>
+__global__ __launch_bounds__(256) void interleave_kernel(SymPlan sp, int nx, int ny, int m, int batch,
+                                                         const float* __restrict__ img, float* __restrict__ rows,
+                                                         float* __restrict__ cols) {
+  const size_t npix = (size_t)nx * ny;
+  const int img0 = blockIdx.z * m, nslot = sp.nh * min(m, batch - img0);
+  float x[G];
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const int ix = blockIdx.x * 16 + tx, iy = blockIdx.y * 16 + ty;
+  if (ix >= nx || iy >= ny) return;
+#pragma unroll
+  for (int s = 0; s < G; ++s) {
+    x[s] = 0.0f;
+    if (s < nslot) {
+      const int k = s >> sp.lg, h = s & (sp.nh - 1);
+      int qx, qy;
+      SymOp::pixel(sp.op[h], nx, ny, ix, iy, &qx, &qy);
+      x[s] = img[(img0 + k) * npix + (size_t)qy * nx + qx];
+    }
+  }
+  if (rows) {
+    rows += blockIdx.z * npix * G;
+    __builtin_memcpy(__builtin_assume_aligned(rows + ((size_t)iy * nx + ix) * G, G < 4 ? 4 * G : 16), x, sizeof(x));
+  }
+  if (cols) {
+    cols += blockIdx.z * npix * G;
+    __builtin_memcpy(__builtin_assume_aligned(cols + ((size_t)ix * ny + iy) * G, G < 4 ? 4 * G : 16), x, sizeof(x));
+  }
 }
 
 // out[i] = sum_k part[k n + i], k ascending (deterministic).
@@ -55,10 +132,36 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const double* __restrict
 }
 
 
-// Widest bin window over every tile and view (host-side, on the host copy of
-// the view table): the LDS-staged A^T kernel is used when it is <= kMaxWindow.
-int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host) {
+// Bin window that holds every tile's window over all views (host-side, on the
+// host copy of the view table).  A point d away from a tile's centre projects
+// to kc - (d . G) / (beta + d . grad beta), G = grad N_0 + kc grad beta, kc
+// the centre's projection.  Over the image, kc is extreme at the corner tiles
+// (a projective map), |G| at extreme kc, and beta, affine, at the corners; so
+// four tiles per view bound every tile's window.  Where that bound is above
+// `enough`, every tile is looked at.
+int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough) {
+  const int tx = (g.nx + kTile - 1) / kTile, ty = (g.ny + kTile - 1) / kTile;
+  const double r = 0.5 * (kTile - 1) + (double)g.h;
   int w = 0;
+  for (int v = 0; v < g.np; ++v) {
+    const ViewGeo& vg = views_host[v];
+    double top = 0.0, room = 1e300;
+    for (int c = 0; c < 4; ++c) {
+      const double cx = ((c & 1) ? (tx - 1) * kTile : 0) + 0.5 * (kTile - 1);
+      const double cy = ((c & 2) ? (ty - 1) * kTile : 0) + 0.5 * (kTile - 1);
+      const double wx = cx * g.dx + vg.w0x, wy = cy * g.dy + vg.w0y;
+      const double be = vg.pux * wy - vg.puy * wx;
+      const double kc = -(vg.e0x * wy - vg.e0y * wx) / be;
+      top = fmax(top, fabs(vg.gx0 + kc * vg.gx1) + fabs(vg.gy0 + kc * vg.gy1));
+      // beta < 0 in front of the source
+      room = fmin(room, -be - r * (fabs((double)vg.gx1) + fabs((double)vg.gy1)));
+    }
+    // floor(kc + hw) - floor(kc - hw) <= 2 hw + 1, the window's margins 2 more
+    const double n = room > 0.0 ? floor(2.0 * r * top / room) + 4.0 : 1e9;
+    w = n < g.nu ? ((int)n > w ? (int)n : w) : g.nu;
+  }
+  if (w <= enough) return w;
+  w = 0;
   for (int v = 0; v < g.np; ++v)
     for (int iy0 = 0; iy0 < g.ny; iy0 += kTile)
       for (int ix0 = 0; ix0 < g.nx; ix0 += kTile) {
@@ -69,21 +172,39 @@ int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host) {
   return w;
 }
 
-// grid (tiles x, tiles y, batch * ngroup): view group k = blockIdx.z % ngroup
-// covers views [k vpg, (k + 1) vpg); with ngroup > 1 it writes FP64 partial
-// images to part[(k * batch + image) * nx * ny + ...] for sum_parts_kernel.
-template <int BASIS, bool USE_LDS>
+// grid (tiles, view groups, image groups): view group k covers views
+// [k vpg, (k + 1) vpg); with more than one group it writes FP64 partial images
+// to part[(k * batch + image) * nx * ny + ...] for sum_parts_kernel.
+// Bound by VALU issue and the LDS reads of records and values (64 bytes per
+// footprint at G = 8).  B1 at 512 x 512, 720 views, 768 bins, per call: 940 us
+// with one value per footprint, 197 us with the scan's 8 symmetries; 2048 x
+// 2048, 1440 views, 3072 bins 29.3 -> 5.5 ms.
+template <int BASIS, int G>
+__global__ __launch_bounds__(256) void bwd_group_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                        const float* __restrict__ sino, float* __restrict__ img,
+                                                        int vpg, int nvc, int win, double* __restrict__ part) {
+  extern __shared__ float4 bwd_lds[];
+  __shared__ int win_lo[kWinViews], win_n[kWinViews];
+  const int k = blockIdx.y, img0 = blockIdx.z * m;
+  const size_t npix = (size_t)g.nx * g.ny;
+  const int v0 = k * vpg, v1 = min(g.np, v0 + vpg);
+  bwd_group_tile<BASIS, G>(g, sp, min(m, batch - img0), sino + (size_t)img0 * g.np * g.nu, img + img0 * npix,
+                           blockIdx.x, bwd_lds, nvc, win, win_lo, win_n, v0, v1,
+                           gridDim.y > 1 ? part + ((size_t)k * batch + img0) * npix : nullptr);
+}
+
+// Tiles whose bin windows are too wide for LDS: records read from global
+// memory (L2), one image and no symmetries.  grid (tiles x, tiles y, batch *
+// ngroup).
+template <int BASIS>
 __global__ __launch_bounds__(256, 8) void bwd_pix_kernel(Proj2DArgs g, const float* __restrict__ sino,
-                                                      float* __restrict__ img, int ngroup, int vpg,
-                                                      double* __restrict__ part) {
-  using Bin = typename Traits<BASIS>::Bin;
-  __shared__ Bin lds[USE_LDS ? kViewChunk : 1][kMaxWindow];
-  __shared__ int win[2 * kViewChunk];
+                                                         float* __restrict__ img, int ngroup, int vpg,
+                                                         double* __restrict__ part) {
   const int k = blockIdx.z % ngroup, b = blockIdx.z / ngroup, batch = gridDim.z / ngroup;
   const size_t nimg = (size_t)g.nx * g.ny;
   const int v0 = k * vpg, v1 = min(g.np, v0 + vpg);
-  bwd_pix_tile<BASIS, USE_LDS>(g, sino + (size_t)b * g.np * g.nu, img + b * nimg, blockIdx.x, blockIdx.y, lds, win,
-                               v0, v1, ngroup > 1 ? part + ((size_t)k * batch + b) * nimg : nullptr);
+  bwd_pix_tile<BASIS, false>(g, sino + (size_t)b * g.np * g.nu, img + b * nimg, blockIdx.x, blockIdx.y, nullptr,
+                             nullptr, v0, v1, ngroup > 1 ? part + ((size_t)k * batch + b) * nimg : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -126,43 +247,98 @@ hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts
   return hipGetLastError();
 }
 
-// nseg > 1 needs part with nseg * batch * np * nu doubles.
-hipError_t launch_forward(int basis, const Proj2DArgs& g, const float* img, float* sino, int batch, int nseg,
-                          double* part, hipStream_t s) {
-  const int waves = g.np * g.nchunk;
-  if (nseg < 1 || (nseg > 1 && !part)) return hipErrorInvalidValue;
-  dim3 grid(waves, batch, nseg), block(64);
-  if (basis == BASIS_B1) fwd_bin_kernel<BASIS_B1><<<grid, block, 0, s>>>(g, img, sino, part);
-  else if (basis == BASIS_B0) fwd_bin_kernel<BASIS_B0><<<grid, block, 0, s>>>(g, img, sino, part);
-  else return hipErrorInvalidValue;
-  if (nseg > 1) {
-    const size_t n = (size_t)batch * g.np * g.nu;
-    sum_parts_kernel<<<(unsigned)std::min<size_t>((n + 255) / 256, 4096), 256, 0, s>>>(part, sino, n, nseg);
-  }
+namespace {
+dim3 grid3(int x, int y, int z) { return dim3((unsigned)x, (unsigned)y, (unsigned)z); }
+
+template <int G>
+hipError_t interleave_g(const Proj2DArgs& g, const GroupRun& r, const float* img, hipStream_t s) {
+  interleave_kernel<G><<<grid3((g.nx + 15) / 16, (g.ny + 15) / 16, r.groups()), 256, 0, s>>>(
+      r.sym, g.nx, g.ny, r.m, r.batch, img, r.rows, r.cols);
   return hipGetLastError();
 }
 
-// ngroup > 1 needs part with ngroup * batch * nx * ny doubles.
-hipError_t launch_backward(int basis, const Proj2DArgs& g, bool use_lds, const float* sino, float* img, int batch,
-                           int ngroup, double* part, hipStream_t s) {
-  if (ngroup < 1 || (ngroup > 1 && !part)) return hipErrorInvalidValue;
-  // views per group, whole view chunks
-  const int vpg = ((g.np + ngroup - 1) / ngroup + kViewChunk - 1) / kViewChunk * kViewChunk;
-  dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, batch * ngroup), block(256);
-  if (basis == BASIS_B1) {
-    if (use_lds) bwd_pix_kernel<BASIS_B1, true><<<grid, block, 0, s>>>(g, sino, img, ngroup, vpg, part);
-    else bwd_pix_kernel<BASIS_B1, false><<<grid, block, 0, s>>>(g, sino, img, ngroup, vpg, part);
-  } else if (basis == BASIS_B0) {
-    if (use_lds) bwd_pix_kernel<BASIS_B0, true><<<grid, block, 0, s>>>(g, sino, img, ngroup, vpg, part);
-    else bwd_pix_kernel<BASIS_B0, false><<<grid, block, 0, s>>>(g, sino, img, ngroup, vpg, part);
-  } else {
-    return hipErrorInvalidValue;
-  }
-  if (ngroup > 1) {
-    const size_t n = (size_t)batch * g.nx * g.ny;
-    sum_parts_kernel<<<(unsigned)std::min<size_t>((n + 255) / 256, 4096), 256, 0, s>>>(part, img, n, ngroup);
-  }
+template <int BASIS, int G>
+hipError_t forward_g(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  const float* rows = r.rows ? r.rows : img;
+  fwd_group_kernel<BASIS, G><<<grid3(r.sym.nrep * g.nchunk, r.groups(), r.split), 64 * kFwdWaves, 0, s>>>(
+      g, r.sym, r.m, r.batch, rows, r.cols, sino, r.part);
   return hipGetLastError();
+}
+
+template <int BASIS, int G>
+hipError_t backward_g(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  const size_t lds = (size_t)r.nvc * r.win * (32 + 4 * G);
+  bwd_group_kernel<BASIS, G><<<grid3(r.sym.ntile, r.split, r.groups()), 256, lds, s>>>(
+      g, r.sym, r.m, r.batch, sino, img, r.vpg, r.nvc, r.win, r.part);
+  return hipGetLastError();
+}
+
+template <int BASIS>
+hipError_t forward_b(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  switch (r.g) {
+    case 1: return forward_g<BASIS, 1>(g, r, img, sino, s);
+    case 2: return forward_g<BASIS, 2>(g, r, img, sino, s);
+    case 4: return forward_g<BASIS, 4>(g, r, img, sino, s);
+    case 8: return forward_g<BASIS, 8>(g, r, img, sino, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int BASIS>
+hipError_t backward_b(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  switch (r.g) {
+    case 1: return backward_g<BASIS, 1>(g, r, sino, img, s);
+    case 2: return backward_g<BASIS, 2>(g, r, sino, img, s);
+    case 4: return backward_g<BASIS, 4>(g, r, sino, img, s);
+    case 8: return backward_g<BASIS, 8>(g, r, sino, img, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+}  // namespace
+
+// The interleaved copies of the images of one launch (r.rows; r.cols too
+// where the caller wants the transposed one).
+hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float* img, hipStream_t s) {
+  switch (r.g) {
+    case 1: return interleave_g<1>(g, r, img, s);
+    case 2: return interleave_g<2>(g, r, img, s);
+    case 4: return interleave_g<4>(g, r, img, s);
+    case 8: return interleave_g<8>(g, r, img, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// r.split > 1 needs r.part with split * batch * np * nu doubles.
+hipError_t launch_forward(int basis, const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino,
+                          hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  hipError_t e = r.rows || r.cols ? launch_interleave(g, r, img, s) : hipSuccess;
+  if (e != hipSuccess) return e;
+  if (basis == BASIS_B1) e = forward_b<BASIS_B1>(g, r, img, sino, s);
+  else if (basis == BASIS_B0) e = forward_b<BASIS_B0>(g, r, img, sino, s);
+  else return hipErrorInvalidValue;
+  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
+  return e;
+}
+
+// r.split > 1 needs r.part with split * batch * nx * ny doubles; r.win = 0
+// reads the records from global memory.
+hipError_t launch_backward(int basis, const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img,
+                           hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  if (basis != BASIS_B1 && basis != BASIS_B0) return hipErrorInvalidValue;
+  hipError_t e;
+  if (r.win > 0) {
+    e = basis == BASIS_B1 ? backward_b<BASIS_B1>(g, r, sino, img, s) : backward_b<BASIS_B0>(g, r, sino, img, s);
+  } else {
+    if (r.sym.nh != 1) return hipErrorInvalidValue;
+    const dim3 grid = grid3((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, r.batch * r.split);
+    if (basis == BASIS_B1) bwd_pix_kernel<BASIS_B1><<<grid, 256, 0, s>>>(g, sino, img, r.split, r.vpg, r.part);
+    else bwd_pix_kernel<BASIS_B0><<<grid, 256, 0, s>>>(g, sino, img, r.split, r.vpg, r.part);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, img, (size_t)r.batch * g.nx * g.ny, r.split, s);
+  return e;
 }
 
 hipError_t launch_count(const Proj2DArgs& g, unsigned long long* out, hipStream_t s) {

@@ -8,6 +8,7 @@
 #include <cstdint>
 
 #include "footprint.hpp"
+#include "group2d.hpp"
 #include "projector.hpp"
 
 namespace sgdct {
@@ -41,20 +42,46 @@ template <> struct Traits<BASIS_B0> {
 // ---------------------------------------------------------------------------
 // A: bin-driven gather.
 // ---------------------------------------------------------------------------
-// One wave: bins [64 chunk, 64 chunk + 64) of view v, wave = v * nchunk + chunk.
-// With nseg > 1 the wave covers only lines [seg L, seg L + L) of its walk
-// (L = ceil(lines / nseg)) and writes its FP64 partial sum, already scaled,
-// to part[v * nu + u]; otherwise it writes the finished value to sino.
-template <int BASIS>
-__device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* __restrict__ img,
-                                             float* __restrict__ sino, int wave, int seg = 0, int nseg = 1,
-                                             double* __restrict__ part = nullptr) {
+// N consecutive floats of a buffer resource at a byte offset (reads past the
+// resource's end return zero).
+template <int N>
+__device__ __forceinline__ void buffer_load_n(__amdgpu_buffer_rsrc_t r, unsigned off, float (&x)[N]) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  if constexpr (N == 1) {
+    x[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+  } else if constexpr (N == 2) {
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+    x[0] = __uint_as_float(v.x);
+    x[1] = __uint_as_float(v.y);
+  } else {
+    static_assert(N % 4 == 0, "whole 16-byte loads");
+#pragma unroll
+    for (int k = 0; k < N; k += 4) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 4 * k, 0);
+      x[k] = __uint_as_float(v.x);
+      x[k + 1] = __uint_as_float(v.y);
+      x[k + 2] = __uint_as_float(v.z);
+      x[k + 3] = __uint_as_float(v.w);
+    }
+  }
+}
+
+// One wave: bins [64 chunk, 64 chunk + 64) of view v, one per lane.  The walk
+// covers the lines m = w0 mod wn of every bin's strip, restricted to lines
+// [seg L, seg L + L) with L = ceil(lines / nseg), and adds
+// sum_pixel conv * x into acc[G] (FP32 along a line, FP64 across lines;
+// without the factors dx dy and scale(bin)).  rows_img holds G values per
+// pixel, [iy][ix][G]; cols_img the same transposed, [ix][iy][G], which the
+// column walks read (null: they read rows_img strided).  Lanes past the last
+// bin add nothing.
+template <int BASIS, int G>
+__device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int chunk, const float* __restrict__ rows_img,
+                                              const float* __restrict__ cols_img, int w0, int wn, int seg, int nseg,
+                                              double (&acc)[G]) {
   using T = Traits<BASIS>;
-  const int lane = threadIdx.x & 63;
-  const int v = wave / g.nchunk;
-  if (v >= g.np) return;
-  const int chunk = wave - v * g.nchunk;
-  const int u = chunk * 64 + lane;
+  const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
+  const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
 
   const ViewGeo vg = g.views[v];
   // Walk rows when the wave's middle ray is closer to the y axis, columns
@@ -62,7 +89,6 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
   const int umid = min(chunk * 64 + 32, g.nu - 1);
   const double mx = vg.e0x + (umid + 0.5) * vg.pux, my = vg.e0y + (umid + 0.5) * vg.puy;
   const bool rows = fabs(my) >= fabs(mx);
-  if (u >= g.nu) return;
 
   const typename T::Bin rec = reinterpret_cast<const typename T::Bin*>(g.bins)[(size_t)v * g.nu + u];
   // N_u and N_{u+1} as affine functions of the pixel indices.
@@ -87,7 +113,8 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
   const double sq = rows ? qcx : qcy, mq = rows ? qcy : qcx;
   const double sr = rows ? rcx : rcy, mr = rows ? rcy : rcx;
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
-  const int smin = rows ? 1 : g.nx, smaj = rows ? g.nx : 1;
+  const bool strided = !rows && !cols_img;
+  const int smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
   const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
   const float dta = (float)(rec.ka * sa), dtb = (float)(rec.kb * sb);
 
@@ -99,8 +126,8 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
     double c1 = (-ra - qc0) / mq, c2 = (-ra - qc0 - sq * last) / mq;
     double c3 = (rb - rc0) / mr, c4 = (rb - rc0 - sr * last) / mr;
     double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    lo = fmax(floor(lo) - 1.0, 0.0);
-    hi = fmin(ceil(hi) + 1.0, (double)(nmaj - 1));
+    lo = fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
+    hi = fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
     m_lo = (int)lo;
     m_hi = (int)hi;
   }
@@ -109,19 +136,20 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
     m_lo = max(m_lo, seg * len);
     m_hi = min(m_hi, seg * len + len - 1);
   }
+  if (!inside) m_hi = -1;
 
   // ta, tb at pixel n of line m in FP64: ta = ka N_u = (a0 + am m) + an n,
   // formed per line from m alone, so that a line's values do not depend on
   // where the walk (or its segment) started.
   const double an = (double)rec.ka * sa, am = (double)rec.ka * ma, a0 = (double)rec.ka * ac0;
   const double bn = (double)rec.kb * sb, bm = (double)rec.kb * mb, b0 = (double)rec.kb * bc0;
-  double acc = 0.0;
 
   // Image reads go through a buffer resource with 32-bit byte offsets (the
-  // image is under 4 GiB; reads past its end would return zero).
+  // G-fold image is under 4 GiB; reads past its end would return zero).
+  const float* const img = (rows || strided) ? rows_img : cols_img;
   const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(img), (short)0, (int)(4u * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
-  const unsigned bstep = 4u * (unsigned)smin;
+      const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
+  const unsigned bstep = 4u * G * (unsigned)smin;
 
   // One line: pixels [flo, fhi] (flo <= fhi) of line m.
   auto walk_line = [&](int m, float flo, float fhi) {
@@ -129,18 +157,26 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
     const double dn = (double)flo, dm = (double)m;
     float ta = (float)__builtin_fma(dn, an, __builtin_fma(dm, am, a0));
     float tb = (float)__builtin_fma(dn, bn, __builtin_fma(dm, bm, b0));
-    unsigned off = 4u * (unsigned)(m * smaj + n0 * smin);
+    unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
     const unsigned end = off + (unsigned)((int)fhi - n0 + 1) * bstep;
-    float accl = 0.0f;
+    float accl[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) accl[k] = 0.0f;
     do {
-      const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(img_rsrc, (int)off, 0, 0));
-      accl = __builtin_fmaf(T::conv(rec, ta, tb), x, accl);
+      float x[G];
+      buffer_load_n<G>(img_rsrc, off, x);
+      const float c = T::conv(rec, ta, tb);
+#pragma unroll
+      for (int k = 0; k < G; ++k) accl[k] = __builtin_fmaf(c, x[k], accl[k]);
       off += bstep;
       ta += dta;
       tb += dtb;
     } while (off != end);
-    acc += (double)accl;
+#pragma unroll
+    for (int k = 0; k < G; ++k) acc[k] += (double)accl[k];
   };
+  // first line of the walk that is w0 mod wn (wn a power of two)
+  const int m_first = m_lo + ((w0 - m_lo) & (wn - 1));
 
   if constexpr (BASIS == BASIS_B1) {
     // Pixel interval of line m: [ceil(lo(m)), floor(hi(m))] from the two
@@ -164,7 +200,7 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
       lo1 = (float)(-mr * isr);
     }
     const float lastn = (float)(nmin - 1);
-    for (int m = m_lo; m <= m_hi; ++m) {
+    for (int m = m_first; m <= m_hi; m += wn) {
       const float fm = (float)m;
       const float flo = fmaxf(ceilf(__builtin_fmaf(fm, lo1, lo0)), 0.0f);
       const float fhi = fminf(floorf(__builtin_fmaf(fm, hi1, hi0)), lastn);
@@ -183,6 +219,7 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
     constexpr double kFar = 1e300;
     double lq0 = -kFar, lq1 = 0.0, uq0 = kFar, uq1 = 0.0;
     double lr0 = -kFar, lr1 = 0.0, ur0 = kFar, ur1 = 0.0;
+    int b_lo = 0, b_hi = nmaj - 1;  // bounds of m from tests with zero slope
     if (sq > 0.0) {
       lq0 = (-ra - qc0) * isq;
       lq1 = -mq * isq;
@@ -190,11 +227,11 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
       uq0 = (-ra - qc0) * isq;
       uq1 = -mq * isq;
     } else if (mq > 0.0) {
-      m_lo = max(m_lo, (int)fmin(ceil((-ra - qc0) / mq), 1e9));
+      b_lo = max(b_lo, (int)fmin(ceil((-ra - qc0) / mq), 1e9));
     } else if (mq < 0.0) {
-      m_hi = min(m_hi, (int)fmax(floor((-ra - qc0) / mq), -1e9));
+      b_hi = min(b_hi, (int)fmax(floor((-ra - qc0) / mq), -1e9));
     } else if (-ra - qc0 > 0.0) {
-      m_hi = -1;
+      b_hi = -1;
     }
     if (sr > 0.0) {
       ur0 = (rb - rc0) * isr;
@@ -203,25 +240,39 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
       lr0 = (rb - rc0) * isr;
       lr1 = -mr * isr;
     } else if (mr > 0.0) {
-      m_hi = min(m_hi, (int)fmax(ceil((rb - rc0) / mr) - 1.0, -1e9));
+      b_hi = min(b_hi, (int)fmax(ceil((rb - rc0) / mr) - 1.0, -1e9));
     } else if (mr < 0.0) {
-      m_lo = max(m_lo, (int)fmin(floor((rb - rc0) / mr) + 1.0, 1e9));
+      b_lo = max(b_lo, (int)fmin(floor((rb - rc0) / mr) + 1.0, 1e9));
     } else if (rb - rc0 <= 0.0) {
-      m_hi = -1;
+      b_hi = -1;
     }
+    m_hi = min(m_hi, b_hi);
     const double lastn = (double)(nmin - 1);
-    for (int m = m_lo; m <= m_hi; ++m) {
+    for (int m = m_first; m <= m_hi; m += wn) {
+      if (m < b_lo) continue;
       const double dm = (double)m;
       const double flo = fmax(fmax(ceil(fma(dm, lq1, lq0)), floor(fma(dm, lr1, lr0)) + 1.0), 0.0);
       const double fhi = fmin(fmin(floor(fma(dm, uq1, uq0)), ceil(fma(dm, ur1, ur0)) - 1.0), lastn);
       if (flo <= fhi) walk_line(m, (float)flo, (float)fhi);
     }
   }
-  const double val = acc * g.dx * g.dy * T::scale(rec);
-  if (part) part[(size_t)v * g.nu + u] = val;
-  else sino[(size_t)v * g.nu + u] = (float)val;
 }
 
+// One wave of the batched work queue: item `wave` = view * nchunk + chunk,
+// every line, finished values to sino.
+template <int BASIS>
+__device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* __restrict__ img,
+                                             float* __restrict__ sino, int wave) {
+  const int v = wave / g.nchunk;
+  if (v >= g.np) return;
+  const int chunk = wave - v * g.nchunk;
+  double acc[1] = {0.0};
+  fwd_bin_lines<BASIS, 1>(g, v, chunk, img, nullptr, 0, 1, 0, 1, acc);
+  const int u = chunk * 64 + (int)(threadIdx.x & 63);
+  if (u >= g.nu) return;
+  const typename Traits<BASIS>::Bin* bins = reinterpret_cast<const typename Traits<BASIS>::Bin*>(g.bins);
+  sino[(size_t)v * g.nu + u] = (float)(acc[0] * g.dx * g.dy * Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]));
+}
 
 // ---------------------------------------------------------------------------
 // A^T: pixel-driven gather.
@@ -232,6 +283,7 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
 __host__ __device__ inline void tile_window(const Proj2DArgs& g, const ViewGeo& vg, int ix0, int iy0, int* lo,
                                             int* n, int cap = kMaxWindow) {
   double umin = 1e300, umax = -1e300;
+#pragma unroll 1  // four divisions at once cost the gather kernels a wave per SIMD
   for (int c = 0; c < 4; ++c) {
     double fx = (c & 1) ? (ix0 + kTile - 1 + g.h) : (ix0 - g.h);
     double fy = (c & 2) ? (iy0 + kTile - 1 + g.h) : (iy0 - g.h);
@@ -360,5 +412,177 @@ __device__ __forceinline__ void bwd_pix_tile(const Proj2DArgs& g, const float* _
   }
 }
 
+
+// Loads of tables that no kernel writes, at wave-uniform addresses, through
+// the constant address space, so that they become scalar loads also after a
+// workgroup barrier (where the compiler can no longer tell that the table has
+// not changed; as vector loads the view record cost A^T a memory latency per
+// view: 303 -> 265 us with cheaper tile windows, 200 us with these and with a
+// bin's staged values loaded together).
+template <class T>
+__device__ __forceinline__ T const_load(const T* p, int i) {
+  typedef const __attribute__((address_space(4))) T* const_ptr;
+  return *((const_ptr)(uintptr_t)p + i);
+}
+
+__device__ __forceinline__ ViewGeo scalar_view(const ViewGeo* views, int v) {
+  const double* d = reinterpret_cast<const double*>(views + __builtin_amdgcn_readfirstlane(v));
+  ViewGeo r{};
+  r.e0x = const_load(d, 0);
+  r.e0y = const_load(d, 1);
+  r.pux = const_load(d, 2);
+  r.puy = const_load(d, 3);
+  r.w0x = const_load(d, 4);
+  r.w0y = const_load(d, 5);
+  const float* f = reinterpret_cast<const float*>(d + 8);
+  r.gx0 = const_load(f, 0);
+  r.gy0 = const_load(f, 1);
+  r.gx1 = const_load(f, 2);
+  r.gy1 = const_load(f, 3);
+  r.db = const_load(f, 4);
+  return r;
+}
+
+// The same gather for G = nh * m values per footprint (group2d.hpp): one
+// 16 x 16 tile of the plan's fundamental domain per 256-thread block, views
+// [v_begin, v_end).  `lds` holds nvc views x win bins: the records as two
+// float4 planes, then the G staged sinogram values of each bin as planes of
+// up to 4, so that 16-byte reads of consecutive bins touch all banks.  Slot
+// s = image * nh + symmetry; slots past nimg * nh repeat the last and
+// write nothing.  Sums go to part[image * nx * ny + pixel] (FP64) or img.
+constexpr int kWinViews = 64;  // views whose bin windows are computed at a time
+
+template <int BASIS, int G>
+__device__ __forceinline__ void bwd_group_tile(const Proj2DArgs& g, const SymPlan& sp, int nimg,
+                                               const float* __restrict__ sino, float* __restrict__ img, int tile,
+                                               float4* lds, int nvc, int win, int* win_lo, int* win_n, int v_begin,
+                                               int v_end, double* __restrict__ part) {
+  using T = Traits<BASIS>;
+  using Bin = typename T::Bin;
+  static_assert(sizeof(Bin) == 32, "two float4s per record");
+  constexpr int GV = G < 4 ? G : 4, GP = G / GV;  // values per staged vector, planes
+  const int tiles_x = (g.nx + kTile - 1) / kTile;
+  const int txy = sp.tile ? sp.tile[tile] : ((tile / tiles_x) << 16 | (tile % tiles_x));
+  const int ix0 = (txy & 0xffff) * kTile, iy0 = (txy >> 16) * kTile;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ix = ix0 + (threadIdx.x & (kTile - 1)), iy = iy0 + threadIdx.x / kTile;
+  const bool valid = ix < g.nx && iy < g.ny;
+  const Bin* bins = reinterpret_cast<const Bin*>(g.bins);
+  const double fx = ix * g.dx, fy = iy * g.dy;
+  const float last = (float)(g.nu - 1);
+  const size_t nsino = (size_t)g.np * g.nu, npix = (size_t)g.nx * g.ny;
+  const int cap = nvc * win, nslot = sp.nh * nimg;
+  float4* const rec_a = lds;
+  float4* const rec_b = lds + cap;
+  float* const ys = reinterpret_cast<float*>(lds + 2 * cap);
+
+  unsigned rev = 0;  // slots whose bins run backwards
+#pragma unroll
+  for (int s = 0; s < G; ++s) rev |= (unsigned)SymOp::reverses(sp.op[min(s, nslot - 1) & (sp.nh - 1)]) << s;
+
+  double acc[G];
+#pragma unroll
+  for (int s = 0; s < G; ++s) acc[s] = 0.0;
+  for (int w0 = v_begin; w0 < v_end; w0 += kWinViews) {
+    const int nw = min(kWinViews, v_end - w0);
+    __syncthreads();  // the previous views' windows and records are read
+    if ((int)threadIdx.x < nw) {
+      int lo, n;
+      tile_window(g, g.views[w0 + threadIdx.x], ix0, iy0, &lo, &n, win);
+      win_lo[threadIdx.x] = lo;
+      win_n[threadIdx.x] = n;
+    }
+    for (int c0 = 0; c0 < nw; c0 += nvc) {
+      const int nv = min(nvc, nw - c0);
+      __syncthreads();
+      for (int j = wv; j < nv; j += 4) {
+        const int v = w0 + c0 + j, lo = win_lo[c0 + j], n = win_n[c0 + j];
+        int row[G];  // sinogram row of each slot (slots past the last repeat it)
+#pragma unroll
+        for (int s = 0; s < G; ++s) {
+          const int sl = min(s, nslot - 1), k = sl >> sp.lg, h = sl & (sp.nh - 1);
+          row[s] = k * g.np + (sp.view ? const_load(sp.view, v * sp.nh + h) : v);
+        }
+        for (int i = lane; i < n; i += 64) {
+          const int u = lo + i;
+          const float4* src = reinterpret_cast<const float4*>(bins + (size_t)v * g.nu + u);
+          Bin r;
+          float4* const rd = reinterpret_cast<float4*>(&r);
+          rd[0] = src[0];
+          rd[1] = src[1];
+          float y[G];
+#pragma unroll
+          for (int s = 0; s < G; ++s)
+            y[s] = sino[(size_t)row[s] * g.nu + ((rev >> s) & 1 ? g.nu - 1 - u : u)];
+          rec_a[j * win + i] = rd[0];
+          rec_b[j * win + i] = rd[1];
+          const float sc = T::scale(r);
+#pragma unroll
+          for (int p = 0; p < GP; ++p)
+#pragma unroll
+            for (int e = 0; e < GV; ++e) ys[(p * cap + j * win + i) * GV + e] = y[p * GV + e] * sc;
+        }
+      }
+      __syncthreads();
+      if (!valid) continue;
+      for (int j = 0; j < nv; ++j) {
+        const ViewGeo vg = scalar_view(g.views, w0 + c0 + j);
+        const double wx = fx + vg.w0x, wy = fy + vg.w0y;
+        const double n0 = vg.e0x * wy - vg.e0y * wx;
+        const double be = vg.pux * wy - vg.puy * wx;
+        const float bef = (float)be;
+        const float kc = -(float)n0 * __builtin_amdgcn_rcpf(bef);
+        const float gx = __builtin_fmaf(kc, vg.gx1, vg.gx0), gy = __builtin_fmaf(kc, vg.gy1, vg.gy0);
+        const float hw = g.h * (__builtin_fabsf(gx) + __builtin_fabsf(gy)) *
+                         __builtin_amdgcn_rcpf(__builtin_fabsf(bef) - vg.db);
+        // clamped corner range (layers/A_B1.cu:150-151), kept inside the
+        // tile's window as in bwd_pix_tile
+        const int wlo = win_lo[c0 + j], wn = win_n[c0 + j];
+        float flo = fminf(fmaxf(floorf(kc - hw), 0.0f), last);
+        float fhi = fminf(fmaxf(floorf(kc + hw), 0.0f), last);
+        flo = fmaxf(flo, (float)wlo);
+        fhi = fminf(fhi, (float)(wlo + wn - 1));
+        const int ulo = (int)flo, cnt = (int)fhi - ulo + 1;
+        float na = (float)__builtin_fma((double)ulo, be, n0);
+        float accv[G];
+#pragma unroll
+        for (int s = 0; s < G; ++s) accv[s] = 0.0f;
+        int at = j * win + ulo - wlo;
+        for (int k = 0; k < cnt; ++k, ++at) {
+          Bin rec;
+          float4* const rd = reinterpret_cast<float4*>(&rec);
+          rd[0] = rec_a[at];
+          rd[1] = rec_b[at];
+          const float nb = na + bef;
+          const float c = T::conv(rec, rec.ka * na, rec.kb * nb);
+#pragma unroll
+          for (int p = 0; p < GP; ++p) {
+            float y[GV];
+            __builtin_memcpy(y, __builtin_assume_aligned(ys + (p * cap + at) * GV, 4 * GV), sizeof(y));
+#pragma unroll
+            for (int e = 0; e < GV; ++e) accv[p * GV + e] = __builtin_fmaf(c, y[e], accv[p * GV + e]);
+          }
+          na = nb;
+        }
+#pragma unroll
+        for (int s = 0; s < G; ++s) acc[s] += (double)accv[s];
+      }
+    }
+  }
+  if (!valid) return;
+  const unsigned own = sp.owner ? sp.owner[(size_t)tile * (kTile * kTile) + threadIdx.x] : 1u;
+#pragma unroll
+  for (int s = 0; s < G; ++s) {
+    if (s >= nslot) continue;
+    const int k = s >> sp.lg, h = s & (sp.nh - 1);
+    if (!((own >> h) & 1)) continue;
+    int qx, qy;
+    SymOp::pixel(sp.op[h], g.nx, g.ny, ix, iy, &qx, &qy);
+    const double val = acc[s] * g.dx * g.dy;
+    const size_t q = k * npix + (size_t)qy * g.nx + qx;
+    if (part) part[q] = val;
+    else img[q] = (float)val;
+  }
+}
 
 }  // namespace sgdct

@@ -1,0 +1,59 @@
+"""Grouped launches: one footprint evaluation serving a scan's symmetric views
+and the images of a batch (sgd_amd/csrc/group2d.hpp).
+
+Full-turn scans with 8, 4 and 2 symmetries (view counts 0 and 2 mod 4, odd;
+square and rectangular images, odd sizes; other start angles; alternating
+source radius) and without any, against the FP64 oracle at the projector's
+parity bar (1e-5 relative L2); a batch of 1..9 images is bit for bit the
+images by themselves.  The view counts are high enough that the symmetries
+are used (256 workgroups of a view and 64 bins)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "8 symmetries": dict(nx=33, ny=33, views=2056, nu=60),
+    "8, two bin chunks": dict(nx=40, ny=40, views=1032, nu=70),
+    "4, rectangle": dict(nx=37, ny=18, views=1032, nu=64),
+    "4, half turns": dict(nx=31, ny=31, views=1034, nu=61),
+    "4, turned start": dict(nx=32, ny=32, views=1028, nu=48, start=0.37),
+    "4, flying spot": dict(nx=30, ny=30, views=1032, nu=52, focal=0.6),
+    "2, odd": dict(nx=21, ny=34, views=521, nu=63),
+    "1": dict(nx=29, ny=29, views=300, nu=55, start=0.2),
+}
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("basis", ["B0", "B1", "SF"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_grouped_matches_oracle(cuda, oracle_exact, basis, name):
+    import torch
+    from pyoracle import Geometry
+    from sgd_amd.torch_ops import Projector
+    c = CASES[name]
+    n = c["views"]
+    ang = c.get("start", 0.0) + 2 * np.pi * np.arange(n) / n
+    drho = c["focal"] * (-1.0) ** np.arange(n) if "focal" in c else None
+    nx, ny, nu = c["nx"], c["ny"], c["nu"]
+    geo = (nx, ny, ang, nu, 1.7, 1.7, 2.9, 1000.0, 500.3)
+    P = Projector(basis, *geo, drho=drho)
+    G = Geometry(oracle_exact, *geo, drho=drho)
+    print(basis, name, c, flush=True)
+    rng = np.random.default_rng(7)
+    x = rng.random((9, ny, nx)).astype(np.float32)
+    y = rng.standard_normal((9, n, nu)).astype(np.float32)
+    xt, yt = torch.from_numpy(x).to(cuda), torch.from_numpy(y).to(cuda)
+    ax, aty = P.forward(xt), P.backward(yt)
+    torch.cuda.synchronize()
+    for k in (0, 8):
+        e1 = rel(ax[k].double().cpu().numpy(), G.forward(basis, x[k].astype(np.float64)))
+        e2 = rel(aty[k].double().cpu().numpy(), G.backward(basis, y[k].astype(np.float64)))
+        print("  image %d: A %.2e  A^T %.2e" % (k, e1, e2), flush=True)
+        assert e1 <= 1e-5 and e2 <= 1e-5, (k, e1, e2)
+    for b in (1, 2, 3, 4, 5, 8):
+        assert torch.equal(P.forward(xt[:b].contiguous()), ax[:b]), b
+        assert torch.equal(P.backward(yt[:b].contiguous()), aty[:b]), b
