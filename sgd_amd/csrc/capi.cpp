@@ -24,10 +24,8 @@ hipError_t launch_backward(int basis, const Proj2DArgs& g, const GroupRun& r, co
                            hipStream_t s);
 int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough);
 hipError_t launch_count(const Proj2DArgs& g, unsigned long long* out, hipStream_t s);
-hipError_t launch_sf_forward(const Proj2DArgs& g, const float* img, float* sino, int batch, int nseg, double* part,
-                             hipStream_t s);
-hipError_t launch_sf_backward(const Proj2DArgs& g, const float* sino, float* img, int batch, int ngroup,
-                              double* part, hipStream_t s);
+hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s);
+hipError_t launch_sf_backward(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s);
 void hex_bin_constants(int basis, const ViewGeo& v, int nu, double dt, void* out);
 size_t hex_bin_size(int basis);
 hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const float* img, float* sino, int batch,
@@ -167,7 +165,7 @@ struct sgdct_projector {
   unsigned long long* d_count = nullptr;
   long long evals = -1;
   bool bwd_lds = false;  // the batched A^T stages bin windows in LDS (B0 / B1)
-  // B0 / B1: the scan's symmetries (group2d.hpp) and A^T's LDS bin window
+  // B0 / B1 / SF: the scan's symmetries (group2d.hpp) and A^T's LDS bin window
   // (0: too wide, records are read from global memory)
   SymPlan sym{};
   int* d_sym = nullptr;
@@ -270,10 +268,11 @@ struct sgdct_batch {
 
 namespace {
 
-bool grouped(int basis) { return basis == BASIS_B0 || basis == BASIS_B1; }
+bool grouped(int basis) { return basis == BASIS_B0 || basis == BASIS_B1 || basis == BASIS_SF; }
 int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views);
 constexpr size_t kLdsBytes = (size_t)64 << 10;
-size_t bwd_lds_bytes(int win, int views, int g) { return (size_t)win * views * (32 + 4 * g); }
+// A^T's staged bins: records (none for SF) and g values each.
+size_t bwd_lds_bytes(int basis, int win, int g) { return (size_t)win * ((basis == BASIS_SF ? 0 : 32) + 4 * g); }
 size_t work_doubles(const sgdct_projector* h);
 SymPlan plain_plan(const sgdct_projector* h);
 int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
@@ -422,7 +421,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
       delete h;
       return nullptr;
     }
-    if (bwd_lds_bytes(w, 1, h->sym.nh) <= kLdsBytes) h->win = w;
+    if (bwd_lds_bytes(basis, w, h->sym.nh) <= kLdsBytes) h->win = w;
   }
   if (splits(basis)) {
     // hexagonal A runs unsplit unless asked: at 296 x 256 points, 1024 views
@@ -694,7 +693,7 @@ constexpr int kDirectEdge = 96;
 
 constexpr size_t kGroupBytes = (size_t)64 << 20;  // several image groups per launch up to this much workspace
 
-// Workspace of a handle: for B0 / B1 one image group of A with as many images
+// Workspace of a handle: for B0 / B1 / SF one image group of A with as many images
 // as fit kMaxGroup values, more while it stays within kGroupBytes; the FP64
 // partial images of A^T.
 size_t work_doubles(const sgdct_projector* h) {
@@ -749,17 +748,15 @@ int part_images(const sgdct_projector* h) {
 
 hipError_t launch_fwd2d(const sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* part,
                         hipStream_t s) {
-  if (h->basis == BASIS_SF) return launch_sf_forward(h->args, img, sino, batch, nseg, part, s);
   return launch_hex_forward(h->basis, h->args, h->dt, img, sino, batch, nseg, part, s);
 }
 
 hipError_t launch_bwd2d(const sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* part,
                         hipStream_t s) {
-  if (h->basis == BASIS_SF) return launch_sf_backward(h->args, sino, img, batch, ngroup, part, s);
   return launch_hex_backward(h->basis, h->args, h->dt, sino, img, batch, ngroup, part, s);
 }
 
-// B0 / B1 A: images in groups of m, as many groups per launch as the
+// B0 / B1 / SF A: images in groups of m, as many groups per launch as the
 // workspace buf[0, cap) holds.  Every image's values are formed the same way
 // whatever the batch.  A workspace too small for one group of one image
 // runs without symmetries, reading the image in place (partial sums, which a
@@ -795,12 +792,13 @@ int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, 
       r.rows = r.g > 1 ? reinterpret_cast<float*>(at) : nullptr;
       r.cols = reinterpret_cast<float*>(at) + n;
     }
-    e = launch_forward(h->basis, h->args, r, img + b0 * ni, sino + b0 * ns, s);
+    e = h->basis == BASIS_SF ? launch_sf_forward(h->args, r, img + b0 * ni, sino + b0 * ns, s)
+                             : launch_forward(h->basis, h->args, r, img + b0 * ni, sino + b0 * ns, s);
   }
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
 }
 
-// B0 / B1 A^T, view groups' FP64 partial images in buf[0, cap).
+// B0 / B1 / SF A^T, view groups' FP64 partial images in buf[0, cap).
 int group_backward(sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* buf, size_t cap,
                    bool plain, hipStream_t s) {
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
@@ -813,15 +811,16 @@ int group_backward(sgdct_projector* h, const float* sino, float* img, int batch,
   r.vpg = (h->np + ngroup - 1) / ngroup;
   const size_t fit = ngroup > 1 ? cap / (ngroup * ni) : (size_t)batch;
   r.m = h->win ? (int)std::min<size_t>({(size_t)batch, (size_t)(kMaxGroup / r.sym.nh), fit}) : 1;
-  while (r.m > 1 && bwd_lds_bytes(r.win, 1, group_size(r.sym.nh, r.m)) > kLdsBytes) --r.m;
+  while (r.m > 1 && bwd_lds_bytes(h->basis, r.win, group_size(r.sym.nh, r.m)) > kLdsBytes) --r.m;
   const int step = (int)std::min<size_t>(batch, fit / r.m * r.m);
   hipError_t e = hipSuccess;
   for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += step) {
     r.batch = std::min(step, batch - b0);
     r.m = std::min(r.m, r.batch);
     r.g = group_size(r.sym.nh, r.m);
-    if (r.win) r.nvc = (int)std::max<size_t>(1, std::min<size_t>(kBwdMaxViews, kBwdStageBytes / bwd_lds_bytes(r.win, 1, r.g)));
-    e = launch_backward(h->basis, h->args, r, sino + b0 * ns, img + b0 * ni, s);
+    if (r.win) r.nvc = (int)std::max<size_t>(1, std::min<size_t>(kBwdMaxViews, kBwdStageBytes / bwd_lds_bytes(h->basis, r.win, r.g)));
+    e = h->basis == BASIS_SF ? launch_sf_backward(h->args, r, sino + b0 * ns, img + b0 * ni, s)
+                             : launch_backward(h->basis, h->args, r, sino + b0 * ns, img + b0 * ni, s);
   }
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
 }

@@ -57,34 +57,20 @@ __global__ __launch_bounds__(64 * kFwdWaves) void fwd_group_kernel(Proj2DArgs g,
   const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
   const int chunk = centre_out(rank, g.nchunk);
   const int v = sp.rep ? sp.rep[rep] : rep;
-  const size_t nsino = (size_t)g.np * g.nu, gpix = (size_t)G * g.nx * g.ny;
-  const int seg = blockIdx.z, nseg = gridDim.z;
+  const size_t gpix = (size_t)G * g.nx * g.ny;
   double acc[G];
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
   fwd_bin_lines<BASIS, G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr,
-                          wv, kFwdWaves, seg, nseg, acc);
+                          wv, kFwdWaves, blockIdx.z, gridDim.z, acc);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
   const int u = chunk * 64 + lane;
   if (u >= g.nu) return;
   const typename Traits<BASIS>::Bin* bins = reinterpret_cast<const typename Traits<BASIS>::Bin*>(g.bins);
-  const float scale = Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]);
-  const int img0 = blockIdx.y * m, nimg = min(m, batch - img0);
-  for (int s = wv; s < sp.nh * nimg; s += kFwdWaves) {
-    const int k = s >> sp.lg, h = s & (sp.nh - 1);
-    const int vh = sp.rep_view ? sp.rep_view[rep * sp.nh + h] : v;
-    if (vh < 0) continue;
-    double t = 0.0;
-#pragma unroll
-    for (int w = 0; w < kFwdWaves; ++w) t += red[w][s][lane];
-    t = t * g.dx * g.dy * scale;
-    const int uh = SymOp::reverses(sp.op[h]) ? g.nu - 1 - u : u;
-    const size_t o = (img0 + k) * nsino + (size_t)vh * g.nu + uh;
-    if (nseg > 1) part[(size_t)seg * batch * nsino + o] = t;
-    else sino[o] = (float)t;
-  }
+  fwd_group_store<G>(g, sp, rep, v, u, m, batch, red, g.dx * g.dy * Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]),
+                     sino, gridDim.z > 1 ? part : nullptr);
 }
 
 // Interleaved copies of the images of one launch: slot s = image * nh + h of
@@ -172,25 +158,16 @@ int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough) 
   return w;
 }
 
-// grid (tiles, view groups, image groups): view group k covers views
-// [k vpg, (k + 1) vpg); with more than one group it writes FP64 partial images
-// to part[(k * batch + image) * nx * ny + ...] for sum_parts_kernel.
-// Bound by VALU issue and the LDS reads of records and values (64 bytes per
-// footprint at G = 8).  B1 at 512 x 512, 720 views, 768 bins, per call: 940 us
-// with one value per footprint, 197 us with the scan's 8 symmetries; 2048 x
-// 2048, 1440 views, 3072 bins 29.3 -> 5.5 ms.
+// grid (tiles, view groups, image groups), bwd_group_block.  Bound by VALU
+// issue and the LDS reads of records and values (64 bytes per footprint at G =
+// 8).  B1 at 512 x 512, 720 views, 768 bins, per call: 940 us with one value
+// per footprint, 197 us with the scan's 8 symmetries; 2048 x 2048, 1440 views,
+// 3072 bins 29.3 -> 5.5 ms.
 template <int BASIS, int G>
 __global__ __launch_bounds__(256) void bwd_group_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
                                                         const float* __restrict__ sino, float* __restrict__ img,
                                                         int vpg, int nvc, int win, double* __restrict__ part) {
-  extern __shared__ float4 bwd_lds[];
-  __shared__ int win_lo[kWinViews], win_n[kWinViews];
-  const int k = blockIdx.y, img0 = blockIdx.z * m;
-  const size_t npix = (size_t)g.nx * g.ny;
-  const int v0 = k * vpg, v1 = min(g.np, v0 + vpg);
-  bwd_group_tile<BASIS, G>(g, sp, min(m, batch - img0), sino + (size_t)img0 * g.np * g.nu, img + img0 * npix,
-                           blockIdx.x, bwd_lds, nvc, win, win_lo, win_n, v0, v1,
-                           gridDim.y > 1 ? part + ((size_t)k * batch + img0) * npix : nullptr);
+  bwd_group_block<FanBwd<BASIS>, G>(g, sp, m, batch, sino, img, vpg, nvc, win, part);
 }
 
 // Tiles whose bin windows are too wide for LDS: records read from global

@@ -8,7 +8,7 @@
 #include <cstdint>
 
 #include "footprint.hpp"
-#include "group2d.hpp"
+#include "group2d_dev.hpp"
 #include "projector.hpp"
 
 namespace sgdct {
@@ -42,31 +42,6 @@ template <> struct Traits<BASIS_B0> {
 // ---------------------------------------------------------------------------
 // A: bin-driven gather.
 // ---------------------------------------------------------------------------
-// N consecutive floats of a buffer resource at a byte offset (reads past the
-// resource's end return zero).
-template <int N>
-__device__ __forceinline__ void buffer_load_n(__amdgpu_buffer_rsrc_t r, unsigned off, float (&x)[N]) {
-  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  if constexpr (N == 1) {
-    x[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
-  } else if constexpr (N == 2) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
-    x[0] = __uint_as_float(v.x);
-    x[1] = __uint_as_float(v.y);
-  } else {
-    static_assert(N % 4 == 0, "whole 16-byte loads");
-#pragma unroll
-    for (int k = 0; k < N; k += 4) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 4 * k, 0);
-      x[k] = __uint_as_float(v.x);
-      x[k + 1] = __uint_as_float(v.y);
-      x[k + 2] = __uint_as_float(v.z);
-      x[k + 3] = __uint_as_float(v.w);
-    }
-  }
-}
-
 // One wave: bins [64 chunk, 64 chunk + 64) of view v, one per lane.  The walk
 // covers the lines m = w0 mod wn of every bin's strip, restricted to lines
 // [seg L, seg L + L) with L = ceil(lines / nseg), and adds
@@ -278,28 +253,6 @@ __device__ __forceinline__ void fwd_bin_wave(const Proj2DArgs& g, const float* _
 // A^T: pixel-driven gather.
 // ---------------------------------------------------------------------------
 
-// Bin window of one view for a pixel tile: bins touched by the tile's box
-// widened by h, from the exact projection of its four corners, +-1 margin.
-__host__ __device__ inline void tile_window(const Proj2DArgs& g, const ViewGeo& vg, int ix0, int iy0, int* lo,
-                                            int* n, int cap = kMaxWindow) {
-  double umin = 1e300, umax = -1e300;
-#pragma unroll 1  // four divisions at once cost the gather kernels a wave per SIMD
-  for (int c = 0; c < 4; ++c) {
-    double fx = (c & 1) ? (ix0 + kTile - 1 + g.h) : (ix0 - g.h);
-    double fy = (c & 2) ? (iy0 + kTile - 1 + g.h) : (iy0 - g.h);
-    double wx = fx * g.dx + vg.w0x, wy = fy * g.dy + vg.w0y;
-    double n0 = vg.e0x * wy - vg.e0y * wx;
-    double be = vg.pux * wy - vg.puy * wx;
-    double uu = -n0 / be;
-    umin = fmin(umin, uu);
-    umax = fmax(umax, uu);
-  }
-  double l = fmax(floor(umin) - 1.0, 0.0), hgh = fmin(floor(umax) + 1.0, (double)(g.nu - 1));
-  int li = (int)l, hi = (int)hgh;
-  *lo = li;
-  *n = hi >= li ? min(hi - li + 1, cap) : 0;
-}
-
 // A^T stages bin records in LDS with the sinogram value (times the footprint
 // scale) in place of the scale: stage() writes it, staged_y() reads it.
 __device__ __forceinline__ void stage(B1Bin& r, float y) { r.scale *= y; }
@@ -412,177 +365,59 @@ __device__ __forceinline__ void bwd_pix_tile(const Proj2DArgs& g, const float* _
   }
 }
 
-
-// Loads of tables that no kernel writes, at wave-uniform addresses, through
-// the constant address space, so that they become scalar loads also after a
-// workgroup barrier (where the compiler can no longer tell that the table has
-// not changed; as vector loads the view record cost A^T a memory latency per
-// view: 303 -> 265 us with cheaper tile windows, 200 us with these and with a
-// bin's staged values loaded together).
-template <class T>
-__device__ __forceinline__ T const_load(const T* p, int i) {
-  typedef const __attribute__((address_space(4))) T* const_ptr;
-  return *((const_ptr)(uintptr_t)p + i);
-}
-
-__device__ __forceinline__ ViewGeo scalar_view(const ViewGeo* views, int v) {
-  const double* d = reinterpret_cast<const double*>(views + __builtin_amdgcn_readfirstlane(v));
-  ViewGeo r{};
-  r.e0x = const_load(d, 0);
-  r.e0y = const_load(d, 1);
-  r.pux = const_load(d, 2);
-  r.puy = const_load(d, 3);
-  r.w0x = const_load(d, 4);
-  r.w0y = const_load(d, 5);
-  const float* f = reinterpret_cast<const float*>(d + 8);
-  r.gx0 = const_load(f, 0);
-  r.gy0 = const_load(f, 1);
-  r.gx1 = const_load(f, 2);
-  r.gy1 = const_load(f, 3);
-  r.db = const_load(f, 4);
-  return r;
-}
-
-// The same gather for G = nh * m values per footprint (group2d.hpp): one
-// 16 x 16 tile of the plan's fundamental domain per 256-thread block, views
-// [v_begin, v_end).  `lds` holds nvc views x win bins: the records as two
-// float4 planes, then the G staged sinogram values of each bin as planes of
-// up to 4, so that 16-byte reads of consecutive bins touch all banks.  Slot
-// s = image * nh + symmetry; slots past nimg * nh repeat the last and
-// write nothing.  Sums go to part[image * nx * ny + pixel] (FP64) or img.
-constexpr int kWinViews = 64;  // views whose bin windows are computed at a time
-
-template <int BASIS, int G>
-__device__ __forceinline__ void bwd_group_tile(const Proj2DArgs& g, const SymPlan& sp, int nimg,
-                                               const float* __restrict__ sino, float* __restrict__ img, int tile,
-                                               float4* lds, int nvc, int win, int* win_lo, int* win_n, int v_begin,
-                                               int v_end, double* __restrict__ part) {
+// A^T of B0 / B1 in the grouped frame (group2d_dev.hpp).
+template <int BASIS> struct FanBwd {
+  using Args = Proj2DArgs;
   using T = Traits<BASIS>;
   using Bin = typename T::Bin;
-  static_assert(sizeof(Bin) == 32, "two float4s per record");
-  constexpr int GV = G < 4 ? G : 4, GP = G / GV;  // values per staged vector, planes
-  const int tiles_x = (g.nx + kTile - 1) / kTile;
-  const int txy = sp.tile ? sp.tile[tile] : ((tile / tiles_x) << 16 | (tile % tiles_x));
-  const int ix0 = (txy & 0xffff) * kTile, iy0 = (txy >> 16) * kTile;
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ix = ix0 + (threadIdx.x & (kTile - 1)), iy = iy0 + threadIdx.x / kTile;
-  const bool valid = ix < g.nx && iy < g.ny;
-  const Bin* bins = reinterpret_cast<const Bin*>(g.bins);
-  const double fx = ix * g.dx, fy = iy * g.dy;
-  const float last = (float)(g.nu - 1);
-  const size_t nsino = (size_t)g.np * g.nu, npix = (size_t)g.nx * g.ny;
-  const int cap = nvc * win, nslot = sp.nh * nimg;
-  float4* const rec_a = lds;
-  float4* const rec_b = lds + cap;
-  float* const ys = reinterpret_cast<float*>(lds + 2 * cap);
+  static constexpr int kRec = 2;  // float4s per record
+  struct Pixel {
+    double fx, fy;
+  };
+  __device__ static __forceinline__ const Proj2DArgs& geo(const Args& a) { return a; }
+  __device__ static __forceinline__ void window(const Args& a, const ViewGeo& vg, int ix0, int iy0, int* lo, int* n,
+                                                int cap) {
+    tile_window(a, vg, ix0, iy0, lo, n, cap);
+  }
+  __device__ static __forceinline__ Pixel pixel(const Args& a, int ix, int iy) { return {ix * a.dx, iy * a.dy}; }
+  __device__ static __forceinline__ bool active(const Args&, int, int) { return true; }
+  __device__ static __forceinline__ void image(const Args& a, int op, int ix, int iy, int* qx, int* qy) {
+    SymOp::pixel(op, a.nx, a.ny, ix, iy, qx, qy);
+  }
+  __device__ static __forceinline__ float value(const float4 (&rec)[kRec], float y) {
+    return y * T::scale(__builtin_bit_cast(Bin, rec));
+  }
+  __device__ static __forceinline__ double result(const Args& a, double acc) { return acc * a.dx * a.dy; }
 
-  unsigned rev = 0;  // slots whose bins run backwards
-#pragma unroll
-  for (int s = 0; s < G; ++s) rev |= (unsigned)SymOp::reverses(sp.op[min(s, nslot - 1) & (sp.nh - 1)]) << s;
-
-  double acc[G];
-#pragma unroll
-  for (int s = 0; s < G; ++s) acc[s] = 0.0;
-  for (int w0 = v_begin; w0 < v_end; w0 += kWinViews) {
-    const int nw = min(kWinViews, v_end - w0);
-    __syncthreads();  // the previous views' windows and records are read
-    if ((int)threadIdx.x < nw) {
-      int lo, n;
-      tile_window(g, g.views[w0 + threadIdx.x], ix0, iy0, &lo, &n, win);
-      win_lo[threadIdx.x] = lo;
-      win_n[threadIdx.x] = n;
-    }
-    for (int c0 = 0; c0 < nw; c0 += nvc) {
-      const int nv = min(nvc, nw - c0);
-      __syncthreads();
-      for (int j = wv; j < nv; j += 4) {
-        const int v = w0 + c0 + j, lo = win_lo[c0 + j], n = win_n[c0 + j];
-        int row[G];  // sinogram row of each slot (slots past the last repeat it)
-#pragma unroll
-        for (int s = 0; s < G; ++s) {
-          const int sl = min(s, nslot - 1), k = sl >> sp.lg, h = sl & (sp.nh - 1);
-          row[s] = k * g.np + (sp.view ? const_load(sp.view, v * sp.nh + h) : v);
-        }
-        for (int i = lane; i < n; i += 64) {
-          const int u = lo + i;
-          const float4* src = reinterpret_cast<const float4*>(bins + (size_t)v * g.nu + u);
-          Bin r;
-          float4* const rd = reinterpret_cast<float4*>(&r);
-          rd[0] = src[0];
-          rd[1] = src[1];
-          float y[G];
-#pragma unroll
-          for (int s = 0; s < G; ++s)
-            y[s] = sino[(size_t)row[s] * g.nu + ((rev >> s) & 1 ? g.nu - 1 - u : u)];
-          rec_a[j * win + i] = rd[0];
-          rec_b[j * win + i] = rd[1];
-          const float sc = T::scale(r);
-#pragma unroll
-          for (int p = 0; p < GP; ++p)
-#pragma unroll
-            for (int e = 0; e < GV; ++e) ys[(p * cap + j * win + i) * GV + e] = y[p * GV + e] * sc;
-        }
-      }
-      __syncthreads();
-      if (!valid) continue;
-      for (int j = 0; j < nv; ++j) {
-        const ViewGeo vg = scalar_view(g.views, w0 + c0 + j);
-        const double wx = fx + vg.w0x, wy = fy + vg.w0y;
-        const double n0 = vg.e0x * wy - vg.e0y * wx;
-        const double be = vg.pux * wy - vg.puy * wx;
-        const float bef = (float)be;
-        const float kc = -(float)n0 * __builtin_amdgcn_rcpf(bef);
-        const float gx = __builtin_fmaf(kc, vg.gx1, vg.gx0), gy = __builtin_fmaf(kc, vg.gy1, vg.gy0);
-        const float hw = g.h * (__builtin_fabsf(gx) + __builtin_fabsf(gy)) *
-                         __builtin_amdgcn_rcpf(__builtin_fabsf(bef) - vg.db);
-        // clamped corner range (layers/A_B1.cu:150-151), kept inside the
-        // tile's window as in bwd_pix_tile
-        const int wlo = win_lo[c0 + j], wn = win_n[c0 + j];
-        float flo = fminf(fmaxf(floorf(kc - hw), 0.0f), last);
-        float fhi = fminf(fmaxf(floorf(kc + hw), 0.0f), last);
-        flo = fmaxf(flo, (float)wlo);
-        fhi = fminf(fhi, (float)(wlo + wn - 1));
-        const int ulo = (int)flo, cnt = (int)fhi - ulo + 1;
-        float na = (float)__builtin_fma((double)ulo, be, n0);
-        float accv[G];
-#pragma unroll
-        for (int s = 0; s < G; ++s) accv[s] = 0.0f;
-        int at = j * win + ulo - wlo;
-        for (int k = 0; k < cnt; ++k, ++at) {
-          Bin rec;
-          float4* const rd = reinterpret_cast<float4*>(&rec);
-          rd[0] = rec_a[at];
-          rd[1] = rec_b[at];
-          const float nb = na + bef;
-          const float c = T::conv(rec, rec.ka * na, rec.kb * nb);
-#pragma unroll
-          for (int p = 0; p < GP; ++p) {
-            float y[GV];
-            __builtin_memcpy(y, __builtin_assume_aligned(ys + (p * cap + at) * GV, 4 * GV), sizeof(y));
-#pragma unroll
-            for (int e = 0; e < GV; ++e) accv[p * GV + e] = __builtin_fmaf(c, y[e], accv[p * GV + e]);
-          }
-          na = nb;
-        }
-#pragma unroll
-        for (int s = 0; s < G; ++s) acc[s] += (double)accv[s];
-      }
+  template <int G>
+  __device__ static __forceinline__ void view(const Args& g, const ViewGeo& vg, const Pixel& p, const Staged<kRec, G>& st,
+                                              int base, int wlo, int wn, float (&accv)[G]) {
+    const double wx = p.fx + vg.w0x, wy = p.fy + vg.w0y;
+    const double n0 = vg.e0x * wy - vg.e0y * wx;
+    const double be = vg.pux * wy - vg.puy * wx;
+    const float bef = (float)be, last = (float)(g.nu - 1);
+    const float kc = -(float)n0 * __builtin_amdgcn_rcpf(bef);
+    const float gx = __builtin_fmaf(kc, vg.gx1, vg.gx0), gy = __builtin_fmaf(kc, vg.gy1, vg.gy0);
+    const float hw = g.h * (__builtin_fabsf(gx) + __builtin_fabsf(gy)) *
+                     __builtin_amdgcn_rcpf(__builtin_fabsf(bef) - vg.db);
+    // clamped corner range (layers/A_B1.cu:150-151), kept inside the tile's
+    // window as in bwd_pix_tile
+    float flo = fminf(fmaxf(floorf(kc - hw), 0.0f), last);
+    float fhi = fminf(fmaxf(floorf(kc + hw), 0.0f), last);
+    flo = fmaxf(flo, (float)wlo);
+    fhi = fminf(fhi, (float)(wlo + wn - 1));
+    const int ulo = (int)flo, cnt = (int)fhi - ulo + 1;
+    float na = (float)__builtin_fma((double)ulo, be, n0);
+    int at = base + ulo - wlo;
+    for (int k = 0; k < cnt; ++k, ++at) {
+      float4 rd[kRec];
+      st.record(at, rd);
+      const Bin rec = __builtin_bit_cast(Bin, rd);
+      const float nb = na + bef;
+      st.add(at, T::conv(rec, rec.ka * na, rec.kb * nb), accv);
+      na = nb;
     }
   }
-  if (!valid) return;
-  const unsigned own = sp.owner ? sp.owner[(size_t)tile * (kTile * kTile) + threadIdx.x] : 1u;
-#pragma unroll
-  for (int s = 0; s < G; ++s) {
-    if (s >= nslot) continue;
-    const int k = s >> sp.lg, h = s & (sp.nh - 1);
-    if (!((own >> h) & 1)) continue;
-    int qx, qy;
-    SymOp::pixel(sp.op[h], g.nx, g.ny, ix, iy, &qx, &qy);
-    const double val = acc[s] * g.dx * g.dy;
-    const size_t q = k * npix + (size_t)qy * g.nx + qx;
-    if (part) part[q] = val;
-    else img[q] = (float)val;
-  }
-}
+};
 
 }  // namespace sgdct

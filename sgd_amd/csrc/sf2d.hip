@@ -18,48 +18,113 @@
 namespace sgdct {
 
 hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts, hipStream_t s);
+hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float* img, hipStream_t s);
 
-// grid (waves / 4, batch, nseg); partial sums as in fwd_bin_kernel.
-__global__ __launch_bounds__(256) void sf_fwd_kernel(Proj2DArgs g, const float* __restrict__ img,
-                                                     float* __restrict__ sino, double* __restrict__ part) {
-  const int b = blockIdx.y, seg = blockIdx.z, nseg = gridDim.z;
-  const size_t nsino = (size_t)g.np * g.nu;
-  sf_fwd_wave(g, img + (size_t)b * g.nx * g.ny, sino + b * nsino, blockIdx.x * 4 + (threadIdx.x >> 6), seg, nseg,
-              nseg > 1 ? part + ((size_t)seg * gridDim.y + b) * nsino : nullptr);
+// A, launched as fwd_group_kernel.  Bound by VALU issue: ~70 instructions per
+// footprint (four corner projections with two reciprocals, the sort and the
+// trapezoid's area) beside one multiply-add per value.  512 x 512, 720 views,
+// 768 bins, per call: one value per footprint 1456 us, the scan's 8
+// symmetries 260 us; 1024 x 1024, 900 views 7.04 -> 1.13 ms; 256 x 256, 90
+// views, batch 5 266 -> 84 us; one value, 721 views from another start angle
+// 1455 -> 1420 us.
+template <int G>
+__global__ __launch_bounds__(64 * kFwdWaves) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                                const float* __restrict__ rows_img,
+                                                                const float* __restrict__ cols_img,
+                                                                float* __restrict__ sino, double* __restrict__ part) {
+  __shared__ double red[kFwdWaves][G][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
+  const int chunk = centre_out(rank, g.nchunk);
+  const int v = sp.rep ? sp.rep[rep] : rep;
+  const size_t gpix = (size_t)G * g.nx * g.ny;
+  double acc[G];
+#pragma unroll
+  for (int s = 0; s < G; ++s) acc[s] = 0.0;
+  sf_fwd_lines<G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr, wv,
+                  kFwdWaves, blockIdx.z, gridDim.z, acc);
+#pragma unroll
+  for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
+  __syncthreads();
+  const int u = chunk * 64 + lane;
+  if (u >= g.nu) return;
+  fwd_group_store<G>(g, sp, rep, v, u, m, batch, red, 1.0, sino, gridDim.z > 1 ? part : nullptr);
 }
 
-// grid (tiles x, tiles y, batch * ngroup); view groups as in bwd_pix_kernel,
-// blocks mapped by xcd_block: SF A^T 0.859 -> 0.840 ms at 512 x 512, 720
-// views, 768 bins (B0 / B1's bwd_pix_kernel and Hl's A^T were slower with it).
-__global__ __launch_bounds__(256) void sf_bwd_kernel(Proj2DArgs g, const float* __restrict__ sino,
-                                                     float* __restrict__ img, int ngroup, int vpg,
-                                                     double* __restrict__ part) {
-  const uint3 blk = xcd_block();
-  const int k = blk.z % ngroup, b = blk.z / ngroup, batch = gridDim.z / ngroup;
+// A^T, launched as bwd_group_kernel; same cases as above: 841 -> 175 us, 4.13
+// -> 0.75 ms, 146 -> 55 us, 869 -> 863 us.  The FP64 projection of the pixel's
+// centre and its sorted corners are formed once per view for all values.
+template <int G>
+__global__ __launch_bounds__(256) void sf_bwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                     const float* __restrict__ sino, float* __restrict__ img, int vpg,
+                                                     int nvc, int win, double* __restrict__ part) {
+  bwd_group_block<SfBwd, G>(g, sp, m, batch, sino, img, vpg, nvc, win, part);
+}
+
+// Tiles whose bin windows are too wide for LDS: sinogram values from global
+// memory, one image and no symmetries.  grid (tiles x, tiles y, batch *
+// ngroup).
+__global__ __launch_bounds__(256) void sf_bwd_wide_kernel(Proj2DArgs g, const float* __restrict__ sino,
+                                                          float* __restrict__ img, int ngroup, int vpg,
+                                                          double* __restrict__ part) {
+  const int k = blockIdx.z % ngroup, b = blockIdx.z / ngroup, batch = gridDim.z / ngroup;
   const size_t nimg = (size_t)g.nx * g.ny;
   const int v0 = k * vpg, v1 = min(g.np, v0 + vpg);
-  sf_bwd_tile(g, sino + (size_t)b * g.np * g.nu, img + b * nimg, blk.x, blk.y, v0, v1,
+  sf_bwd_tile(g, sino + (size_t)b * g.np * g.nu, img + b * nimg, blockIdx.x, blockIdx.y, v0, v1,
               ngroup > 1 ? part + ((size_t)k * batch + b) * nimg : nullptr);
 }
 
-hipError_t launch_sf_forward(const Proj2DArgs& g, const float* img, float* sino, int batch, int nseg, double* part,
-                             hipStream_t s) {
-  if (nseg < 1 || (nseg > 1 && !part)) return hipErrorInvalidValue;
-  const int waves = g.np * g.nchunk;
-  sf_fwd_kernel<<<dim3((waves + 3) / 4, batch, nseg), dim3(256), 0, s>>>(g, img, sino, part);
-  if (nseg > 1) return launch_sum_parts(part, sino, (size_t)batch * g.np * g.nu, nseg, s);
+namespace {
+template <int G>
+hipError_t sf_forward_g(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  const dim3 grid((unsigned)(r.sym.nrep * g.nchunk), (unsigned)r.groups(), (unsigned)r.split);
+  sf_fwd_kernel<G><<<grid, 64 * kFwdWaves, 0, s>>>(g, r.sym, r.m, r.batch, r.rows ? r.rows : img, r.cols, sino, r.part);
   return hipGetLastError();
 }
 
-hipError_t launch_sf_backward(const Proj2DArgs& g, const float* sino, float* img, int batch, int ngroup,
-                              double* part, hipStream_t s) {
-  if (ngroup < 1 || (ngroup > 1 && !part)) return hipErrorInvalidValue;
-  const int vpg = (g.np + ngroup - 1) / ngroup;
-  dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, batch * ngroup);
-  sf_bwd_kernel<<<grid, dim3(256), 0, s>>>(g, sino, img, ngroup, vpg, part);
-  if (ngroup > 1) return launch_sum_parts(part, img, (size_t)batch * g.nx * g.ny, ngroup, s);
+template <int G>
+hipError_t sf_backward_g(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  const dim3 grid((unsigned)r.sym.ntile, (unsigned)r.split, (unsigned)r.groups());
+  sf_bwd_kernel<G><<<grid, 256, (size_t)r.nvc * r.win * 4 * G, s>>>(g, r.sym, r.m, r.batch, sino, img, r.vpg, r.nvc,
+                                                                   r.win, r.part);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  hipError_t e = r.rows || r.cols ? launch_interleave(g, r, img, s) : hipSuccess;
+  if (e != hipSuccess) return e;
+  if (r.g == 1) e = sf_forward_g<1>(g, r, img, sino, s);
+  else if (r.g == 2) e = sf_forward_g<2>(g, r, img, sino, s);
+  else if (r.g == 4) e = sf_forward_g<4>(g, r, img, sino, s);
+  else if (r.g == 8) e = sf_forward_g<8>(g, r, img, sino, s);
+  else return hipErrorInvalidValue;
+  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
+  return e;
+}
+
+hipError_t launch_sf_backward(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  hipError_t e;
+  if (r.win == 0) {
+    if (r.sym.nh != 1) return hipErrorInvalidValue;
+    const dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, (unsigned)(r.batch * r.split));
+    sf_bwd_wide_kernel<<<grid, 256, 0, s>>>(g, sino, img, r.split, r.vpg, r.part);
+    e = hipGetLastError();
+  } else if (r.g == 1) {
+    e = sf_backward_g<1>(g, r, sino, img, s);
+  } else if (r.g == 2) {
+    e = sf_backward_g<2>(g, r, sino, img, s);
+  } else if (r.g == 4) {
+    e = sf_backward_g<4>(g, r, sino, img, s);
+  } else if (r.g == 8) {
+    e = sf_backward_g<8>(g, r, sino, img, s);
+  } else {
+    return hipErrorInvalidValue;
+  }
+  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, img, (size_t)r.batch * g.nx * g.ny, r.split, s);
+  return e;
 }
 
 }  // namespace sgdct
-

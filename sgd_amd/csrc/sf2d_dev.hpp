@@ -5,6 +5,7 @@
 
 #include <cmath>
 
+#include "group2d_dev.hpp"
 #include "projector.hpp"
 
 namespace sgdct {
@@ -58,25 +59,19 @@ __device__ __forceinline__ float sf_weight(float dx, float wx, float wy) {
   return dx * __builtin_amdgcn_sqrtf(r2) * __builtin_amdgcn_rcpf(fmaxf(fabsf(wx), fabsf(wy)));
 }
 
-// A: bin-driven gather (same strip walk as fwd_bin_kernel, corner rule h = 1/2).
-// One wave: bins [64 chunk, 64 chunk + 64) of view v, wave = chunk * np + v
-// (chunk-major: the four waves of a workgroup walk the same bins of adjacent
-// views, nearly the same pixels; SF A 1.505 -> 1.468 ms at 512 x 512, 720
-// views, 768 bins against view-major order).
-// nseg > 1: lines [seg L, seg L + L) only, FP64 partial sum to part[v nu + u].
-__device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __restrict__ img,
-                                            float* __restrict__ sino, int wave, int seg = 0, int nseg = 1,
-                                            double* __restrict__ part = nullptr) {
-  const int lane = threadIdx.x & 63;
-  const int chunk = wave / g.np;
-  if (chunk >= g.nchunk) return;
-  const int v = wave - chunk * g.np;
-  const int u = chunk * 64 + lane;
+// A: bin-driven gather (the strip walk of fwd_bin_lines, corner rule h = 1/2).
+// One wave: bins [64 chunk, 64 chunk + 64) of view v, lines m = w0 mod wn of
+// segment seg of nseg, sums into acc[G]; images as in fwd_bin_lines.
+template <int G>
+__device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chunk, const float* __restrict__ rows_img,
+                                             const float* __restrict__ cols_img, int w0, int wn, int seg, int nseg,
+                                             double (&acc)[G]) {
+  const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
+  const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
   const ViewGeo vg = g.views[v];
   const int umid = min(chunk * 64 + 32, g.nu - 1);
   const double mx = vg.e0x + (umid + 0.5) * vg.pux, my = vg.e0y + (umid + 0.5) * vg.puy;
   const bool rows = fabs(my) >= fabs(mx);
-  if (u >= g.nu) return;
 
   const double eax = vg.e0x + u * vg.pux, eay = vg.e0y + u * vg.puy;
   const double ebx = eax + vg.pux, eby = eay + vg.puy;
@@ -86,7 +81,8 @@ __device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __
   const double sa = rows ? acx : acy, ma = rows ? acy : acx;
   const double sb = rows ? bcx : bcy, mb = rows ? bcy : bcx;
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
-  const size_t smin = rows ? 1 : g.nx, smaj = rows ? g.nx : 1;
+  const bool strided = !rows && !cols_img;
+  const int smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
   const double isa = sa != 0.0 ? 1.0 / sa : 0.0, isb = sb != 0.0 ? 1.0 / sb : 0.0;
   // beta(ix, iy) = cross(pu, w): affine, gradient (gx1, gy1) per index step
   const double bcxx = -vg.puy * g.dx, bcyy = vg.pux * g.dy, bc00 = vg.pux * vg.w0y - vg.puy * vg.w0x;
@@ -107,16 +103,20 @@ __device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __
     double c1 = (-ra - ac0) / ma, c2 = (-ra - ac0 - sa * last) / ma;
     double c3 = (rb - bc0) / mb, c4 = (rb - bc0 - sb * last) / mb;
     double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    m_lo = (int)fmax(floor(lo) - 1.0, 0.0);
-    m_hi = (int)fmin(ceil(hi) + 1.0, (double)(nmaj - 1));
+    m_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
+    m_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
   }
   if (nseg > 1) {
     const int len = (nmaj + nseg - 1) / nseg;
     m_lo = max(m_lo, seg * len);
     m_hi = min(m_hi, seg * len + len - 1);
   }
-  double acc = 0.0;
-  for (int m = m_lo; m <= m_hi; ++m) {
+  if (!inside) m_hi = -1;
+  const float* const img = (rows || strided) ? rows_img : cols_img;
+  const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
+  const unsigned bstep = 4u * G * (unsigned)smin;
+  for (int m = m_lo + ((w0 - m_lo) & (wn - 1)); m <= m_hi; m += wn) {
     const double r1 = -ra - ma * m - ac0;
     const double r2 = rb - mb * m - bc0;
     double lo = 0.0, hi = (double)(nmin - 1);
@@ -132,13 +132,17 @@ __device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __
     float nu_ = (float)(acx * ixs + acy * iys + ac0);
     float be = (float)(bcxx * ixs + bcyy * iys + bc00);
     float wx = (float)(ixs * g.dx + vg.w0x), wy = (float)(iys * g.dy + vg.w0y);
-    const float* p = img + (size_t)m * smaj + (size_t)n0 * smin;
-    float accl = 0.0f;
+    unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
+    float accl[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) accl[k] = 0.0f;
     // corner projections relative to edge u, -N_u(c) / beta(c), of the
     // trailing corners of the line's first pixel
     float t1 = -(nu_ - w_n - c_n) * __builtin_amdgcn_rcpf(be - w_b - c_b);
     float t2 = -(nu_ - w_n + c_n) * __builtin_amdgcn_rcpf(be - w_b + c_b);
     for (int n = n0; n <= n1; ++n) {
+      float x[G];
+      buffer_load_n<G>(img_rsrc, off, x);
       const float l1 = -(nu_ + w_n - c_n) * __builtin_amdgcn_rcpf(be + w_b - c_b);
       const float l2 = -(nu_ + w_n + c_n) * __builtin_amdgcn_rcpf(be + w_b + c_b);
       const Trap t = make_trap(t1, t2, l1, l2);
@@ -146,17 +150,29 @@ __device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __
       t2 = l2;
       const float gm = trap_gamma(t, 0.0f, 1.0f);
       const float val = (gm > 1e-7f) ? gm * sf_weight(fdx, wx, wy) : 0.0f;
-      accl = __builtin_fmaf(val, *p, accl);
-      p += smin;
+#pragma unroll
+      for (int k = 0; k < G; ++k) accl[k] = __builtin_fmaf(val, x[k], accl[k]);
+      off += bstep;
       nu_ += dN;
       be += dB;
       wx += dwx;
       wy += dwy;
     }
-    acc += (double)accl;
+#pragma unroll
+    for (int k = 0; k < G; ++k) acc[k] += (double)accl[k];
   }
-  if (part) part[(size_t)v * g.nu + u] = acc;
-  else sino[(size_t)v * g.nu + u] = (float)acc;
+}
+
+// One wave of the batched work queue: item `wave` = chunk * np + view, every
+// line, finished values to sino.
+__device__ __forceinline__ void sf_fwd_wave(const Proj2DArgs& g, const float* __restrict__ img,
+                                            float* __restrict__ sino, int wave) {
+  const int chunk = wave / g.np;
+  if (chunk >= g.nchunk) return;
+  const int v = wave - chunk * g.np, u = chunk * 64 + (int)(threadIdx.x & 63);
+  double acc[1] = {0.0};
+  sf_fwd_lines<1>(g, v, chunk, img, nullptr, 0, 1, 0, 1, acc);
+  if (u < g.nu) sino[(size_t)v * g.nu + u] = (float)acc[0];
 }
 
 
@@ -206,5 +222,57 @@ __device__ __forceinline__ void sf_bwd_tile(const Proj2DArgs& g, const float* __
   else img[(size_t)iy * g.nx + ix] = (float)acc;
 }
 
+// A^T in the grouped frame (group2d_dev.hpp): no records, the sinogram values
+// of a tile's bins staged in LDS.  sf_bwd_tile's arithmetic per view.
+struct SfBwd {
+  using Args = Proj2DArgs;
+  static constexpr int kRec = 0;
+  struct Pixel {
+    double fx, fy;
+  };
+  __device__ static __forceinline__ const Proj2DArgs& geo(const Args& a) { return a; }
+  __device__ static __forceinline__ void window(const Args& a, const ViewGeo& vg, int ix0, int iy0, int* lo, int* n,
+                                                int cap) {
+    tile_window(a, vg, ix0, iy0, lo, n, cap);
+  }
+  __device__ static __forceinline__ Pixel pixel(const Args& a, int ix, int iy) { return {ix * a.dx, iy * a.dy}; }
+  __device__ static __forceinline__ bool active(const Args&, int, int) { return true; }
+  __device__ static __forceinline__ void image(const Args& a, int op, int ix, int iy, int* qx, int* qy) {
+    SymOp::pixel(op, a.nx, a.ny, ix, iy, qx, qy);
+  }
+  __device__ static __forceinline__ float value(const float4 (&)[1], float y) { return y; }
+  __device__ static __forceinline__ double result(const Args&, double acc) { return acc; }
+
+  template <int G>
+  __device__ static __forceinline__ void view(const Args& g, const ViewGeo& vg, const Pixel& p, const Staged<kRec, G>& st,
+                                              int base, int wlo, int wn, float (&accv)[G]) {
+    const double wx = p.fx + vg.w0x, wy = p.fy + vg.w0y;
+    const double n0 = vg.e0x * wy - vg.e0y * wx;
+    const double be = vg.pux * wy - vg.puy * wx;
+    const double kc = -n0 / be;
+    const double kfl = floor(kc);
+    const float kf = (float)(kc - kfl);
+    const float kcf = (float)kc, bef = (float)be;
+    const float gx = 0.5f * __builtin_fmaf(kcf, vg.gx1, vg.gx0), gy = 0.5f * __builtin_fmaf(kcf, vg.gy1, vg.gy0);
+    const float bx = 0.5f * vg.gx1, by = 0.5f * vg.gy1;
+    // corner c: k*(c) - kc = -(d.G) / (beta + d.grad beta)
+    const float q0 = kf + (gx + gy) * __builtin_amdgcn_rcpf(bef - bx - by);
+    const float q1 = kf + (gx - gy) * __builtin_amdgcn_rcpf(bef - bx + by);
+    const float q2 = kf - (gx - gy) * __builtin_amdgcn_rcpf(bef + bx - by);
+    const float q3 = kf - (gx + gy) * __builtin_amdgcn_rcpf(bef + bx + by);
+    const Trap t = make_trap(q0, q1, q2, q3);
+    const int ki = (int)kfl;
+    // bins of the trapezoid, inside the detector and the tile's window
+    const int ulo = max(ki + (int)floorf(t.q0), wlo), uhi = min(ki + (int)floorf(t.q3), wlo + wn - 1);
+    const float w = sf_weight((float)g.dx, (float)wx, (float)wy);
+    for (int u = ulo; u <= uhi; ++u) {
+      const float s1 = (float)(u - ki);
+      const float gm = trap_gamma(t, s1, s1 + 1.0f);
+      st.add(base + u - wlo, (gm > 1e-7f) ? gm : 0.0f, accv);
+    }
+#pragma unroll
+    for (int s = 0; s < G; ++s) accv[s] *= w;
+  }
+};
 
 }  // namespace sgdct
