@@ -28,10 +28,11 @@ hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float
 hipError_t launch_sf_backward(const Proj2DArgs& g, const GroupRun& r, const float* sino, float* img, hipStream_t s);
 void hex_bin_constants(int basis, const ViewGeo& v, int nu, double dt, void* out);
 size_t hex_bin_size(int basis);
-hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const float* img, float* sino, int batch,
-                              int nseg, double* part, hipStream_t s);
-hipError_t launch_hex_backward(int basis, const Proj2DArgs& g, double dt, const float* sino, float* img, int batch,
-                               int ngroup, double* part, hipStream_t s);
+hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const GroupRun& r, const float* img,
+                              float* sino, hipStream_t s);
+hipError_t launch_hex_backward(int basis, const Proj2DArgs& g, double dt, const GroupRun& r, const float* sino,
+                               float* img, hipStream_t s);
+int hex_tile_window(const Proj2DArgs& g, double dt, const ViewGeo* views);
 hipError_t launch_hex_count(const Proj2DArgs& g, double dt, unsigned long long* out, hipStream_t s);
 hipError_t launch_tv_grad(const float* x, float* g, int nx, int ny, int batch, float eps, hipStream_t s);
 hipError_t launch_tv_descent(float* x, float* g, double* part, const double* step, int nx, int ny, int batch,
@@ -160,15 +161,24 @@ struct sgdct_projector {
   void* d_bins = nullptr;
   float* d_img = nullptr;   // staging for the host-array entry points
   float* d_sino = nullptr;
+  double* d_host_part = nullptr;  // their partial sums
+  size_t host_part_cap = 0;
   float* h_img = nullptr;   // pinned
   float* h_sino = nullptr;  // pinned
   unsigned long long* d_count = nullptr;
   long long evals = -1;
   bool bwd_lds = false;  // the batched A^T stages bin windows in LDS (B0 / B1)
-  // B0 / B1 / SF: the scan's symmetries (group2d.hpp) and A^T's LDS bin window
+  // the scan's symmetries (group2d.hpp) and A^T's LDS bin window
   // (0: too wide, records are read from global memory)
   SymPlan sym{};
   int* d_sym = nullptr;
+  struct Lattice {
+    hipStream_t stream;
+    bool taken;
+    double* p;
+  };
+  std::vector<Lattice> lattices;
+  std::mutex lattice_mu;
   int win = 0;
   // B0 / B1 / SF: A splits each bin's walk into line segments and A^T the views
   // into groups; fwd_auto / bwd_auto are chosen at creation from one image's
@@ -218,8 +228,10 @@ struct sgdct_projector {
     if (d_views) (void)hipFree(d_views);
     if (d_bins) (void)hipFree(d_bins);
     if (d_sym) (void)hipFree(d_sym);
+    for (auto& l : lattices) (void)hipFree(l.p);
     if (d_img) (void)hipFree(d_img);
     if (d_sino) (void)hipFree(d_sino);
+    if (d_host_part) (void)hipFree(d_host_part);
     if (d_count) (void)hipFree(d_count);
     if (d_part) (void)hipFree(d_part);
     release_cone();
@@ -268,20 +280,22 @@ struct sgdct_batch {
 
 namespace {
 
-bool grouped(int basis) { return basis == BASIS_B0 || basis == BASIS_B1 || basis == BASIS_SF; }
 int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views);
+constexpr int kAutoMaxSplit = 24;  // automatic splits stop here
 constexpr size_t kLdsBytes = (size_t)64 << 10;
-// A^T's staged bins: records (none for SF) and g values each.
-size_t bwd_lds_bytes(int basis, int win, int g) { return (size_t)win * ((basis == BASIS_SF ? 0 : 32) + 4 * g); }
+size_t record_bytes(int basis);
+// A^T's staged bins: a record (none for SF) and g values each.
+size_t bwd_lds_bytes(int basis, int win, int g) { return (size_t)win * (record_bytes(basis) + 4 * g); }
 size_t work_doubles(const sgdct_projector* h);
+double* new_lattice(sgdct_projector* h);
 SymPlan plain_plan(const sgdct_projector* h);
 int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
 int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
-int auto_fwd_split(const sgdct_projector* h);
 int auto_bwd_split(const sgdct_projector* h);
 int ensure_part(sgdct_projector* h, size_t doubles);
 void release_part(sgdct_projector* h);
 size_t part_need(const sgdct_projector* h);
+size_t host_part_doubles(const sgdct_projector* h);
 int part_images(const sgdct_projector* h);
 
 // Per-(view, bin) constants, FP64 on the host, stored FP32 like the
@@ -341,6 +355,13 @@ void bin_constants(int basis, const ViewGeo& v, int nu, double dx, double dy, vo
 }
 
 bool is_hex(int basis) { return basis == BASIS_H0 || basis == BASIS_HL; }
+
+// Bytes of a basis's per-(view, bin) record.
+size_t record_bytes(int basis) {
+  if (basis == BASIS_B1) return sizeof(B1Bin);
+  if (basis == BASIS_B0) return sizeof(B0Bin);
+  return is_hex(basis) ? hex_bin_size(basis) : 0;
+}
 // fan-beam handles split both A (line or row segments) and A^T (view groups)
 bool splits(int basis) { return basis == BASIS_B0 || basis == BASIS_B1 || basis == BASIS_SF || is_hex(basis); }
 
@@ -385,10 +406,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     v.gy1 = (float)(v.pux * dy);
     v.db = (float)(h->h * (std::fabs(v.puy * dx) + std::fabs(v.pux * dy)));
   }
-  size_t rec = 0;
-  if (basis == BASIS_B1) rec = sizeof(B1Bin);
-  else if (basis == BASIS_B0) rec = sizeof(B0Bin);
-  else if (is_hex(basis)) rec = hex_bin_size(basis);
+  const size_t rec = record_bytes(basis);
   std::vector<unsigned char> bins(rec * (size_t)np * nu);
   for (int p = 0; p < np && rec; ++p) {
     unsigned char* dst = bins.data() + rec * (size_t)p * nu;
@@ -413,9 +431,10 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
   a.dx = dx; a.dy = dy;
   a.h = h->h;
   a.nchunk = (nu + 63) / 64;
-  // 2 bins of slack for FP64 contraction differences between host and device
-  if (grouped(basis)) {
-    const int w = max_tile_window(a, views.data(), kMaxWindow - 2) + 2;
+  if (splits(basis)) {
+    // 2 bins of slack for FP64 contraction differences between host and device
+    const int w = (is_hex(basis) ? hex_tile_window(a, dt, views.data())
+                                 : max_tile_window(a, views.data(), kMaxWindow - 2)) + 2;
     h->bwd_lds = w <= kMaxWindow;
     if (setup_symmetry(h, views) != SGDCT_OK) {
       delete h;
@@ -428,9 +447,9 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     // and 1024 bins, 2..16 row segments took one image from 1.11 to 1.20..1.40
     // ms (H0) and a batch of 64 from 59 to 64..84 ms (measured when A walked
     // lattice rows only, before steep waves walked the vertical lines)
-    h->fwd_auto = is_hex(basis) ? 1 : auto_fwd_split(h);
+    h->fwd_auto = is_hex(basis) ? 1 : kAutoMaxSplit;
     h->bwd_auto = auto_bwd_split(h);
-    if (ensure_part(h, work_doubles(h)) != SGDCT_OK) {
+    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || (is_hex(basis) && !new_lattice(h))) {
       delete h;
       return nullptr;
     }
@@ -442,6 +461,16 @@ size_t img_elems(const sgdct_projector* h) { return (size_t)h->nx * h->ny * h->n
 size_t sino_elems(const sgdct_projector* h) { return (size_t)h->np * h->nu * h->nv; }
 
 int ensure_staging(sgdct_projector* h) {
+  // a split_config since the last call may ask for more partial sums
+  const size_t need = host_part_doubles(h);
+  if (need > h->host_part_cap) {
+    if (h->d_host_part) (void)hipFree(h->d_host_part);
+    h->d_host_part = nullptr;
+    h->host_part_cap = 0;
+    const hipError_t e = hipMalloc(&h->d_host_part, need * sizeof(double));
+    if (e != hipSuccess) return hip_fail(e, "staging allocation");
+    h->host_part_cap = need;
+  }
   if (h->d_img) return SGDCT_OK;
   const size_t ni = img_elems(h), ns = sino_elems(h);
   hipError_t e = hipMalloc(&h->d_img, ni * sizeof(float));
@@ -559,41 +588,28 @@ int cone_backward(sgdct_projector* h, const float* proj, float* vol, int batch, 
   return SGDCT_OK;
 }
 
-// Launch-size targets of the automatic splits (one image): enough waves for
-// the GPU's 8192 wave slots (256 CUs x 4 SIMDs x 8) to turn over about 24
-// times in A (its per-wave work is uneven) and 12 times in A^T.  B1 at
-// 512 x 512, 720 views, 768 bins thus runs 24 segments and 24 view groups:
-// A 0.942 ms, A^T 0.922 ms, against 0.960 / 0.932 ms at 16 / 16.
-constexpr long long kFwdWaveTarget = 200000, kBwdWaveTarget = 98304, kBwdBlockTarget = 4600, kBwdSmallBlocks = 1024;
+// Workgroups A^T's view groups aim at: three turns of the 1536 that are
+// resident at G = 8 (512 x 512, 720 views, 8 symmetries: 1536 workgroups 219
+// us, 2300 209, 4600 197; 1024 x 1024, 1440 views 1.83, 1.51, 1.35 ms), twelve
+// waves per wave slot without symmetries.
+constexpr long long kBwdWaveTarget = 98304, kBwdBlockTarget = 4600, kBwdSmallBlocks = 1024;
 // A^T stages as many views at a time as fill 16 KB of LDS (16, 24, 32 KB: 200
 // us at 512 x 512, 720 views; 48 KB, which costs a workgroup per CU, 210 us).
 constexpr size_t kBwdStageBytes = (size_t)16 << 10;
 constexpr int kBwdMaxViews = 8;
-constexpr int kAutoMaxSplit = 24;  // automatic splits stop here
 constexpr int kMaxSplit = 32;      // sgdct_split_config accepts 1..kMaxSplit
 
-int auto_fwd_split(const sgdct_projector* h) {
-  if (grouped(h->basis)) return kAutoMaxSplit;
-  const long long waves = (long long)h->np * h->args.nchunk;
-  return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, (kFwdWaveTarget + waves - 1) / waves));
-}
 
 int auto_bwd_split(const sgdct_projector* h) {
-  if (grouped(h->basis)) {
-    const long long tiles = h->win ? h->sym.ntile : plain_plan(h).ntile;
-    // groups of >= 16 views while they add blocks up to kBwdBlockTarget; a
-    // small image, which leaves the GPU idle, takes groups of >= 4 views up
-    // to kBwdSmallBlocks (64 x 64, 60 views: 29.2 us at 16 views per group,
-    // 14.4 us at 4; 512 x 512, 90 views, batch 8: 205 us at 16, 257 us at 4)
-    const long long target = h->sym.nh > 1 ? kBwdBlockTarget / tiles : (kBwdWaveTarget / 4 + tiles - 1) / tiles;
-    const long long many = std::min<long long>(h->np / 16, target);
-    const long long few = std::min<long long>(h->np / 4, kBwdSmallBlocks / tiles);
-    return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, std::max(many, few)));
-  }
-  const long long waves = 4LL * ((h->nx + kTile - 1) / kTile) * ((h->ny + kTile - 1) / kTile);
-  const long long by_views = std::max(1, h->np / (4 * kViewChunk));  // groups of >= 16 views
-  return (int)std::max(1LL, std::min<long long>(std::min<long long>(kAutoMaxSplit, by_views),
-                                                (kBwdWaveTarget + waves - 1) / waves));
+  const long long tiles = h->win ? h->sym.ntile : plain_plan(h).ntile;
+  // groups of >= 16 views while they add blocks up to kBwdBlockTarget; a
+  // small image, which leaves the GPU idle, takes groups of >= 4 views up
+  // to kBwdSmallBlocks (64 x 64, 60 views: 29.2 us at 16 views per group,
+  // 14.4 us at 4; 512 x 512, 90 views, batch 8: 205 us at 16, 257 us at 4)
+  const long long target = h->sym.nh > 1 ? kBwdBlockTarget / tiles : (kBwdWaveTarget / 4 + tiles - 1) / tiles;
+  const long long many = std::min<long long>(h->np / 16, target);
+  const long long few = std::min<long long>(h->np / 4, kBwdSmallBlocks / tiles);
+  return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, std::max(many, few)));
 }
 
 // The identity only.
@@ -631,7 +647,11 @@ int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views) {
   // mirrors and half turns for any grid, axis swaps for square ones
   unsigned allowed = 1u | 1u << SymOp::kFlipX | 1u << SymOp::kFlipY | 1u << (SymOp::kFlipX | SymOp::kFlipY);
   if (h->nx == h->ny && h->dx == h->dy) allowed = 0xff;
-  const SymTables t = find_symmetries(views, h->nx, h->ny, h->nu, allowed, most, 4e-12 * (h->lsd + h->lso));
+  // a hexagonal lattice has no quarter turns, and its rows keep their parity
+  // under a vertical mirror when their number is odd
+  if (is_hex(h->basis)) allowed &= (h->ny & 1) ? 0x55 : (1u | 1u << SymOp::kFlipX);
+  const SymTables t = find_symmetries(views, h->nx, h->ny, h->nu, allowed, most, 4e-12 * (h->lsd + h->lso),
+                                      is_hex(h->basis));
   if (t.nh() == 1) return SGDCT_OK;
   const size_t nr = t.rep.size(), nv = t.rep_view.size(), np = t.view.size(), nt = t.tile.size();
   std::vector<int> all(nr + nv + np + nt + (t.owner.size() + 3) / 4);
@@ -674,6 +694,7 @@ int group_size(int nh, int m) {
 // 4332 workgroups) 453 / 422 us; 64 x 64, 60 views 11.9 / 9.7 us (a launch
 // more).
 int grid_segments(const sgdct_projector* h, int n) {
+  if (is_hex(h->basis)) return n;  // one wave per (view, chunk)
   const long long blocks = (long long)h->sym.nrep * h->args.nchunk;
   const size_t bytes = (size_t)h->nx * h->ny * h->sym.nh * sizeof(float);
   const bool more = std::max(h->nx, h->ny) > 96 && (blocks < 2048 || bytes > ((size_t)16 << 20));
@@ -684,7 +705,7 @@ int grid_segments(const sgdct_projector* h, int n) {
 // in doubles, for image groups of m images.
 size_t fwd_group_doubles(const sgdct_projector* h, int nh, int nseg, int m) {
   const size_t n = (((size_t)h->nx * h->ny * group_size(nh, m) + 3) / 4 * 4) / 2;
-  return (nseg > 1 ? ((size_t)nseg * m * h->np * h->nu + 1) / 2 * 2 : 0) + 2 * n;
+  return (nseg > 1 ? ((size_t)nseg * m * h->np * h->nu + 1) / 2 * 2 : 0) + (is_hex(h->basis) ? 1 : 2) * n;
 }
 
 // One image of at most this edge without symmetries is read in place: its
@@ -693,17 +714,51 @@ constexpr int kDirectEdge = 96;
 
 constexpr size_t kGroupBytes = (size_t)64 << 20;  // several image groups per launch up to this much workspace
 
-// Workspace of a handle: for B0 / B1 / SF one image group of A with as many images
+// Workspace of a handle: one image group of A with as many images
 // as fit kMaxGroup values, more while it stays within kGroupBytes; the FP64
 // partial images of A^T.
-size_t work_doubles(const sgdct_projector* h) {
-  const size_t part = part_images(h) * part_need(h);
-  if (!grouped(h->basis)) return part;
+size_t fwd_work_doubles(const sgdct_projector* h, int nseg) {
   const int m = std::max(1, max_group(h) / h->sym.nh);
-  size_t need = fwd_group_doubles(h, h->sym.nh, grid_segments(h, fwd_segments(h)), m);
-  need *= std::max<size_t>(1, std::min<size_t>(16, kGroupBytes / sizeof(double) / need));
-  const int bs = bwd_groups(h);
-  return std::max(need, bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0);
+  const size_t need = fwd_group_doubles(h, h->sym.nh, nseg, m);
+  return need * std::max<size_t>(1, std::min<size_t>(16, kGroupBytes / sizeof(double) / need));
+}
+
+size_t work_doubles(const sgdct_projector* h) {
+  const int nseg = grid_segments(h, fwd_segments(h)), bs = bwd_groups(h);
+  const size_t fwd = is_hex(h->basis) && nseg == 1 ? 0 : fwd_work_doubles(h, nseg);
+  return std::max(fwd, bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0);
+}
+
+// Interleaved lattices of the hexagonal A, whose unsplit launches share no
+// other memory: one buffer per stream that calls it, so that a handle's calls
+// on different streams may overlap.  The first is made with the handle and
+// taken by the first stream; a stream past kLattices, and one under capture
+// (whose graph may be launched anywhere), gets none and runs without groups.
+constexpr size_t kLattices = 4;
+
+double* new_lattice(sgdct_projector* h) {
+  double* p = nullptr;
+  const hipError_t e = hipMalloc(&p, fwd_work_doubles(h, 1) * sizeof(double));
+  if (e != hipSuccess) {
+    hip_fail(e, "interleaved lattice");
+    return nullptr;
+  }
+  h->lattices.push_back({nullptr, false, p});
+  return p;
+}
+
+// Called with h->lattice_mu held, which the caller keeps until its kernels are
+// enqueued.
+double* lattice_of(sgdct_projector* h, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+  else if (st != hipStreamCaptureStatusNone) return nullptr;
+  for (auto& l : h->lattices)
+    if (l.taken && l.stream == s) return l.p;
+  if (h->lattices.back().taken && (h->lattices.size() >= kLattices || !new_lattice(h))) return nullptr;
+  h->lattices.back().taken = true;
+  h->lattices.back().stream = s;
+  return h->lattices.back().p;
 }
 
 // Room for `doubles` partial sums.
@@ -746,33 +801,37 @@ int part_images(const sgdct_projector* h) {
 }
 
 
-hipError_t launch_fwd2d(const sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* part,
-                        hipStream_t s) {
-  return launch_hex_forward(h->basis, h->args, h->dt, img, sino, batch, nseg, part, s);
+hipError_t launch_fwd2d(const sgdct_projector* h, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  if (h->basis == BASIS_SF) return launch_sf_forward(h->args, r, img, sino, s);
+  if (is_hex(h->basis)) return launch_hex_forward(h->basis, h->args, h->dt, r, img, sino, s);
+  return launch_forward(h->basis, h->args, r, img, sino, s);
 }
 
-hipError_t launch_bwd2d(const sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* part,
-                        hipStream_t s) {
-  return launch_hex_backward(h->basis, h->args, h->dt, sino, img, batch, ngroup, part, s);
+hipError_t launch_bwd2d(const sgdct_projector* h, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  if (h->basis == BASIS_SF) return launch_sf_backward(h->args, r, sino, img, s);
+  if (is_hex(h->basis)) return launch_hex_backward(h->basis, h->args, h->dt, r, sino, img, s);
+  return launch_backward(h->basis, h->args, r, sino, img, s);
 }
 
-// B0 / B1 / SF A: images in groups of m, as many groups per launch as the
+// A: images in groups of m, as many groups per launch as the
 // workspace buf[0, cap) holds.  Every image's values are formed the same way
 // whatever the batch.  A workspace too small for one group of one image
 // runs without symmetries, reading the image in place (partial sums, which a
 // fixed split needs, must fit).
 int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* buf, size_t cap,
-                  bool plain, hipStream_t s) {
+                  hipStream_t s) {
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
   nseg = grid_segments(h, nseg);
   if (nseg > 1 && (!buf || cap < nseg * ns)) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
   GroupRun r;
-  r.sym = plain ? plain_plan(h) : h->sym;
+  r.sym = h->sym;
   r.split = nseg;
-  r.m = plain ? 1 : std::max(1, std::min(batch, max_group(h) / r.sym.nh));
+  r.m = std::max(1, std::min(batch, max_group(h) / r.sym.nh));
+  // a small launch takes fewer images per group and more workgroups
+  while (r.m > 1 && (long long)r.sym.nrep * h->args.nchunk * ((batch + r.m - 1) / r.m) < kSymBlocks) r.m >>= 1;
   while (r.m > 1 && fwd_group_doubles(h, r.sym.nh, nseg, r.m) > cap) --r.m;
   const size_t per = fwd_group_doubles(h, r.sym.nh, nseg, r.m);
-  const bool interleave = buf && per <= cap && (r.sym.nh * r.m > 1 || std::max(h->nx, h->ny) > kDirectEdge);
+  const bool interleave = buf && per <= cap && (r.sym.nh * r.m > 1 || (!is_hex(h->basis) && std::max(h->nx, h->ny) > kDirectEdge));
   if (!interleave) r.sym = plain_plan(h), r.m = 1;
   r.g = group_size(r.sym.nh, r.m);
   const size_t groups = interleave ? cap / per : (nseg > 1 ? cap / (nseg * ns) : (size_t)batch);
@@ -790,21 +849,25 @@ int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, 
       if ((at - buf) & 1) ++at;  // 16-byte alignment
       const size_t n = (ni * r.g + 3) / 4 * 4 * r.groups();
       r.rows = r.g > 1 ? reinterpret_cast<float*>(at) : nullptr;
-      r.cols = reinterpret_cast<float*>(at) + n;
+      r.cols = is_hex(h->basis) ? nullptr : reinterpret_cast<float*>(at) + n;
     }
-    e = h->basis == BASIS_SF ? launch_sf_forward(h->args, r, img + b0 * ni, sino + b0 * ns, s)
-                             : launch_forward(h->basis, h->args, r, img + b0 * ni, sino + b0 * ns, s);
+    e = launch_fwd2d(h, r, img + b0 * ni, sino + b0 * ns, s);
   }
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
 }
 
-// B0 / B1 / SF A^T, view groups' FP64 partial images in buf[0, cap).
+// Views A^T stages at a time.
+int stage_views(const sgdct_projector* h, const GroupRun& r) {
+  return (int)std::max<size_t>(1, std::min<size_t>(kBwdMaxViews, kBwdStageBytes / bwd_lds_bytes(h->basis, r.win, r.g)));
+}
+
+// A^T, view groups' FP64 partial images in buf[0, cap).
 int group_backward(sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* buf, size_t cap,
-                   bool plain, hipStream_t s) {
+                   hipStream_t s) {
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
   if (ngroup > 1 && (!buf || cap < ngroup * ni)) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
   GroupRun r;
-  r.sym = h->win && !plain ? h->sym : plain_plan(h);
+  r.sym = h->win ? h->sym : plain_plan(h);
   r.split = ngroup;
   r.part = ngroup > 1 ? buf : nullptr;
   r.win = h->win;
@@ -818,68 +881,83 @@ int group_backward(sgdct_projector* h, const float* sino, float* img, int batch,
     r.batch = std::min(step, batch - b0);
     r.m = std::min(r.m, r.batch);
     r.g = group_size(r.sym.nh, r.m);
-    if (r.win) r.nvc = (int)std::max<size_t>(1, std::min<size_t>(kBwdMaxViews, kBwdStageBytes / bwd_lds_bytes(h->basis, r.win, r.g)));
-    e = h->basis == BASIS_SF ? launch_sf_backward(h->args, r, sino + b0 * ns, img + b0 * ni, s)
-                             : launch_backward(h->basis, h->args, r, sino + b0 * ns, img + b0 * ni, s);
+    if (r.win) r.nvc = stage_views(h, r);
+    e = launch_bwd2d(h, r, sino + b0 * ns, img + b0 * ni, s);
   }
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
 }
 
-// Fan-beam A of `batch` images with each bin's walk in `nseg` line segments,
-// the FP64 partial sums in part[0, cap) (doubles): as many images per launch
-// as the buffer holds, so every image is computed the same way whatever the
-// batch size or the buffer.
-int fan_forward(sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* part, size_t cap,
-                bool plain, hipStream_t s) {
-  if (grouped(h->basis)) return group_forward(h, img, sino, batch, nseg, part, cap, plain, s);
-  hipError_t e = hipSuccess;
-  const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu, per = (size_t)nseg * ns;
-  if (nseg == 1) {
-    e = launch_fwd2d(h, img, sino, batch, 1, nullptr, s);
-  } else {
-    if (!part || cap < per) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
-    const int bc = (int)std::min<size_t>(batch, cap / per);
-    for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += bc)
-      e = launch_fwd2d(h, img + b0 * ni, sino + b0 * ns, std::min(bc, batch - b0), nseg, part, s);
+int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s) {
+  if (is_cone(h->basis)) return cone_forward(h, img, sino, batch, s);
+  if (is_hex(h->basis) && fwd_segments(h) == 1) {
+    std::lock_guard<std::mutex> lock(h->lattice_mu);
+    double* const buf = lattice_of(h, s);
+    return group_forward(h, img, sino, batch, 1, buf, buf ? fwd_work_doubles(h, 1) : 0, s);
   }
+  return group_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, s);
+}
+
+int run_backward(sgdct_projector* h, const float* sino, float* img, int batch, hipStream_t s) {
+  if (is_cone(h->basis)) return cone_backward(h, sino, img, batch, s);
+  return group_backward(h, sino, img, batch, bwd_groups(h), h->d_part, h->part_cap, s);
+}
+
+// The FP64 host-array entry points evaluate every view by itself and add its
+// lines and views in an order of their own (contiguous line segments, whole
+// groups of views), which neither the scan's symmetries nor the launch shape
+// of the device entry points change: what they return for a view is the same
+// to the last bit whichever other views the handle holds.  That costs little
+// while the conversions and copies of their arrays are most of a call (256 x
+// 256, 360 views: the kernels are 0.2 of 0.46 ms per pair).  From kHostPairs
+// (pixel, view) pairs on the kernels are most of it, and the call takes the
+// device entry points' launches.
+constexpr double kHostPairs = 1.5e8;
+bool host_alone(const sgdct_projector* h) {
+  return !is_cone(h->basis) && (double)h->nx * h->ny * h->np < kHostPairs;
+}
+
+int host_segments(const sgdct_projector* h) {
+  if (h->fwd_split || is_hex(h->basis)) return fwd_segments(h);
+  const long long waves = (long long)h->np * h->args.nchunk;
+  return (int)std::max(1LL, std::min<long long>(kAutoMaxSplit, (200000 + waves - 1) / waves));
+}
+
+int host_groups(const sgdct_projector* h) {
+  if (h->bwd_split) return h->bwd_split;
+  const long long waves = 4LL * plain_plan(h).ntile, by_views = std::max(1, h->np / 16);
+  return (int)std::max(1LL, std::min<long long>(std::min<long long>(kAutoMaxSplit, by_views),
+                                                (kBwdWaveTarget + waves - 1) / waves));
+}
+
+size_t host_part_doubles(const sgdct_projector* h) {
+  if (!host_alone(h)) return 0;
+  const size_t fs = host_segments(h), bs = host_groups(h);
+  return std::max(fs > 1 ? fs * h->np * h->nu : 0, bs > 1 ? bs * h->nx * h->ny : 0);
+}
+
+int run_host_forward(sgdct_projector* h) {
+  if (!host_alone(h)) return run_forward(h, h->d_img, h->d_sino, 1, nullptr);
+  GroupRun r;
+  r.sym = plain_plan(h);
+  r.lone = true;
+  r.split = host_segments(h);
+  r.part = r.split > 1 ? h->d_host_part : nullptr;
+  const hipError_t e = launch_fwd2d(h, r, h->d_img, h->d_sino, nullptr);
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
 }
 
-// Fan-beam A^T with the views in `ngroup` groups, partial sums as above.
-int fan_backward(sgdct_projector* h, const float* sino, float* img, int batch, int ngroup, double* part, size_t cap,
-                 bool plain, hipStream_t s) {
-  if (grouped(h->basis)) return group_backward(h, sino, img, batch, ngroup, part, cap, plain, s);
-  hipError_t e = hipSuccess;
-  const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu, per = (size_t)ngroup * ni;
-  if (ngroup == 1) {
-    e = launch_bwd2d(h, sino, img, batch, 1, nullptr, s);
-  } else {
-    if (!part || cap < per) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
-    const int bc = (int)std::min<size_t>(batch, cap / per);
-    for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += bc)
-      e = launch_bwd2d(h, sino + b0 * ns, img + b0 * ni, std::min(bc, batch - b0), ngroup, part, s);
-  }
+int run_host_backward(sgdct_projector* h) {
+  if (!host_alone(h)) return run_backward(h, h->d_sino, h->d_img, 1, nullptr);
+  GroupRun r;
+  r.sym = plain_plan(h);
+  r.split = host_groups(h);
+  r.part = r.split > 1 ? h->d_host_part : nullptr;
+  r.win = h->win;
+  r.vpg = (h->np + r.split - 1) / r.split;
+  if (h->basis == BASIS_B0 || h->basis == BASIS_B1) r.vpg = (r.vpg + kViewChunk - 1) / kViewChunk * kViewChunk;
+  if (r.win) r.nvc = stage_views(h, r);
+  const hipError_t e = launch_bwd2d(h, r, h->d_sino, h->d_img, nullptr);
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
-}
-
-// plain: every view's footprints by themselves, without the scan's
-// symmetries, so that a view's values do not depend (in the last FP32 bit) on
-// which other views the handle holds.  The FP64 host-array entry points run
-// this way while the conversions and copies of their arrays are most of the
-// call (256 x 256, 360 views: the kernels are 0.18 of 0.46 ms per pair); from
-// kHostPairs (pixel, view) pairs on the kernels are, and they take the
-// symmetries.
-constexpr double kHostPairs = 1.5e8;
-bool host_plain(const sgdct_projector* h) { return (double)h->nx * h->ny * h->np < kHostPairs; }
-
-int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s, bool plain = false) {
-  if (is_cone(h->basis)) return cone_forward(h, img, sino, batch, s);
-  return fan_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, plain, s);
-}
-
-int run_backward(sgdct_projector* h, const float* sino, float* img, int batch, hipStream_t s, bool plain = false) {
-  if (is_cone(h->basis)) return cone_backward(h, sino, img, batch, s);
-  return fan_backward(h, sino, img, batch, bwd_groups(h), h->d_part, h->part_cap, plain, s);
 }
 
 // Footprint evaluations of the reference's cone-beam forward
@@ -976,7 +1054,7 @@ int host_forward(double* b, double* x, sgdct_projector* h) {
     const size_t ni = (size_t)nx * ny, ns = (size_t)h->np * h->nu;
     e = hipMemcpy(h->d_img, h->h_img, ni * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "upload image");
-    rc = run_forward(h, h->d_img, h->d_sino, 1, nullptr, host_plain(h));
+    rc = run_host_forward(h);
     if (rc) return rc;
     e = hipMemcpy(h->h_sino, h->d_sino, ns * sizeof(float), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "download sinogram");
@@ -1003,7 +1081,7 @@ int host_backward(double* b, double* x, sgdct_projector* h) {
     for (size_t i = 0; i < ns; ++i) h->h_sino[i] = (float)b[i];
     e = hipMemcpy(h->d_sino, h->h_sino, ns * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "upload sinogram");
-    rc = run_backward(h, h->d_sino, h->d_img, 1, nullptr, host_plain(h));
+    rc = run_host_backward(h);
     if (rc) return rc;
     e = hipMemcpy(h->h_img, h->d_img, ni * sizeof(float), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "download image");
@@ -1519,8 +1597,8 @@ int sgdct_project_dev_noalloc(sgdct_projector* h, int direction, const float* in
     n = (int)std::max<size_t>(1, kScratchDoubles / unit);
   }
   hipStream_t s = (hipStream_t)stream;
-  return direction == 0 ? fan_forward(h, in, out, batch, n, part, kScratchDoubles, false, s)
-                        : fan_backward(h, in, out, batch, n, part, kScratchDoubles, false, s);
+  return direction == 0 ? group_forward(h, in, out, batch, n, part, kScratchDoubles, s)
+                        : group_backward(h, in, out, batch, n, part, kScratchDoubles, s);
 }
 
 int sgdct_shape(const sgdct_projector* h, int* out) {

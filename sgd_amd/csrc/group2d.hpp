@@ -44,6 +44,14 @@ struct SymOp {
     *ox = x;
     *oy = y;
   }
+  // point (ic, il) of a hexagonal lattice (odd rows hold nx - 1 points, half a
+  // column on; their slot nx - 1 is no point and maps to such a slot).  A
+  // vertical mirror keeps a row's parity only when ny is odd.
+  __host__ __device__ static __forceinline__ void hex_point(int op, int nx, int ny, int ix, int iy, int* ox, int* oy) {
+    const int n = nx - (iy & 1);
+    *ox = (op & kFlipX) && ix < n ? n - 1 - ix : ix;
+    *oy = (op & kFlipY) ? ny - 1 - iy : iy;
+  }
   __host__ __device__ static __forceinline__ void point(int op, double x, double y, double* ox, double* oy) {
     const double a = (op & kSwap) ? y : x, b = (op & kSwap) ? x : y;
     *ox = (op & kFlipX) ? -a : a;
@@ -71,7 +79,8 @@ struct GroupRun {
   SymPlan sym;
   int g = 1;              // values per footprint, >= sym.nh * m (1, 2, 4 or 8)
   int m = 1, batch = 1;
-  int split = 1;          // A: line segments, A^T: view groups
+  int split = 1;          // A: grid segments, A^T: view groups
+  bool lone = false;      // A (g = 1): one wave per workgroup
   double* part = nullptr; // FP64 partial sums (split > 1)
   float* rows = nullptr;  // A: interleaved images (null: g = 1, read in place)
   float* cols = nullptr;  // A: their transposes (null: column walks read strided)
@@ -83,6 +92,8 @@ struct GroupRun {
 // Waves of an A workgroup share one (view, 64-bin chunk): wave w walks the
 // lines m = w mod kFwdWaves of every bin's strip, and the FP64 sums of the
 // waves are added in wave order through LDS.
+// A lone run has one wave per workgroup, which walks whole segments line by
+// line.
 constexpr int kFwdWaves = 8;
 
 // The chunk a workgroup takes: centre chunks (whose strips are longest) first,

@@ -87,25 +87,25 @@ __host__ __device__ inline void tile_window(const Proj2DArgs& g, const ViewGeo& 
   *n = hi >= li ? min(hi - li + 1, cap) : 0;
 }
 
-// Sums of an A workgroup's waves (kFwdWaves, red[wave][slot][lane]) in wave
-// order, times the bin's factor, to the outputs of every slot: view h v, bin u
+// Sums of an A workgroup's W waves (red[wave][slot][lane]) in wave order,
+// times the bin's factors, to the outputs of every slot: view h v, bin u
 // (reversed where h mirrors).  All threads of the workgroup call this after
 // writing red and a barrier.
-template <int G>
+template <int G, int W>
 __device__ __forceinline__ void fwd_group_store(const Proj2DArgs& g, const SymPlan& sp, int rep, int v, int u, int m,
-                                                int batch, const double (*red)[G][64], double factor,
+                                                int batch, const double (*red)[G][64], double f0, double f1, double f2,
                                                 float* __restrict__ sino, double* __restrict__ part) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int img0 = blockIdx.y * m, nimg = min(m, batch - img0);
   const size_t nsino = (size_t)g.np * g.nu;
-  for (int s = wv; s < sp.nh * nimg; s += kFwdWaves) {
+  for (int s = wv; s < sp.nh * nimg; s += W) {
     const int k = s >> sp.lg, h = s & (sp.nh - 1);
     const int vh = sp.rep_view ? sp.rep_view[rep * sp.nh + h] : v;
     if (vh < 0) continue;
     double t = 0.0;
 #pragma unroll
-    for (int w = 0; w < kFwdWaves; ++w) t += red[w][s][lane];
-    t *= factor;
+    for (int w = 0; w < W; ++w) t += red[w][s][lane];
+    t = t * f0 * f1 * f2;
     const int uh = SymOp::reverses(sp.op[h]) ? g.nu - 1 - u : u;
     const size_t o = (img0 + k) * nsino + (size_t)vh * g.nu + uh;
     if (part) part[(size_t)blockIdx.z * batch * nsino + o] = t;

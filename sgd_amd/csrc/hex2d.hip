@@ -19,7 +19,9 @@
 #include <cmath>
 
 #include "footprint.hpp"
+#include "group2d_dev.hpp"
 #include "projector.hpp"
+#include "symmetry.hpp"
 
 namespace sgdct {
 
@@ -95,61 +97,35 @@ struct HexArgs {
   double dt;
 };
 
-// A: bin-driven gather over lattice rows.
-// grid (waves / 4, batch, nseg), wave = chunk * np + view.  With nseg > 1,
-// segment k = blockIdx.z takes
-// lines [k L, k L + L) of its walk (rows or vertical lines, L = ceil(lines /
-// nseg)) and writes its FP64
-// sum, already scaled, to part[(k * batch + image) * np * nu + v * nu + u];
-// sum_parts_kernel adds the segments in order.
-// STAGE: the row walk reads the lattice from LDS.  The strips of a wave's 64
-// adjacent bins lie along the rows there and each lane walks rows of its own,
-// so direct reads touch a cache line per lane and instruction, and the lines
-// a wave is working on outgrow the vector L1.  Instead the wave walks the
-// lattice in slabs of cw columns (32, halved while the slab's rows do not fit
-// in the wave's kHexStage floats): it copies the rows its lanes reach in the
-// slab into LDS with coalesced loads, then every lane walks its rows of the
-// slab there.  The footprint arithmetic is that of the direct walk; the
-// point order within a row is the same, the FP32 partial sums restart at each
-// slab.  A slab whose rows do not fit even at the narrowest width is read
-// directly.
-// Waves whose middle ray is within atan(kHexStageSlope dy / dx) of the rows
-// stage (22 degrees on the 0.5 mm Hl lattice); steeper strips cross each row
-// in a few points, and the slabs would split their short runs.
-constexpr int kHexStage = 2048, kHexCW = 32, kHexCWMin = 8;
-constexpr double kHexStageSlope = 1.4;
-
-__device__ __forceinline__ void hex_wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// The G values of a lattice point.
+template <int G>
+__device__ __forceinline__ void load_point(const float* p, float (&x)[G]) {
+  __builtin_memcpy(x, __builtin_assume_aligned(p, G < 4 ? 4 * G : 16), sizeof(x));
 }
 
-template <int HB, bool STAGE>
-__global__ __launch_bounds__(256) void hex_fwd_kernel(HexArgs ha, const float* __restrict__ img,
-                                                      float* __restrict__ sino, double* __restrict__ part) {
+// A: bin-driven gather along lattice rows, or along the vertical lines k = 2 ic
+// + (il & 1) (x = k dx / 2, every other row) when the wave's middle ray gives a
+// strip more points per vertical line (|ray_y| dx > 2 dy |ray_x|): steep strips
+// cross every row with only a point or two in each.  The choice is uniform
+// over the wave.
+// One wave: bins [64 chunk, 64 chunk + 64) of view v, one per lane; of every
+// line's points the w-th of wn equal ranges of columns (row walk) or rows
+// (vertical walk), of the lines segment seg of nseg.  Adds sum conv * x into
+// acc[G] (FP32 along a line, FP64 across lines; without dx dy).  img holds G
+// values per point.  Lanes past the last bin add nothing.
+// The strips lie along the lines, so splitting the points keeps every lane of
+// every wave busy, where splitting the lines would leave a lane only the few
+// it crosses; and a wave's lanes stay within one narrow range of columns or
+// rows at a time, which keeps the lines they touch in the vector L1 (walking
+// the whole lattice, near-row strips needed their rows staged in LDS for
+// that).
+template <int HB, int G>
+__device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chunk, const float* __restrict__ img, int w,
+                                              int wn, int seg, int nseg, double (&acc)[G]) {
   using T = HexTraits<HB>;
   const Proj2DArgs& g = ha.g;
-  constexpr int kWaves = 4;
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * kWaves + (threadIdx.x >> 6);
-  // chunk-major: the waves of a workgroup take the same 64 bins of adjacent
-  // views, so they walk nearly the same lattice points (shared L1 lines) and
-  // reach the lattice together or miss it together (a workgroup holds its
-  // slots until its longest wave ends; the 74 mm tall Hl lattice leaves three
-  // quarters of a view's bins empty near the row direction).  Against
-  // view-major order: H0 A 1.094 -> 0.834 ms, Hl 1.258 -> 0.944 ms (296 x 256,
-  // 1024 views, 1024 bins, one image); with the LDS staging below Hl 0.651 ms.
-  const int chunk = wave / g.np, v = wave - chunk * g.np;
-  if (chunk >= g.nchunk) return;
-  // with STAGE every lane of the wave takes part in the staging: lanes past
-  // the last bin walk nothing and store nothing
-  const int u_lane = chunk * 64 + lane;
-  const bool lane_ok = u_lane < g.nu;
-  if (!STAGE && !lane_ok) return;
-  const int u = lane_ok ? u_lane : g.nu - 1;
-  const int seg = blockIdx.z, nseg = gridDim.z;
-  img += (size_t)blockIdx.y * g.nx * g.ny;
+  const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
+  const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
   const ViewGeo vg = g.views[v];
   const typename T::Bin rec = reinterpret_cast<const typename T::Bin*>(g.bins)[(size_t)v * g.nu + u];
 
@@ -158,130 +134,68 @@ __global__ __launch_bounds__(256) void hex_fwd_kernel(HexArgs ha, const float* _
   // N(ic', il) = s * ic' + m * il + c, ic' = ic + (il odd) / 2
   const double sa = -eay * g.dx, ma = eax * g.dy, ca = eax * vg.w0y - eay * vg.w0x;
   const double sb = -eby * g.dx, mb = ebx * g.dy, cb = ebx * vg.w0y - eby * vg.w0x;
-  // pixel-set edges (clamped end bins see one more bin), as in fwd_bin_kernel
+  // pixel-set edges (clamped end bins see one more bin), as in fwd_bin_lines
   const double lax = (u == 0) ? eax - vg.pux : eax, lay = (u == 0) ? eay - vg.puy : eay;
   const double lbx = (u == g.nu - 1) ? ebx + vg.pux : ebx, lby = (u == g.nu - 1) ? eby + vg.puy : eby;
   const double sq = -lay * g.dx, mq = lax * g.dy, cq = lax * vg.w0y - lay * vg.w0x;
   const double sr = -lby * g.dx, mr = lbx * g.dy, cr = lbx * vg.w0y - lby * vg.w0x;
   const double rq = hex_reach(-lay, lax, ha.dt), rr = hex_reach(-lby, lbx, ha.dt);
-
   const double ka = rec.ka, kb = rec.kb;
-  double acc = 0.0;
-  // Walk lattice rows, or the vertical lines k = 2 ic + (il & 1) (x = k dx / 2,
-  // every other row) when the wave's middle ray gives a strip more points per
-  // vertical line (|ray_y| dx > 2 dy |ray_x|): steep strips cross every row
-  // with only a point or two in each.  The choice is uniform over the wave.
+  const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
+  const double imq = mq != 0.0 ? 1.0 / mq : 0.0, imr = mr != 0.0 ? 1.0 / mr : 0.0;
+
+  // One line: points i0, i0 + step, ... <= i1, `stride` floats apart.
+  auto walk = [&](const float* p, int i0, int i1, int step, size_t stride, float ta, float tb, float dta, float dtb) {
+    float accl[G], xn[G];
+#pragma unroll
+    for (int s = 0; s < G; ++s) accl[s] = 0.0f;
+    // the next point's values are requested one step ahead (the index clamped
+    // to the line's last point, so the read needs no branch), which overlaps
+    // their latency with the footprint evaluation
+    load_point<G>(p + (size_t)i0 * stride, xn);
+    for (int i = i0; i <= i1; i += step) {
+      float xc[G];
+#pragma unroll
+      for (int s = 0; s < G; ++s) xc[s] = xn[s];
+      load_point<G>(p + (size_t)min(i + step, i1) * stride, xn);
+      const float c = T::conv(rec, ta, tb);
+#pragma unroll
+      for (int s = 0; s < G; ++s) accl[s] = __builtin_fmaf(c, xc[s], accl[s]);
+      ta += dta;
+      tb += dtb;
+    }
+#pragma unroll
+    for (int s = 0; s < G; ++s) acc[s] += (double)accl[s];
+  };
+
   const int umid = min(chunk * 64 + 32, g.nu - 1);
   const double rmx = vg.e0x + (umid + 0.5) * vg.pux, rmy = vg.e0y + (umid + 0.5) * vg.puy;
   if (fabs(rmy) * g.dx <= 2.0 * g.dy * fabs(rmx)) {
-    // rows the strip can reach: between the crossings of its two boundary
-    // lines with the first and last column (ic' = 0 and nc), one row of margin
+    const int c_lo = g.nx * w / wn, c_hi = g.nx * (w + 1) / wn - 1;
+    // rows the strip can reach within the columns: between the crossings of
+    // its two boundary lines with ic' = c_lo and c_hi + 1, one row of margin
     int il_lo = 0, il_hi = g.ny - 1;
     if (mq != 0.0 && mr != 0.0) {
-      const double last = (double)g.nx;
-      const double c1 = (-rq - cq) / mq, c2 = (-rq - cq - sq * last) / mq;
-      const double c3 = (rr - cr) / mr, c4 = (rr - cr - sr * last) / mr;
+      const double x0 = (double)c_lo, x1 = (double)(c_hi + 1);
+      const double c1 = (-rq - cq - sq * x0) * imq, c2 = (-rq - cq - sq * x1) * imq;
+      const double c3 = (rr - cr - sr * x0) * imr, c4 = (rr - cr - sr * x1) * imr;
       const double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-      il_lo = (int)fmax(floor(lo) - 1.0, 0.0);
-      il_hi = (int)fmin(ceil(hi) + 1.0, (double)(g.ny - 1));
+      il_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)g.ny);
+      il_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(g.ny - 1)), -1.0);
     }
     if (nseg > 1) {
       const int len = (g.ny + nseg - 1) / nseg;
       il_lo = max(il_lo, seg * len);
       il_hi = min(il_hi, seg * len + len - 1);
     }
-    if (!lane_ok) il_lo = 1, il_hi = 0;
-    if (STAGE && fabs(rmy) * g.dx <= kHexStageSlope * g.dy * fabs(rmx)) {
-      __shared__ float stage_all[STAGE ? kWaves * kHexStage : 1];
-      float* st = stage_all + (threadIdx.x >> 6) * kHexStage;
-      const double kas = ka * sa, kbs = kb * sb;
-      const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
-      const double imq = mq != 0.0 ? 1.0 / mq : 0.0, imr = mr != 0.0 ? 1.0 / mr : 0.0;
-      const float dta = (float)kas, dtb = (float)kbs;
-      // the lane's rows within the slab ic' in [x0, x1]: between the
-      // crossings of its boundary lines with the slab's edges, one row of margin
-      auto slab_rows = [&](double x0, double x1, int& lo_r, int& hi_r) {
-        lo_r = il_lo;
-        hi_r = il_hi;
-        if (mq != 0.0 && mr != 0.0) {
-          const double c1 = (-rq - cq - sq * x0) * imq, c2 = (-rq - cq - sq * x1) * imq;
-          const double c3 = (rr - cr - sr * x0) * imr, c4 = (rr - cr - sr * x1) * imr;
-          const double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-          lo_r = max(lo_r, (int)fmin(fmax(floor(lo) - 1.0, -1.0), (double)g.ny));
-          hi_r = min(hi_r, (int)fmin(fmax(ceil(hi) + 1.0, -1.0), (double)g.ny));
-        }
-      };
-      for (int c0 = 0; c0 < g.nx;) {
-        int cw = kHexCW, lo_r, hi_r, R0, R1;
-        for (;;) {
-          slab_rows((double)c0, (double)(c0 + cw), lo_r, hi_r);
-          const bool any = lo_r <= hi_r;
-          R0 = __ockl_wfred_min_i32(any ? lo_r : 0x7fffffff);
-          R1 = __ockl_wfred_max_i32(any ? hi_r : -1);
-          if (R0 > R1 || (R1 - R0 + 1) * (cw + 1) <= kHexStage || cw == kHexCWMin) break;
-          cw >>= 1;
-        }
-        const int c1 = c0 + cw - 1;
-        if (R0 <= R1) {
-          const int ls = cw + 1;
-          const bool staged = (R1 - R0 + 1) * ls <= kHexStage;  // uniform over the wave
-          if (staged) {
-            const int lg = __builtin_ctz(cw), n_el = (R1 - R0 + 1) << lg;
-            hex_wave_lds_sync();  // the previous slab's reads come first
-            for (int e = lane; e < n_el; e += 64) {
-              const int r = e >> lg, c = e & (cw - 1);
-              st[r * ls + c] = img[(size_t)(R0 + r) * g.nx + min(c0 + c, g.nx - 1)];
-            }
-            hex_wave_lds_sync();
-          }
-          for (int il = lo_r; il <= hi_r; ++il) {
-            const double sh = (il & 1) ? 0.5 : 0.0;
-            const double r1 = -rq - __builtin_fma(mq, (double)il, cq) - sq * sh;  // need sq * ic >= r1
-            const double r2 = rr - __builtin_fma(mr, (double)il, cr) - sr * sh;   // need sr * ic <  r2
-            double lo = (double)c0, hi = (double)min(c1, g.nx - 1 - (il & 1));
-            if (sq > 0.0) lo = fmax(lo, ceil(r1 * isq));
-            else if (sq < 0.0) hi = fmin(hi, floor(r1 * isq));
-            else if (r1 > 0.0) continue;
-            if (sr > 0.0) hi = fmin(hi, ceil(r2 * isr) - 1.0);
-            else if (sr < 0.0) lo = fmax(lo, floor(r2 * isr) + 1.0);
-            else if (r2 <= 0.0) continue;
-            if (lo > hi) continue;
-            const int n0 = (int)lo, n1 = (int)hi;
-            float ta = (float)__builtin_fma(kas, n0 + sh, ka * __builtin_fma(ma, (double)il, ca));
-            float tb = (float)__builtin_fma(kbs, n0 + sh, kb * __builtin_fma(mb, (double)il, cb));
-            float accl = 0.0f;
-            if (staged) {
-              const float* q = st + (il - R0) * ls - c0;
-              for (int n = n0; n <= n1; ++n) {
-                accl = __builtin_fmaf(T::conv(rec, ta, tb), q[n], accl);
-                ta += dta;
-                tb += dtb;
-              }
-            } else {
-              const float* p = img + (size_t)il * g.nx;
-              for (int n = n0; n <= n1; ++n) {
-                accl = __builtin_fmaf(T::conv(rec, ta, tb), p[n], accl);
-                ta += dta;
-                tb += dtb;
-              }
-            }
-            acc += (double)accl;
-          }
-        }
-        c0 += cw;
-      }
-    } else {
-    // terms linear in the row index, carried from row to row in FP64
-    double q_il = mq * il_lo + cq, r_il = mr * il_lo + cr;
-    double ta_il = ka * (ma * il_lo + ca), tb_il = kb * (mb * il_lo + cb);
-    const double dta_il = ka * ma, dtb_il = kb * mb, kas = ka * sa, kbs = kb * sb;
-    const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
+    if (!inside) il_hi = -1;
+    const double kas = ka * sa, kbs = kb * sb;
     const float dta = (float)kas, dtb = (float)kbs;
-    for (int il = il_lo; il <= il_hi; ++il, q_il += mq, r_il += mr, ta_il += dta_il, tb_il += dtb_il) {
+    for (int il = il_lo; il <= il_hi; ++il) {
       const double sh = (il & 1) ? 0.5 : 0.0;
-      const double r1 = -rq - q_il - sq * sh;  // need sq * ic >= r1
-      const double r2 = rr - r_il - sr * sh;   // need sr * ic <  r2
-      double lo = 0.0, hi = (double)(g.nx - 1 - (il & 1));
+      const double r1 = -rq - __builtin_fma(mq, (double)il, cq) - sq * sh;  // need sq * ic >= r1
+      const double r2 = rr - __builtin_fma(mr, (double)il, cr) - sr * sh;   // need sr * ic <  r2
+      double lo = (double)c_lo, hi = (double)min(c_hi, g.nx - 1 - (il & 1));
       if (sq > 0.0) lo = fmax(lo, ceil(r1 * isq));
       else if (sq < 0.0) hi = fmin(hi, floor(r1 * isq));
       else if (r1 > 0.0) continue;
@@ -289,45 +203,32 @@ __global__ __launch_bounds__(256) void hex_fwd_kernel(HexArgs ha, const float* _
       else if (sr < 0.0) lo = fmax(lo, floor(r2 * isr) + 1.0);
       else if (r2 <= 0.0) continue;
       if (lo > hi) continue;
-      const int n0 = (int)lo, n1 = (int)hi;
-      float ta = (float)__builtin_fma(kas, n0 + sh, ta_il);
-      float tb = (float)__builtin_fma(kbs, n0 + sh, tb_il);
-      const float* p = img + (size_t)il * g.nx;
-      float accl = 0.0f;
-      // the next point's value is requested one step ahead (the index clamped
-      // to the row's last point, so the read needs no branch), which overlaps
-      // its latency with the footprint evaluation
-      float xn = p[n0];
-      for (int n = n0; n <= n1; ++n) {
-        const float xc = xn;
-        xn = p[min(n + 1, n1)];
-        accl = __builtin_fmaf(T::conv(rec, ta, tb), xc, accl);
-        ta += dta;
-        tb += dtb;
-      }
-      acc += (double)accl;
-    }
+      const int n0 = (int)lo;
+      walk(img + (size_t)il * g.nx * G, n0, (int)hi, 1, G,
+           (float)__builtin_fma(kas, n0 + sh, ka * __builtin_fma(ma, (double)il, ca)),
+           (float)__builtin_fma(kbs, n0 + sh, kb * __builtin_fma(mb, (double)il, cb)), dta, dtb);
     }
   } else {
-    // vertical lines the strip can reach: between the crossings of its two
-    // boundary lines with the first and last row, one line of margin
+    const int r_lo = g.ny * w / wn, r_hi = g.ny * (w + 1) / wn - 1;
+    // vertical lines the strip can reach within the rows: between the
+    // crossings of its two boundary lines with rows r_lo and r_hi, one line of
+    // margin
     const int kmax = 2 * g.nx - 2;
     int k_lo = 0, k_hi = kmax;
     if (sq != 0.0 && sr != 0.0) {
-      const double last = (double)(g.ny - 1);
-      const double c1 = (-rq - cq) / sq, c2 = (-rq - cq - mq * last) / sq;
-      const double c3 = (rr - cr) / sr, c4 = (rr - cr - mr * last) / sr;
+      const double y0 = (double)r_lo, y1 = (double)r_hi;
+      const double c1 = (-rq - cq - mq * y0) * isq, c2 = (-rq - cq - mq * y1) * isq;
+      const double c3 = (rr - cr - mr * y0) * isr, c4 = (rr - cr - mr * y1) * isr;
       const double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-      k_lo = (int)fmax(floor(2.0 * lo) - 2.0, 0.0);
-      k_hi = (int)fmin(ceil(2.0 * hi) + 2.0, (double)kmax);
+      k_lo = (int)fmin(fmax(floor(2.0 * lo) - 2.0, 0.0), (double)(kmax + 1));
+      k_hi = (int)fmax(fmin(ceil(2.0 * hi) + 2.0, (double)kmax), -1.0);
     }
     if (nseg > 1) {
       const int len = (kmax + nseg) / nseg;
       k_lo = max(k_lo, seg * len);
       k_hi = min(k_hi, seg * len + len - 1);
     }
-    if (!lane_ok) k_lo = 1, k_hi = 0;
-    const double imq = mq != 0.0 ? 1.0 / mq : 0.0, imr = mr != 0.0 ? 1.0 / mr : 0.0;
+    if (!inside) k_hi = -1;
     const double kam = ka * ma, kbm = kb * mb;
     const float dta = (float)(2.0 * kam), dtb = (float)(2.0 * kbm);
     for (int k = k_lo; k <= k_hi; ++k) {
@@ -335,7 +236,7 @@ __global__ __launch_bounds__(256) void hex_fwd_kernel(HexArgs ha, const float* _
       const double xh = 0.5 * k;                   // ic' of the line
       const double r1 = -rq - cq - sq * xh;        // need mq * il >= r1
       const double r2 = rr - cr - sr * xh;         // need mr * il <  r2
-      double lo = (double)par, hi = (double)(g.ny - 1);
+      double lo = (double)r_lo, hi = (double)r_hi;
       if (mq > 0.0) lo = fmax(lo, ceil(r1 * imq));
       else if (mq < 0.0) hi = fmin(hi, floor(r1 * imq));
       else if (r1 > 0.0) continue;
@@ -347,30 +248,163 @@ __global__ __launch_bounds__(256) void hex_fwd_kernel(HexArgs ha, const float* _
       i0 += (i0 ^ par) & 1;  // rows of the line's parity
       i1 -= (i1 ^ par) & 1;
       if (i0 > i1) continue;
-      float ta = (float)__builtin_fma(kam, (double)i0, ka * (sa * xh + ca));
-      float tb = (float)__builtin_fma(kbm, (double)i0, kb * (sb * xh + cb));
-      const float* p = img + (k >> 1);
-      float accl = 0.0f;
-      float xn = p[(size_t)i0 * g.nx];
-      for (int il = i0; il <= i1; il += 2) {
-        const float xc = xn;
-        xn = p[(size_t)min(il + 2, i1) * g.nx];
-        accl = __builtin_fmaf(T::conv(rec, ta, tb), xc, accl);
-        ta += dta;
-        tb += dtb;
-      }
-      acc += (double)accl;
+      walk(img + (size_t)(k >> 1) * G, i0, i1, 2, (size_t)g.nx * G,
+           (float)__builtin_fma(kam, (double)i0, ka * (sa * xh + ca)),
+           (float)__builtin_fma(kbm, (double)i0, kb * (sb * xh + cb)), dta, dtb);
     }
   }
-  if (!lane_ok) return;
-  const size_t out = (size_t)v * g.nu + u, nsino = (size_t)g.np * g.nu;
-  if (nseg > 1) part[((size_t)seg * gridDim.y + blockIdx.y) * nsino + out] = acc * g.dx * g.dy;
-  else sino[blockIdx.y * nsino + out] = (float)(acc * g.dx * g.dy);
+}
+
+// grid (nrep * nchunk, image groups, nseg): W waves take one representative
+// view and 64-bin chunk, and their FP64 sums are added in wave order through
+// LDS.  Chunk-major: workgroups in flight take the same bins of adjacent views,
+// so they walk nearly the same points and reach the lattice together or miss
+// it together.  Bound by VALU issue (H0: six trapezoid antiderivatives, ~75
+// instructions per footprint; Hl ~35) and, at G = 8, by the vector L1.  Per
+// call, one value per footprint and one wave per (view, chunk) -> now: H0 256
+// x 296 points, 1024 views, 1024 bins 840 -> 476 us; Hl, batch 64 30.8 -> 7.1
+// ms; Hl 40 x 46, 60 views, batch 3 76 -> 20 us.
+template <int HB, int G, int W>
+__global__ __launch_bounds__(64 * W) void hex_fwd_kernel(HexArgs ha, SymPlan sp, int m, int batch,
+                                                         const float* __restrict__ img, float* __restrict__ sino,
+                                                         double* __restrict__ part) {
+  __shared__ double red[W][G][64];
+  const Proj2DArgs& g = ha.g;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
+  const int chunk = centre_out(rank, g.nchunk);
+  const int v = sp.rep ? sp.rep[rep] : rep;
+  double acc[G];
+#pragma unroll
+  for (int s = 0; s < G; ++s) acc[s] = 0.0;
+  hex_fwd_lines<HB, G>(ha, v, chunk, img + (size_t)blockIdx.y * G * g.nx * g.ny, wv, W, blockIdx.z, gridDim.z, acc);
+#pragma unroll
+  for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
+  __syncthreads();
+  const int u = chunk * 64 + lane;
+  if (u >= g.nu) return;
+  fwd_group_store<G, W>(g, sp, rep, v, u, m, batch, red, g.dx, g.dy, 1.0, sino, gridDim.z > 1 ? part : nullptr);
+}
+
+// Interleaved copies of the lattices of one launch (interleave_kernel on the
+// hexagonal lattice: a mirror maps the points of an odd row among its nc - 1).
+template <int G>
+__global__ __launch_bounds__(256) void hex_interleave_kernel(SymPlan sp, int nx, int ny, int m, int batch,
+                                                             const float* __restrict__ img, float* __restrict__ rows) {
+  const size_t npix = (size_t)nx * ny;
+  const int img0 = blockIdx.z * m, nslot = sp.nh * min(m, batch - img0);
+  const int ix = blockIdx.x * 16 + (threadIdx.x & 15), iy = blockIdx.y * 16 + (threadIdx.x >> 4);
+  if (ix >= nx || iy >= ny) return;
+  float x[G];
+#pragma unroll
+  for (int s = 0; s < G; ++s) {
+    x[s] = 0.0f;
+    if (s < nslot) {
+      const int k = s >> sp.lg, h = s & (sp.nh - 1);
+      int qx, qy;
+      SymOp::hex_point(sp.op[h], nx, ny, ix, iy, &qx, &qy);
+      x[s] = img[(img0 + k) * npix + (size_t)qy * nx + qx];
+    }
+  }
+  rows += blockIdx.z * npix * G;
+  __builtin_memcpy(__builtin_assume_aligned(rows + ((size_t)iy * nx + ix) * G, G < 4 ? 4 * G : 16), x, sizeof(x));
+}
+
+// Box that holds the footprints of a 16 x 16 point tile: its centre relative
+// to point (0, 0) of the tile and its half extents (one circumradius and the
+// half-column shift of odd rows around the points).
+__host__ __device__ inline void hex_tile_box(const HexArgs& a, double* cx, double* cy, double* hx, double* hy) {
+  *cx = 0.5 * kTile * a.g.dx;
+  *cy = 0.5 * (kTile - 1) * a.g.dy;
+  *hx = (0.5 * kTile + 0.5) * a.g.dx + a.dt;
+  *hy = 0.5 * (kTile + 1) * a.g.dy + a.dt;
+}
+
+// A^T in the grouped frame (group2d_dev.hpp).
+template <int HB> struct HexBwd {
+  using Args = HexArgs;
+  using T = HexTraits<HB>;
+  using Bin = typename T::Bin;
+  static constexpr int kRec = sizeof(Bin) / 16;
+  static_assert(sizeof(Bin) % 16 == 0, "bin records are whole float4s");
+  struct Pixel {
+    double fx, fy;
+  };
+  __device__ static __forceinline__ const Proj2DArgs& geo(const Args& a) { return a.g; }
+  __device__ static __forceinline__ void window(const Args& a, const ViewGeo& vg, int ix0, int iy0, int* lo, int* n,
+                                                int cap) {
+    double cx, cy, hx, hy, umin = 1e300, umax = -1e300;
+    hex_tile_box(a, &cx, &cy, &hx, &hy);
+#pragma unroll 1
+    for (int c = 0; c < 4; ++c) {
+      const double wx = ix0 * a.g.dx + cx + ((c & 1) ? hx : -hx) + vg.w0x;
+      const double wy = iy0 * a.g.dy + cy + ((c & 2) ? hy : -hy) + vg.w0y;
+      const double uu = -(vg.e0x * wy - vg.e0y * wx) / (vg.pux * wy - vg.puy * wx);
+      umin = fmin(umin, uu);
+      umax = fmax(umax, uu);
+    }
+    const int l = (int)fmax(floor(umin) - 1.0, 0.0), h = (int)fmin(floor(umax) + 1.0, (double)(a.g.nu - 1));
+    *lo = l;
+    *n = h >= l ? min(h - l + 1, cap) : 0;
+  }
+  __device__ static __forceinline__ Pixel pixel(const Args& a, int ic, int il) {
+    return {(ic + ((il & 1) ? 0.5 : 0.0)) * a.g.dx, il * a.g.dy};
+  }
+  __device__ static __forceinline__ bool active(const Args& a, int ic, int il) {
+    return !((il & 1) && ic == a.g.nx - 1);
+  }
+  __device__ static __forceinline__ void image(const Args& a, int op, int ic, int il, int* qx, int* qy) {
+    SymOp::hex_point(op, a.g.nx, a.g.ny, ic, il, qx, qy);
+  }
+  __device__ static __forceinline__ float value(const float4 (&)[kRec], float y) { return y; }
+  __device__ static __forceinline__ double result(const Args& a, double acc) { return acc * a.g.dx * a.g.dy; }
+
+  template <int G>
+  __device__ static __forceinline__ void view(const Args& a, const ViewGeo& vg, const Pixel& p,
+                                              const Staged<kRec, G>& st, int base, int wlo, int wn, float (&accv)[G]) {
+    const double wx = p.fx + vg.w0x, wy = p.fy + vg.w0y;
+    const double n0 = vg.e0x * wy - vg.e0y * wx;
+    const double be = vg.pux * wy - vg.puy * wx;
+    const float bef = (float)be;
+    // bin range in FP32 (it only bounds the bins visited; a bin gained or
+    // lost at a rounding boundary carries a vanishing footprint)
+    const float kc = -(float)n0 * __builtin_amdgcn_rcpf(bef);
+    // k*(vertex) - kc = -(d . G) / (beta + d . grad beta), G = grad N_0 + kc grad beta
+    const float gx = -__builtin_fmaf(kc, (float)vg.puy, (float)vg.e0y);
+    const float gy = __builtin_fmaf(kc, (float)vg.pux, (float)vg.e0x);
+    const float dt = (float)a.dt;
+    const float hw = hex_reach_f(gx, gy, dt) *
+                     __builtin_amdgcn_rcpf(__builtin_fabsf(bef) - hex_reach_f(-(float)vg.puy, (float)vg.pux, dt));
+    const float last = (float)(a.g.nu - 1);
+    const int ulo = max((int)fminf(fmaxf(floorf(kc - hw), 0.0f), last), wlo);
+    const int uhi = min((int)fminf(fmaxf(floorf(kc + hw), 0.0f), last), wlo + wn - 1);
+    float na = (float)(n0 + (double)ulo * be);
+    for (int u = ulo; u <= uhi; ++u) {
+      const int at = base + u - wlo;
+      float4 rd[kRec];
+      st.record(at, rd);
+      const Bin rec = __builtin_bit_cast(Bin, rd);
+      const float nb = na + bef;
+      st.add(at, T::conv(rec, rec.ka * na, rec.kb * nb), accv);
+      na = nb;
+    }
+  }
+};
+
+// Launched as bwd_group_kernel; bound by the LDS reads of the records (80 bytes
+// per footprint for H0) and VALU issue.  Same cases as hex_fwd_kernel: 728 ->
+// 437 us, 33.2 -> 5.5 ms, 39 -> 14 us.
+template <int HB, int G>
+__global__ __launch_bounds__(256) void hex_bwd_group_kernel(HexArgs ha, SymPlan sp, int m, int batch,
+                                                            const float* __restrict__ sino, float* __restrict__ img,
+                                                            int vpg, int nvc, int win, double* __restrict__ part) {
+  bwd_group_block<HexBwd<HB>, G>(ha, sp, m, batch, sino, img, vpg, nvc, win, part);
 }
 
 constexpr int kHexH0Window = 72;
 
-// A^T: lattice-point-driven gather, 16 x 16 point tiles, LDS bin windows.
+// A^T where the tiles' bin windows are too wide for the grouped frame's LDS:
+// lattice-point-driven gather, 16 x 16 point tiles, LDS bin windows.
 // grid (tiles, tiles, batch * ngroup), H0's blocks mapped by xcd_block: z =
 // b * ngroup + k takes views
 // [k vpg, (k+1) vpg); with ngroup > 1 it writes its FP64 sum to
@@ -569,30 +603,110 @@ void hex_bin_constants(int basis, const ViewGeo& v, int nu, double dt, void* out
 
 size_t hex_bin_size(int basis) { return basis == BASIS_H0 ? sizeof(H0Bin) : sizeof(HlBin); }
 
-// nseg > 1 needs part with nseg * batch * np * nu doubles.
-hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const float* img, float* sino, int batch,
-                              int nseg, double* part, hipStream_t s) {
-  if (nseg < 1 || (nseg > 1 && !part)) return hipErrorInvalidValue;
-  HexArgs ha{g, dt};
-  const int waves = g.np * g.nchunk;
-  if (basis == BASIS_H0)
-    hex_fwd_kernel<BASIS_H0, false><<<dim3((waves + 3) / 4, batch, nseg), dim3(256), 0, s>>>(ha, img, sino, part);
-  else
-    hex_fwd_kernel<BASIS_HL, true><<<dim3((waves + 3) / 4, batch, nseg), dim3(256), 0, s>>>(ha, img, sino, part);
-  if (nseg > 1) return launch_sum_parts(part, sino, (size_t)batch * g.np * g.nu, nseg, s);
+// Bins per view that hold every tile's window (host-side).
+int hex_tile_window(const Proj2DArgs& g, double dt, const ViewGeo* views) {
+  const HexArgs a{g, dt};
+  double cx, cy, hx, hy;
+  hex_tile_box(a, &cx, &cy, &hx, &hy);
+  return window_bound(g, views, cx, cy, hx, hy);
+}
+
+namespace {
+template <int HB, int G, int W>
+hipError_t hex_forward_g(const HexArgs& ha, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  const Proj2DArgs& g = ha.g;
+  if (r.rows)
+    hex_interleave_kernel<G><<<dim3((unsigned)(g.nx + 15) / 16, (unsigned)(g.ny + 15) / 16, (unsigned)r.groups()), 256,
+                               0, s>>>(r.sym, g.nx, g.ny, r.m, r.batch, img, r.rows);
+  const dim3 grid((unsigned)(r.sym.nrep * g.nchunk), (unsigned)r.groups(), (unsigned)r.split);
+  hex_fwd_kernel<HB, G, W><<<grid, 64 * W, 0, s>>>(ha, r.sym, r.m, r.batch, r.rows ? r.rows : img, sino, r.part);
   return hipGetLastError();
 }
 
-hipError_t launch_hex_backward(int basis, const Proj2DArgs& g, double dt, const float* sino, float* img, int batch,
-                               int ngroup, double* part, hipStream_t s) {
-  if (ngroup < 1 || (ngroup > 1 && !part)) return hipErrorInvalidValue;
-  HexArgs ha{g, dt};
-  const int vpg = (g.np + ngroup - 1) / ngroup;
-  dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, batch * ngroup), block(256);
-  if (basis == BASIS_H0) hex_bwd_kernel<BASIS_H0><<<grid, block, 0, s>>>(ha, sino, img, ngroup, vpg, part);
-  else hex_bwd_kernel<BASIS_HL><<<grid, block, 0, s>>>(ha, sino, img, ngroup, vpg, part);
-  if (ngroup > 1) return launch_sum_parts(part, img, (size_t)batch * g.nx * g.ny, ngroup, s);
+template <int HB, int G>
+hipError_t hex_backward_g(const HexArgs& ha, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  const dim3 grid((unsigned)r.sym.ntile, (unsigned)r.split, (unsigned)r.groups());
+  const size_t lds = (size_t)r.nvc * r.win * (16 * HexBwd<HB>::kRec + 4 * G);
+  hex_bwd_group_kernel<HB, G><<<grid, 256, lds, s>>>(ha, r.sym, r.m, r.batch, sino, img, r.vpg, r.nvc, r.win, r.part);
   return hipGetLastError();
+}
+
+// Waves per (view, chunk): as many as a launch of one image needs to fill the
+// GPU, since every wave repeats a strip's set-up and shortens its lines.  A at
+// 8 / 4 / 2 waves, us: H0 128 x 147, 360 views (1448 workgroups) 52 / 62 / 94;
+// H0 256 x 296, 1024 views (8208) 543 / 496 / 476, batch 16 2398 / 2164 / 1963;
+// Hl, batch 64 8525 / 7805 / 7107, one image without symmetries (16368) 738 /
+// 619 / 570.  The choice follows the handle, not the batch, so that an image's
+// sums associate alike in every batch.
+int hex_waves(const Proj2DArgs& g, const GroupRun& r) {
+  const long long n = (long long)r.sym.nrep * g.nchunk;
+  return r.lone ? 1 : (n < 2048 ? 8 : (n < 6000 ? 4 : 2));
+}
+
+template <int HB, int G>
+hipError_t hex_forward_w(const HexArgs& ha, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  switch (hex_waves(ha.g, r)) {
+    case 8: return hex_forward_g<HB, G, 8>(ha, r, img, sino, s);
+    case 4: return hex_forward_g<HB, G, 4>(ha, r, img, sino, s);
+    case 2: return hex_forward_g<HB, G, 2>(ha, r, img, sino, s);
+    default: return hex_forward_g<HB, 1, 1>(ha, r, img, sino, s);  // lone: one value per point
+  }
+}
+
+template <int HB>
+hipError_t hex_forward_b(const HexArgs& ha, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
+  if (r.lone && r.g != 1) return hipErrorInvalidValue;
+  switch (r.g) {
+    case 1: return hex_forward_w<HB, 1>(ha, r, img, sino, s);
+    case 2: return hex_forward_w<HB, 2>(ha, r, img, sino, s);
+    case 4: return hex_forward_w<HB, 4>(ha, r, img, sino, s);
+    case 8: return hex_forward_w<HB, 8>(ha, r, img, sino, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int HB>
+hipError_t hex_backward_b(const HexArgs& ha, const GroupRun& r, const float* sino, float* img, hipStream_t s) {
+  switch (r.g) {
+    case 1: return hex_backward_g<HB, 1>(ha, r, sino, img, s);
+    case 2: return hex_backward_g<HB, 2>(ha, r, sino, img, s);
+    case 4: return hex_backward_g<HB, 4>(ha, r, sino, img, s);
+    case 8: return hex_backward_g<HB, 8>(ha, r, sino, img, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+}  // namespace
+
+// r.split > 1 needs r.part with split * batch * np * nu doubles.
+hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const GroupRun& r, const float* img,
+                              float* sino, hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  const HexArgs ha{g, dt};
+  const hipError_t e = basis == BASIS_H0 ? hex_forward_b<BASIS_H0>(ha, r, img, sino, s)
+                                         : hex_forward_b<BASIS_HL>(ha, r, img, sino, s);
+  if (e == hipSuccess && r.split > 1)
+    return launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
+  return e;
+}
+
+// r.split > 1 needs r.part with split * batch * nc * nl doubles.
+hipError_t launch_hex_backward(int basis, const Proj2DArgs& g, double dt, const GroupRun& r, const float* sino,
+                               float* img, hipStream_t s) {
+  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  const HexArgs ha{g, dt};
+  hipError_t e;
+  if (r.win > 0) {
+    e = basis == BASIS_H0 ? hex_backward_b<BASIS_H0>(ha, r, sino, img, s)
+                          : hex_backward_b<BASIS_HL>(ha, r, sino, img, s);
+  } else {
+    if (r.sym.nh != 1) return hipErrorInvalidValue;
+    const dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, (unsigned)(r.batch * r.split));
+    if (basis == BASIS_H0) hex_bwd_kernel<BASIS_H0><<<grid, 256, 0, s>>>(ha, sino, img, r.split, r.vpg, r.part);
+    else hex_bwd_kernel<BASIS_HL><<<grid, 256, 0, s>>>(ha, sino, img, r.split, r.vpg, r.part);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, img, (size_t)r.batch * g.nx * g.ny, r.split, s);
+  return e;
 }
 
 // Explicit system matrix (h0_matrix_generation / hl_matrix_generation; the

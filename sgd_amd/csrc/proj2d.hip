@@ -27,6 +27,7 @@
 #include <cstdint>
 
 #include "proj2d_dev.hpp"
+#include "symmetry.hpp"
 
 namespace sgdct {
 
@@ -46,13 +47,12 @@ hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts
 // 202 us (one workgroup per CU).  Column walks read the transposed copy, so
 // that both walks read consecutive pixels (512 x 512, 721 views without
 // symmetries, read in place 947 us, with the copy 782 us).
-template <int BASIS, int G>
-__global__ __launch_bounds__(64 * kFwdWaves) void fwd_group_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
-                                                                   const float* __restrict__ rows_img,
-                                                                   const float* __restrict__ cols_img,
-                                                                   float* __restrict__ sino,
-                                                                   double* __restrict__ part) {
-  __shared__ double red[kFwdWaves][G][64];
+template <int BASIS, int G, int W>
+__global__ __launch_bounds__(64 * W) void fwd_group_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                           const float* __restrict__ rows_img,
+                                                           const float* __restrict__ cols_img,
+                                                           float* __restrict__ sino, double* __restrict__ part) {
+  __shared__ double red[W][G][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
   const int chunk = centre_out(rank, g.nchunk);
@@ -62,15 +62,15 @@ __global__ __launch_bounds__(64 * kFwdWaves) void fwd_group_kernel(Proj2DArgs g,
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
   fwd_bin_lines<BASIS, G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr,
-                          wv, kFwdWaves, blockIdx.z, gridDim.z, acc);
+                          wv, W, blockIdx.z, gridDim.z, acc);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
   const int u = chunk * 64 + lane;
   if (u >= g.nu) return;
   const typename Traits<BASIS>::Bin* bins = reinterpret_cast<const typename Traits<BASIS>::Bin*>(g.bins);
-  fwd_group_store<G>(g, sp, rep, v, u, m, batch, red, g.dx * g.dy * Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]),
-                     sino, gridDim.z > 1 ? part : nullptr);
+  fwd_group_store<G, W>(g, sp, rep, v, u, m, batch, red, g.dx, g.dy,
+                        Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]), sino, gridDim.z > 1 ? part : nullptr);
 }
 
 // Interleaved copies of the images of one launch: slot s = image * nh + h of
@@ -119,33 +119,11 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const double* __restrict
 
 
 // Bin window that holds every tile's window over all views (host-side, on the
-// host copy of the view table).  A point d away from a tile's centre projects
-// to kc - (d . G) / (beta + d . grad beta), G = grad N_0 + kc grad beta, kc
-// the centre's projection.  Over the image, kc is extreme at the corner tiles
-// (a projective map), |G| at extreme kc, and beta, affine, at the corners; so
-// four tiles per view bound every tile's window.  Where that bound is above
-// `enough`, every tile is looked at.
+// host copy of the view table): the bound from the corner tiles, or, where
+// that is above `enough`, every tile looked at.
 int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough) {
-  const int tx = (g.nx + kTile - 1) / kTile, ty = (g.ny + kTile - 1) / kTile;
-  const double r = 0.5 * (kTile - 1) + (double)g.h;
-  int w = 0;
-  for (int v = 0; v < g.np; ++v) {
-    const ViewGeo& vg = views_host[v];
-    double top = 0.0, room = 1e300;
-    for (int c = 0; c < 4; ++c) {
-      const double cx = ((c & 1) ? (tx - 1) * kTile : 0) + 0.5 * (kTile - 1);
-      const double cy = ((c & 2) ? (ty - 1) * kTile : 0) + 0.5 * (kTile - 1);
-      const double wx = cx * g.dx + vg.w0x, wy = cy * g.dy + vg.w0y;
-      const double be = vg.pux * wy - vg.puy * wx;
-      const double kc = -(vg.e0x * wy - vg.e0y * wx) / be;
-      top = fmax(top, fabs(vg.gx0 + kc * vg.gx1) + fabs(vg.gy0 + kc * vg.gy1));
-      // beta < 0 in front of the source
-      room = fmin(room, -be - r * (fabs((double)vg.gx1) + fabs((double)vg.gy1)));
-    }
-    // floor(kc + hw) - floor(kc - hw) <= 2 hw + 1, the window's margins 2 more
-    const double n = room > 0.0 ? floor(2.0 * r * top / room) + 4.0 : 1e9;
-    w = n < g.nu ? ((int)n > w ? (int)n : w) : g.nu;
-  }
+  const double half = 0.5 * (kTile - 1), r = half + (double)g.h;
+  int w = window_bound(g, views_host, half * g.dx, half * g.dy, r * g.dx, r * g.dy);
   if (w <= enough) return w;
   w = 0;
   for (int v = 0; v < g.np; ++v)
@@ -234,10 +212,10 @@ hipError_t interleave_g(const Proj2DArgs& g, const GroupRun& r, const float* img
   return hipGetLastError();
 }
 
-template <int BASIS, int G>
+template <int BASIS, int G, int W>
 hipError_t forward_g(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
   const float* rows = r.rows ? r.rows : img;
-  fwd_group_kernel<BASIS, G><<<grid3(r.sym.nrep * g.nchunk, r.groups(), r.split), 64 * kFwdWaves, 0, s>>>(
+  fwd_group_kernel<BASIS, G, W><<<grid3(r.sym.nrep * g.nchunk, r.groups(), r.split), 64 * W, 0, s>>>(
       g, r.sym, r.m, r.batch, rows, r.cols, sino, r.part);
   return hipGetLastError();
 }
@@ -253,10 +231,11 @@ hipError_t backward_g(const Proj2DArgs& g, const GroupRun& r, const float* sino,
 template <int BASIS>
 hipError_t forward_b(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
   switch (r.g) {
-    case 1: return forward_g<BASIS, 1>(g, r, img, sino, s);
-    case 2: return forward_g<BASIS, 2>(g, r, img, sino, s);
-    case 4: return forward_g<BASIS, 4>(g, r, img, sino, s);
-    case 8: return forward_g<BASIS, 8>(g, r, img, sino, s);
+    case 1:
+      return r.lone ? forward_g<BASIS, 1, 1>(g, r, img, sino, s) : forward_g<BASIS, 1, kFwdWaves>(g, r, img, sino, s);
+    case 2: return forward_g<BASIS, 2, kFwdWaves>(g, r, img, sino, s);
+    case 4: return forward_g<BASIS, 4, kFwdWaves>(g, r, img, sino, s);
+    case 8: return forward_g<BASIS, 8, kFwdWaves>(g, r, img, sino, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -27,12 +27,12 @@ hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float
 // symmetries 260 us; 1024 x 1024, 900 views 7.04 -> 1.13 ms; 256 x 256, 90
 // views, batch 5 266 -> 84 us; one value, 721 views from another start angle
 // 1455 -> 1420 us.
-template <int G>
-__global__ __launch_bounds__(64 * kFwdWaves) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
-                                                                const float* __restrict__ rows_img,
-                                                                const float* __restrict__ cols_img,
-                                                                float* __restrict__ sino, double* __restrict__ part) {
-  __shared__ double red[kFwdWaves][G][64];
+template <int G, int W>
+__global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
+                                                        const float* __restrict__ rows_img,
+                                                        const float* __restrict__ cols_img, float* __restrict__ sino,
+                                                        double* __restrict__ part) {
+  __shared__ double red[W][G][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int rank = blockIdx.x / sp.nrep, rep = blockIdx.x - rank * sp.nrep;
   const int chunk = centre_out(rank, g.nchunk);
@@ -42,13 +42,13 @@ __global__ __launch_bounds__(64 * kFwdWaves) void sf_fwd_kernel(Proj2DArgs g, Sy
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
   sf_fwd_lines<G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr, wv,
-                  kFwdWaves, blockIdx.z, gridDim.z, acc);
+                  W, blockIdx.z, gridDim.z, acc);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
   const int u = chunk * 64 + lane;
   if (u >= g.nu) return;
-  fwd_group_store<G>(g, sp, rep, v, u, m, batch, red, 1.0, sino, gridDim.z > 1 ? part : nullptr);
+  fwd_group_store<G, W>(g, sp, rep, v, u, m, batch, red, 1.0, 1.0, 1.0, sino, gridDim.z > 1 ? part : nullptr);
 }
 
 // A^T, launched as bwd_group_kernel; same cases as above: 841 -> 175 us, 4.13
@@ -75,10 +75,10 @@ __global__ __launch_bounds__(256) void sf_bwd_wide_kernel(Proj2DArgs g, const fl
 }
 
 namespace {
-template <int G>
+template <int G, int W>
 hipError_t sf_forward_g(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
   const dim3 grid((unsigned)(r.sym.nrep * g.nchunk), (unsigned)r.groups(), (unsigned)r.split);
-  sf_fwd_kernel<G><<<grid, 64 * kFwdWaves, 0, s>>>(g, r.sym, r.m, r.batch, r.rows ? r.rows : img, r.cols, sino, r.part);
+  sf_fwd_kernel<G, W><<<grid, 64 * W, 0, s>>>(g, r.sym, r.m, r.batch, r.rows ? r.rows : img, r.cols, sino, r.part);
   return hipGetLastError();
 }
 
@@ -95,10 +95,11 @@ hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float
   if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
   hipError_t e = r.rows || r.cols ? launch_interleave(g, r, img, s) : hipSuccess;
   if (e != hipSuccess) return e;
-  if (r.g == 1) e = sf_forward_g<1>(g, r, img, sino, s);
-  else if (r.g == 2) e = sf_forward_g<2>(g, r, img, sino, s);
-  else if (r.g == 4) e = sf_forward_g<4>(g, r, img, sino, s);
-  else if (r.g == 8) e = sf_forward_g<8>(g, r, img, sino, s);
+  if (r.g == 1 && r.lone) e = sf_forward_g<1, 1>(g, r, img, sino, s);
+  else if (r.g == 1) e = sf_forward_g<1, kFwdWaves>(g, r, img, sino, s);
+  else if (r.g == 2) e = sf_forward_g<2, kFwdWaves>(g, r, img, sino, s);
+  else if (r.g == 4) e = sf_forward_g<4, kFwdWaves>(g, r, img, sino, s);
+  else if (r.g == 8) e = sf_forward_g<8, kFwdWaves>(g, r, img, sino, s);
   else return hipErrorInvalidValue;
   if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
   return e;

@@ -20,6 +20,34 @@ struct SymTables {
   int nh() const { return (int)op.size(); }
 };
 
+// Bins that hold the projection of every pixel tile's box in every view,
+// +-1 margin.  Tile (0, 0)'s box has its centre (cx, cy) from pixel (0, 0) and
+// half extents (hx, hy), the other tiles' lie kTile pixels apart.  A point d
+// away from a box's centre projects to kc - (d . G) / (beta + d . grad beta), G
+// = grad N_0 + kc grad beta, kc the centre's projection.  Over the image, kc is
+// extreme at the corner tiles (a projective map), |G| at extreme kc, and beta,
+// affine, at the corners; so four tiles per view bound every window.
+inline int window_bound(const Proj2DArgs& g, const ViewGeo* views, double cx, double cy, double hx, double hy) {
+  const int tx = (g.nx + kTile - 1) / kTile, ty = (g.ny + kTile - 1) / kTile;
+  int w = 0;
+  for (int v = 0; v < g.np; ++v) {
+    const ViewGeo& vg = views[v];
+    double top = 0.0, room = 1e300;
+    for (int c = 0; c < 4; ++c) {
+      const double wx = ((c & 1) ? (tx - 1) * kTile : 0) * g.dx + cx + vg.w0x;
+      const double wy = ((c & 2) ? (ty - 1) * kTile : 0) * g.dy + cy + vg.w0y;
+      const double be = vg.pux * wy - vg.puy * wx;  // < 0 in front of the source
+      const double kc = -(vg.e0x * wy - vg.e0y * wx) / be;
+      top = std::max(top, hx * std::fabs(vg.e0y + kc * vg.puy) + hy * std::fabs(vg.e0x + kc * vg.pux));
+      room = std::min(room, -be - (hx * std::fabs(vg.puy) + hy * std::fabs(vg.pux)));
+    }
+    // floor(kc + hw) - floor(kc - hw) <= 2 hw + 1, the window's margins 2 more
+    const double n = room > 0.0 ? std::floor(2.0 * top / room) + 4.0 : 1e9;
+    w = n < g.nu ? std::max(w, (int)n) : g.nu;
+  }
+  return w;
+}
+
 // Views per symmetry op: perm[v] is the view op maps v onto, empty if some
 // view has no partner.  Source, first edge ray and detector step have to
 // agree within tol (the FP64 rounding of the angles); every view is the
@@ -63,9 +91,9 @@ inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int 
 // The symmetries of a scan of nx x ny pixels, at most `most` of them: the
 // group of every grid symmetry that permutes the views, or its subgroup
 // without axis swaps, or that subgroup's first element of order two.
-// `allowed` has a bit for each op the grid admits.
+// `allowed` has a bit for each op the grid admits; hex: a hexagonal lattice.
 inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int ny, int nu, unsigned allowed, int most,
-                                 double tol) {
+                                 double tol, bool hex = false) {
   SymTables t;
   const int np = (int)views.size();
   std::vector<int> perm[kMaxSym];
@@ -125,7 +153,8 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
         for (int x = i * kTile; x < x1; ++x)
           for (int h = 0; h < nh; ++h) {
             int qx, qy;
-            SymOp::pixel(found[h], nx, ny, x, y, &qx, &qy);
+            if (hex) SymOp::hex_point(found[h], nx, ny, x, y, &qx, &qy);
+            else SymOp::pixel(found[h], nx, ny, x, y, &qx, &qy);
             char& c = covered[(size_t)qy * nx + qx];
             if (c) continue;
             c = 1;

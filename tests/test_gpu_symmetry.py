@@ -5,8 +5,9 @@ Full-turn scans with 8, 4 and 2 symmetries (view counts 0 and 2 mod 4, odd;
 square and rectangular images, odd sizes; other start angles; alternating
 source radius) and without any, against the FP64 oracle at the projector's
 parity bar (1e-5 relative L2); a batch of 1..9 images is bit for bit the
-images by themselves.  The view counts are high enough that the symmetries
-are used (256 workgroups of a view and 64 bins)."""
+images by themselves.  The hexagonal lattices likewise.  The view counts are
+high enough that the symmetries are used (256 workgroups of a view and 64
+bins)."""
 import numpy as np
 import pytest
 
@@ -57,3 +58,65 @@ def test_grouped_matches_oracle(cuda, oracle_exact, basis, name):
     for b in (1, 2, 3, 4, 5, 8):
         assert torch.equal(P.forward(xt[:b].contiguous()), ax[:b]), b
         assert torch.equal(P.backward(yt[:b].contiguous()), aty[:b]), b
+
+
+HEX = {
+    "4 symmetries, odd rows": dict(nl=33, nc=20, views=1030, nu=70),
+    "2, even rows": dict(nl=24, nc=19, views=1028, nu=63),
+    "2, odd views": dict(nl=21, nc=18, views=521, nu=75),
+    "1": dict(nl=22, nc=17, views=300, nu=60, start=0.2),
+    "1, many workgroups": dict(nl=9, nc=8, views=3000, nu=140, start=0.2),
+    "2, most workgroups": dict(nl=10, nc=9, views=6200, nu=130),
+}
+
+
+@pytest.mark.parametrize("basis", ["H0", "Hl"])
+@pytest.mark.parametrize("name", list(HEX))
+def test_grouped_hex_matches_oracle(cuda, oracle_exact, basis, name):
+    import torch
+    from pyoracle import HexGeometry
+    from sgd_amd.torch_ops import Projector
+    c = HEX[name]
+    n, nl, nc = c["views"], c["nl"], c["nc"]
+    ang = c.get("start", 0.0) + 2 * np.pi * np.arange(n) / n
+    geo = (nl, nc, ang, c["nu"], 1.3, 1.1, 1000.0, 500.3)
+    P = Projector.hexagonal(basis, *geo)
+    G = HexGeometry(oracle_exact, *geo)
+    print(basis, name, c, flush=True)
+    rng = np.random.default_rng(8)
+    x = rng.random((9, nl, nc)).astype(np.float32)
+    x[:, 1::2, -1] = 0.0
+    y = rng.standard_normal((9, n, c["nu"])).astype(np.float32)
+    xt, yt = torch.from_numpy(x).to(cuda), torch.from_numpy(y).to(cuda)
+    ax, aty = P.forward(xt), P.backward(yt)
+    torch.cuda.synchronize()
+    for k in (0, 8):
+        e1 = rel(ax[k].double().cpu().numpy(), G.forward(basis, x[k].astype(np.float64)))
+        e2 = rel(aty[k].double().cpu().numpy(), G.backward(basis, y[k].astype(np.float64)))
+        print("  image %d: A %.2e  A^T %.2e" % (k, e1, e2), flush=True)
+        assert e1 <= 1e-5 and e2 <= 1e-5, (k, e1, e2)
+    assert (aty[:, 1::2, -1] == 0).all()
+    for b in (1, 2, 3, 5, 8):
+        assert torch.equal(P.forward(xt[:b].contiguous()), ax[:b]), b
+        assert torch.equal(P.backward(yt[:b].contiguous()), aty[:b]), b
+
+
+def test_hex_forward_on_two_streams(cuda):
+    """One handle's A on two streams at once (each has its own interleaved
+    lattice) equals the calls one after the other."""
+    import torch
+    from sgd_amd.torch_ops import Projector
+    ang = 2 * np.pi * np.arange(1024) / 1024
+    P = Projector.hexagonal("Hl", 80, 64, ang, 256, 1.0, 1.2, 1000.0, 500.0)
+    g = torch.Generator(device=cuda).manual_seed(3)
+    xs = [torch.randn((8,) + P.img_shape, device=cuda, generator=g) for _ in range(6)]
+    ref = [P.forward(x) for x in xs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for k, x in enumerate(xs):
+        with torch.cuda.stream(streams[k % 2]):
+            outs.append(P.forward(x))
+    torch.cuda.synchronize()
+    for a, b in zip(ref, outs):
+        assert torch.equal(a, b)
