@@ -187,17 +187,20 @@ int sgdct_project_dev_noalloc(sgdct_projector *h, int direction, const float *in
                               void *stream);
 
 /* Fan-beam launch shape (no reference counterpart).  A splits every bin's
- * pixel walk into `fwd_split` line segments (on hexagonal handles: segments of
- * the lattice rows, or of the vertical lattice lines a wave walks when its
- * strips are steep) and A^T the views into `bwd_split` groups, each writing
- * FP64 partial sums that a second kernel adds
- * in a fixed order (results are deterministic, independent of the batch size,
- * and agree across splits to FP64 rounding).  0 = automatic: chosen at
- * creation from one image's launch size (a launch of few waves splits, up to
- * 24 ways; hexagonal A stays unsplit); 1..32 = fixed.  The partial-sum workspace (2 images per launch,
- * or up to 16 while it stays within 64 MiB; larger batches take several
- * launches) is allocated at creation and by this call, never inside a
- * projection.  Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
+ * pixel walk into `fwd_split` line segments (eight of them, where there are as
+ * many, the waves of a workgroup, the others grid segments where those pay; on
+ * hexagonal handles grid segments of the lattice rows, or of the vertical
+ * lattice lines a wave walks when its strips are steep) and A^T the views into
+ * `bwd_split` groups.  Grid segments and groups write FP64 partial sums that a
+ * second kernel adds in a fixed order (results are deterministic, independent
+ * of the batch size, and agree across splits to FP64 rounding).  0 =
+ * automatic: chosen at creation from one image's launch size (24 segments;
+ * hexagonal A stays unsplit); 1..32 = fixed.  The workspace (partial sums,
+ * interleaved images of A; more images per launch while it stays within 64
+ * MiB, larger batches take several launches) is allocated at creation and by
+ * this call, never inside a projection on the handle's stream (a hexagonal
+ * handle's A takes one interleaved lattice for each stream it is called on, up
+ * to four, and runs without one on others and under capture).  Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
 int sgdct_split_config(sgdct_projector *h, int fwd_split, int bwd_split);
 
 /* Shape query: out[0..3] = nx, ny, np, nu (hexagonal: nc, nl, np, nu);
@@ -239,8 +242,9 @@ int sgdct_tv_descent(float *x, float *g, double *work, const double *step, int n
 
 /* ---- batched slices (no reference counterpart: the reference projects one
  * slice per call and launches one kernel per view, layers/A_B1.cu:512-541) --
- * Many B0 / B1 / SF projectors of uneven size, view count and basis run as
- * one persistent launch per direction over a device work queue (A: 64-bin
+ * Many B0 / B1 / SF projectors of uneven size, view count and basis in one
+ * call: one launch per slice (see sgdct_batch_config), or one persistent
+ * launch per direction over a device work queue (A: 64-bin
  * waves of one view, A^T: 16x16 pixel tiles), slices ordered by decreasing
  * per-item cost.  Results equal the per-projector entry points to one FP32
  * rounding per element (those may split a walk or the views into FP64
@@ -254,9 +258,11 @@ sgdct_batch *sgdct_batch_create(sgdct_projector *const *slices, int nslice);
 void sgdct_batch_destroy(sgdct_batch *b);
 int sgdct_batch_layout(const sgdct_batch *b, long long *img_off, long long *sino_off);
 /* Launch shape: persistent blocks per CU for A and A^T (1..32, or 0 for one
- * launch per slice through the slices' own projector kernels and workspaces)
- * and slice order of the persistent queue (0: decreasing per-item cost, 1: as
- * given); set by the autotuner.  Defaults: 8, 8, 0. */
+ * launch per slice through the slices' own projector kernels, on the batch's
+ * workspace) and slice order of the persistent queue (0: decreasing per-item
+ * cost, 1: as given); set by the autotuner.  Until then each direction runs
+ * one launch per slice, or, for more than 16 small slices, the persistent
+ * queue at 8 blocks per CU, order 0. */
 int sgdct_batch_config(sgdct_batch *b, int fwd_blocks_per_cu, int bwd_blocks_per_cu, int order);
 int sgdct_batch_forward(sgdct_batch *b, const float *img, float *sino, void *stream);
 int sgdct_batch_backward(sgdct_batch *b, const float *sino, float *img, void *stream);

@@ -87,6 +87,8 @@ class SliceBatch:
         _lib.check(L.sgdct_batch_layout(h, io, so), "batch layout")
         self.img_off, self.sino_off = list(io), list(so)
         self.device = self.projectors[0].device
+        # the persistent shape, used where the batch's own choice (one launch
+        # per slice, or the persistent queue) is the queue
         self.config = (8, 8, 0)
 
     def close(self):

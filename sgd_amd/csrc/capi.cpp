@@ -253,10 +253,13 @@ struct sgdct_batch {
   unsigned int* d_counters = nullptr;
   BatchPlan plan{};
   // Persistent blocks per CU of A and A^T; 0 = one launch per slice (each
-  // projector's own split kernels).  Defaults: the autotuner's persistent
-  // choice on 256 uneven slices (A^T at 8 blocks per CU: 165.5 ms against
-  // 200.8 ms at 4).
+  // projector's own split kernels, on the batch's workspace d_part).  Until
+  // sgdct_batch_config sets them they follow auto_blocks; 8 is the autotuner's
+  // persistent choice on 256 uneven slices (A^T at 8 blocks per CU: 165.5 ms
+  // against 200.8 ms at 4).
   int fwd_bpc = 8, bwd_bpc = 8, order = 0;
+  double* d_part = nullptr;
+  size_t part_cap = 0;
   struct Graph {
     hipGraphExec_t exec = nullptr;
     const void* in = nullptr;
@@ -275,6 +278,7 @@ struct sgdct_batch {
     if (d_order) (void)hipFree(d_order);
     if (d_prefix) (void)hipFree(d_prefix);
     if (d_counters) (void)hipFree(d_counters);
+    if (d_part) (void)hipFree(d_part);
   }
 };
 
@@ -1180,13 +1184,47 @@ int batch_upload_plan(sgdct_batch* b) {
   return SGDCT_OK;
 }
 
+// Workspace that the slices' launches need one after the other.
+int batch_workspace(sgdct_batch* b) {
+  size_t need = 0;
+  for (const sgdct_projector* h : b->proj) need = std::max(need, work_doubles(h));
+  if (need == 0) return SGDCT_OK;
+  const hipError_t e = hipMalloc(&b->d_part, need * sizeof(double));
+  if (e != hipSuccess) return hip_fail(e, "batch workspace");
+  b->part_cap = need;
+  return SGDCT_OK;
+}
+
+// Launches of a batch that nobody has configured: one per slice, which splits
+// and shares footprints, unless many small slices make the launches' own time
+// the larger part (then the persistent queue, 8 blocks per CU).  A / A^T,
+// per-slice against persistent, us: 8 slices of 64^2, 60 views 78 / 100
+// against 178 / 116, of 256^2, 361 views 972 / 1096 against 1541 / 1289; 64
+// slices of 64^2 617 / 837 against 280 / 202, of 256^2 7.8 / 8.8 against 10.4 /
+// 8.3 ms; 16 helical slices of 128^2..768^2 13.3 / 12.2 against 18.2 / 12.8
+// ms; 5 slices with two symmetries each 3.4 / 3.2 against 8.0 / 5.6 ms.
+int auto_blocks(const sgdct_batch* b, int dir) {
+  if (b->n <= 16) return 0;
+  double items = 0.0, sym = 0.0;
+  for (int i = 0; i < b->n; ++i) {
+    items += (double)b->fwd_items[i] / b->n;
+    sym += (double)b->proj[i]->sym.nh / b->n;
+  }
+  return items * sym >= (dir == 0 ? 2000.0 : 4000.0) ? 0 : 8;
+}
+
 int batch_run(sgdct_batch* b, int dir, const float* in, float* out, hipStream_t s) {
   if ((dir == 0 ? b->fwd_bpc : b->bwd_bpc) == 0) {
-    // one launch per slice, in slice order, on the slices' own handles
+    // one launch per slice, in slice order, the slices' own splits
     for (int i = 0; i < b->n; ++i) {
       sgdct_projector* h = b->proj[i];
-      const int rc = dir == 0 ? run_forward(h, in + b->img_off[i], out + b->sino_off[i], 1, s)
-                              : run_backward(h, in + b->sino_off[i], out + b->img_off[i], 1, s);
+      // the batch's workspace, so that the slices' handles stay free for other
+      // callers; a split raised since the batch was made has its room there
+      const bool own = work_doubles(h) <= b->part_cap;
+      double* const part = own ? b->d_part : h->d_part;
+      const size_t cap = own ? b->part_cap : h->part_cap;
+      const int rc = dir == 0 ? group_forward(h, in + b->img_off[i], out + b->sino_off[i], 1, fwd_segments(h), part, cap, s)
+                              : group_backward(h, in + b->sino_off[i], out + b->img_off[i], 1, bwd_groups(h), part, cap, s);
       if (rc) return rc;
     }
     return SGDCT_OK;
@@ -1465,6 +1503,12 @@ sgdct_batch* sgdct_batch_create(sgdct_projector* const* slices, int nslice) {
     return nullptr;
   }
   if (batch_upload_plan(b) != SGDCT_OK) {
+    delete b;
+    return nullptr;
+  }
+  b->fwd_bpc = auto_blocks(b, 0);
+  b->bwd_bpc = auto_blocks(b, 1);
+  if (batch_workspace(b) != SGDCT_OK) {
     delete b;
     return nullptr;
   }
