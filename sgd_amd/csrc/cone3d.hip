@@ -53,10 +53,8 @@ namespace sgdct {
 // axial transpose in windows of kMaxNv.  Neither bounds nz or nv.
 constexpr int kMaxNz = 512;
 constexpr int kMaxNv = 512;
-// The in-plane kernels give each wave RCW chunks of 64 detector rows (a grid
-// dimension runs over the chunk groups): with RCW < nv / 64 more waves are in
-// flight on the row profiles, at the price of recomputing the in-plane weight
-// once per group.  RCW = kAllRows keeps every row in one wave (nv <= 512).
+// The in-plane kernels give each wave RCW chunks of 64 detector rows, at most
+// kAllRows (a grid dimension runs over the chunk groups).
 constexpr int kAllRows = 8;
 constexpr float kGammaEps = 1e-7f; // A_B1_3D.cu:300 skips gamma <= eps
 
@@ -289,11 +287,11 @@ __global__ __launch_bounds__(256) void axial_fwd_kernel(Cone3DArgs a, int p0, co
 }
 
 // ---------------------------------------------------------------------------
-// proj[p][j][u] = sum over the columns c of bin u's strip of conv(u, c) Y[c][j].
-// Wave per (view, bin); the strip walk is the 2-D B1 A kernel's with the bin
-// wave-uniform.  Grid: ceil(nu / 4) * nview blocks, view = blockIdx % nview
-// (consecutive blocks, which the dispatcher spreads over the XCDs, take
-// different views; the blocks of one view share an XCD's L2 when nview is 8).
+// In-plane kernels.  Their weights do not depend on the detector row, so lanes
+// cover the rows (RCW chunks of 64 per wave) where row profiles are read and
+// added up, and pairs (column, bin) where the weights are evaluated: one
+// evaluation gives up to 64 weights, which the row loop then reads lane by
+// lane into scalar registers.
 // ---------------------------------------------------------------------------
 // SF in-plane weight of cell u for pixel (ix, iy): area of the pixel's unit
 // trapezoid over the cell times 2 / (sum of its widths), from the corner
@@ -316,15 +314,45 @@ __device__ __forceinline__ float sf_cell_weight(const ViewGeo& vg, const Proj2DA
   return width > 0.0f ? gm * 2.0f / width : 0.0f;
 }
 
+// Lane `l`'s value, wave-uniform (l too).
+__device__ __forceinline__ float lane_value(float x, int l) {
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(x), l));
+}
+
+// min / max over each group of four lanes
+__device__ __forceinline__ int quad_min(int x) {
+  x = min(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xf, 0xf, true));   // lanes 1 0 3 2
+  return min(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xf, 0xf, true));  // lanes 2 3 0 1
+}
+__device__ __forceinline__ int quad_max(int x) {
+  x = max(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xf, 0xf, true));
+  return max(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xf, 0xf, true));
+}
+
+// proj[p][j][u] = sum over the columns c of bin u's strip of conv(u, c) Y[c][j].
+// A workgroup of four waves takes kFwdBins adjacent bins of one view; wave w
+// walks the lines m = w mod 4 of their strips (the 2-D A's walk), and the
+// waves' FP64 sums are added in wave order through LDS.  Per line the wave
+// finds the columns that its four strips cover together, requests the row
+// profiles of the first kFwdCols of them, and evaluates the weights meanwhile
+// (lane = 4 column + bin); a column's profile is read once for the bins it
+// touches, and a bin takes only columns of its own strip.  Grid: ceil(nu / 4) *
+// nview blocks, view = blockIdx % nview (consecutive blocks, which the
+// dispatcher spreads over the XCDs, take different views; the blocks of one
+// view share an XCD's L2 when nview is 8).
+constexpr int kFwdBins = 4, kFwdCols = 4;
+
 template <int M, int RCW>
 __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int nview, const float* __restrict__ Y,
                                                        float* __restrict__ proj) {
+  __shared__ double red[2][kFwdBins][RCW][64];
   const Proj2DArgs& g = a.g;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kc0 = blockIdx.y * RCW;  // this wave's detector-row chunks
-  const int pl = blockIdx.x % nview;
-  const int u = (blockIdx.x / nview) * 4 + wv;
-  if (u >= g.nu) return;
+  const int pl = blockIdx.x % nview, u0 = (blockIdx.x / nview) * kFwdBins;
+  const int lb = lane & (kFwdBins - 1), lt = lane / kFwdBins;  // this lane's bin and column of a weight evaluation
+  const bool live = u0 + lb < g.nu;
+  const int u = live ? u0 + lb : g.nu - 1;
   const int v = p0 + pl;
   const int ncol = g.nx * g.ny;
   const ViewGeo vg = g.views[v];
@@ -333,7 +361,9 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
 
   const double eax = vg.e0x + u * vg.pux, eay = vg.e0y + u * vg.puy;
   const double ebx = eax + vg.pux, eby = eay + vg.puy;
-  const double mx = eax + 0.5 * vg.pux, my = eay + 0.5 * vg.puy;
+  // walk direction from the bins' middle ray (uniform over the workgroup)
+  const double um = u0 + 0.5 * min(kFwdBins, g.nu - u0);
+  const double mx = vg.e0x + um * vg.pux, my = vg.e0y + um * vg.puy;
   const bool rows = fabs(my) >= fabs(mx);
   const double acx = -eay * g.dx, acy = eax * g.dy, ac0 = eax * vg.w0y - eay * vg.w0x;
   const double bcx = -eby * g.dx, bcy = ebx * g.dy, bc0 = ebx * vg.w0y - eby * vg.w0x;
@@ -352,7 +382,6 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
   const double sr = rows ? rcx : rcy, mr = rows ? rcy : rcx;
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
   const int smin = rows ? 1 : g.nx, smaj = rows ? g.nx : 1;
-  const float dta = (float)(rec.ka * sa), dtb = (float)(rec.kb * sb);
 
   int m_lo = 0, m_hi = nmaj - 1;
   if (mq != 0.0 && mr != 0.0) {
@@ -360,9 +389,10 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
     double c1 = (-ra - qc0) / mq, c2 = (-ra - qc0 - sq * last) / mq;
     double c3 = (rb - rc0) / mr, c4 = (rb - rc0 - sr * last) / mr;
     double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    m_lo = (int)fmax(floor(lo) - 1.0, 0.0);
-    m_hi = (int)fmin(ceil(hi) + 1.0, (double)(nmaj - 1));
+    m_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
+    m_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
   }
+  if (!live) m_lo = nmaj, m_hi = -1;
   double lo0 = 0.0, lo1 = 0.0, hi0 = nmin - 1, hi1 = 0.0;
   if (sq > 0.0 && sr > 0.0) {
     lo0 = (-ra - qc0) / sq; lo1 = -mq / sq; hi0 = (rb - rc0) / sr; hi1 = -mr / sr;
@@ -371,96 +401,121 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
   }
   const double an = (double)rec.ka * sa, am = (double)rec.ka * ma, a0 = (double)rec.ka * ac0;
   const double bn = (double)rec.kb * sb, bm = (double)rec.kb * mb, b0 = (double)rec.kb * bc0;
+  const int b_lo = __builtin_amdgcn_readfirstlane(quad_min(m_lo)), b_hi = __builtin_amdgcn_readfirstlane(quad_max(m_hi));
 
-  double acc[RCW];
+  double acc[kFwdBins][RCW];
 #pragma unroll
-  for (int k = 0; k < RCW; ++k) acc[k] = 0.0;
+  for (int b = 0; b < kFwdBins; ++b)
+#pragma unroll
+    for (int k = 0; k < RCW; ++k) acc[b][k] = 0.0;
   // Row-profile reads of a column: every lane loads (rows past nv read the
   // last row and are never stored), so the loads need no per-lane branch.
-  const float* ybase = Y + (size_t)pl * ncol * a.nv + kc0 * 64 + lane;
-  const int jmax = a.nv - 1 - kc0 * 64 - lane;  // offset of the last row
-  auto load_col = [&](int m, int n, float* y) {
-    const float* yc = ybase + (size_t)(m * smaj + n * smin) * a.nv;
+  const float* ybase = Y + (size_t)pl * ncol * a.nv;
+  int joff[RCW];
 #pragma unroll
-    for (int k = 0; k < RCW; ++k)
-      if ((kc0 + k) * 64 < a.nv) y[k] = yc[min(k * 64, jmax)];
-  };
-  // strip range of line m (empty when n0 > n1)
-  auto line_range = [&](int m, int& n0, int& n1) {
-    n0 = (int)fmax(ceil(fma((double)m, lo1, lo0)), 0.0);
-    n1 = (int)fmin(floor(fma((double)m, hi1, hi0)), (double)(nmin - 1));
-  };
-  // Lines are walked in order; within a line the next column's profile is
-  // loaded while the current column's weight is computed, and the last
-  // column of a line loads the first of the next line.
-  float ycur[RCW], ynext[RCW];
+  for (int k = 0; k < RCW; ++k) joff[k] = min((kc0 + k) * 64 + lane, a.nv - 1);
+  for (int m = b_lo + ((wv - b_lo) & 3); m <= b_hi; m += 4) {
+    // this lane's bin: columns [n0, n1] of line m
+    int n0 = (int)fmax(ceil(fma((double)m, lo1, lo0)), 0.0);
+    int n1 = (int)fmin(floor(fma((double)m, hi1, hi0)), (double)(nmin - 1));
+    if (m < m_lo || m > m_hi || n0 > n1) n0 = 0x7fffffff, n1 = -1;
+    const int c_lo = __builtin_amdgcn_readfirstlane(quad_min(n0)), c_hi = __builtin_amdgcn_readfirstlane(quad_max(n1));
+    if (c_lo > c_hi) continue;
+    float accl[kFwdBins][RCW];
 #pragma unroll
-  for (int k = 0; k < RCW; ++k) ycur[k] = ynext[k] = 0.0f;
-  int n0, n1;
-  // m_lo is not clamped from above: a strip that misses the volume has
-  // m_lo > m_hi and loads nothing
-  n0 = 0;
-  n1 = -1;
-  if (m_lo <= m_hi) line_range(m_lo, n0, n1);
-  if (n0 <= n1) load_col(m_lo, n0, ycur);
-  for (int m = m_lo; m <= m_hi; ++m) {
-    int q0 = 0, q1 = -1;  // next line's range
-    if (m < m_hi) line_range(m + 1, q0, q1);
-    if (n0 <= n1) {
-      float ta = (float)fma((double)n0, an, fma((double)m, am, a0));
-      float tb = (float)fma((double)n0, bn, fma((double)m, bm, b0));
-      float accl[RCW];
+    for (int b = 0; b < kFwdBins; ++b)
 #pragma unroll
-      for (int k = 0; k < RCW; ++k) accl[k] = 0.0f;
-      for (int n = n0; n <= n1; ++n) {
-        if (n < n1) load_col(m, n + 1, ynext);
-        else if (q0 <= q1) load_col(m + 1, q0, ynext);
-        float w;
-        if (M == CONE_B1) {
-          w = b1_mean(rec, ta, tb) * rec.scale;
-        } else {
-          const int ix = rows ? n : m, iy = rows ? m : n;
-          w = sf_cell_weight(vg, g, u, ix, iy);
-        }
+      for (int k = 0; k < RCW; ++k) accl[b][k] = 0.0f;
+    float w = 0.0f;
+    for (int c0 = c_lo; c0 <= c_hi; c0 += kFwdCols) {
+      float y[kFwdCols][RCW];
 #pragma unroll
-        for (int k = 0; k < RCW; ++k) {
-          accl[k] = __builtin_fmaf(w, ycur[k], accl[k]);
-          ycur[k] = ynext[k];
-        }
-        ta += dta;
-        tb += dtb;
+      for (int i = 0; i < kFwdCols; ++i) {
+        const float* yc = ybase + (size_t)(m * smaj + min(c0 + i, c_hi) * smin) * a.nv;
+#pragma unroll
+        for (int k = 0; k < RCW; ++k) y[i][k] = yc[joff[k]];
       }
+      if (((c0 - c_lo) & (64 / kFwdBins - 1)) == 0) {  // weights of the next 16 columns
+        const int n = c0 + lt;
+        w = 0.0f;
+        if (n >= n0 && n <= n1) {
+          if (M == CONE_B1) {
+            const float ta = (float)fma((double)n, an, fma((double)m, am, a0));
+            const float tb = (float)fma((double)n, bn, fma((double)m, bm, b0));
+            w = b1_mean(rec, ta, tb) * rec.scale;
+          } else {
+            w = sf_cell_weight(vg, g, u, rows ? n : m, rows ? m : n);
+          }
+        }
+      }
+      const int l0 = ((c0 - c_lo) & (64 / kFwdBins - 1)) * kFwdBins;
 #pragma unroll
-      for (int k = 0; k < RCW; ++k) acc[k] += (double)accl[k];
-    } else if (q0 <= q1) {
-      load_col(m + 1, q0, ycur);
+      for (int i = 0; i < kFwdCols; ++i) {
+        if (c0 + i > c_hi) break;
+#pragma unroll
+        for (int b = 0; b < kFwdBins; ++b) {
+          const float wb = lane_value(w, l0 + i * kFwdBins + b);
+          if (wb != 0.0f) {
+#pragma unroll
+            for (int k = 0; k < RCW; ++k) accl[b][k] = __builtin_fmaf(wb, y[i][k], accl[b][k]);
+          }
+        }
+      }
     }
-    n0 = q0;
-    n1 = q1;
+#pragma unroll
+    for (int b = 0; b < kFwdBins; ++b)
+#pragma unroll
+      for (int k = 0; k < RCW; ++k) acc[b][k] += (double)accl[b][k];
   }
-  float* out = proj + (size_t)v * a.nv * g.nu + u;
+  // waves 2, 3 onto 0, 1, then 1 onto 0
+#pragma unroll
+  for (int half = 2; half >= 1; half >>= 1) {
+    if (wv >= half && wv < 2 * half) {
+#pragma unroll
+      for (int b = 0; b < kFwdBins; ++b)
+#pragma unroll
+        for (int k = 0; k < RCW; ++k) red[wv - half][b][k][lane] = acc[b][k];
+    }
+    __syncthreads();
+    if (wv < half) {
+#pragma unroll
+      for (int b = 0; b < kFwdBins; ++b)
+#pragma unroll
+        for (int k = 0; k < RCW; ++k) acc[b][k] += red[wv][b][k][lane];
+    }
+    __syncthreads();
+  }
+  if (wv != 0) return;
+  float* out = proj + (size_t)v * a.nv * g.nu + u0;
 #pragma unroll
   for (int k = 0; k < RCW; ++k) {
     const int j = (kc0 + k) * 64 + lane;
-    if (j < a.nv) out[(size_t)j * g.nu] = (float)acc[k];
+    if (j >= a.nv) continue;
+#pragma unroll
+    for (int b = 0; b < kFwdBins; ++b)
+      if (u0 + b < g.nu) out[(size_t)j * g.nu + b] = (float)acc[b][k];
   }
 }
 
-// ---------------------------------------------------------------------------
-// Yb[pl][c][j] = sum_u conv(u, c) projT[pl][u][j].  Wave per (column, view),
-// the column's clamped corner range (A_B1_3D.cu:117-151) wave-uniform.
-// ---------------------------------------------------------------------------
+// Yb[pl][c][j] = sum_u conv(u, c) projT[pl][u][j], u over the column's clamped
+// corner range (A_B1_3D.cu:117-151).  Wave per kBwdCols adjacent columns of a
+// view: lane = 8 column + bin evaluates the weights of the first 8 bins of
+// every column at once (further ones as the column's loop reaches them), then
+// the columns take their bins' detector rows in turn, kBwdBins at a time.
+constexpr int kBwdCols = 8, kBwdBins = 6;
+
 template <int M, int RCW>
 __global__ __launch_bounds__(256) void conv_bwd_kernel(Cone3DArgs a, int p0, const float* __restrict__ projT,
                                                        float* __restrict__ Yb) {
   const Proj2DArgs& g = a.g;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int ncol = g.nx * g.ny;
-  const int c = blockIdx.x * 4 + wv, pl = blockIdx.y;
+  const int col0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + wv) * kBwdCols), pl = blockIdx.y;
   const int kc0 = blockIdx.z * RCW;  // this wave's detector-row chunks
-  if (c >= ncol) return;
+  if (col0 >= ncol) return;
   const int v = p0 + pl;
-  const int ix = c % g.nx, iy = c / g.nx;
+  const int lt = lane & 7, lc = min(col0 + lane / 8, ncol - 1);  // this lane's bin slot and column
+  const int ix = lc % g.nx, iy = lc / g.nx;
   const ViewGeo& vg = g.views[v];
   const B1Bin* bins = M == CONE_B1 ? reinterpret_cast<const B1Bin*>(g.bins) + (size_t)v * g.nu : nullptr;
   const double wx = ix * g.dx + vg.w0x, wy = iy * g.dy + vg.w0y;
@@ -473,46 +528,58 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(Cone3DArgs a, int p0, con
   const float last = (float)(g.nu - 1);
   const int ulo = (int)fminf(fmaxf(floorf(kc - hw), 0.0f), last);
   const int uhi = (int)fminf(fmaxf(floorf(kc + hw), 0.0f), last);
-  float acc[RCW];
+  auto weight = [&](int u) {
+    float w = 0.0f;
+    if (u <= uhi) {
+      if (M == CONE_B1) {
+        const B1Bin rec = bins[u];
+        const float ta = rec.ka * (float)fma((double)u, be, n0), tb = rec.kb * (float)fma((double)(u + 1), be, n0);
+        w = b1_mean(rec, ta, tb) * rec.scale;
+      } else {
+        w = sf_cell_weight(vg, g, u, ix, iy);
+      }
+    }
+    return w;
+  };
+  const float w_first = weight(ulo + lt);
+  // every lane loads (rows past nv read the last row and are never stored)
+  const float* rows0 = projT + (size_t)pl * g.nu * a.nv;
+  int joff[RCW];
 #pragma unroll
-  for (int k = 0; k < RCW; ++k) acc[k] = 0.0f;
-  // every lane loads (rows past nv read the last row and are never stored);
-  // the next bin's rows are loaded while the current bin's weight is computed
-  const float* rows0 = projT + (size_t)pl * g.nu * a.nv + kc0 * 64 + lane;
-  const int jmax = a.nv - 1 - kc0 * 64 - lane;
-  auto load_bin = [&](int u, float* y) {
-    const float* row = rows0 + (size_t)u * a.nv;
+  for (int k = 0; k < RCW; ++k) joff[k] = min((kc0 + k) * 64 + lane, a.nv - 1);
+  const int ncols = min(kBwdCols, ncol - col0);
+  for (int c = 0; c < ncols; ++c) {
+    const int u0 = __builtin_amdgcn_readlane(ulo, 8 * c), u1 = __builtin_amdgcn_readlane(uhi, 8 * c);
+    float acc[RCW];
+#pragma unroll
+    for (int k = 0; k < RCW; ++k) acc[k] = 0.0f;
+    float w = w_first;
+    int w0 = u0;  // bin of slot 0 of w
+    for (int ub = u0; ub <= u1; ub += kBwdBins) {
+      float y[kBwdBins][RCW];
+#pragma unroll
+      for (int i = 0; i < kBwdBins; ++i) {
+        const float* row = rows0 + (size_t)min(ub + i, u1) * a.nv;
+#pragma unroll
+        for (int k = 0; k < RCW; ++k) y[i][k] = row[joff[k]];
+      }
+      if (ub > u0) {  // slots of this column's further bins
+        w = weight(ub + lt);
+        w0 = ub;
+      }
+#pragma unroll
+      for (int i = 0; i < kBwdBins; ++i) {
+        if (ub + i > u1) break;
+        const float wi = lane_value(w, 8 * c + ub + i - w0);
+#pragma unroll
+        for (int k = 0; k < RCW; ++k) acc[k] = __builtin_fmaf(wi, y[i][k], acc[k]);
+      }
+    }
+    float* out = Yb + ((size_t)pl * ncol + col0 + c) * a.nv;
 #pragma unroll
     for (int k = 0; k < RCW; ++k)
-      if ((kc0 + k) * 64 < a.nv) y[k] = row[min(k * 64, jmax)];
-  };
-  float ycur[RCW], ynext[RCW];
-#pragma unroll
-  for (int k = 0; k < RCW; ++k) ycur[k] = ynext[k] = 0.0f;
-  load_bin(ulo, ycur);
-  float na = (float)fma((double)ulo, be, n0);
-  for (int u = ulo; u <= uhi; ++u) {
-    if (u < uhi) load_bin(u + 1, ynext);
-    const float nb = na + bef;
-    float w;
-    if (M == CONE_B1) {
-      const B1Bin rec = bins[u];
-      const float ta = rec.ka * na, tb = rec.kb * nb;
-      w = b1_mean(rec, ta, tb) * rec.scale;
-    } else {
-      w = sf_cell_weight(vg, g, u, ix, iy);
-    }
-#pragma unroll
-    for (int k = 0; k < RCW; ++k) {
-      acc[k] = __builtin_fmaf(w, ycur[k], acc[k]);
-      ycur[k] = ynext[k];
-    }
-    na = nb;
+      if ((kc0 + k) * 64 + lane < a.nv) out[(kc0 + k) * 64 + lane] = acc[k];
   }
-  float* out = Yb + ((size_t)pl * ncol + c) * a.nv + kc0 * 64 + lane;
-#pragma unroll
-  for (int k = 0; k < RCW; ++k)
-    if ((kc0 + k) * 64 + lane < a.nv) out[k * 64] = acc[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -620,6 +687,13 @@ hipError_t launch_transpose(const float* in, float* out, int rows, int cols, int
   return hipGetLastError();
 }
 
+// Chunks of 64 detector rows per wave of the in-plane kernels: at most
+// kAllRows, as few as hold the rows of a group.
+static int row_chunks(const Cone3DArgs& a) {
+  const int groups = (a.nrc + kAllRows - 1) / kAllRows, per = (a.nrc + groups - 1) / groups;
+  return (per + 1) / 2 * 2;
+}
+
 template <int M>
 static void cone_forward_chunk(const Cone3DArgs& a, int p0, int nview, const float* xT, float* Y, float* proj,
                                hipStream_t s) {
@@ -627,21 +701,28 @@ static void cone_forward_chunk(const Cone3DArgs& a, int p0, int nview, const flo
   const size_t lds = sizeof(float) * 4 * kAxialFields * std::min(a.nz, kMaxNz);  // 4 waves
   if (a.nz > kMaxNz) axial_fwd_kernel<M, true><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
   else axial_fwd_kernel<M, false><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
-  // every row in one wave: with the next column's profile loaded during the
-  // weight computation, splitting the rows over more waves (each computing
-  // the weights again) no longer pays (B1, 16 views of 256^2 x 384: 2 chunks
-  // of 64 rows per wave 67 ms per call, 3 chunks 61 ms, all 55 ms)
-  constexpr int RCW = kAllRows;
-  const int groups = (a.nrc + RCW - 1) / RCW;
-  conv_fwd_kernel<M, RCW><<<dim3(((a.g.nu + 3) / 4) * nview, groups), dim3(256), 0, s>>>(a, p0, nview, Y, proj);
+  const int groups = (a.nrc + kAllRows - 1) / kAllRows;
+  const dim3 grid(((a.g.nu + kFwdBins - 1) / kFwdBins) * nview, groups);
+  switch (row_chunks(a)) {
+    case 2: conv_fwd_kernel<M, 2><<<grid, dim3(256), 0, s>>>(a, p0, nview, Y, proj); break;
+    case 4: conv_fwd_kernel<M, 4><<<grid, dim3(256), 0, s>>>(a, p0, nview, Y, proj); break;
+    case 6: conv_fwd_kernel<M, 6><<<grid, dim3(256), 0, s>>>(a, p0, nview, Y, proj); break;
+    default: conv_fwd_kernel<M, 8><<<grid, dim3(256), 0, s>>>(a, p0, nview, Y, proj); break;
+  }
 }
 
 template <int M>
 static void cone_backward_chunk(const Cone3DArgs& a, int p0, int nview, const float* projT, float* Yb, float* xT,
                                 int accumulate, hipStream_t s) {
   const int ncol = a.g.nx * a.g.ny;
-  const int groups = (a.nrc + kAllRows - 1) / kAllRows;  // 512 detector rows per wave
-  conv_bwd_kernel<M, kAllRows><<<dim3((ncol + 3) / 4, nview, groups), dim3(256), 0, s>>>(a, p0, projT, Yb);
+  const int groups = (a.nrc + kAllRows - 1) / kAllRows;
+  const dim3 cgrid((ncol + 4 * kBwdCols - 1) / (4 * kBwdCols), nview, groups);
+  switch (row_chunks(a)) {
+    case 2: conv_bwd_kernel<M, 2><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
+    case 4: conv_bwd_kernel<M, 4><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
+    case 6: conv_bwd_kernel<M, 6><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
+    default: conv_bwd_kernel<M, 8><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
+  }
   const dim3 grid((ncol + 3) / 4, (a.nz + kMaxNz - 1) / kMaxNz);
   if (a.nv > kMaxNv || a.nz > kMaxNz)
     axial_bwd_kernel<M, true><<<grid, dim3(256), 0, s>>>(a, p0, nview, Yb, xT, accumulate);
