@@ -41,7 +41,9 @@ hipError_t launch_resid(const float* b, const float* ax, const float* w, float* 
 hipError_t launch_update(float* x, const float* c, const float* v, float lam, int positivity, size_t n, size_t per,
                          hipStream_t s);
 hipError_t launch_axpy(float* x, const float* g, float a, size_t n, hipStream_t s);
-hipError_t launch_transpose(const float* in, float* out, int rows, int cols, int batch, hipStream_t s);
+hipError_t launch_transpose(const float* in, float* out, int rows, int cols, int batch, const int* map,
+                            hipStream_t s);
+bool cone_groups_fit(int nz, int nv);
 hipError_t launch_cone_forward_chunk(int model, const Cone3DArgs& a, int p0, int nview, const float* xT, float* Y,
                                      float* proj, hipStream_t s);
 hipError_t launch_cone_backward_chunk(int model, const Cone3DArgs& a, int p0, int nview, const float* projT,
@@ -206,6 +208,10 @@ struct sgdct_projector {
   // (in-plane kernels on the caller's stream, volume updates in pass order on
   // cone_s2) gained nothing (39.0 -> 39.9 ms) and is not used.
   float* d_Y2 = nullptr;
+  // views in slots, classes of symmetric views together (Cone3DArgs)
+  Cone3DArgs cone{};
+  int nslot = 0;
+  int* d_cone = nullptr;
   hipStream_t cone_s2 = nullptr;
   hipEvent_t cone_ev[2] = {nullptr, nullptr};
 
@@ -234,6 +240,7 @@ struct sgdct_projector {
     if (d_host_part) (void)hipFree(d_host_part);
     if (d_count) (void)hipFree(d_count);
     if (d_part) (void)hipFree(d_part);
+    if (d_cone) (void)hipFree(d_cone);
     release_cone();
     if (h_img) (void)hipHostFree(h_img);
     if (h_sino) (void)hipHostFree(h_sino);
@@ -497,7 +504,7 @@ int ensure_staging(sgdct_projector* h) {
 }
 
 Cone3DArgs cone_args(const sgdct_projector* h) {
-  Cone3DArgs a;
+  Cone3DArgs a = h->cone;
   a.g = h->args;
   a.nz = h->nz;
   a.nv = h->nv;
@@ -511,6 +518,51 @@ Cone3DArgs cone_args(const sgdct_projector* h) {
   return a;
 }
 
+// Lays the views out in slots.  The axial trapezoids of B1 and SF-TT run from
+// x - off to x + off at the column's y, so that mirrors and half turns keep
+// them, and quarter turns only SF-TR's, which have no extent in the plane; the
+// detector's bins play no part in them.
+int setup_cone(sgdct_projector* h) {
+  h->nslot = h->np;
+  h->cone.nh = 1;
+  if (!cone_groups_fit(h->nz, h->nv) || h->nx > 0xffff || h->ny > 0x7fff) return SGDCT_OK;
+  std::vector<ViewGeo> views(h->np);
+  hipError_t e = hipMemcpy(views.data(), h->d_views, sizeof(ViewGeo) * h->np, hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return hip_fail(e, "cone-beam symmetries");
+  unsigned allowed = 1u | 1u << SymOp::kFlipX | 1u << SymOp::kFlipY | 1u << (SymOp::kFlipX | SymOp::kFlipY);
+  if (h->cone_model == 1 && h->nx == h->ny && h->dx == h->dy) allowed = 0xff;
+  const SymTables t = find_symmetries(views, h->nx, h->ny, h->nu, allowed, kMaxSym, 4e-12 * (h->lsd + h->lso), false,
+                                      false, 1);
+  const int nh = t.nh();
+  if (nh == 1) return SGDCT_OK;
+  const size_t ns = t.rep_view.size(), nd = t.tile.size();
+  std::vector<int> all(ns + ns * nh + nd + (nd + 3) / 4, 0);
+  for (size_t s = 0; s < ns; ++s) {
+    all[s] = t.rep_view[s];
+    const size_t cls = s / nh * nh;
+    for (int k = 0; k < nh && t.rep_view[s] >= 0; ++k) {
+      const int w = t.view[(size_t)t.rep_view[s] * nh + k];
+      for (int q = 0; q < nh; ++q)
+        if (t.rep_view[cls + q] == w) all[ns + s * nh + k] = q;
+    }
+  }
+  std::copy(t.tile.begin(), t.tile.end(), all.begin() + ns + ns * nh);
+  std::memcpy(all.data() + ns + ns * nh + nd, t.owner.data(), t.owner.size());
+  e = hipMalloc(&h->d_cone, all.size() * sizeof(int));
+  if (e == hipSuccess) e = hipMemcpy(h->d_cone, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice);
+  if (e != hipSuccess) return hip_fail(e, "cone-beam symmetries");
+  h->nslot = (int)ns;
+  Cone3DArgs& a = h->cone;
+  a.nh = nh;
+  for (int k = 0; k < nh; ++k) a.op[k] = t.op[k];
+  a.slot_view = h->d_cone;
+  a.peer = h->d_cone + ns;
+  a.dom = h->d_cone + ns + ns * nh;
+  a.own = reinterpret_cast<const unsigned char*>(h->d_cone + ns + ns * nh + nd);
+  a.ndom = (int)nd;
+  return SGDCT_OK;
+}
+
 bool is_cone(int basis) { return basis == BASIS_B1_3D || basis == BASIS_SF_3D; }
 
 int ensure_cone_workspace(sgdct_projector* h) {
@@ -521,11 +573,16 @@ int ensure_cone_workspace(sgdct_projector* h) {
   // columns x 384 rows), a multiple of 8 so that every XCD takes whole views
   size_t chunk = std::max<size_t>(1, ((size_t)2 << 30) / per_view);
   if (chunk >= 8) chunk -= chunk % 8;
-  h->chunk = (int)std::min<size_t>(chunk, (size_t)h->np);
+  if (chunk < 8 && h->cone.nh > 1) {  // passes of a few views each take them one by one
+    h->cone.nh = 1;
+    h->cone.slot_view = nullptr;
+    h->nslot = h->np;
+  }
+  h->chunk = (int)std::min<size_t>(chunk, (size_t)h->nslot);
   hipError_t e = hipMalloc(&h->d_xT, ncol * h->nz * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&h->d_Y, (size_t)h->chunk * per_view);
   if (e == hipSuccess) e = hipMalloc(&h->d_projT, (size_t)h->chunk * h->nu * h->nv * sizeof(float));
-  if (e == hipSuccess && h->np > h->chunk) {
+  if (e == hipSuccess && h->nslot > h->chunk) {
     e = hipMalloc(&h->d_Y2, (size_t)h->chunk * per_view);
     // non-blocking: no implicit ordering against the null stream; every
     // dependency is an explicit event
@@ -548,15 +605,15 @@ int cone_forward(sgdct_projector* h, const float* vol, float* proj, int batch, h
   for (int b = 0; b < batch; ++b) {
     const float* x = vol + (size_t)b * ncol * h->nz;
     float* y = proj + (size_t)b * h->np * h->nv * h->nu;
-    hipError_t e = launch_transpose(x, h->d_xT, h->nz, ncol, 1, s);
+    hipError_t e = launch_transpose(x, h->d_xT, h->nz, ncol, 1, nullptr, s);
     // odd passes on cone_s2 with d_Y2, after the transpose; the caller's
     // stream waits for them before the next image's transpose and at the end
     const bool two = h->cone_s2 != nullptr;
     if (two && e == hipSuccess) e = hipEventRecord(h->cone_ev[0], s);
     if (two && e == hipSuccess) e = hipStreamWaitEvent(h->cone_s2, h->cone_ev[0], 0);
-    for (int p0 = 0, k = 0; p0 < h->np && e == hipSuccess; p0 += h->chunk, ++k) {
+    for (int p0 = 0, k = 0; p0 < h->nslot && e == hipSuccess; p0 += h->chunk, ++k) {
       const bool odd = two && (k & 1);
-      e = launch_cone_forward_chunk(h->cone_model, a, p0, std::min(h->chunk, h->np - p0), h->d_xT,
+      e = launch_cone_forward_chunk(h->cone_model, a, p0, std::min(h->chunk, h->nslot - p0), h->d_xT,
                                     odd ? h->d_Y2 : h->d_Y, y, odd ? h->cone_s2 : s);
     }
     if (two) {
@@ -580,13 +637,14 @@ int cone_backward(sgdct_projector* h, const float* proj, float* vol, int batch, 
     const float* y = proj + (size_t)b * h->np * h->nv * h->nu;
     float* x = vol + (size_t)b * ncol * h->nz;
     hipError_t e = hipSuccess;
-    for (int p0 = 0; p0 < h->np && e == hipSuccess; p0 += h->chunk) {
-      const int nview = std::min(h->chunk, h->np - p0);
-      e = launch_transpose(y + (size_t)p0 * h->nv * h->nu, h->d_projT, h->nv, h->nu, nview, s);
+    for (int p0 = 0; p0 < h->nslot && e == hipSuccess; p0 += h->chunk) {
+      const int nview = std::min(h->chunk, h->nslot - p0);
+      const float* from = a.slot_view ? y : y + (size_t)p0 * h->nv * h->nu;
+      e = launch_transpose(from, h->d_projT, h->nv, h->nu, nview, a.slot_view ? a.slot_view + p0 : nullptr, s);
       if (e == hipSuccess)
         e = launch_cone_backward_chunk(h->cone_model, a, p0, nview, h->d_projT, h->d_Y, h->d_xT, p0 > 0, s);
     }
-    if (e == hipSuccess) e = launch_transpose(h->d_xT, x, ncol, h->nz, 1, s);
+    if (e == hipSuccess) e = launch_transpose(h->d_xT, x, ncol, h->nz, 1, nullptr, s);
     if (e != hipSuccess) return hip_fail(e, "cone-beam backward launch");
   }
   return SGDCT_OK;
@@ -1401,6 +1459,10 @@ sgdct_projector* b1_3d_init(int nx, int ny, int nz, int np, int nu, int nv, doub
   h->nv = nv;
   h->dz = dz;
   h->dv = dv;
+  if (setup_cone(h) != SGDCT_OK) {
+    delete h;
+    return nullptr;
+  }
   return h;
 }
 
@@ -1429,6 +1491,10 @@ sgdct_projector* sf3d_init(int nx, int ny, int nz, int np, int nu, int nv, doubl
   h->nv = nv;
   h->dz = dz;
   h->dv = dv;
+  if (setup_cone(h) != SGDCT_OK) {
+    delete h;
+    return nullptr;
+  }
   return h;
 }
 

@@ -42,6 +42,7 @@
 #include <cstdint>
 
 #include "footprint.hpp"
+#include "group2d.hpp"
 #include "projector.hpp"
 #include "sf2d_dev.hpp"
 
@@ -286,6 +287,86 @@ __global__ __launch_bounds__(256) void axial_fwd_kernel(Cone3DArgs a, int p0, co
   }
 }
 
+// Column c under symmetry op.
+__device__ __forceinline__ int image_column(const Proj2DArgs& g, int op, int c) {
+  int qx, qy;
+  SymOp::pixel(op, g.nx, g.ny, c % g.nx, c / g.nx, &qx, &qy);
+  return qy * g.nx + qx;
+}
+
+// The same for the G views of a class at once: the trapezoids of (view, c) are
+// staged once, with the voxel values of the G columns h c, and every overlap is
+// formed once for G row sums.  Block: two columns of the class's first view,
+// 128 threads each; grid (ceil(ncol / 2), classes in the pass).  nz <= kMaxNz.
+// Dynamic LDS: per column and voxel 6 + G floats and one of padding to an odd
+// stride.  Bound by the LDS reads of the records and, at G = 4, by the stores
+// of Y.  256^3 voxels, 360 views, 512 x 384, classes of 4: A as a whole 40.0 ->
+// 20.4 ms against one view at a time.
+template <int M, int G>
+__global__ __launch_bounds__(256) void axial_fwd_group_kernel(Cone3DArgs a, int p0, const float* __restrict__ xT,
+                                                              float* __restrict__ Y) {
+  extern __shared__ float axial_lds[];
+  constexpr int F = (6 + G) | 1;
+  const int t = threadIdx.x & 127, half = threadIdx.x >> 7;
+  float* const R = axial_lds + (size_t)half * F * a.nz;
+  const int ncol = a.g.nx * a.g.ny;
+  const int c = blockIdx.x * 2 + half, s0 = blockIdx.y * G;
+  const bool live = c < ncol;
+  ColumnAxial ca{};
+  int col[G];
+  if (live) {
+    ca = column_axial<M>(a, a.g.views[a.slot_view[p0 + s0]], c % a.g.nx, c / a.g.nx);
+#pragma unroll
+    for (int h = 0; h < G; ++h) col[h] = image_column(a.g, a.op[h], c);
+    for (int iz = t; iz < a.nz; iz += 128) {
+      const AxialTrap tr = voxel_trap<M>(a, ca, iz);
+      float* const r = R + F * iz;
+      r[0] = tr.v0;
+      r[1] = tr.v1;
+      r[2] = tr.v2;
+      r[3] = tr.v3;
+      r[4] = tr.i01;
+      r[5] = tr.i23;
+#pragma unroll
+      for (int h = 0; h < G; ++h) r[6 + h] = xT[(size_t)col[h] * a.nz + iz] * tr.cf;
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+  // first voxel that reaches a row, as in axial_fwd_kernel
+  const float ikhi = 1.0f / fmaxf(ca.ka, ca.kb), iklo = 1.0f / fminf(ca.ka, ca.kb);
+  const float zoff = 0.5f * (float)(a.nz - 1) - 0.5f;
+  for (int j = t; j < a.nv; j += 128) {
+    const float fj = (float)j + row_off<M>();
+    const float est = __builtin_fmaf(fj - a.vc, fj >= a.vc ? ikhi : iklo, zoff);
+    int lo = (int)fminf(fmaxf(ceilf(est), 0.0f), (float)a.nz);
+    while (lo > 0 && R[F * (lo - 1) + 3] >= fj) --lo;
+    while (lo < a.nz && R[F * lo + 3] < fj) ++lo;
+    float acc[G];
+#pragma unroll
+    for (int h = 0; h < G; ++h) acc[h] = 0.0f;
+    for (int iz = lo; iz < a.nz; ++iz) {
+      const float* const r = R + F * iz;
+      if (!(r[0] < fj + 1.0f)) break;
+      AxialTrap tr;
+      tr.v0 = r[0];
+      tr.v1 = r[1];
+      tr.v2 = r[2];
+      tr.v3 = r[3];
+      tr.i01 = r[4];
+      tr.i23 = r[5];
+      const float gm = trap_gamma(fj, tr);
+      if (keep_gamma<M>(gm)) {
+#pragma unroll
+        for (int h = 0; h < G; ++h) acc[h] = __builtin_fmaf(r[6 + h], gm, acc[h]);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < G; ++h)
+      if (a.slot_view[p0 + s0 + h] >= 0) Y[((size_t)(s0 + h) * ncol + col[h]) * a.nv + j] = acc[h];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // In-plane kernels.  Their weights do not depend on the detector row, so lanes
 // cover the rows (RCW chunks of 64 per wave) where row profiles are read and
@@ -353,7 +434,8 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
   const int lb = lane & (kFwdBins - 1), lt = lane / kFwdBins;  // this lane's bin and column of a weight evaluation
   const bool live = u0 + lb < g.nu;
   const int u = live ? u0 + lb : g.nu - 1;
-  const int v = p0 + pl;
+  const int v = slot_view(a, p0 + pl);
+  if (v < 0) return;  // the whole workgroup
   const int ncol = g.nx * g.ny;
   const ViewGeo vg = g.views[v];
   B1Bin rec{};
@@ -512,8 +594,8 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(Cone3DArgs a, int p0, con
   const int ncol = g.nx * g.ny;
   const int col0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + wv) * kBwdCols), pl = blockIdx.y;
   const int kc0 = blockIdx.z * RCW;  // this wave's detector-row chunks
-  if (col0 >= ncol) return;
-  const int v = p0 + pl;
+  const int v = slot_view(a, p0 + pl);
+  if (col0 >= ncol || v < 0) return;
   const int lt = lane & 7, lc = min(col0 + lane / 8, ncol - 1);  // this lane's bin slot and column
   const int ix = lc % g.nx, iy = lc / g.nx;
   const ViewGeo& vg = g.views[v];
@@ -661,18 +743,114 @@ __global__ __launch_bounds__(256) void axial_bwd_kernel(Cone3DArgs a, int p0, in
   }
 }
 
+// The same for the G columns h c of a column c of the fundamental domain: the
+// trapezoid of (view, voxel) serves voxel h c of the views h v, whose row
+// profiles are staged side by side (one 16-byte LDS read per row at G = 4).
+// Block: 256 voxels of one column; grid (ndom, ceil(nz / 256)).  The next
+// view's profiles are requested before the current view's rows are gathered.
+// nv <= kGroupRows.  Bound by the reads of the profiles (1.6 GB per 16 views of
+// the case above); A^T as a whole 34.3 -> 21.3 ms.
+constexpr int kGroupRows = 512;
+
+template <int M, int G>
+__global__ __launch_bounds__(256) void axial_bwd_group_kernel(Cone3DArgs a, int p0, int nview,
+                                                              const float* __restrict__ Yb, float* __restrict__ xT,
+                                                              int accumulate) {
+  extern __shared__ __attribute__((aligned(16))) float prof[];  // [nv][G]
+  constexpr int kPre = (kGroupRows * G + 255) / 256;
+  const int ncol = a.g.nx * a.g.ny;
+  const int xy = a.dom[blockIdx.x], ix = xy & 0xffff, iy = xy >> 16;
+  const unsigned own = a.own[blockIdx.x];
+  const int iz = blockIdx.y * 256 + threadIdx.x;
+  int col[G];
+#pragma unroll
+  for (int h = 0; h < G; ++h) col[h] = image_column(a.g, a.op[h], iy * a.g.nx + ix);
+  double acc[G];
+#pragma unroll
+  for (int h = 0; h < G; ++h) acc[h] = 0.0;
+  const int rows = a.nv;
+  float pre[kPre];
+  auto fetch = [&](int s) {
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      const int cls = s / G * G;
+      const float* src = Yb + ((size_t)(cls + a.peer[(size_t)(p0 + s) * G + h]) * ncol + col[h]) * rows;
+#pragma unroll
+      for (int k = 0; k < kPre / G; ++k) {
+        const int j = k * 256 + (int)threadIdx.x;
+        pre[h * (kPre / G) + k] = j < rows ? src[j] : 0.0f;
+      }
+    }
+  };
+  auto next_slot = [&](int s) {
+    while (s < nview && a.slot_view[p0 + s] < 0) ++s;
+    return s;
+  };
+  const float lastj = (float)(rows - 1), ro = row_off<M>();
+  int s = next_slot(0);
+  if (s < nview) fetch(s);
+  while (s < nview) {
+    __syncthreads();  // the previous view's reads come first
+#pragma unroll
+    for (int k = 0; k < kPre / G; ++k) {
+      const int j = k * 256 + (int)threadIdx.x;
+      if (j < rows) {
+#pragma unroll
+        for (int h = 0; h < G; ++h) prof[j * G + h] = pre[h * (kPre / G) + k];
+      }
+    }
+    __syncthreads();
+    const int sn = next_slot(s + 1);
+    if (sn < nview) fetch(sn);
+    if (iz < a.nz) {
+      const ColumnAxial ca = column_axial<M>(a, a.g.views[a.slot_view[p0 + s]], ix, iy);
+      int k0;
+      const AxialTrap tr = voxel_trap_rel<M>(a, ca, iz, &k0);
+      // rows relative to k0 (small integers plus ro: exact)
+      const int jlo = (int)fminf(fmaxf(floorf(tr.v0 - ro) + (float)k0, 0.0f), lastj);
+      const int jhi = (int)fminf(fmaxf(floorf(tr.v3 - ro) + (float)k0, 0.0f), lastj);
+      float sum[G];
+#pragma unroll
+      for (int h = 0; h < G; ++h) sum[h] = 0.0f;
+      float sj = (float)(jlo - k0) + ro;
+      for (int j = jlo; j <= jhi; ++j, sj += 1.0f) {
+        const float gm = trap_gamma(sj, tr);
+        if (keep_gamma<M>(gm)) {
+          float y[G];
+          __builtin_memcpy(y, __builtin_assume_aligned(prof + j * G, G < 4 ? 4 * G : 16), sizeof(y));
+#pragma unroll
+          for (int h = 0; h < G; ++h) sum[h] = __builtin_fmaf(gm, y[h], sum[h]);
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < G; ++h) acc[h] += (double)(tr.cf * sum[h]);
+    }
+    s = sn;
+  }
+  if (iz >= a.nz) return;
+#pragma unroll
+  for (int h = 0; h < G; ++h) {
+    if (!((own >> h) & 1)) continue;
+    float* const out = xT + (size_t)col[h] * a.nz + iz;
+    *out = (float)((accumulate ? (double)*out : 0.0) + acc[h]);
+  }
+}
+
 // ---------------------------------------------------------------------------
-// out[b][c][r] = in[b][r][c] for a batch of rows x cols matrices.
+// out[b][c][r] = in[map(b)][r][c] for a batch of rows x cols matrices (map null:
+// the identity; an entry -1: nothing).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void transpose_kernel(const float* __restrict__ in, float* __restrict__ out,
-                                                        int rows, int cols) {
+                                                        int rows, int cols, const int* __restrict__ map) {
   __shared__ float tile[32][33];
-  const size_t off = (size_t)blockIdx.z * rows * cols;
+  const int src = map ? map[blockIdx.z] : (int)blockIdx.z;
+  if (src < 0) return;
+  const size_t off = (size_t)blockIdx.z * rows * cols, in_off = (size_t)src * rows * cols;
   const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
   for (int k = ty; k < 32; k += 8) {
     const int r = r0 + k, c = c0 + tx;
-    if (r < rows && c < cols) tile[k][tx] = in[off + (size_t)r * cols + c];
+    if (r < rows && c < cols) tile[k][tx] = in[in_off + (size_t)r * cols + c];
   }
   __syncthreads();
   for (int k = ty; k < 32; k += 8) {
@@ -681,9 +859,10 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float* __restrict_
   }
 }
 
-hipError_t launch_transpose(const float* in, float* out, int rows, int cols, int batch, hipStream_t s) {
+hipError_t launch_transpose(const float* in, float* out, int rows, int cols, int batch, const int* map,
+                            hipStream_t s) {
   dim3 grid((cols + 31) / 32, (rows + 31) / 32, batch);
-  transpose_kernel<<<grid, dim3(256), 0, s>>>(in, out, rows, cols);
+  transpose_kernel<<<grid, dim3(256), 0, s>>>(in, out, rows, cols, map);
   return hipGetLastError();
 }
 
@@ -698,9 +877,17 @@ template <int M>
 static void cone_forward_chunk(const Cone3DArgs& a, int p0, int nview, const float* xT, float* Y, float* proj,
                                hipStream_t s) {
   const int ncol = a.g.nx * a.g.ny;
-  const size_t lds = sizeof(float) * 4 * kAxialFields * std::min(a.nz, kMaxNz);  // 4 waves
-  if (a.nz > kMaxNz) axial_fwd_kernel<M, true><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
-  else axial_fwd_kernel<M, false><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
+  if (a.nh > 1) {
+    const dim3 grid((ncol + 1) / 2, nview / a.nh);
+    const size_t lds = sizeof(float) * 2 * ((6 + a.nh) | 1) * a.nz;
+    if (a.nh == 2) axial_fwd_group_kernel<M, 2><<<grid, dim3(256), lds, s>>>(a, p0, xT, Y);
+    else if (a.nh == 4) axial_fwd_group_kernel<M, 4><<<grid, dim3(256), lds, s>>>(a, p0, xT, Y);
+    else if (M == CONE_SF_TR) axial_fwd_group_kernel<M, 8><<<grid, dim3(256), lds, s>>>(a, p0, xT, Y);
+  } else {
+    const size_t lds = sizeof(float) * 4 * kAxialFields * std::min(a.nz, kMaxNz);  // 4 waves
+    if (a.nz > kMaxNz) axial_fwd_kernel<M, true><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
+    else axial_fwd_kernel<M, false><<<dim3((ncol + 3) / 4, nview), dim3(256), lds, s>>>(a, p0, xT, Y);
+  }
   const int groups = (a.nrc + kAllRows - 1) / kAllRows;
   const dim3 grid(((a.g.nu + kFwdBins - 1) / kFwdBins) * nview, groups);
   switch (row_chunks(a)) {
@@ -723,12 +910,23 @@ static void cone_backward_chunk(const Cone3DArgs& a, int p0, int nview, const fl
     case 6: conv_bwd_kernel<M, 6><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
     default: conv_bwd_kernel<M, 8><<<cgrid, dim3(256), 0, s>>>(a, p0, projT, Yb); break;
   }
+  if (a.nh > 1) {
+    const dim3 dgrid(a.ndom, (a.nz + 255) / 256);
+    const size_t lds = sizeof(float) * a.nh * a.nv;
+    if (a.nh == 2) axial_bwd_group_kernel<M, 2><<<dgrid, dim3(256), lds, s>>>(a, p0, nview, Yb, xT, accumulate);
+    else if (a.nh == 4) axial_bwd_group_kernel<M, 4><<<dgrid, dim3(256), lds, s>>>(a, p0, nview, Yb, xT, accumulate);
+    else if (M == CONE_SF_TR) axial_bwd_group_kernel<M, 8><<<dgrid, dim3(256), lds, s>>>(a, p0, nview, Yb, xT, accumulate);
+    return;
+  }
   const dim3 grid((ncol + 3) / 4, (a.nz + kMaxNz - 1) / kMaxNz);
   if (a.nv > kMaxNv || a.nz > kMaxNz)
     axial_bwd_kernel<M, true><<<grid, dim3(256), 0, s>>>(a, p0, nview, Yb, xT, accumulate);
   else
     axial_bwd_kernel<M, false><<<grid, dim3(256), 0, s>>>(a, p0, nview, Yb, xT, accumulate);
 }
+
+// Sizes the grouped axial kernels take.
+bool cone_groups_fit(int nz, int nv) { return nz <= kMaxNz && nv <= kGroupRows; }
 
 hipError_t launch_cone_forward_chunk(int model, const Cone3DArgs& a, int p0, int nview, const float* xT, float* Y,
                                      float* proj, hipStream_t s) {

@@ -56,7 +56,20 @@ struct Cone3DArgs {
   float dz;
   double du;        // |pu|
   float fac;        // separable footprints: lsd^2 dx dy dz / (du dv)
+  // Views in slots, nh to a class of views that the symmetries op[] map onto
+  // each other (group2d.hpp; nh = 1: every view by itself, slot_view null =
+  // slot s is view s).  The axial trapezoids of (view, column) are those of
+  // (h view, h column).
+  int nh;
+  int op[8];
+  const int* slot_view;       // [nslot] view of a slot, -1 where a class repeats one
+  const int* peer;            // [nslot][nh] slot of h view, counted from the class's first
+  const int* dom;             // columns of the fundamental domain, iy << 16 | ix
+  const unsigned char* own;   // bit h: column h c is written by this one
+  int ndom;
 };
+
+__device__ __forceinline__ int slot_view(const Cone3DArgs& a, int s) { return a.slot_view ? a.slot_view[s] : s; }
 
 // One slice of a batched persistent launch (batch.hip): a 2-D projector's
 // arguments and its images' offsets in the packed batch buffers.

@@ -16,7 +16,7 @@ struct SymTables {
   std::vector<int> rep, rep_view;   // [nrep], [nrep][nh]
   std::vector<int> view;            // [np][nh]
   std::vector<int> tile;            // tiles of the fundamental domain
-  std::vector<unsigned char> owner; // [ntile][kTile * kTile]
+  std::vector<unsigned char> owner; // [ntile][edge * edge], edge = kTile unless asked otherwise
   int nh() const { return (int)op.size(); }
 };
 
@@ -49,10 +49,10 @@ inline int window_bound(const Proj2DArgs& g, const ViewGeo* views, double cx, do
 }
 
 // Views per symmetry op: perm[v] is the view op maps v onto, empty if some
-// view has no partner.  Source, first edge ray and detector step have to
-// agree within tol (the FP64 rounding of the angles); every view is the
+// view has no partner.  Source, first edge ray (`edges`) and detector step have
+// to agree within tol (the FP64 rounding of the angles); every view is the
 // partner of exactly one.
-inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int nu, int op, double tol) {
+inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int nu, int op, double tol, bool edges) {
   const int np = (int)views.size();
   std::vector<std::pair<double, int>> by_angle(np);
   for (int v = 0; v < np; ++v) by_angle[v] = {std::atan2(views[v].py, views[v].px), v};
@@ -74,9 +74,9 @@ inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int 
       auto it = std::lower_bound(by_angle.begin(), by_angle.end(), std::make_pair(t - eps, -1));
       for (; it != by_angle.end() && it->first <= t + eps && perm[v] < 0; ++it) {
         const ViewGeo& b = views[it->second];
-        const double err = std::max({std::fabs(b.px - p[0]), std::fabs(b.py - p[1]), std::fabs(b.e0x - e[0]),
-                                     std::fabs(b.e0y - e[1]), nu * std::fabs(b.pux - d[0]),
-                                     nu * std::fabs(b.puy - d[1])});
+        double err = std::max({std::fabs(b.px - p[0]), std::fabs(b.py - p[1]), nu * std::fabs(b.pux - d[0]),
+                               nu * std::fabs(b.puy - d[1])});
+        if (edges) err = std::max({err, std::fabs(b.e0x - e[0]), std::fabs(b.e0y - e[1])});
         if (!used[it->second] && err <= tol) {
           used[it->second] = 1;
           perm[v] = it->second;
@@ -91,16 +91,18 @@ inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int 
 // The symmetries of a scan of nx x ny pixels, at most `most` of them: the
 // group of every grid symmetry that permutes the views, or its subgroup
 // without axis swaps, or that subgroup's first element of order two.
-// `allowed` has a bit for each op the grid admits; hex: a hexagonal lattice.
+// `allowed` has a bit for each op the grid admits; hex: a hexagonal lattice;
+// edges = false: the detector's bins need not map onto each other; edge: tile
+// edge of the fundamental domain.
 inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int ny, int nu, unsigned allowed, int most,
-                                 double tol, bool hex = false) {
+                                 double tol, bool hex = false, bool edges = true, int edge = kTile) {
   SymTables t;
   const int np = (int)views.size();
   std::vector<int> perm[kMaxSym];
   std::vector<int> found{0};
   for (int op = 1; op < kMaxSym && most > 1; ++op) {
     if (!((allowed >> op) & 1)) continue;
-    perm[op] = view_permutation(views, nu, op, tol);
+    perm[op] = view_permutation(views, nu, op, tol, edges);
     if (!perm[op].empty()) found.push_back(op);
   }
   if ((int)found.size() > most) {
@@ -138,19 +140,19 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
   // tiles in raster order until every pixel is the image of a tile's pixel;
   // the first pair (pixel, op) that reaches a pixel writes it
   std::vector<char> covered((size_t)nx * ny, 0);
-  const int tx = (nx + kTile - 1) / kTile, ty = (ny + kTile - 1) / kTile;
+  const int tx = (nx + edge - 1) / edge, ty = (ny + edge - 1) / edge;
   for (int j = 0; j < ty; ++j)
     for (int i = 0; i < tx; ++i) {
-      const int x1 = std::min(nx, (i + 1) * kTile), y1 = std::min(ny, (j + 1) * kTile);
+      const int x1 = std::min(nx, (i + 1) * edge), y1 = std::min(ny, (j + 1) * edge);
       bool need = false;
-      for (int y = j * kTile; y < y1 && !need; ++y)
-        for (int x = i * kTile; x < x1 && !need; ++x) need = !covered[(size_t)y * nx + x];
+      for (int y = j * edge; y < y1 && !need; ++y)
+        for (int x = i * edge; x < x1 && !need; ++x) need = !covered[(size_t)y * nx + x];
       if (!need) continue;
       t.tile.push_back(j << 16 | i);
       const size_t o = t.owner.size();
-      t.owner.resize(o + kTile * kTile, 0);
-      for (int y = j * kTile; y < y1; ++y)
-        for (int x = i * kTile; x < x1; ++x)
+      t.owner.resize(o + edge * edge, 0);
+      for (int y = j * edge; y < y1; ++y)
+        for (int x = i * edge; x < x1; ++x)
           for (int h = 0; h < nh; ++h) {
             int qx, qy;
             if (hex) SymOp::hex_point(found[h], nx, ny, x, y, &qx, &qy);
@@ -158,7 +160,7 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
             char& c = covered[(size_t)qy * nx + qx];
             if (c) continue;
             c = 1;
-            t.owner[o + (size_t)(y - j * kTile) * kTile + (x - i * kTile)] |= (unsigned char)(1 << h);
+            t.owner[o + (size_t)(y - j * edge) * edge + (x - i * edge)] |= (unsigned char)(1 << h);
           }
     }
   return t;

@@ -120,3 +120,47 @@ def test_hex_forward_on_two_streams(cuda):
     torch.cuda.synchronize()
     for a, b in zip(ref, outs):
         assert torch.equal(a, b)
+
+
+CONE = {
+    "views on the axes": dict(nx=12, ny=12, views=8),
+    "3 classes of 4": dict(nx=13, ny=13, views=12, start=np.pi / 12),
+    "rectangle": dict(nx=15, ny=10, views=12),
+    "half turns": dict(nx=11, ny=11, views=10, start=0.3),
+    "quarter turns": dict(nx=10, ny=10, views=12, start=0.3),
+    "odd": dict(nx=9, ny=14, views=9),
+    "none": dict(nx=9, ny=9, views=7, start=0.2),
+    "many rows": dict(nx=6, ny=6, views=8, nz=300, nv=500),
+    "most rows": dict(nx=6, ny=6, views=4, nz=20, nv=512),
+    "too many rows": dict(nx=6, ny=6, views=4, nz=20, nv=513),
+    "too many voxels": dict(nx=5, ny=5, views=4, nz=513, nv=60),
+}
+
+
+@pytest.mark.parametrize("model", ["B1", "SF-TR", "SF-TT"])
+@pytest.mark.parametrize("name", list(CONE))
+def test_cone_classes_match_oracle(cuda, oracle_exact, model, name):
+    """Cone beam: axial trapezoids shared by the views of a class, on either
+    side of the sizes the grouped kernels take."""
+    import torch
+    from pyoracle import Geometry3
+    from sgd_amd.torch_ops import Projector
+    c = dict(dict(nz=21, nv=40, start=0.0), **CONE[name])
+    ang = c["start"] + 2 * np.pi * np.arange(c["views"]) / c["views"]
+    geo = (c["nx"], c["ny"], c["nz"], ang, 45, c["nv"], 1.1, 1.1, 0.9, 1.3, 1.2, 300.0, 150.3)
+    P = Projector.cone_beam(*geo, model=model)
+    G = Geometry3(oracle_exact, *geo)
+    print(model, name, c, flush=True)
+    rng = np.random.default_rng(9)
+    x = rng.random((2,) + P.img_shape).astype(np.float32)
+    y = rng.random((2,) + P.sino_shape).astype(np.float32)
+    xt, yt = torch.from_numpy(x).to(cuda), torch.from_numpy(y).to(cuda)
+    ax, aty = P.forward(xt), P.backward(yt)
+    torch.cuda.synchronize()
+    tv = model == "SF-TT"
+    for k in (0, 1):
+        xd, yd = x[k].astype(np.float64), y[k].astype(np.float64)
+        e1 = rel(ax[k].double().cpu().numpy(), G.forward(xd) if model == "B1" else G.sf_forward(xd, trap_v=tv))
+        e2 = rel(aty[k].double().cpu().numpy(), G.backward(yd) if model == "B1" else G.sf_backward(yd, trap_v=tv))
+        print("  A %.2e  A^T %.2e" % (e1, e2), flush=True)
+        assert e1 <= 1e-5 and e2 <= 1e-5, (k, e1, e2)
