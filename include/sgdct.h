@@ -290,6 +290,16 @@ int sgdct_nn_conv3x3(const void *in, const void *w, const float *bias, void *out
 int sgdct_nn_conv3x3_ex(const void *in, const void *in2, int c0, const void *w, const float *bias, void *out,
                         const void *mask, int B, int H, int W, int cin, int cout, int relu, int out_f32,
                         void *stream);
+/* Input gradient of a convolution of [upsample2(low), skip]: in (cin channels)
+ * the bf16 output gradient, w the flipped weights; low_out (B, H/2, W/2, c0) =
+ * the first c0 of the cout gradient channels summed over 2x2 blocks and masked
+ * by low_mask > 0, gskip (B, H, W, cout - c0) the others (sgdct_nn_conv3x3 with
+ * out_f32 followed by sgdct_nn_upcat_back; the workspace holds the gradient in
+ * between where the two do not run as one, and is empty where they do). */
+long long sgdct_nn_conv3x3_upback_workspace(int B, int H, int W, int cin, int cout, int c0);
+int sgdct_nn_conv3x3_upback(const void *in, const void *w, void *low_out, const void *low_mask, float *gskip,
+                            float *workspace, long long workspace_floats, int B, int H, int W, int cin, int cout,
+                            int c0, void *stream);
 long long sgdct_nn_wgrad_workspace(int B, int H, int W, int cin, int cout);
 /* dw[co][k] = sum over pixels of dy[m][co] x[m + tap(k)][c(k)] */
 int sgdct_nn_wgrad(const void *x, const void *dy, float *dw, float *workspace, long long workspace_floats, int B,

@@ -89,6 +89,8 @@ def lib():
         "sgdct_nn_wgrad_workspace": [_i] * 5,
         "sgdct_nn_wgrad": [_v, _v, _v, _v, _ll] + [_i] * 5 + [_v],
         "sgdct_nn_conv3x3_ex": [_v, _v, _i, _v, _v, _v, _v] + [_i] * 7 + [_v],
+        "sgdct_nn_conv3x3_upback_workspace": [_i] * 6,
+        "sgdct_nn_conv3x3_upback": [_v] * 6 + [_ll] + [_i] * 6 + [_v],
         "sgdct_nn_wgrad_ex": [_v, _v, _i, _v, _v, _v, _v, _ll] + [_i] * 5 + [_v],
         "sgdct_nn_colsum_workspace": [_ll, _i],
         "sgdct_nn_colsum": [_v, _v, _v, _ll, _ll, _i, _v],

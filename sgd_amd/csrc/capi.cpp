@@ -55,6 +55,9 @@ hipError_t launch_hex_matgen(int basis, const Proj2DArgs& g, double dt, bool wri
 hipError_t launch_batch_forward(const BatchPlan& P, int blocks, const float* img, float* sino, hipStream_t s);
 hipError_t nn_conv3x3(const void* in, const void* in2, int c0, const void* w, const float* bias, void* out,
                       const void* mask, int B, int H, int W, int cin, int cout, int relu, int out_f32, hipStream_t s);
+bool nn_upback_fused(int cin, int cout, int c0);
+hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
+                             int H, int W, int cin, int cout, int c0, hipStream_t s);
 long long nn_wgrad_splits(long long M);
 hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float* dw, float* db, float* partial, int B,
                     int H, int W, int cin, int cout, hipStream_t s);
@@ -1750,6 +1753,28 @@ int sgdct_nn_conv3x3_ex(const void* in, const void* in2, int c0, const void* w, 
     return fail(SGDCT_EINVAL, "bad conv3x3 concatenation (0 < c0 < cin, c0 % 8 == 0, even H and W)");
   return nn_ret(nn_conv3x3(in, in2, c0, w, bias, out, mask, B, H, W, cin, cout, relu, out_f32, (hipStream_t)stream),
                 "conv3x3");
+}
+
+long long sgdct_nn_conv3x3_upback_workspace(int B, int H, int W, int cin, int cout, int c0) {
+  if (!dims_ok(B, H, W) || cin <= 0 || cout <= 0 || c0 <= 0 || c0 >= cout) return fail(SGDCT_EINVAL, "bad upback shape");
+  return nn_upback_fused(cin, cout, c0) ? 0 : (long long)B * H * W * cout;
+}
+
+int sgdct_nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* gskip,
+                            float* workspace, long long workspace_floats, int B, int H, int W, int cin, int cout,
+                            int c0, void* stream) {
+  if (!in || !w || !low_out || !low_mask || !gskip || !dims_ok(B, H, W) || H % 2 || W % 2 || cin <= 0 || cin % 8 ||
+      cout <= 0 || c0 <= 0 || c0 >= cout)
+    return fail(SGDCT_EINVAL, "bad conv3x3_upback arguments");
+  hipStream_t s = (hipStream_t)stream;
+  if (nn_upback_fused(cin, cout, c0))
+    return nn_ret(nn_conv3x3_upback(in, w, low_out, low_mask, gskip, B, H, W, cin, cout, c0, s), "conv3x3_upback");
+  if (!workspace || workspace_floats < sgdct_nn_conv3x3_upback_workspace(B, H, W, cin, cout, c0))
+    return fail(SGDCT_EINVAL, "conv3x3_upback workspace too small");
+  hipError_t e = nn_conv3x3(in, nullptr, 0, w, nullptr, workspace, nullptr, B, H, W, cin, cout, 0, 1, s);
+  if (e == hipSuccess)
+    e = nn_upcat_back(workspace, nullptr, low_out, low_mask, gskip, 0, B, H, W, c0, cout - c0, s);
+  return nn_ret(e, "conv3x3_upback");
 }
 
 long long sgdct_nn_wgrad_workspace(int B, int H, int W, int cin, int cout) {

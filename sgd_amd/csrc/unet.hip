@@ -46,6 +46,13 @@ struct ConvArgs {
   const bf16* mask;    // [B][H][W][cout] or null: out = value * (mask > 0)
   const bf16* in2;     // [B][H][W][cin - c0] or null (see conv_in)
   int c0;
+  // Output as the gradient of a concatenation [upsample2(low), skip] (halo
+  // kernel; null low_out: the plain output): channels [0, low_c) are summed
+  // over 2 x 2 blocks, masked and stored in bf16, the others go to skip_out.
+  bf16* low_out;          // [B][H/2][W/2][low_c]
+  const bf16* low_mask;
+  float* skip_out;        // [B][H][W][cout - low_c]
+  int low_c;
 };
 
 // Address of the 8 input channels c .. c + 7 at pixel (b, y, x).  With in2 the
@@ -415,6 +422,39 @@ __global__ __launch_bounds__(256) void conv3x3_halo_kernel(ConvArgs a) {
       for (int r = 0; r < 4; ++r)
         etile[((wm * TM + i) * TW + 4 * g + r) * ES + wn * (BN / WN) + 16 * j + r16] = acc[i][j][r];
   __syncthreads();
+  if (a.low_out && nb < a.low_c) {
+    // 2 x 2 sums (low_c is a multiple of BN; tiles start at even pixels)
+    for (int q = tid; q < EG / 4; q += 256) {
+      const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
+      const int ly = p / (TW / 2), lx = p - ly * (TW / 2);
+      const int oy = (y0 >> 1) + ly, ox = (x0 >> 1) + lx;
+      if (2 * oy >= a.H || 2 * ox >= a.W) continue;
+      const float* const e0 = etile + (2 * ly * TW + 2 * lx) * ES + c8;
+      const long long o = (((long long)b * (a.H >> 1) + oy) * (a.W >> 1) + ox) * a.low_c + nb + c8;
+      const i16x8 mk = __builtin_bit_cast(i16x8, *reinterpret_cast<const bf16x8*>(a.low_mask + o));
+      bf16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = e0[e] + e0[ES + e] + e0[TW * ES + e] + e0[(TW + 1) * ES + e];
+        h[e] = (bf16)(__uint_as_float((unsigned)(unsigned short)mk[e] << 16) > 0.0f ? v : 0.0f);
+      }
+      *reinterpret_cast<bf16x8*>(a.low_out + o) = h;
+    }
+    return;
+  }
+  if (a.low_out) {
+    const int cs = a.cout - a.low_c;
+    for (int q = tid; q < EG; q += 256) {
+      const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
+      const int oy = y0 + p / TW, ox = x0 + p % TW;
+      if (oy >= a.H || ox >= a.W) continue;
+      float* const op = a.skip_out + (((long long)b * a.H + oy) * a.W + ox) * cs + nb - a.low_c + c8;
+      const float* const e0 = etile + p * ES + c8;
+      *reinterpret_cast<f32x4*>(op) = f32x4{e0[0], e0[1], e0[2], e0[3]};
+      *reinterpret_cast<f32x4*>(op + 4) = f32x4{e0[4], e0[5], e0[6], e0[7]};
+    }
+    return;
+  }
   for (int q = tid; q < EG; q += 256) {
     const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
     const int oy = y0 + p / TW, ox = x0 + p % TW, co = nb + c8;
@@ -705,6 +745,58 @@ __global__ void pool2_kernel(const bf16* __restrict__ src, bf16* __restrict__ ds
   dst[i] = (bf16)(0.25f * s);
 }
 
+// 8 bf16 of one 16-byte vector as floats
+__device__ __forceinline__ void unpack8(const bf16* p, float (&x)[8]) {
+  const i16x8 u = __builtin_bit_cast(i16x8, *reinterpret_cast<const bf16x8*>(p));
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = __uint_as_float((unsigned)(unsigned short)u[e] << 16);
+}
+
+// pool2_kernel for C % 8 == 0, one thread per 8 channels of a pixel (16-byte
+// accesses; element-wise it issued four 2-byte loads and two 64-bit divisions
+// per value: 92 -> 43 us for the three levels of 8 x 512 x 512 x 32).  grid.y = b.
+__global__ __launch_bounds__(256) void pool2_vec_kernel(const bf16* __restrict__ src, bf16* __restrict__ dst, int H,
+                                                        int W, int C8) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= H * W * C8) return;
+  const int p = i / C8, c = (i - p * C8) * 8, y = p / W, x = p - y * W, C = C8 * 8;
+  const size_t row = (size_t)2 * W * C;
+  const bf16* const s = src + (((size_t)blockIdx.y * 2 * H + 2 * y) * 2 * W + 2 * x) * C + c;
+  float v0[8], v1[8], v2[8], v3[8];
+  unpack8(s, v0);
+  unpack8(s + C, v1);
+  unpack8(s + row, v2);
+  unpack8(s + row + C, v3);
+  bf16x8 h;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) h[e] = (bf16)(0.25f * (v0[e] + v1[e] + v2[e] + v3[e]));
+  *reinterpret_cast<bf16x8*>(dst + (size_t)blockIdx.y * H * W * C + (size_t)i * 8) = h;
+}
+
+// pool2_back_kernel with out for C % 8 == 0, one thread per 8 channels of a
+// source pixel: bound by its 9 bytes per value (455 -> 173 us for the three
+// levels of 8 x 512 x 512 x 32; 99 us, 6.1 TB/s, at the largest).  grid.y = b.
+__global__ __launch_bounds__(256) void pool2_back_vec_kernel(const float* __restrict__ dv,
+                                                             const float* __restrict__ gsrc, bf16* __restrict__ out,
+                                                             const bf16* __restrict__ mask, int H, int W, int C8) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= 4 * H * W * C8) return;
+  const int p = i / C8, c = (i - p * C8) * 8, y = p / (2 * W), x = p - y * 2 * W, C = C8 * 8;
+  const size_t o = (size_t)blockIdx.y * 4 * H * W * C + (size_t)i * 8;
+  const f32x4* const d = reinterpret_cast<const f32x4*>(dv + (((size_t)blockIdx.y * H + y / 2) * W + x / 2) * C + c);
+  const f32x4* const s = reinterpret_cast<const f32x4*>(gsrc + o);
+  const f32x4 d0 = d[0], d1 = d[1], s0 = s[0], s1 = s[1];
+  float m[8];
+  unpack8(mask + o, m);
+  bf16x8 h;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = (e < 4 ? s0[e & 3] : s1[e & 3]) + 0.25f * (e < 4 ? d0[e & 3] : d1[e & 3]);
+    h[e] = (bf16)(m[e] > 0.0f ? v : 0.0f);
+  }
+  *reinterpret_cast<bf16x8*>(out + o) = h;
+}
+
 // g_src[b][2y+i][2x+j][c] += dv[b][y][x][c] / 4   (one thread per source element)
 // gsrc += dv / 4 over each 2x2 block; with out (bf16) the sum, masked by
 // mask > 0, goes to out instead (the last contribution to that gradient)
@@ -849,6 +941,60 @@ __global__ __launch_bounds__(256) void head_wgrad_kernel(const float* __restrict
   }
 }
 
+// head_back_kernel with out and head_wgrad_kernel in one pass over d0, for C =
+// 8 C8 with C8 a power of two up to 16: block `split` takes 4096 rows, C8
+// threads per row with 8 channels each.  Bound by its 4 C + 12 bytes per row
+// (mask and d0 being the same tensor, as in the network, 6 C bytes less than
+// the two kernels moved): 443 -> 69 us at 8 x 512 x 512 x 32.
+__global__ __launch_bounds__(256) void head_back_vec_kernel(const float* __restrict__ y,
+                                                            const float* __restrict__ target,
+                                                            const float* __restrict__ w, const bf16* __restrict__ d0,
+                                                            float* __restrict__ dy, bf16* __restrict__ out,
+                                                            const bf16* __restrict__ mask, float* __restrict__ part,
+                                                            long long M, int C8, float scale) {
+  __shared__ float red[256][9];
+  const int lg = threadIdx.x & (C8 - 1), rl = threadIdx.x / C8, nrl = 256 / C8, C = C8 * 8;
+  const long long r0 = (long long)blockIdx.x * 4096, r1 = r0 + 4096 < M ? r0 + 4096 : M;
+  const bool same = mask == d0;
+  float wc[8], acc[9];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) wc[e] = w[lg * 8 + e];
+#pragma unroll
+  for (int e = 0; e < 9; ++e) acc[e] = 0.0f;
+  for (long long r = r0 + rl; r < r1; r += nrl) {
+    const float d = scale * (y[r] - target[r]);
+    const long long o = r * C + lg * 8;
+    float v[8], m[8];
+    unpack8(d0 + o, v);
+    if (same) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] = v[e];
+    } else {
+      unpack8(mask + o, m);
+    }
+    bf16x8 h;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float g = d * wc[e];
+      h[e] = (bf16)(m[e] > 0.0f ? g : 0.0f);
+      acc[e] = __builtin_fmaf(d, v[e], acc[e]);
+    }
+    *reinterpret_cast<bf16x8*>(out + o) = h;
+    if (lg == 0) dy[r] = d;
+    acc[8] += d;
+  }
+#pragma unroll
+  for (int e = 0; e < 9; ++e) red[threadIdx.x][e] = acc[e];
+  __syncthreads();
+  // column c: the row lanes of its channel group, in order; column C: dy
+  for (int c = threadIdx.x; c <= C; c += 256) {
+    const int e = c < C ? c & 7 : 8, g = c < C ? c >> 3 : 0;
+    float t = 0.0f;
+    for (int k = 0; k < nrl; ++k) t += red[k * C8 + g][e];
+    part[(size_t)blockIdx.x * (C + 1) + c] = t;
+  }
+}
+
 // out = bf16(g * (act > 0))
 __global__ void relu_mask_kernel(const float* __restrict__ g, const bf16* __restrict__ act, bf16* __restrict__ out,
                                  long long n) {
@@ -902,29 +1048,50 @@ static inline unsigned blocks_for(long long n, int t = 256) { return (unsigned)(
 
 // 3x3 convolutions with cin % 32 == 0 (or cin == 8) and cout % 32 == 0 run
 // the halo-tiled kernel; the others the K-step-staged one.
-constexpr bool kHaloConv = true;
+static bool halo_conv(int cin, int cout) { return (cin % 32 == 0 || cin == 8) && cout % 32 == 0; }
+
+// 16-row tiles for 32 output channels, 8-row tiles and 64-channel blocks
+// otherwise.
+static int halo_block(int cout) { return cout % 64 == 0 ? 64 : 32; }
+
+static hipError_t launch_halo(const ConvArgs& a, hipStream_t s) {
+  const unsigned tiles16 = (unsigned)((a.W + 15) / 16), img = (unsigned)a.B;
+  if (halo_block(a.cout) == 64) {
+    const dim3 grid(tiles16 * (unsigned)((a.H + 7) / 8) * img, a.cout / 64);
+    if (a.cin == 8) conv3x3_halo_kernel<8, 64, 2, 2, 8><<<grid, 256, 0, s>>>(a);
+    else conv3x3_halo_kernel<8, 64, 2, 2, 32><<<grid, 256, 0, s>>>(a);
+  } else {
+    const dim3 grid(tiles16 * (unsigned)((a.H + 15) / 16) * img, a.cout / 32);
+    if (a.cin == 8) conv3x3_halo_kernel<16, 32, 4, 1, 8><<<grid, 256, 0, s>>>(a);
+    else conv3x3_halo_kernel<16, 32, 4, 1, 32><<<grid, 256, 0, s>>>(a);
+  }
+  return hipGetLastError();
+}
+
+// Whether nn_conv3x3_upback runs in one kernel: whole blocks of output
+// channels on either side of the concatenation.
+bool nn_upback_fused(int cin, int cout, int c0) { return halo_conv(cin, cout) && c0 % halo_block(cout) == 0; }
+
+// Input gradient of a convolution of [upsample2(low), skip], low's part summed
+// over 2 x 2 blocks and masked, in the convolution's epilogue: the FP32
+// gradient of the concatenation, written and read again, is 1.6 GB at 8 x 512 x
+// 512 x (64 + 32), and the two passes that split it took 614 us over the three
+// levels; the convolution itself takes no longer (250 -> 238 us at the largest).
+hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
+                             int H, int W, int cin, int cout, int c0, hipStream_t s) {
+  if (!nn_upback_fused(cin, cout, c0)) return hipErrorInvalidValue;
+  ConvArgs a{static_cast<const bf16*>(in), static_cast<const bf16*>(w), nullptr, nullptr, B, H, W, cin, cout, 0, 1,
+             nullptr, nullptr, 0, static_cast<bf16*>(low_out), static_cast<const bf16*>(low_mask), skip_out, c0};
+  return launch_halo(a, s);
+}
 
 hipError_t nn_conv3x3(const void* in, const void* in2, int c0, const void* w, const float* bias, void* out,
                       const void* mask, int B, int H, int W, int cin, int cout, int relu, int out_f32, hipStream_t s) {
   ConvArgs a{static_cast<const bf16*>(in), static_cast<const bf16*>(w), bias, out, B, H, W, cin, cout, relu, out_f32,
-             static_cast<const bf16*>(mask), static_cast<const bf16*>(in2), c0};
+             static_cast<const bf16*>(mask), static_cast<const bf16*>(in2), c0, nullptr, nullptr, nullptr, 0};
   const long long M = (long long)B * H * W;
   if (cin % 8 != 0) return hipErrorInvalidValue;
-  if (kHaloConv && (cin % 32 == 0 || cin == 8) && cout % 32 == 0) {
-    // halo-tiled kernel: 16-row tiles for 32 output channels, 8-row tiles
-    // and 64-channel blocks otherwise
-    const unsigned tiles16 = (unsigned)((W + 15) / 16), img = (unsigned)B;
-    if (cout % 64 == 0) {
-      const dim3 grid(tiles16 * (unsigned)((H + 7) / 8) * img, cout / 64);
-      if (cin == 8) conv3x3_halo_kernel<8, 64, 2, 2, 8><<<grid, 256, 0, s>>>(a);
-      else conv3x3_halo_kernel<8, 64, 2, 2, 32><<<grid, 256, 0, s>>>(a);
-    } else {
-      const dim3 grid(tiles16 * (unsigned)((H + 15) / 16) * img, cout / 32);
-      if (cin == 8) conv3x3_halo_kernel<16, 32, 4, 1, 8><<<grid, 256, 0, s>>>(a);
-      else conv3x3_halo_kernel<16, 32, 4, 1, 32><<<grid, 256, 0, s>>>(a);
-    }
-    return hipGetLastError();
-  }
+  if (halo_conv(cin, cout)) return launch_halo(a, s);
   if (cout % 128 == 0) {
     conv3x3_lds_kernel<128, 128, 2, 2><<<dim3(blocks_for(M, 128), cout / 128), 256, 0, s>>>(a);
   } else if (cout % 64 == 0) {
@@ -974,7 +1141,19 @@ hipError_t nn_pad_input(const float* x, void* out8, long long n, hipStream_t s) 
   return hipGetLastError();
 }
 
+// The vector kernels take 8 channels as aligned vectors, index one image in 32
+// bits and the image by grid.y.
+static bool aligned16(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
+}
+static bool vec8(long long per_image, int B, int C) { return C % 8 == 0 && per_image < (1LL << 31) && B < 65536; }
+
 hipError_t nn_pool2(const void* src, void* dst, int B, int H, int W, int C, hipStream_t s) {
+  if (vec8((long long)H * W * C, B, C) && aligned16(src, dst)) {
+    const dim3 grid(blocks_for((long long)H * W * (C / 8)), (unsigned)B);
+    pool2_vec_kernel<<<grid, 256, 0, s>>>(static_cast<const bf16*>(src), static_cast<bf16*>(dst), H, W, C / 8);
+    return hipGetLastError();
+  }
   pool2_kernel<<<blocks_for((long long)B * H * W * C), 256, 0, s>>>(static_cast<const bf16*>(src),
                                                                    static_cast<bf16*>(dst), B, H, W, C);
   return hipGetLastError();
@@ -982,6 +1161,12 @@ hipError_t nn_pool2(const void* src, void* dst, int B, int H, int W, int C, hipS
 
 hipError_t nn_pool2_back(const float* dv, float* gsrc, void* out, const void* mask, int B, int H, int W, int C,
                          hipStream_t s) {
+  if (out && vec8(4LL * H * W * C, B, C) && aligned16(dv, gsrc, out, mask)) {
+    const dim3 grid(blocks_for(4LL * H * W * (C / 8)), (unsigned)B);
+    pool2_back_vec_kernel<<<grid, 256, 0, s>>>(dv, gsrc, static_cast<bf16*>(out), static_cast<const bf16*>(mask), H, W,
+                                               C / 8);
+    return hipGetLastError();
+  }
   pool2_back_kernel<<<blocks_for((long long)B * 4 * H * W * C), 256, 0, s>>>(
       dv, gsrc, static_cast<bf16*>(out), static_cast<const bf16*>(mask), B, H, W, C);
   return hipGetLastError();
@@ -1012,6 +1197,15 @@ hipError_t nn_head(const void* d0, const float* w, const float* b, const float* 
 hipError_t nn_head_back(const float* y, const float* target, const float* w, const void* d0, float* dy, float* gd0,
                         void* gd0_out, const void* mask, float* gw, float* partial, long long M, int C,
                         hipStream_t s) {
+  const int c8 = C / 8;
+  if (gd0_out && C % 8 == 0 && c8 <= 16 && (c8 & (c8 - 1)) == 0 && aligned16(d0, gd0_out, mask)) {
+    const long long nb = (M + 4095) / 4096;
+    head_back_vec_kernel<<<(unsigned)nb, 256, 0, s>>>(y, target, w, static_cast<const bf16*>(d0), dy,
+                                                      static_cast<bf16*>(gd0_out), static_cast<const bf16*>(mask),
+                                                      partial, M, c8, 2.0f / (float)M);
+    reduce_partials_kernel<<<blocks_for(C + 1), 256, 0, s>>>(partial, gw, C + 1, (int)nb);
+    return hipGetLastError();
+  }
   head_back_kernel<<<blocks_for(M * C), 256, 0, s>>>(y, target, w, dy, gd0, static_cast<bf16*>(gd0_out),
                                                  static_cast<const bf16*>(mask), M, C, 2.0f / (float)M);
   const long long ns = (M + 4095) / 4096;

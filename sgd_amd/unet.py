@@ -242,16 +242,19 @@ class UNet:
             gy2 = self._get("gy%d_a" % l, (B, h, w, ca.cout), bf)
             self._input_grad(cb, gy, gy2, B, h, w, mask=t["dec%d_a" % l])
             self._conv_grads(ca, t["dec%d_in" % l], gy2, B, h, w)
-            gin = self._get("gin%d" % l, (B, h, w, ca.cin), f32)
-            self._input_grad(ca, gy2, gin, B, h, w)
-            cs = genc[l].shape[3]
-            cu = ca.cin - cs
             if l + 1 < L_ - 1:
                 low_out, low_mask = gyb[l + 1], t["dec%d_b" % (l + 1)]
             else:
                 low_out, low_mask = gyeb[L_ - 1], t["enc%d_b" % (L_ - 1)]
-            self._chk(L.sgdct_nn_upcat_back(_vp(gin), None, _vp(low_out), _vp(low_mask), _vp(genc[l]), 0, B, h, w,
-                                            cu, cs, self._s()), "upcat_back")
+            # the input gradient of the concatenation, split as it is stored:
+            # the level below's masked 2x2 sums, the skip part in FP32
+            cu = ca.cin - genc[l].shape[3]
+            n = L.sgdct_nn_conv3x3_upback_workspace(B, h, w, ca.cout, ca.cin, cu)
+            gin = self._get("gin%d" % l, (n,), f32) if n > 0 else None
+            self._chk(L.sgdct_nn_flip_weights(_vp(ca.w16), _vp(ca.wt16), ca.cin, ca.cout, self._s()), "flip")
+            self._chk(L.sgdct_nn_conv3x3_upback(_vp(gy2), _vp(ca.wt16), _vp(low_out), _vp(low_mask), _vp(genc[l]),
+                                                _vp(gin) if n > 0 else None, n, B, h, w, ca.cout, ca.cin, cu,
+                                                self._s()), "conv3x3_upback " + ca.name)
         for l in range(L_ - 1, -1, -1):
             h, w = H >> l, W >> l
             ca, cb = self.convs["enc%d_a" % l], self.convs["enc%d_b" % l]
