@@ -58,7 +58,7 @@ hipError_t nn_conv3x3(const void* in, const void* in2, int c0, const void* w, co
 bool nn_upback_fused(int cin, int cout, int c0);
 hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
                              int H, int W, int cin, int cout, int c0, hipStream_t s);
-long long nn_wgrad_splits(long long M);
+long long nn_wgrad_parts(int B, int H, int W, int cin, int cout);
 hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float* dw, float* db, float* partial, int B,
                     int H, int W, int cin, int cout, hipStream_t s);
 hipError_t nn_colsum_bf16(const void* a, float* out, float* partial, long long M, int C, hipStream_t s);
@@ -1779,7 +1779,7 @@ int sgdct_nn_conv3x3_upback(const void* in, const void* w, void* low_out, const 
 
 long long sgdct_nn_wgrad_workspace(int B, int H, int W, int cin, int cout) {
   if (!dims_ok(B, H, W) || cin <= 0 || cout <= 0) return fail(SGDCT_EINVAL, "bad wgrad shape");
-  return nn_wgrad_splits((long long)B * H * W) * cout * (9LL * cin + 1);
+  return nn_wgrad_parts(B, H, W, cin, cout) * cout * (9LL * cin + 1);
 }
 
 int sgdct_nn_wgrad(const void* x, const void* dy, float* dw, float* workspace, long long workspace_floats, int B,

@@ -664,19 +664,226 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
   }
 }
 
-// out[i] = sum_s partial[s][i] (fixed order)
-__global__ void reduce_partials_kernel(const float* __restrict__ partial, float* __restrict__ out, long long n,
-                                       int nsplit) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float p4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  int k = 0;
-  for (; k + 3 < nsplit; k += 4) {
+// ---------------------------------------------------------------------------
+// The same gradient with its operands staged once per spatial tile and input-
+// channel chunk, for cin and cout multiples of 32 (or cin 8): the block walks tiles of 4 x
+// 32 pixels, stages a tile's dY [128 pixels][CO_T] and the (6 x 34)-pixel halo
+// of 32 input channels of X in LDS, and forms all nine taps' products from
+// them (288 columns k of dW), where wgrad_kernel gathers X once per tap.  Each
+// wave holds 32 co x 9 taps x 16 channels (18 MFMA tiles): CO_T 64: waves =
+// co halves x channel halves; CO_T 32: channel halves x row pairs of the tile,
+// added through LDS at the end.  One MFMA step is one row of 32 pixels, so the
+// three fragments (kx) of a halo row serve the three taps ky whose tile rows
+// lie at it: 26 fragment reads per 72 MFMAs, where a step of two 16-pixel rows
+// needs 88 and is bound by them.  Double-buffered LDS, the next tile's loads in
+// flight during the MFMAs, one barrier per tile; pixels outside the image stage
+// dY = 0.  CC = 8 (the network's first layer, bound by reading dY): 32 co x 9
+// taps x 8 channels per wave as five tiles of two taps each (the tenth is
+// dropped), the waves one tile row each.
+// At 8 x 512 x 512: 32 -> 32 channels 211 -> 77 us (268 MB; 500 TF/s), 96 -> 32
+// 476 -> 200 us, 8 -> 32 180 -> 48 us; at 8 x 256 x 256 64 -> 64 167 -> 57 us
+// (680 TF/s), 192 -> 64 339 -> 143 us.
+// ---------------------------------------------------------------------------
+constexpr int kWgTH = 4, kWgTW = 32;
+
+template <int CO_T, int CC>
+__global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int tiles_per_split) {
+  static_assert(CC == 32 ? CO_T == 64 || CO_T == 32 : CC == 8 && CO_T == 32, "co tile 64 or 32");
+  constexpr int PW = CC == 8 ? 4 : CO_T == 32 ? 2 : 1, TR = kWgTH / PW;  // waves along the rows; rows per wave
+  constexpr int NP = kWgTH * kWgTW, HH = kWgTH + 2, HW = kWgTW + 2;
+  constexpr int SD = CO_T + 16, SX = CC == 8 ? 8 : 48;  // LDS row strides (bf16)
+  constexpr int XG = CC / 8, NB = CC == 8 ? 5 : 9;       // groups per halo pixel; column tiles per wave
+  constexpr int DG = CO_T / 8, DC = NP * DG / 256, NX = HH * HW * XG, XC = (NX + 255) / 256;  // 16-byte groups
+  constexpr int BUF = NP * SD + HH * HW * SX;
+  static_assert(2 * BUF * (int)sizeof(bf16) >= (CC == 8 ? 1 : 2) * 8 * NB * 64 * (int)sizeof(float), "the final sums fit the tiles");
+  __shared__ __attribute__((aligned(16))) bf16 smem[2 * BUF];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int wa = wv & 1, wb = wv >> 1;
+  const int wco = CO_T == 64 ? wa * 32 : 0;     // this wave's first co
+  const int wch = CC == 8 ? 0 : (CO_T == 64 ? wb : wa) * 16;  // and input channel
+  const int part = PW == 4 ? wv : PW == 2 ? wb : 0, wr = part * TR;  // and tile row
+  const int K = 9 * a.cin;
+  const int co0 = blockIdx.x * CO_T, ch0 = blockIdx.y * CC;
+  const int tiles_x = (a.W + kWgTW - 1) / kWgTW, tiles_y = (a.H + kWgTH - 1) / kWgTH;
+  const int ntile = tiles_x * tiles_y * a.B;
+  const int t_begin = blockIdx.z * tiles_per_split, t_end = min(ntile, t_begin + tiles_per_split);
+
+  f32x4 acc[2][NB];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) p4[j] += partial[(size_t)(k + j) * n + i];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const bool bias = a.bias_partial && blockIdx.y == 0;
+  float bs[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+
+  bf16x8 rd[DC], rx[XC];
+  auto load = [&](int t) {
+    const int tx = t % tiles_x, r = t / tiles_x, ty = r % tiles_y, b = r / tiles_y;
+    const int x0 = tx * kWgTW, y0 = ty * kWgTH;
+#pragma unroll
+    for (int i = 0; i < DC; ++i) {
+      const int q = tid + 256 * i, p = q / DG, cg = (q % DG) * 8;
+      const int y = y0 + p / kWgTW, x = x0 + p % kWgTW;
+      rd[i] = zero8();
+      if (y < a.H && x < a.W)
+        rd[i] = *reinterpret_cast<const bf16x8*>(a.dy + (((size_t)b * a.H + y) * a.W + x) * a.cout + co0 + cg);
+    }
+#pragma unroll
+    for (int i = 0; i < XC; ++i) {
+      const int q = tid + 256 * i, p = q / XG, cg = (q % XG) * 8;
+      const int hy = p / HW, y = y0 + hy - 1, x = x0 + p - hy * HW - 1;
+      rx[i] = zero8();
+      if (q < NX && y >= 0 && y < a.H && x >= 0 && x < a.W)
+        rx[i] = *reinterpret_cast<const bf16x8*>(conv_in(a.x, a.x2, a.c0, a.H, a.W, a.cin, b, y, x, ch0 + cg));
+    }
+  };
+  if (t_begin < t_end) load(t_begin);
+  for (int t = t_begin; t < t_end; ++t) {
+    bf16* const sd = smem + ((t - t_begin) & 1) * BUF;
+    bf16* const sx = sd + NP * SD;
+#pragma unroll
+    for (int i = 0; i < DC; ++i) {
+      const int q = tid + 256 * i;
+      *reinterpret_cast<bf16x8*>(&sd[(q / DG) * SD + (q % DG) * 8]) = rd[i];
+      if (bias) {
+        const i16x8 u = __builtin_bit_cast(i16x8, rd[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bs[e] += __uint_as_float((unsigned)(unsigned short)u[e] << 16);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < XC; ++i) {
+      const int q = tid + 256 * i;
+      if (q < NX) *reinterpret_cast<bf16x8*>(&sx[(q / XG) * SX + (q % XG) * 8]) = rx[i];
+    }
+    __syncthreads();
+    if (t + 1 < t_end) load(t + 1);
+    const int row = 8 * g + (r16 >> 2), col = 4 * (r16 & 3);
+    if constexpr (CC == 8) {
+      const bf16x8 a0 = tr_fragment(sd, wr * kWgTW + row, col, SD);
+      const bf16x8 a1 = tr_fragment(sd, wr * kWgTW + row, 16 + col, SD);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int tap = min(2 * j + ((r16 & 3) >> 1), 8);
+        const bf16x8 fb = tr_fragment(sx, (wr + tap / 3) * HW + row + tap % 3, 4 * (r16 & 1), SX);
+        acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, fb, acc[0][j], 0, 0, 0);
+        acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, fb, acc[1][j], 0, 0, 0);
+      }
+      continue;
+    }
+    bf16x8 fa[TR][2];
+#pragma unroll
+    for (int hr = 0; hr < TR + 2; ++hr) {  // halo rows wr + hr; tile rows wr + hr - ky
+      if (hr < TR) {
+        fa[hr][0] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + col, SD);
+        fa[hr][1] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + 16 + col, SD);
+      }
+#pragma unroll
+      for (int kx = 0; kx < 3; ++kx) {
+        const bf16x8 fb = tr_fragment(sx, (wr + hr) * HW + row + kx, wch + col, SX);
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) {
+          const int r = hr - ky, j = (3 * ky + kx) % NB;
+          if (r < 0 || r >= TR) continue;
+          acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][0], fb, acc[0][j], 0, 0, 0);
+          acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][1], fb, acc[1][j], 0, 0, 0);
+        }
+      }
+    }
   }
-  for (int j = 0; k < nsplit; ++k, ++j) p4[j & 3] += partial[(size_t)k * n + i];
-  out[i] = (p4[0] + p4[1]) + (p4[2] + p4[3]);
+  float* const red = reinterpret_cast<float*>(smem);
+  float* const mine = red + (PW == 2 ? wa : 0) * 8 * NB * 64 + lane;
+#pragma unroll
+  for (int k = 1; k < PW; ++k) {  // the waves' sums, in the order of their rows
+    __syncthreads();
+    if (part == k)
+#pragma unroll
+      for (int i = 0; i < 2 * NB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mine[(4 * i + r) * 64] = acc[i / NB][i % NB][r];
+    __syncthreads();
+    if (part == 0)
+#pragma unroll
+      for (int i = 0; i < 2 * NB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i / NB][i % NB][r] += mine[(4 * i + r) * 64];
+  }
+  if (part == 0) {
+    float* const out = a.partial + (size_t)blockIdx.z * a.cout * K;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int co = co0 + wco + 16 * i + 4 * g + r, k = CC == 8 ? 16 * j + r16 : j * a.cin + ch0 + wch + r16;
+          if (CC == 32 || k < K) out[(size_t)co * K + k] = acc[i][j][r];
+        }
+  }
+  if (bias) {
+    // the threads of a channel group, added in thread order through LDS
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[tid * 8 + e] = bs[e];
+    __syncthreads();
+    if (tid < CO_T) {
+      const int grp = tid / 8, e = tid % 8;
+      float t = 0.0f;
+      for (int j = grp; j < 256; j += DG) t += red[j * 8 + e];
+      a.bias_partial[(size_t)blockIdx.z * a.cout + co0 + tid] = t;
+    }
+  }
+}
+
+// out[i] = sum_s partial[s][i] in a fixed order: 64 columns per block, four per
+// thread (16-byte loads), 16 threads per column with every 16th partial each,
+// added in thread order.  Two arrays (the weights' n, the bias's n2) in one
+// launch.  Bound by reading the partials: 10.5 -> 7.2 us a launch on average
+// over a gradient step at 8 x 512 x 512, against one thread per column.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ partial,
+                                                              float* __restrict__ out, long long n,
+                                                              const float* __restrict__ partial2,
+                                                              float* __restrict__ out2, int n2, int nsplit) {
+  __shared__ f32x4 red[16][16];
+  const int c = threadIdx.x & 15, s = threadIdx.x >> 4;
+  const long long nb = (n + 63) / 64;
+  const bool second = blockIdx.x >= nb;
+  const long long i = ((long long)blockIdx.x - (second ? nb : 0)) * 64 + 4 * c, m = second ? n2 : n;
+  const float* const p = second ? partial2 : partial;
+  f32x4 t = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (i + 4 <= m) {
+    f32x4 u = t;
+    int k = s;
+    for (; k + 48 < nsplit; k += 64) {
+      const f32x4 v0 = *reinterpret_cast<const f32x4u*>(p + (size_t)k * m + i);
+      const f32x4 v1 = *reinterpret_cast<const f32x4u*>(p + (size_t)(k + 16) * m + i);
+      const f32x4 v2 = *reinterpret_cast<const f32x4u*>(p + (size_t)(k + 32) * m + i);
+      const f32x4 v3 = *reinterpret_cast<const f32x4u*>(p + (size_t)(k + 48) * m + i);
+      t += v0 + v1;
+      u += v2 + v3;
+    }
+    for (; k < nsplit; k += 16) t += *reinterpret_cast<const f32x4u*>(p + (size_t)k * m + i);
+    t += u;
+  } else {
+    for (int k = s; k < nsplit; k += 16)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < m) t[e] += p[(size_t)k * m + i + e];
+  }
+  red[s][c] = t;
+  __syncthreads();
+  if (s == 0) {
+    f32x4 u = red[0][c];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) u += red[k][c];
+    float* const o = second ? out2 : out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < m) o[i + e] = u[e];
+  }
 }
 
 // Column sums of an [M][C] bf16 or FP32 matrix into partial[split][C]: block
@@ -1076,7 +1283,8 @@ bool nn_upback_fused(int cin, int cout, int c0) { return halo_conv(cin, cout) &&
 // over 2 x 2 blocks and masked, in the convolution's epilogue: the FP32
 // gradient of the concatenation, written and read again, is 1.6 GB at 8 x 512 x
 // 512 x (64 + 32), and the two passes that split it took 614 us over the three
-// levels; the convolution itself takes no longer (250 -> 238 us at the largest).
+// levels; the step's 32-channel-block convolutions, the largest of these among
+// them, take no longer for it (910 -> 882 us together).
 hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
                              int H, int W, int cin, int cout, int c0, hipStream_t s) {
   if (!nn_upback_fused(cin, cout, c0)) return hipErrorInvalidValue;
@@ -1110,30 +1318,65 @@ long long nn_wgrad_splits(long long M) {
   return n < 1 ? 1 : n;
 }
 
-// partial holds nsplit * cout * (9 cin + 1) floats: the weight partials,
-// then (with db) the bias partials.
+static hipError_t reduce_partials(const float* partial, float* out, long long n, const float* partial2, float* out2,
+                                  int n2, long long rows, hipStream_t s) {
+  const long long nb = (n + 63) / 64 + (n2 + 63) / 64;
+  reduce_partials_kernel<<<(unsigned)nb, 256, 0, s>>>(partial, out, n, partial2, out2, n2, (int)rows);
+  return hipGetLastError();
+}
+
+static bool halo_wgrad(int cin, int cout) { return (cin % 32 == 0 || cin == 8) && cout % 32 == 0; }
+static int halo_wgrad_co(int cin, int cout) { return cin != 8 && cout % 64 == 0 ? 64 : 32; }
+
+// Pixel-range splits of wgrad_halo_kernel: as many as give the launch its two
+// workgroups per CU at once, with at least 4 tiles each.
+static int halo_wgrad_splits(int B, int H, int W, int cin, int cout) {
+  const long long ntile = (long long)B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH);
+  const long long blocks = (long long)(cout / halo_wgrad_co(cin, cout)) * (cin == 8 ? 1 : cin / 32);
+  long long n = 512 / blocks;
+  if (n > ntile / 4) n = ntile / 4;
+  return (int)(n < 1 ? 1 : n);
+}
+
+// Rows of partial sums a weight gradient may need: each holds cout * (9 cin +
+// 1) floats, the weight partials of all rows first, then the bias partials.
+long long nn_wgrad_parts(int B, int H, int W, int cin, int cout) {
+  const long long n = nn_wgrad_splits((long long)B * H * W);
+  if (!halo_wgrad(cin, cout)) return n;
+  const long long h = halo_wgrad_splits(B, H, W, cin, cout);
+  return h > n ? h : n;
+}
+
 hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float* dw, float* db, float* partial, int B,
                     int H, int W, int cin, int cout, hipStream_t s) {
   const long long M = (long long)B * H * W;
-  const long long ns = nn_wgrad_splits(M);
-  const long long per = ((M + ns - 1) / ns + 63) / 64 * 64;
   const int K = 9 * cin;
-  float* bpart = db ? partial + ns * cout * K : nullptr;
+  const bool halo = halo_wgrad(cin, cout) && (!x2 || c0 % 32 == 0) &&
+                    (long long)B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH) < (1LL << 30);
+  long long parts = nn_wgrad_splits(M);
+  const long long per = ((M + parts - 1) / parts + 63) / 64 * 64;
   WgradArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(dy), partial, B, H, W, cin, cout, per,
-              static_cast<const bf16*>(x2), c0, bpart};
-  if (cout <= 32) wgrad_kernel<32><<<dim3(1, (K + 127) / 128, (unsigned)ns), 256, 0, s>>>(a);
-  else wgrad_kernel<64><<<dim3((cout + 63) / 64, (K + 63) / 64, (unsigned)ns), 256, 0, s>>>(a);
-  const long long n = (long long)cout * K;
-  reduce_partials_kernel<<<blocks_for(n), 256, 0, s>>>(partial, dw, n, (int)ns);
-  if (db) reduce_partials_kernel<<<blocks_for(cout), 256, 0, s>>>(bpart, db, cout, (int)ns);
-  return hipGetLastError();
+              static_cast<const bf16*>(x2), c0, nullptr};
+  if (halo) {
+    const int ns = halo_wgrad_splits(B, H, W, cin, cout);
+    const int ntile = B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH), tps = (ntile + ns - 1) / ns;
+    parts = ns;
+    a.bias_partial = db ? partial + parts * cout * K : nullptr;
+    if (cin == 8) wgrad_halo_kernel<32, 8><<<dim3(cout / 32, 1, ns), 256, 0, s>>>(a, tps);
+    else if (cout % 64 == 0) wgrad_halo_kernel<64, 32><<<dim3(cout / 64, cin / 32, ns), 256, 0, s>>>(a, tps);
+    else wgrad_halo_kernel<32, 32><<<dim3(cout / 32, cin / 32, ns), 256, 0, s>>>(a, tps);
+  } else {
+    a.bias_partial = db ? partial + parts * cout * K : nullptr;
+    if (cout <= 32) wgrad_kernel<32><<<dim3(1, (K + 127) / 128, (unsigned)parts), 256, 0, s>>>(a);
+    else wgrad_kernel<64><<<dim3((cout + 63) / 64, (K + 63) / 64, (unsigned)parts), 256, 0, s>>>(a);
+  }
+  return reduce_partials(partial, dw, (long long)cout * K, a.bias_partial, db, db ? cout : 0, parts, s);
 }
 
 hipError_t nn_colsum_bf16(const void* a, float* out, float* partial, long long M, int C, hipStream_t s) {
   const long long ns = (M + 4095) / 4096;
   colsum_kernel<bf16><<<(unsigned)ns, 256, 0, s>>>(static_cast<const bf16*>(a), partial, M, C, 4096);
-  reduce_partials_kernel<<<blocks_for(C), 256, 0, s>>>(partial, out, C, (int)ns);
-  return hipGetLastError();
+  return reduce_partials(partial, out, C, nullptr, nullptr, 0, ns, s);
 }
 
 hipError_t nn_pad_input(const float* x, void* out8, long long n, hipStream_t s) {
@@ -1203,15 +1446,13 @@ hipError_t nn_head_back(const float* y, const float* target, const float* w, con
     head_back_vec_kernel<<<(unsigned)nb, 256, 0, s>>>(y, target, w, static_cast<const bf16*>(d0), dy,
                                                       static_cast<bf16*>(gd0_out), static_cast<const bf16*>(mask),
                                                       partial, M, c8, 2.0f / (float)M);
-    reduce_partials_kernel<<<blocks_for(C + 1), 256, 0, s>>>(partial, gw, C + 1, (int)nb);
-    return hipGetLastError();
+    return reduce_partials(partial, gw, C + 1, nullptr, nullptr, 0, nb, s);
   }
   head_back_kernel<<<blocks_for(M * C), 256, 0, s>>>(y, target, w, dy, gd0, static_cast<bf16*>(gd0_out),
                                                  static_cast<const bf16*>(mask), M, C, 2.0f / (float)M);
   const long long ns = (M + 4095) / 4096;
   head_wgrad_kernel<<<(unsigned)ns, 256, 0, s>>>(dy, static_cast<const bf16*>(d0), partial, M, C, 4096);
-  reduce_partials_kernel<<<blocks_for(C + 1), 256, 0, s>>>(partial, gw, C + 1, (int)ns);
-  return hipGetLastError();
+  return reduce_partials(partial, gw, C + 1, nullptr, nullptr, 0, ns, s);
 }
 
 hipError_t nn_relu_mask(const float* g, const void* act, void* out, long long n, hipStream_t s) {
