@@ -666,20 +666,20 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
 
 // ---------------------------------------------------------------------------
 // The same gradient with its operands staged once per spatial tile and input-
-// channel chunk, for cin and cout multiples of 32 (or cin 8): the block walks tiles of 4 x
+// channel chunk, for cin and cout multiples of 16 (or cin 8): the block walks tiles of 4 x
 // 32 pixels, stages a tile's dY [128 pixels][CO_T] and the (6 x 34)-pixel halo
-// of 32 input channels of X in LDS, and forms all nine taps' products from
-// them (288 columns k of dW), where wgrad_kernel gathers X once per tap.  Each
-// wave holds 32 co x 9 taps x 16 channels (18 MFMA tiles): CO_T 64: waves =
-// co halves x channel halves; CO_T 32: channel halves x row pairs of the tile,
-// added through LDS at the end.  One MFMA step is one row of 32 pixels, so the
+// of CC input channels of X in LDS, and forms all nine taps' products from
+// them, where wgrad_kernel gathers X once per tap.  Each wave holds up to 32 co
+// x 9 taps x 16 channels (18 MFMA tiles).  CC = 32: CO_T 64: waves = co halves
+// x channel halves; CO_T 32: channel halves x row pairs of the tile, added
+// through LDS at the end; CC = 16: one tile row per wave.  One MFMA step is one row of 32 pixels, so the
 // three fragments (kx) of a halo row serve the three taps ky whose tile rows
 // lie at it: 26 fragment reads per 72 MFMAs, where a step of two 16-pixel rows
 // needs 88 and is bound by them.  Double-buffered LDS, the next tile's loads in
 // flight during the MFMAs, one barrier per tile; pixels outside the image stage
 // dY = 0.  CC = 8 (the network's first layer, bound by reading dY): 32 co x 9
 // taps x 8 channels per wave as five tiles of two taps each (the tenth is
-// dropped), the waves one tile row each.
+// dropped), one tile row per wave.
 // At 8 x 512 x 512: 32 -> 32 channels 211 -> 77 us (268 MB; 500 TF/s), 96 -> 32
 // 476 -> 200 us, 8 -> 32 180 -> 48 us; at 8 x 256 x 256 64 -> 64 167 -> 57 us
 // (680 TF/s), 192 -> 64 339 -> 143 us.
@@ -688,20 +688,20 @@ constexpr int kWgTH = 4, kWgTW = 32;
 
 template <int CO_T, int CC>
 __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int tiles_per_split) {
-  static_assert(CC == 32 ? CO_T == 64 || CO_T == 32 : CC == 8 && CO_T == 32, "co tile 64 or 32");
-  constexpr int PW = CC == 8 ? 4 : CO_T == 32 ? 2 : 1, TR = kWgTH / PW;  // waves along the rows; rows per wave
+  static_assert(CC == 32 ? CO_T == 64 || CO_T == 32 : (CC == 8 || CC == 16) && CO_T <= 32, "tile");
+  constexpr int PW = CC < 32 ? 4 : CO_T == 32 ? 2 : 1, TR = kWgTH / PW;  // waves along the rows; rows per wave
   constexpr int NP = kWgTH * kWgTW, HH = kWgTH + 2, HW = kWgTW + 2;
-  constexpr int SD = CO_T + 16, SX = CC == 8 ? 8 : 48;  // LDS row strides (bf16)
-  constexpr int XG = CC / 8, NB = CC == 8 ? 5 : 9;       // groups per halo pixel; column tiles per wave
+  constexpr int SD = CO_T + 16, SX = CC < 32 ? CC : 48;  // LDS row strides (bf16)
+  constexpr int XG = CC / 8, NB = CC == 8 ? 5 : 9, NI = CO_T == 16 ? 1 : 2;  // groups per halo pixel; tiles per wave
   constexpr int DG = CO_T / 8, DC = NP * DG / 256, NX = HH * HW * XG, XC = (NX + 255) / 256;  // 16-byte groups
   constexpr int BUF = NP * SD + HH * HW * SX;
-  static_assert(2 * BUF * (int)sizeof(bf16) >= (CC == 8 ? 1 : 2) * 8 * NB * 64 * (int)sizeof(float), "the final sums fit the tiles");
+  static_assert(2 * BUF * (int)sizeof(bf16) >= (CC < 32 ? 1 : 2) * 4 * NI * NB * 64 * (int)sizeof(float), "the final sums fit the tiles");
   __shared__ __attribute__((aligned(16))) bf16 smem[2 * BUF];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int r16 = lane & 15, g = lane >> 4;
   const int wa = wv & 1, wb = wv >> 1;
   const int wco = CO_T == 64 ? wa * 32 : 0;     // this wave's first co
-  const int wch = CC == 8 ? 0 : (CO_T == 64 ? wb : wa) * 16;  // and input channel
+  const int wch = CC < 32 ? 0 : (CO_T == 64 ? wb : wa) * 16;  // and input channel
   const int part = PW == 4 ? wv : PW == 2 ? wb : 0, wr = part * TR;  // and tile row
   const int K = 9 * a.cin;
   const int co0 = blockIdx.x * CO_T, ch0 = blockIdx.y * CC;
@@ -709,9 +709,9 @@ __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int til
   const int ntile = tiles_x * tiles_y * a.B;
   const int t_begin = blockIdx.z * tiles_per_split, t_end = min(ntile, t_begin + tiles_per_split);
 
-  f32x4 acc[2][NB];
+  f32x4 acc[NI][NB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const bool bias = a.bias_partial && blockIdx.y == 0;
@@ -760,25 +760,26 @@ __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int til
     __syncthreads();
     if (t + 1 < t_end) load(t + 1);
     const int row = 8 * g + (r16 >> 2), col = 4 * (r16 & 3);
+    bf16x8 fa[TR][NI];
     if constexpr (CC == 8) {
-      const bf16x8 a0 = tr_fragment(sd, wr * kWgTW + row, col, SD);
-      const bf16x8 a1 = tr_fragment(sd, wr * kWgTW + row, 16 + col, SD);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) fa[0][i] = tr_fragment(sd, wr * kWgTW + row, 16 * i + col, SD);
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const int tap = min(2 * j + ((r16 & 3) >> 1), 8);
         const bf16x8 fb = tr_fragment(sx, (wr + tap / 3) * HW + row + tap % 3, 4 * (r16 & 1), SX);
-        acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, fb, acc[0][j], 0, 0, 0);
-        acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, fb, acc[1][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0][i], fb, acc[i][j], 0, 0, 0);
       }
       continue;
     }
-    bf16x8 fa[TR][2];
 #pragma unroll
     for (int hr = 0; hr < TR + 2; ++hr) {  // halo rows wr + hr; tile rows wr + hr - ky
-      if (hr < TR) {
-        fa[hr][0] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + col, SD);
-        fa[hr][1] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + 16 + col, SD);
-      }
+      if (hr < TR)
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          fa[hr][i] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + 16 * i + col, SD);
 #pragma unroll
       for (int kx = 0; kx < 3; ++kx) {
         const bf16x8 fb = tr_fragment(sx, (wr + hr) * HW + row + kx, wch + col, SX);
@@ -786,39 +787,40 @@ __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int til
         for (int ky = 0; ky < 3; ++ky) {
           const int r = hr - ky, j = (3 * ky + kx) % NB;
           if (r < 0 || r >= TR) continue;
-          acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][0], fb, acc[0][j], 0, 0, 0);
-          acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][1], fb, acc[1][j], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < NI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][i], fb, acc[i][j], 0, 0, 0);
         }
       }
     }
   }
   float* const red = reinterpret_cast<float*>(smem);
-  float* const mine = red + (PW == 2 ? wa : 0) * 8 * NB * 64 + lane;
+  float* const mine = red + (PW == 2 ? wa : 0) * 4 * NI * NB * 64 + lane;
 #pragma unroll
   for (int k = 1; k < PW; ++k) {  // the waves' sums, in the order of their rows
     __syncthreads();
     if (part == k)
 #pragma unroll
-      for (int i = 0; i < 2 * NB; ++i)
+      for (int i = 0; i < NI * NB; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mine[(4 * i + r) * 64] = acc[i / NB][i % NB][r];
     __syncthreads();
     if (part == 0)
 #pragma unroll
-      for (int i = 0; i < 2 * NB; ++i)
+      for (int i = 0; i < NI * NB; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i / NB][i % NB][r] += mine[(4 * i + r) * 64];
   }
   if (part == 0) {
     float* const out = a.partial + (size_t)blockIdx.z * a.cout * K;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int co = co0 + wco + 16 * i + 4 * g + r, k = CC == 8 ? 16 * j + r16 : j * a.cin + ch0 + wch + r16;
-          if (CC == 32 || k < K) out[(size_t)co * K + k] = acc[i][j][r];
+          if (CC != 8 || k < K) out[(size_t)co * K + k] = acc[i][j][r];
         }
   }
   if (bias) {
@@ -1325,14 +1327,19 @@ static hipError_t reduce_partials(const float* partial, float* out, long long n,
   return hipGetLastError();
 }
 
-static bool halo_wgrad(int cin, int cout) { return (cin % 32 == 0 || cin == 8) && cout % 32 == 0; }
-static int halo_wgrad_co(int cin, int cout) { return cin != 8 && cout % 64 == 0 ? 64 : 32; }
+// wgrad_halo_kernel's shapes and its tile: input channels per chunk (0: none),
+// output channels per block.  16-channel tiles serve what 32 does not divide.
+static int halo_wgrad_cc(int cin, int cout) {
+  if (cout % 16 != 0) return 0;
+  return cin == 8 ? 8 : cin % 32 == 0 && cout % 32 == 0 ? 32 : cin % 16 == 0 ? 16 : 0;
+}
+static int halo_wgrad_co(int cc, int cout) { return cc == 32 && cout % 64 == 0 ? 64 : cout % 32 == 0 ? 32 : 16; }
 
 // Pixel-range splits of wgrad_halo_kernel: as many as give the launch its two
 // workgroups per CU at once, with at least 4 tiles each.
-static int halo_wgrad_splits(int B, int H, int W, int cin, int cout) {
+static int halo_wgrad_splits(int B, int H, int W, int cin, int cout, int cc) {
   const long long ntile = (long long)B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH);
-  const long long blocks = (long long)(cout / halo_wgrad_co(cin, cout)) * (cin == 8 ? 1 : cin / 32);
+  const long long blocks = (long long)(cout / halo_wgrad_co(cc, cout)) * (cin / cc);
   long long n = 512 / blocks;
   if (n > ntile / 4) n = ntile / 4;
   return (int)(n < 1 ? 1 : n);
@@ -1342,8 +1349,9 @@ static int halo_wgrad_splits(int B, int H, int W, int cin, int cout) {
 // 1) floats, the weight partials of all rows first, then the bias partials.
 long long nn_wgrad_parts(int B, int H, int W, int cin, int cout) {
   const long long n = nn_wgrad_splits((long long)B * H * W);
-  if (!halo_wgrad(cin, cout)) return n;
-  const long long h = halo_wgrad_splits(B, H, W, cin, cout);
+  const int cc = halo_wgrad_cc(cin, cout);
+  if (cc == 0) return n;
+  const long long h = halo_wgrad_splits(B, H, W, cin, cout, cc);
   return h > n ? h : n;
 }
 
@@ -1351,20 +1359,25 @@ hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float
                     int H, int W, int cin, int cout, hipStream_t s) {
   const long long M = (long long)B * H * W;
   const int K = 9 * cin;
-  const bool halo = halo_wgrad(cin, cout) && (!x2 || c0 % 32 == 0) &&
+  const int cc = halo_wgrad_cc(cin, cout);
+  const bool halo = cc != 0 && (!x2 || c0 % cc == 0) &&
                     (long long)B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH) < (1LL << 30);
   long long parts = nn_wgrad_splits(M);
   const long long per = ((M + parts - 1) / parts + 63) / 64 * 64;
   WgradArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(dy), partial, B, H, W, cin, cout, per,
               static_cast<const bf16*>(x2), c0, nullptr};
   if (halo) {
-    const int ns = halo_wgrad_splits(B, H, W, cin, cout);
+    const int ns = halo_wgrad_splits(B, H, W, cin, cout, cc), co = halo_wgrad_co(cc, cout);
+    const dim3 grid(cout / co, cin / cc, ns);
     const int ntile = B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH), tps = (ntile + ns - 1) / ns;
     parts = ns;
     a.bias_partial = db ? partial + parts * cout * K : nullptr;
-    if (cin == 8) wgrad_halo_kernel<32, 8><<<dim3(cout / 32, 1, ns), 256, 0, s>>>(a, tps);
-    else if (cout % 64 == 0) wgrad_halo_kernel<64, 32><<<dim3(cout / 64, cin / 32, ns), 256, 0, s>>>(a, tps);
-    else wgrad_halo_kernel<32, 32><<<dim3(cout / 32, cin / 32, ns), 256, 0, s>>>(a, tps);
+    if (cc == 32 && co == 64) wgrad_halo_kernel<64, 32><<<grid, 256, 0, s>>>(a, tps);
+    else if (cc == 32) wgrad_halo_kernel<32, 32><<<grid, 256, 0, s>>>(a, tps);
+    else if (cc == 16 && co == 32) wgrad_halo_kernel<32, 16><<<grid, 256, 0, s>>>(a, tps);
+    else if (cc == 16) wgrad_halo_kernel<16, 16><<<grid, 256, 0, s>>>(a, tps);
+    else if (co == 32) wgrad_halo_kernel<32, 8><<<grid, 256, 0, s>>>(a, tps);
+    else wgrad_halo_kernel<16, 8><<<grid, 256, 0, s>>>(a, tps);
   } else {
     a.bias_partial = db ? partial + parts * cout * K : nullptr;
     if (cout <= 32) wgrad_kernel<32><<<dim3(1, (K + 127) / 128, (unsigned)parts), 256, 0, s>>>(a);

@@ -2,10 +2,10 @@
 FP64 on the CPU, on bf16-valued operands: the products are exact in FP32 and
 only the order of their sums differs, relative L2 error <= 1e-5 over the array.
 
-Tile-staged form (cin, cout multiples of 32): 64- and 32-channel output tiles,
-images smaller than a tile, cut tiles, one split and many, the decoder's
-concatenation; gathered form: other channel counts, a concatenation off the
-32-channel chunks.
+Tile-staged form (cin, cout multiples of 16, cin 8): 64-, 32- and 16-channel
+output tiles, images smaller than a tile, cut tiles, one split and many, the
+decoder's concatenation; gathered form: other channel counts, a concatenation
+off the channel chunks.
 """
 import ctypes
 
@@ -20,7 +20,8 @@ def _vp(t):
 
 @pytest.mark.parametrize("B,H,W,cin,cout,c0", [
     (1, 3, 5, 32, 32, 0), (2, 37, 50, 32, 64, 0), (3, 64, 80, 64, 32, 0), (1, 18, 34, 96, 32, 64),
-    (2, 20, 20, 192, 64, 128), (1, 9, 16, 32, 128, 0), (2, 12, 20, 8, 32, 0), (1, 5, 70, 8, 96, 0), (1, 10, 12, 64, 32, 48),
+    (2, 20, 20, 192, 64, 128), (1, 9, 16, 32, 128, 0), (2, 12, 20, 8, 32, 0), (1, 5, 70, 8, 96, 0), (1, 9, 40, 8, 16, 0),
+    (2, 14, 36, 16, 16, 0), (1, 8, 34, 48, 16, 32), (1, 20, 10, 48, 96, 16), (1, 6, 6, 48, 32, 8), (1, 7, 9, 24, 16, 0), (1, 10, 12, 64, 32, 48),
     (1, 11, 13, 32, 40, 0)])
 def test_weight_gradient(cuda, B, H, W, cin, cout, c0):
     import torch
