@@ -291,82 +291,96 @@ __global__ __launch_bounds__(256) void conv3x3_lds_kernel(ConvArgs a) {
   }
 }
 
+// How a block of conv3x3_halo_kernel proceeds: one item, a run of items whose
+// weights stay in LDS (one chunk, one block of output channels), any run.
+enum HaloRun { kOneItem, kWeightsStay, kAnyRun };
+
+// v, with 0 where the activation is not positive
+__device__ __forceinline__ bf16x8 relu_masked(const bf16* v, const bf16* act) {
+  bf16x8 x = *reinterpret_cast<const bf16x8*>(v);
+  const i16x8 m = __builtin_bit_cast(i16x8, *reinterpret_cast<const bf16x8*>(act));
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (!(__uint_as_float((unsigned)(unsigned short)m[e] << 16) > 0.0f)) x[e] = (bf16)0.0f;
+  return x;
+}
+
 // ---------------------------------------------------------------------------
 // Halo-tiled 3x3 convolution, the same implicit GEMM with its operands staged
-// once per block and input-channel chunk: the block's output tile is TH x 16
-// pixels x BN channels, and for each chunk of CC input channels it stages in
-// LDS the (TH + 2) x 18 pixel halo of the tile (80-byte pixel rows for
-// CC = 32) and the chunk's BN x 9 x CC weights (rows of 9 CC + 8 bf16), from
-// which every tap's A and B fragments are read; the next chunk's operands are
-// loaded into registers meanwhile.  Nine taps thus reuse one staged slab
-// instead of re-gathering the tile's pixels per tap.  CC = 32 (cin % 32 == 0):
-// a K step is one tap x 32 channels; CC = 8 (cin == 8): a K step is four
-// taps x 8 channels (lane group g takes tap 4 s + g).  Wave (wm, wn)
-// computes TM tile rows x TN 16-channel tiles.
+// once per tile and input-channel chunk: a tile is TH x 16 output pixels x BN
+// channels, and for each chunk of CC input channels the block stages in LDS the
+// (TH + 2) x 18 pixel halo of the tile (80-byte pixel rows for CC = 32) and the
+// chunk's BN x 9 x CC weights (rows of 9 CC + 8 bf16), from which every tap's A
+// and B fragments are read.  Nine taps thus reuse one staged slab instead of
+// re-gathering the tile's pixels per tap.  CC = 32 (cin % 32 == 0): a K step is
+// one tap x 32 channels; CC = 16, 8 (cin == CC): a K step is 32 / CC taps (lane
+// group g takes tap (32 / CC) s + 8 g / CC).  Wave (wm, wn) computes TM tile
+// rows x TN 16-channel tiles.
+//
+// A block walks a run of items, tiles x blocks of output channels (run_halo).
+// The next chunk's operands, or the next item's, are loaded into registers
+// during the MFMAs, and the weights of a single chunk stay in LDS; each wave
+// finishes its own rows through LDS of its own without a block barrier.  With
+// an item per block the first chunk's load and the epilogue were not
+// overlapped, as much as two chunks' work.  8 x 512 x 512, 32 -> 32 channels:
+// 93 -> 73 us (268 MB), 8 -> 32: 56 -> 47 us; 8 x 256 x 256, 64 -> 64: 86 -> 69
+// us (560 TF/s); 8 x 64 x 64, 256 -> 256: 62 -> 59 us.  Bound by memory at 32
+// channels, by the loads' latency and the barriers of a chunk beyond.
 // ---------------------------------------------------------------------------
-template <int TH, int BN, int WM, int WN, int CC>
-__global__ __launch_bounds__(256) void conv3x3_halo_kernel(ConvArgs a) {
-  static_assert(WM * WN == 4 && TH % WM == 0, "four waves, whole tile rows per wave");
+template <int TH, int BN, int WM, int WN, int CC, HaloRun RUN>
+__global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_kernel(ConvArgs a) {
+  static_assert(WM * WN == 4 && TH % (2 * WM) == 0, "four waves, whole pairs of tile rows per wave");
   constexpr int TW = 16, HH = TH + 2, HWD = TW + 2;
   constexpr int PS = CC == 32 ? 40 : CC;          // LDS pixel stride (bf16)
   constexpr int WR = 9 * CC + 8;                  // LDS weight row (bf16)
   constexpr int TM = TH / WM, TN = BN / WN / 16;  // MFMA tiles per wave
+  constexpr int CW = 16 * TN, CG = CW / 8;        // a wave's channels; 16-byte groups of them
   constexpr int GP = CC / 8;                      // 16-byte groups per halo pixel / weight tap
   constexpr int NG = HH * HWD * GP;               // groups per halo
   constexpr int NW = BN * 9 * GP;                 // groups per weight slab
   constexpr int HC = (NG + 255) / 256, WC = (NW + 255) / 256;  // groups per thread
   constexpr int TPS = 32 / CC;                    // taps per K step
   constexpr int NKS = (9 + TPS - 1) / TPS;        // K steps per chunk
-  constexpr int ES = BN + 4;                      // epilogue tile row (floats)
-  constexpr int NSTAGE = HH * HWD * PS + BN * WR, NEPI = TH * TW * ES * 2;  // bf16 units
-  __shared__ __attribute__((aligned(16))) bf16 smem[NSTAGE > NEPI ? NSTAGE : NEPI];
-  bf16* const halo = smem;
-  bf16* const wts = smem + HH * HWD * PS;
+  constexpr int ES = CW + 8, FS = CW + 4;         // a wave's epilogue pixel rows (bf16, FP32)
+  constexpr int EB = TW * FS * 2;                 // and tile row of them (bf16 units)
+  static_assert(TM / 2 * 8 * ES <= EB && TW * ES <= EB, "the epilogue's tiles fit");
+  __shared__ __attribute__((aligned(16))) bf16 halo[HH * HWD * PS];
+  __shared__ __attribute__((aligned(16))) bf16 wts[BN * WR];
+  __shared__ __attribute__((aligned(16))) bf16 etiles[4 * EB];
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int wm = wv % WM, wn = wv / WM;
   const int r16 = lane & 15, g = lane >> 4;
   const int tiles_x = (a.W + TW - 1) / TW, tiles_y = (a.H + TH - 1) / TH;
-  int t = blockIdx.x;
-  const int tx = t % tiles_x;
-  t /= tiles_x;
-  const int ty = t % tiles_y, b = t / tiles_y;
-  const int x0 = tx * TW, y0 = ty * TH;
-  const int nb = blockIdx.y * BN;
-  const int K = 9 * a.cin, nchunk = a.cin / CC;
+  const int K = 9 * a.cin, nchunk = a.cin / CC, nblk = a.cout / BN;
+  const int nitem = tiles_x * tiles_y * a.B * nblk, G = (int)gridDim.x;
+  // tile * nblk + block of output channels; the blocks of an XCD (every 8th)
+  // take neighbouring items
+  int item = RUN != kOneItem && G % 8 == 0 ? blockIdx.x % 8 * (G / 8) + blockIdx.x / 8 : blockIdx.x;
 
   bf16x8 rh[HC], rw[WC];
-  auto load = [&](int cc) {
+  auto load_halo = [&](int it, int cc) {
+    const int t = it / nblk, tx = t % tiles_x, rest = t / tiles_x, ty = rest % tiles_y, b = rest / tiles_y;
 #pragma unroll
     for (int i = 0; i < HC; ++i) {
       const int q = tid + 256 * i, p = q / GP, cg = (q % GP) * 8;
       const int hy = p / HWD, hx = p - hy * HWD;
-      const int iy = y0 + hy - 1, ix = x0 + hx - 1;
+      const int iy = ty * TH + hy - 1, ix = tx * TW + hx - 1;
       bf16x8 v = zero8();
       if (q < NG && iy >= 0 && iy < a.H && ix >= 0 && ix < a.W)
         v = *reinterpret_cast<const bf16x8*>(conv_in(a.in, a.in2, a.c0, a.H, a.W, a.cin, b, iy, ix, cc * CC + cg));
       rh[i] = v;
     }
+  };
+  auto load_weights = [&](int it, int cc) {
+    const int nb = it % nblk * BN;
 #pragma unroll
     for (int i = 0; i < WC; ++i) {
       const int q = tid + 256 * i, n = q / (9 * GP), rem = q - n * (9 * GP);
       const int tp = rem / GP, cg = (rem - tp * GP) * 8;
       bf16x8 v = zero8();
-      if (q < NW && nb + n < a.cout)
-        v = *reinterpret_cast<const bf16x8*>(a.w + (size_t)(nb + n) * K + tp * a.cin + cc * CC + cg);
+      if (q < NW) v = *reinterpret_cast<const bf16x8*>(a.w + (size_t)(nb + n) * K + tp * a.cin + cc * CC + cg);
       rw[i] = v;
-    }
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int i = 0; i < HC; ++i) {
-      const int q = tid + 256 * i, p = q / GP, cg = (q % GP) * 8;
-      if (q < NG) *reinterpret_cast<bf16x8*>(&halo[p * PS + cg]) = rh[i];
-    }
-#pragma unroll
-    for (int i = 0; i < WC; ++i) {
-      const int q = tid + 256 * i, n = q / (9 * GP), rem = q - n * (9 * GP);
-      if (q < NW) *reinterpret_cast<bf16x8*>(&wts[n * WR + rem * 8]) = rw[i];
     }
   };
 
@@ -377,111 +391,147 @@ __global__ __launch_bounds__(256) void conv3x3_halo_kernel(ConvArgs a) {
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // per-lane fragment bases: A at tile row wm TM, pixel r16, channels
-  // (8 g) % CC; B at weight row wn BN / WN + r16
+  // (8 g) % CC; B at weight row wn CW + r16
   const bf16* const abase = &halo[((wm * TM) * HWD + r16) * PS + (8 * g) % CC];
-  const bf16* const bbase = &wts[(wn * (BN / WN) + r16) * WR + (8 * g) % CC];
-  load(0);
-  for (int cc = 0; cc < nchunk; ++cc) {
-    if (cc > 0) __syncthreads();  // the previous chunk's reads come first
-    store();
-    __syncthreads();
-    if (cc + 1 < nchunk) load(cc + 1);
+  const bf16* const bbase = &wts[(wn * CW + r16) * WR + (8 * g) % CC];
+  bf16* const etile = etiles + wv * EB;
+  load_halo(item, 0);
+  load_weights(item, 0);
+  auto store_weights = [&]() {
+#pragma unroll
+    for (int i = 0; i < WC; ++i) {
+      const int q = tid + 256 * i, n = q / (9 * GP), rem = q - n * (9 * GP);
+      if (q < NW) *reinterpret_cast<bf16x8*>(&wts[n * WR + rem * 8]) = rw[i];
+    }
+  };
+  if (RUN == kWeightsStay) store_weights();
+  for (int next; item < nitem; item = next) {
+    next = RUN == kOneItem ? nitem : item + G;
+    const int nb = item % nblk * BN;
+    float bv[TN];
+    if (RUN != kOneItem)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[nb + wn * CW + 16 * j + r16] : 0.0f;
+    for (int cc = 0; cc < (RUN == kWeightsStay ? 1 : nchunk); ++cc) {
+      __syncthreads();  // the previous chunk's reads come first
+#pragma unroll
+      for (int i = 0; i < HC; ++i) {
+        const int q = tid + 256 * i, p = q / GP, cg = (q % GP) * 8;
+        if (q < NG) *reinterpret_cast<bf16x8*>(&halo[p * PS + cg]) = rh[i];
+      }
+      if (RUN != kWeightsStay) store_weights();
+      __syncthreads();
+      const bool last = RUN == kWeightsStay || cc + 1 == nchunk;
+      if (!last || (RUN != kOneItem && next < nitem)) {
+        const int it = RUN != kOneItem && last ? next : item, c = last ? 0 : cc + 1;
+        load_halo(it, c);
+        if (RUN != kWeightsStay) load_weights(it, c);
+      }
 #pragma unroll 1
-    for (int ks = 0; ks < NKS; ++ks) {
-      // this lane's tap in K step ks and its halo offsets (0..2)
-      const int tg = ks * TPS + (8 * g) / CC;
-      const int dy = tg / 3, dx = tg - 3 * dy;
-      const bool tv = tg < 9;
-      const bf16* const ap = abase + (dy * HWD + dx) * PS;
-      const bf16* const bp = bbase + tg * CC;
-      bf16x8 fa[TM], fb[TN];
+      for (int ks = 0; ks < NKS; ++ks) {
+        // this lane's tap in K step ks and its halo offsets (0..2)
+        const int tg = ks * TPS + (8 * g) / CC;
+        const int dy = tg / 3, dx = tg - 3 * dy;
+        const bool tv = tg < 9;
+        const bf16* const ap = abase + (dy * HWD + dx) * PS;
+        const bf16* const bp = bbase + tg * CC;
+        bf16x8 fa[TM], fb[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = tv ? *reinterpret_cast<const bf16x8*>(ap + i * HWD * PS) : zero8();
+        for (int i = 0; i < TM; ++i) fa[i] = tv ? *reinterpret_cast<const bf16x8*>(ap + i * HWD * PS) : zero8();
 #pragma unroll
-      for (int j = 0; j < TN; ++j) fb[j] = tv ? *reinterpret_cast<const bf16x8*>(bp + 16 * j * WR) : zero8();
+        for (int j = 0; j < TN; ++j) fb[j] = tv ? *reinterpret_cast<const bf16x8*>(bp + 16 * j * WR) : zero8();
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+      }
+    }
+    // D layout: lane holds pixels 4 g + r of tile row wm TM + i, channel r16
+    const int tile = item / nblk, tx = tile % tiles_x, rest = tile / tiles_x, ty = rest % tiles_y, b = rest / tiles_y;
+    const int x0 = tx * TW, y0 = ty * TH + wm * TM, co = nb + wn * CW;
+    if (RUN == kOneItem)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[co + 16 * j + r16] : 0.0f;
+    if (a.low_out && nb < a.low_c) {
+      // 2 x 2 sums (low_c is a multiple of BN; tiles start at even pixels)
+      const int H2 = a.H >> 1, W2 = a.W >> 1;
+#pragma unroll
+      for (int i = 0; i < TM; i += 2)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-  }
-
-  // Epilogue through LDS: the block's FP32 tile [pixel][channel] (row stride
-  // BN + 4 floats) replaces the staged operands, then each thread finishes 8
-  // channels of one pixel with 16-byte loads (mask) and stores.
-  constexpr int EG = TH * TW * BN / 8;  // epilogue groups
-  float* const etile = reinterpret_cast<float*>(smem);
-  __syncthreads();
-  // D layout: lane holds rows 4 g + r (pixels of tile row wm TM + i) of column r16
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        etile[((wm * TM + i) * TW + 4 * g + r) * ES + wn * (BN / WN) + 16 * j + r16] = acc[i][j][r];
-  __syncthreads();
-  if (a.low_out && nb < a.low_c) {
-    // 2 x 2 sums (low_c is a multiple of BN; tiles start at even pixels)
-    for (int q = tid; q < EG / 4; q += 256) {
-      const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
-      const int ly = p / (TW / 2), lx = p - ly * (TW / 2);
-      const int oy = (y0 >> 1) + ly, ox = (x0 >> 1) + lx;
-      if (2 * oy >= a.H || 2 * ox >= a.W) continue;
-      const float* const e0 = etile + (2 * ly * TW + 2 * lx) * ES + c8;
-      const long long o = (((long long)b * (a.H >> 1) + oy) * (a.W >> 1) + ox) * a.low_c + nb + c8;
-      const i16x8 mk = __builtin_bit_cast(i16x8, *reinterpret_cast<const bf16x8*>(a.low_mask + o));
-      bf16x8 h;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = e0[e] + e0[ES + e] + e0[TW * ES + e] + e0[(TW + 1) * ES + e];
-        h[e] = (bf16)(__uint_as_float((unsigned)(unsigned short)mk[e] << 16) > 0.0f ? v : 0.0f);
+          for (int r = 0; r < 4; r += 2)
+            etile[(i / 2 * 8 + 2 * g + r / 2) * ES + 16 * j + r16] =
+                (bf16)(acc[i][j][r] + acc[i][j][r + 1] + acc[i + 1][j][r] + acc[i + 1][j][r + 1]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int q = lane; q < TM / 2 * 8 * CG; q += 64) {
+        const int p = q / CG, c8 = (q - p * CG) * 8;
+        const int oy = (y0 >> 1) + p / 8, ox = (x0 >> 1) + p % 8;
+        if (oy >= H2 || ox >= W2) continue;
+        const long long o = (((long long)b * H2 + oy) * W2 + ox) * a.low_c + co + c8;
+        *reinterpret_cast<bf16x8*>(a.low_out + o) = relu_masked(&etile[p * ES + c8], a.low_mask + o);
       }
-      *reinterpret_cast<bf16x8*>(a.low_out + o) = h;
-    }
-    return;
-  }
-  if (a.low_out) {
-    const int cs = a.cout - a.low_c;
-    for (int q = tid; q < EG; q += 256) {
-      const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
-      const int oy = y0 + p / TW, ox = x0 + p % TW;
-      if (oy >= a.H || ox >= a.W) continue;
-      float* const op = a.skip_out + (((long long)b * a.H + oy) * a.W + ox) * cs + nb - a.low_c + c8;
-      const float* const e0 = etile + p * ES + c8;
-      *reinterpret_cast<f32x4*>(op) = f32x4{e0[0], e0[1], e0[2], e0[3]};
-      *reinterpret_cast<f32x4*>(op + 4) = f32x4{e0[4], e0[5], e0[6], e0[7]};
-    }
-    return;
-  }
-  for (int q = tid; q < EG; q += 256) {
-    const int p = q / (BN / 8), c8 = (q - p * (BN / 8)) * 8;
-    const int oy = y0 + p / TW, ox = x0 + p % TW, co = nb + c8;
-    if (oy >= a.H || ox >= a.W || co >= a.cout) continue;
-    const long long o = (((long long)b * a.H + oy) * a.W + ox) * a.cout + co;
-    float v[8];
+    } else if (a.low_out || a.out_f32) {
+      // FP32 output, a tile row at a time
+      float* const out = a.low_out ? a.skip_out : static_cast<float*>(a.out);
+      float* const ftile = reinterpret_cast<float*>(etile);
+      const int c0 = a.low_out ? a.low_c : 0, C = a.cout - c0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      v[e] = etile[p * ES + c8 + e] + (a.bias ? a.bias[co + e] : 0.0f);
-      if (a.relu) v[e] = fmaxf(v[e], 0.0f);
-    }
-    if (a.mask) {
-      const i16x8 mk = __builtin_bit_cast(i16x8, *reinterpret_cast<const bf16x8*>(a.mask + o));
+      for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (!(__uint_as_float((unsigned)(unsigned short)mk[e] << 16) > 0.0f)) v[e] = 0.0f;
-    }
-    if (a.out_f32) {
-      float* const op = static_cast<float*>(a.out) + o;
-      *reinterpret_cast<f32x4*>(op) = f32x4{v[0], v[1], v[2], v[3]};
-      *reinterpret_cast<f32x4*>(op + 4) = f32x4{v[4], v[5], v[6], v[7]};
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float v = acc[i][j][r] + bv[j];
+            if (a.relu) v = fmaxf(v, 0.0f);
+            ftile[(4 * g + r) * FS + 16 * j + r16] = v;
+          }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = lane; q < TW * CW / 4; q += 64) {
+          const int p = q / (CW / 4), c4 = (q - p * (CW / 4)) * 4;
+          const int oy = y0 + i, ox = x0 + p;
+          if (oy >= a.H || ox >= a.W) continue;
+          const long long o = (((long long)b * a.H + oy) * a.W + ox) * C + co - c0 + c4;
+          f32x4 v = *reinterpret_cast<const f32x4*>(&ftile[p * FS + c4]);
+          if (a.mask)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (!((float)a.mask[o + e] > 0.0f)) v[e] = 0.0f;
+          *reinterpret_cast<f32x4*>(out + o) = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
     } else {
-      bf16x8 h;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) h[e] = (bf16)v[e];
-      *reinterpret_cast<bf16x8*>(static_cast<bf16*>(a.out) + o) = h;
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float v = acc[i][j][r] + bv[j];
+            if (a.relu) v = fmaxf(v, 0.0f);
+            etile[(4 * g + r) * ES + 16 * j + r16] = (bf16)v;
+          }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane < TW * CG) {
+          const int p = lane / CG, c8 = (lane - p * CG) * 8;
+          const int oy = y0 + i, ox = x0 + p;
+          const long long o = (((long long)b * a.H + oy) * a.W + ox) * a.cout + co + c8;
+          if (oy < a.H && ox < a.W)
+            *reinterpret_cast<bf16x8*>(static_cast<bf16*>(a.out) + o) =
+                a.mask ? relu_masked(&etile[p * ES + c8], a.mask + o)
+                       : *reinterpret_cast<const bf16x8*>(&etile[p * ES + c8]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
 }
 
@@ -1255,26 +1305,38 @@ __global__ void to_bf16_kernel(const float* __restrict__ src, bf16* __restrict__
 // ---------------------------------------------------------------------------
 static inline unsigned blocks_for(long long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
-// 3x3 convolutions with cin % 32 == 0 (or cin == 8) and cout % 32 == 0 run
-// the halo-tiled kernel; the others the K-step-staged one.
-static bool halo_conv(int cin, int cout) { return (cin % 32 == 0 || cin == 8) && cout % 32 == 0; }
+// 3x3 convolutions with cin % 32 == 0 (or cin 16 or 8) and cout % 16 == 0 run
+// the halo-tiled kernel; the others the K-step-staged ones.
+static bool halo_conv(int cin, int cout) { return (cin % 32 == 0 || cin == 16 || cin == 8) && cout % 16 == 0; }
 
-// 16-row tiles for 32 output channels, 8-row tiles and 64-channel blocks
-// otherwise.
-static int halo_block(int cout) { return cout % 64 == 0 ? 64 : 32; }
+// 8-row tiles and 64-channel blocks where cout allows, else 16-row tiles.
+static int halo_block(int cout) { return cout % 64 == 0 ? 64 : cout % 32 == 0 ? 32 : 16; }
+
+// Blocks walk runs of items, two per CU (three with registers and LDS for it
+// were slower: 73 -> 89 us for 32 -> 32 channels at 8 x 512 x 512).  32- and 16-
+// channel blocks do so only where their weights stay; with the registers for
+// reloading them an item per block, three per CU, is faster (96 -> 32 channels:
+// 178 us against 186 in runs).
+template <int TH, int BN, int WM, int WN, int CC, HaloRun RUN>
+static hipError_t run_halo(const ConvArgs& a, hipStream_t s) {
+  const long long nitem = (long long)((a.W + 15) / 16) * ((a.H + TH - 1) / TH) * a.B * (a.cout / BN);
+  if (nitem >= 1LL << 30) return hipErrorInvalidValue;
+  const long long blocks = RUN == kOneItem ? nitem : 512;
+  conv3x3_halo_kernel<TH, BN, WM, WN, CC, RUN><<<(unsigned)(nitem < blocks ? nitem : blocks), 256, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+template <int CC>
+static hipError_t run_halo_cc(const ConvArgs& a, hipStream_t s) {
+  const int bn = halo_block(a.cout);
+  const bool stay = a.cin == CC && a.cout == bn;
+  if (bn == 64) return run_halo<8, 64, 2, 2, CC, kAnyRun>(a, s);
+  if (bn == 32) return stay ? run_halo<16, 32, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 32, 4, 1, CC, kOneItem>(a, s);
+  return stay ? run_halo<16, 16, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 16, 4, 1, CC, kOneItem>(a, s);
+}
 
 static hipError_t launch_halo(const ConvArgs& a, hipStream_t s) {
-  const unsigned tiles16 = (unsigned)((a.W + 15) / 16), img = (unsigned)a.B;
-  if (halo_block(a.cout) == 64) {
-    const dim3 grid(tiles16 * (unsigned)((a.H + 7) / 8) * img, a.cout / 64);
-    if (a.cin == 8) conv3x3_halo_kernel<8, 64, 2, 2, 8><<<grid, 256, 0, s>>>(a);
-    else conv3x3_halo_kernel<8, 64, 2, 2, 32><<<grid, 256, 0, s>>>(a);
-  } else {
-    const dim3 grid(tiles16 * (unsigned)((a.H + 15) / 16) * img, a.cout / 32);
-    if (a.cin == 8) conv3x3_halo_kernel<16, 32, 4, 1, 8><<<grid, 256, 0, s>>>(a);
-    else conv3x3_halo_kernel<16, 32, 4, 1, 32><<<grid, 256, 0, s>>>(a);
-  }
-  return hipGetLastError();
+  return a.cin == 8 ? run_halo_cc<8>(a, s) : a.cin == 16 ? run_halo_cc<16>(a, s) : run_halo_cc<32>(a, s);
 }
 
 // Whether nn_conv3x3_upback runs in one kernel: whole blocks of output
