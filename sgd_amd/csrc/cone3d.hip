@@ -72,19 +72,7 @@ struct AxialTrap {
   float i01, i23;  // 1 / (2 (v1 - v0)), 1 / (2 (v3 - v2)); 0 on a flat side
 };
 
-// v_med3_f32: clamp of s into [lo, hi] (lo <= hi) in one instruction, with no
-// NaN quieting of the operands (every value here is finite)
-__device__ __forceinline__ float clampf(float s, float lo, float hi) { return __builtin_amdgcn_fmed3f(s, lo, hi); }
-
 __device__ __forceinline__ float inv_or_zero(float w) { return w > 0.0f ? 0.5f * __builtin_amdgcn_rcpf(w) : 0.0f; }
-
-// 1 / d for a normal double d of float range: the float reciprocal (relative
-// error ~6e-8) refined by one Newton step (error ~4e-15), in place of the
-// double division's longer sequence
-__device__ __forceinline__ double recip(double d) {
-  const double r0 = (double)__builtin_amdgcn_rcpf((float)d);
-  return __builtin_fma(r0, __builtin_fma(-d, r0, 1.0), r0);
-}
 
 struct ColumnAxial {
   float ka, kb;        // ldz / depth at the two x corners (SF-TR: both the centre)
@@ -182,9 +170,9 @@ __device__ __forceinline__ float row_off() {
 // for a side of zero width, which never overlaps.
 __device__ __forceinline__ float trap_gamma(float s, const AxialTrap& t) {
   const float e = s + 1.0f;
-  const float s0 = clampf(s, t.v0, t.v1), e0 = clampf(e, t.v0, t.v1);
-  const float s1 = clampf(s, t.v1, t.v2), e1 = clampf(e, t.v1, t.v2);
-  const float s2 = clampf(s, t.v2, t.v3), e2 = clampf(e, t.v2, t.v3);
+  const float s0 = clamp3(s, t.v0, t.v1), e0 = clamp3(e, t.v0, t.v1);
+  const float s1 = clamp3(s, t.v1, t.v2), e1 = clamp3(e, t.v1, t.v2);
+  const float s2 = clamp3(s, t.v2, t.v3), e2 = clamp3(e, t.v2, t.v3);
   const float g0 = (e0 - s0) * (e0 + s0 - 2.0f * t.v0) * t.i01;
   const float g2 = (e2 - s2) * (2.0f * t.v3 - s2 - e2) * t.i23;
   return g0 + (e1 - s1) + g2;
@@ -389,7 +377,7 @@ __device__ __forceinline__ float sf_cell_weight(const ViewGeo& vg, const Proj2DA
   const float q1 = -(nc - hx + hy) / (bc - bx + by);
   const float q2 = -(nc + hx - hy) / (bc + bx - by);
   const float q3 = -(nc + hx + hy) / (bc + bx + by);
-  const Trap t = make_trap(q0, q1, q2, q3);
+  const Trap t = sorted_trap(q0, q1, q2, q3);
   const float width = (t.q3 - t.q0) + (t.q2 - t.q1);
   const float gm = trap_gamma(t, 0.0f, 1.0f);
   return width > 0.0f ? gm * 2.0f / width : 0.0f;

@@ -20,13 +20,15 @@ namespace sgdct {
 hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts, hipStream_t s);
 hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float* img, hipStream_t s);
 
-// A, launched as fwd_group_kernel.  Bound by VALU issue: ~70 instructions per
-// footprint (four corner projections with two reciprocals, the sort and the
-// trapezoid's area) beside one multiply-add per value.  512 x 512, 720 views,
-// 768 bins, per call: one value per footprint 1456 us, the scan's 8
-// symmetries 260 us; 1024 x 1024, 900 views 7.04 -> 1.13 ms; 256 x 256, 90
-// views, batch 5 266 -> 84 us; one value, 721 views from another start angle
-// 1455 -> 1420 us.
+// A, launched as fwd_group_kernel.  Bound by VALU issue: 57 instructions per
+// footprint, five of them reciprocals and roots at a quarter of the rate (two
+// new corner projections, the merge of two sorted pairs, the trapezoid's area),
+// and about as many per line, beside one multiply-add per value.  512 x 512,
+// 720 views, 768 bins, per call: one value per footprint 1456 us, the scan's 8
+// symmetries 212 us; 1024 x 1024, 900 views 7.04 -> 0.90 ms; 256 x 256, 90
+// views, batch 5 266 -> 72 us; one value, 721 views from another start angle
+// 1455 -> 1133 us.  (FP64 line intervals, a four-value sort, compared ramps and
+// the weight's reciprocal per pixel: 260, 1130, 84, 1418 us.)
 template <int G, int W>
 __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
                                                         const float* __restrict__ rows_img,
@@ -51,9 +53,11 @@ __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp
   fwd_group_store<G, W>(g, sp, rep, v, u, m, batch, red, 1.0, 1.0, 1.0, sino, gridDim.z > 1 ? part : nullptr);
 }
 
-// A^T, launched as bwd_group_kernel; same cases as above: 841 -> 175 us, 4.13
-// -> 0.75 ms, 146 -> 55 us, 869 -> 863 us.  The FP64 projection of the pixel's
-// centre and its sorted corners are formed once per view for all values.
+// A^T, launched as bwd_group_kernel; same cases as above: 841 -> 151 us, 4.13
+// -> 0.64 ms, 146 -> 49 us, 869 -> 664 us.  The FP64 projection of the pixel's
+// centre and its sorted corners are formed once per view for all values, and
+// each bin's area from one new edge (both edges per bin, and a double division
+// per view: 174 us in the first case).
 template <int G>
 __global__ __launch_bounds__(256) void sf_bwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
                                                      const float* __restrict__ sino, float* __restrict__ img, int vpg,

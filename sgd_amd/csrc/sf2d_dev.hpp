@@ -4,52 +4,82 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "group2d_dev.hpp"
 #include "projector.hpp"
 
 namespace sgdct {
 
-struct Trap {
-  float q0, q1, q2, q3, ir, iff;  // sorted corners, 1/(2(q1-q0)), 1/(2(q3-q2))
-};
-
-// min / max of finite values as v_med3_f32 against -inf / +inf: exact, one
-// instruction, and no NaN quieting of the operands (fminf / fmaxf add it)
+// min / max / clamp of finite values as v_med3_f32: exact, one instruction, and
+// no NaN quieting of the operands (fminf / fmaxf add it)
 __device__ __forceinline__ float min2f(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, -__builtin_inff()); }
 __device__ __forceinline__ float max2f(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
+__device__ __forceinline__ float clamp3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
 
-__device__ __forceinline__ void sort4(float& a, float& b, float& c, float& d) {
-  float t;
-  t = min2f(a, b); b = max2f(a, b); a = t;
-  t = min2f(c, d); d = max2f(c, d); c = t;
-  t = min2f(a, c); c = max2f(a, c); a = t;
-  t = min2f(b, d); d = max2f(b, d); b = t;
-  t = min2f(b, c); c = max2f(b, c); b = t;
+// 1 / d for a normal double d of float range: the float reciprocal (relative
+// error ~6e-8) refined by one Newton step (error ~4e-15), in place of the
+// double division's longer sequence
+__device__ __forceinline__ double recip(double d) {
+  const double r0 = (double)__builtin_amdgcn_rcpf((float)d);
+  return __builtin_fma(r0, __builtin_fma(-d, r0, 1.0), r0);
 }
 
-__device__ __forceinline__ Trap make_trap(float q0, float q1, float q2, float q3) {
-  sort4(q0, q1, q2, q3);
+// Unit-height trapezoid over sorted corners, 1 / (q1 - q0) and 1 / (q3 - q2)
+// (finite for an empty ramp, whose terms are then zero).
+struct Trap {
+  float q0, q1, q2, q3, ir, iff;
+};
+
+__device__ __forceinline__ void sort2(float a, float b, float& lo, float& hi) {
+  lo = min2f(a, b);
+  hi = max2f(a, b);
+}
+
+// Trapezoid of two pairs of corners, each sorted.
+__device__ __forceinline__ Trap make_trap(float a0, float a1, float b0, float b1) {
   Trap t;
-  t.q0 = q0; t.q1 = q1; t.q2 = q2; t.q3 = q3;
-  t.ir = __builtin_amdgcn_rcpf(2.0f * (q1 - q0));
-  t.iff = __builtin_amdgcn_rcpf(2.0f * (q3 - q2));
+  t.q0 = min2f(a0, b0);
+  t.q3 = max2f(a1, b1);
+  sort2(max2f(a0, b0), min2f(a1, b1), t.q1, t.q2);
+  t.ir = __builtin_amdgcn_rcpf(max2f(t.q1 - t.q0, 1e-30f));
+  t.iff = __builtin_amdgcn_rcpf(max2f(t.q3 - t.q2, 1e-30f));
   return t;
 }
 
-// Area of the unit-height trapezoid over [s1, s2] (layers/A_SF.cu:48-84).
+__device__ __forceinline__ Trap sorted_trap(float a, float b, float c, float d) {
+  float a0, a1, b0, b1;
+  sort2(a, b, a0, a1);
+  sort2(c, d, b0, b1);
+  return make_trap(a0, a1, b0, b1);
+}
+
+// Area of the trapezoid over [s1, s2] (layers/A_SF.cu:48-84), the ramps'
+// squares differenced as products of sum and difference.  A walk over adjacent
+// intervals passes what it holds of the last edge on: start() at the first
+// edge, next() per further edge.
+struct TrapWalk {
+  float b, m, e;  // clamped distances into the rising ramp, flat top, falling ramp
+  __device__ __forceinline__ void start(const Trap& t, float s) {
+    b = clamp3(s, t.q0, t.q1) - t.q0;
+    m = clamp3(s, t.q1, t.q2);
+    e = t.q3 - clamp3(s, t.q2, t.q3);
+  }
+  __device__ __forceinline__ float next(const Trap& t, float s) {
+    TrapWalk n;
+    n.start(t, s);
+    const float ramps =
+        __builtin_fmaf((e - n.e) * (e + n.e), t.iff, (n.b - b) * (n.b + b) * t.ir);
+    const float area = __builtin_fmaf(0.5f, ramps, n.m - m);
+    *this = n;
+    return area;
+  }
+};
+
 __device__ __forceinline__ float trap_gamma(const Trap& t, float s1, float s2) {
-  float b1 = fmaxf(s1, t.q0), b2 = fminf(s2, t.q1);
-  float d0 = b2 - t.q0, d1 = b1 - t.q0;
-  float g = (b2 > b1) ? (d0 * d0 - d1 * d1) * t.ir : 0.0f;
-  b1 = fmaxf(s1, t.q1);
-  b2 = fminf(s2, t.q2);
-  g += fmaxf(b2 - b1, 0.0f);
-  b1 = fmaxf(s1, t.q2);
-  b2 = fminf(s2, t.q3);
-  float e1 = b1 - t.q3, e2 = b2 - t.q3;
-  g += (b2 > b1) ? (e1 * e1 - e2 * e2) * t.iff : 0.0f;
-  return g;
+  TrapWalk w;
+  w.start(t, s1);
+  return w.next(t, s2);
 }
 
 // dx / max(|cos t|, |sin t|) of the ray through (wx, wy) from the source;
@@ -83,19 +113,19 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
   const bool strided = !rows && !cols_img;
   const int smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
-  const double isa = sa != 0.0 ? 1.0 / sa : 0.0, isb = sb != 0.0 ? 1.0 / sb : 0.0;
-  // beta(ix, iy) = cross(pu, w): affine, gradient (gx1, gy1) per index step
+  // beta(ix, iy) = cross(pu, w): affine, steps (bcxx, bcyy) per index
   const double bcxx = -vg.puy * g.dx, bcyy = vg.pux * g.dy, bc00 = vg.pux * vg.w0y - vg.puy * vg.w0x;
-  const float dN = (float)sa, dB = (float)(rows ? bcxx : bcyy);
-  const float dwx = rows ? (float)g.dx : 0.0f, dwy = rows ? 0.0f : (float)g.dy;
-  // corner offsets (+-1/2, +-1/2) of N_u and beta
-  const float nx_ = 0.5f * (float)acx, ny_ = 0.5f * (float)acy;
-  const float bx_ = 0.5f * (float)bcxx, by_ = 0.5f * (float)bcyy;
-  const float fdx = (float)g.dx;
-  // corner offsets along the walk (w) and across it (c): the corners on the
-  // leading side (+w) of one pixel are the trailing side (-w) of the next
-  const float w_n = rows ? nx_ : ny_, c_n = rows ? ny_ : nx_;
-  const float w_b = rows ? bx_ : by_, c_b = rows ? by_ : bx_;
+  const double sB = rows ? bcxx : bcyy, mB = rows ? bcyy : bcxx;
+  const float dN = (float)sa, dB = (float)sB;
+  // source -> pixel centre, along the walk (moving) and across it (fixed)
+  const double dmov = rows ? g.dx : g.dy, dfix = rows ? g.dy : g.dx;
+  const double w0mov = rows ? vg.w0x : vg.w0y, w0fix = rows ? vg.w0y : vg.w0x;
+  const float fdmov = (float)dmov, fdx = (float)g.dx;
+  // offsets of N_u and beta from a pixel's centre to its corners across the
+  // walk on the leading side (nl, bl) and the trailing side (-nl, -bl): the
+  // leading corners of one pixel are the trailing ones of the next
+  const float w_n = 0.5f * (float)sa, c_n = 0.5f * (float)ma, w_b = 0.5f * (float)sB, c_b = 0.5f * (float)mB;
+  const float nl1 = w_n - c_n, nl2 = w_n + c_n, bl1 = w_b - c_b, bl2 = w_b + c_b;
 
   int m_lo = 0, m_hi = nmaj - 1;
   if (ma != 0.0 && mb != 0.0) {
@@ -116,51 +146,81 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
   const unsigned bstep = 4u * G * (unsigned)smin;
-  for (int m = m_lo + ((w0 - m_lo) & (wn - 1)); m <= m_hi; m += wn) {
-    const double r1 = -ra - ma * m - ac0;
-    const double r2 = rb - mb * m - bc0;
-    double lo = 0.0, hi = (double)(nmin - 1);
-    if (sa > 0.0) lo = fmax(lo, ceil(r1 * isa));
-    else if (sa < 0.0) hi = fmin(hi, floor(r1 * isa));
-    else if (r1 > 0.0) continue;
-    if (sb > 0.0) hi = fmin(hi, ceil(r2 * isb) - 1.0);
-    else if (sb < 0.0) lo = fmax(lo, floor(r2 * isb) + 1.0);
-    else if (r2 <= 0.0) continue;
-    if (lo > hi) continue;
-    const int n0 = (int)lo, n1 = (int)hi;
-    const int ixs = rows ? n0 : m, iys = rows ? m : n0;
-    float nu_ = (float)(acx * ixs + acy * iys + ac0);
-    float be = (float)(bcxx * ixs + bcyy * iys + bc00);
-    float wx = (float)(ixs * g.dx + vg.w0x), wy = (float)(iys * g.dy + vg.w0y);
-    unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
-    float accl[G];
-#pragma unroll
-    for (int k = 0; k < G; ++k) accl[k] = 0.0f;
-    // corner projections relative to edge u, -N_u(c) / beta(c), of the
-    // trailing corners of the line's first pixel
-    float t1 = -(nu_ - w_n - c_n) * __builtin_amdgcn_rcpf(be - w_b - c_b);
-    float t2 = -(nu_ - w_n + c_n) * __builtin_amdgcn_rcpf(be - w_b + c_b);
-    for (int n = n0; n <= n1; ++n) {
-      float x[G];
-      buffer_load_n<G>(img_rsrc, off, x);
-      const float l1 = -(nu_ + w_n - c_n) * __builtin_amdgcn_rcpf(be + w_b - c_b);
-      const float l2 = -(nu_ + w_n + c_n) * __builtin_amdgcn_rcpf(be + w_b + c_b);
-      const Trap t = make_trap(t1, t2, l1, l2);
-      t1 = l1;
-      t2 = l2;
-      const float gm = trap_gamma(t, 0.0f, 1.0f);
-      const float val = (gm > 1e-7f) ? gm * sf_weight(fdx, wx, wy) : 0.0f;
-#pragma unroll
-      for (int k = 0; k < G; ++k) accl[k] = __builtin_fmaf(val, x[k], accl[k]);
-      off += bstep;
-      nu_ += dN;
-      be += dB;
-      wx += dwx;
-      wy += dwy;
-    }
-#pragma unroll
-    for (int k = 0; k < G; ++k) acc[k] += (double)accl[k];
+  // Pixel interval of line m, from N_u + R_u >= 0 and N_{u+1} - R_{u+1} < 0:
+  // [ceil(lo(m)), floor(hi(m))], affine in m, in FP32 and widened by its error
+  // bound: the trapezoid's own area decides at the boundary, where it is zero.
+  // sa and sb share a sign where the strip is within ~45 degrees of the walk
+  // direction, as the wave's orientation has it; otherwise the lane walks whole
+  // lines.
+  const float lastn = (float)(nmin - 1);
+  float lo0 = 0.0f, lo1 = 0.0f, hi0 = lastn, hi1 = 0.0f;
+  if ((sa > 0.0 && sb > 0.0) || (sa < 0.0 && sb < 0.0)) {
+    const float p0 = (float)((-ra - ac0) / sa), p1 = (float)(-ma / sa);
+    const float r0 = (float)((rb - bc0) / sb), r1 = (float)(-mb / sb);
+    lo0 = sa > 0.0 ? p0 : r0;
+    lo1 = sa > 0.0 ? p1 : r1;
+    hi0 = sa > 0.0 ? r0 : p0;
+    hi1 = sa > 0.0 ? r1 : p1;
+    const float most = (float)nmaj;
+    lo0 -= 4e-7f * __builtin_fmaf(fabsf(lo1), most, fabsf(lo0)) + 1e-5f;
+    hi0 += 4e-7f * __builtin_fmaf(fabsf(hi1), most, fabsf(hi0)) + 1e-5f;
   }
+  // The weight's larger coordinate is the fixed one (reciprocal once per line)
+  // if every lane's strip stays inside 45 degrees: at a line's end pixels the
+  // moving coordinate exceeds the ray's by at most the strip's half width and a
+  // pixel.
+  const double f0 = __builtin_fma((double)m_lo, dfix, w0fix), f1 = __builtin_fma((double)m_hi, dfix, w0fix);
+  const double slope = fmax(fabs(rows ? eax / eay : eay / eax), fabs(rows ? ebx / eby : eby / ebx));
+  const bool own = __ballot(inside && !(f0 * f1 > 0.0 && fmin(fabs(f0), fabs(f1)) * (0.999 - slope) >
+                                                             2.0 * (fabs(dmov) + fabs(dfix)))) == 0;
+  auto walk = [&](auto own_c) {
+    for (int m = m_lo + ((w0 - m_lo) & (wn - 1)); m <= m_hi; m += wn) {
+      const float fm = (float)m;
+      const float flo = fmaxf(ceilf(__builtin_fmaf(fm, lo1, lo0)), 0.0f);
+      const float fhi = fminf(floorf(__builtin_fmaf(fm, hi1, hi0)), lastn);
+      if (!(flo <= fhi)) continue;
+      const int n0 = (int)flo;
+      const double dm = (double)m, dn = (double)flo;
+      float nu_ = (float)__builtin_fma(dn, sa, __builtin_fma(dm, ma, ac0));
+      float be = (float)__builtin_fma(dn, sB, __builtin_fma(dm, mB, bc00));
+      float wm = (float)__builtin_fma(dn, dmov, w0mov);
+      const float wf = (float)__builtin_fma(dm, dfix, w0fix);
+      const float ifix = __builtin_amdgcn_rcpf(fabsf(wf)), wf2 = wf * wf;
+      unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
+      const unsigned end = off + (unsigned)((int)fhi - n0 + 1) * bstep;
+      float accl[G];
+#pragma unroll
+      for (int k = 0; k < G; ++k) accl[k] = 0.0f;
+      // corner projections relative to edge u, -N_u(c) / beta(c), of the
+      // trailing corners of the line's first pixel
+      float t1, t2;
+      sort2((nl2 - nu_) * __builtin_amdgcn_rcpf(be - bl2), (nl1 - nu_) * __builtin_amdgcn_rcpf(be - bl1), t1, t2);
+      do {
+        float x[G];
+        buffer_load_n<G>(img_rsrc, off, x);
+        float l1, l2;
+        sort2(-(nu_ + nl1) * __builtin_amdgcn_rcpf(be + bl1), -(nu_ + nl2) * __builtin_amdgcn_rcpf(be + bl2), l1, l2);
+        const Trap t = make_trap(t1, t2, l1, l2);
+        t1 = l1;
+        t2 = l2;
+        const float gm = trap_gamma(t, 0.0f, 1.0f);
+        // dx / max(|cos|, |sin|) of the ray through the pixel's centre
+        const float il = decltype(own_c)::value ? ifix : __builtin_amdgcn_rcpf(fmaxf(fabsf(wm), fabsf(wf)));
+        const float w = fdx * __builtin_amdgcn_sqrtf(__builtin_fmaf(wm, wm, wf2)) * il;
+        const float val = (gm > 1e-7f) ? gm * w : 0.0f;
+#pragma unroll
+        for (int k = 0; k < G; ++k) accl[k] = __builtin_fmaf(val, x[k], accl[k]);
+        off += bstep;
+        nu_ += dN;
+        be += dB;
+        wm += fdmov;
+      } while (off != end);
+#pragma unroll
+      for (int k = 0; k < G; ++k) acc[k] += (double)accl[k];
+    }
+  };
+  if (own) walk(std::true_type{});
+  else walk(std::false_type{});
 }
 
 // One wave of the batched work queue: item `wave` = chunk * np + view, every
@@ -199,21 +259,22 @@ __device__ __forceinline__ void sf_bwd_tile(const Proj2DArgs& g, const float* __
     const float gx = 0.5f * __builtin_fmaf(kcf, vg.gx1, vg.gx0), gy = 0.5f * __builtin_fmaf(kcf, vg.gy1, vg.gy0);
     const float bx = 0.5f * vg.gx1, by = 0.5f * vg.gy1;
     // corner c: k*(c) - kc = -(d.G) / (beta + d.grad beta)
-    const float q0 = kf + (gx + gy) * __builtin_amdgcn_rcpf(bef - bx - by);
-    const float q1 = kf + (gx - gy) * __builtin_amdgcn_rcpf(bef - bx + by);
-    const float q2 = kf - (gx - gy) * __builtin_amdgcn_rcpf(bef + bx - by);
-    const float q3 = kf - (gx + gy) * __builtin_amdgcn_rcpf(bef + bx + by);
-    const Trap t = make_trap(q0, q1, q2, q3);
+    const Trap t = sorted_trap(kf + (gx + gy) * __builtin_amdgcn_rcpf(bef - bx - by),
+                               kf + (gx - gy) * __builtin_amdgcn_rcpf(bef - bx + by),
+                               kf - (gx - gy) * __builtin_amdgcn_rcpf(bef + bx - by),
+                               kf - (gx + gy) * __builtin_amdgcn_rcpf(bef + bx + by));
     const int ki = (int)kfl;
     const int jlo = (int)floorf(t.q0), jhi = (int)floorf(t.q3);
     if (ki + jhi < 0 || ki + jlo > g.nu - 1) continue;
     const int ulo = max(ki + jlo, 0), uhi = min(ki + jhi, g.nu - 1);
     const float w = sf_weight(fdx, (float)wx, (float)wy);
     const float* row = sino + (size_t)v * g.nu;
-    float accv = 0.0f;
+    float accv = 0.0f, edge = (float)(ulo - ki);
+    TrapWalk walk;
+    walk.start(t, edge);
     for (int u = ulo; u <= uhi; ++u) {
-      const float s1 = (float)(u - ki);
-      const float gm = trap_gamma(t, s1, s1 + 1.0f);
+      edge += 1.0f;
+      const float gm = walk.next(t, edge);
       accv = __builtin_fmaf((gm > 1e-7f) ? gm : 0.0f, row[u], accv);
     }
     acc += (double)(accv * w);
@@ -249,26 +310,29 @@ struct SfBwd {
     const double wx = p.fx + vg.w0x, wy = p.fy + vg.w0y;
     const double n0 = vg.e0x * wy - vg.e0y * wx;
     const double be = vg.pux * wy - vg.puy * wx;
-    const double kc = -n0 / be;
+    const double kc = -n0 * recip(be);
     const double kfl = floor(kc);
     const float kf = (float)(kc - kfl);
     const float kcf = (float)kc, bef = (float)be;
     const float gx = 0.5f * __builtin_fmaf(kcf, vg.gx1, vg.gx0), gy = 0.5f * __builtin_fmaf(kcf, vg.gy1, vg.gy0);
     const float bx = 0.5f * vg.gx1, by = 0.5f * vg.gy1;
     // corner c: k*(c) - kc = -(d.G) / (beta + d.grad beta)
-    const float q0 = kf + (gx + gy) * __builtin_amdgcn_rcpf(bef - bx - by);
-    const float q1 = kf + (gx - gy) * __builtin_amdgcn_rcpf(bef - bx + by);
-    const float q2 = kf - (gx - gy) * __builtin_amdgcn_rcpf(bef + bx - by);
-    const float q3 = kf - (gx + gy) * __builtin_amdgcn_rcpf(bef + bx + by);
-    const Trap t = make_trap(q0, q1, q2, q3);
+    const Trap t = sorted_trap(kf + (gx + gy) * __builtin_amdgcn_rcpf(bef - bx - by),
+                               kf + (gx - gy) * __builtin_amdgcn_rcpf(bef - bx + by),
+                               kf - (gx - gy) * __builtin_amdgcn_rcpf(bef + bx - by),
+                               kf - (gx + gy) * __builtin_amdgcn_rcpf(bef + bx + by));
     const int ki = (int)kfl;
     // bins of the trapezoid, inside the detector and the tile's window
     const int ulo = max(ki + (int)floorf(t.q0), wlo), uhi = min(ki + (int)floorf(t.q3), wlo + wn - 1);
     const float w = sf_weight((float)g.dx, (float)wx, (float)wy);
-    for (int u = ulo; u <= uhi; ++u) {
-      const float s1 = (float)(u - ki);
-      const float gm = trap_gamma(t, s1, s1 + 1.0f);
-      st.add(base + u - wlo, (gm > 1e-7f) ? gm : 0.0f, accv);
+    float edge = (float)(ulo - ki);
+    TrapWalk walk;
+    walk.start(t, edge);
+    int at = base + ulo - wlo;
+    for (int u = ulo; u <= uhi; ++u, ++at) {
+      edge += 1.0f;
+      const float gm = walk.next(t, edge);
+      st.add(at, (gm > 1e-7f) ? gm : 0.0f, accv);
     }
 #pragma unroll
     for (int s = 0; s < G; ++s) accv[s] *= w;
