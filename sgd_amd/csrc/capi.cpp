@@ -166,7 +166,7 @@ struct sgdct_projector {
   void* d_bins = nullptr;
   float* d_img = nullptr;   // staging for the host-array entry points
   float* d_sino = nullptr;
-  double* d_host_part = nullptr;  // their partial sums
+  double* d_host_part = nullptr;  // their partial sums and transposed image
   size_t host_part_cap = 0;
   float* h_img = nullptr;   // pinned
   float* h_sino = nullptr;  // pinned
@@ -996,8 +996,8 @@ int host_groups(const sgdct_projector* h) {
 
 size_t host_part_doubles(const sgdct_projector* h) {
   if (!host_alone(h)) return 0;
-  const size_t fs = host_segments(h), bs = host_groups(h);
-  return std::max(fs > 1 ? fs * h->np * h->nu : 0, bs > 1 ? bs * h->nx * h->ny : 0);
+  const size_t fs = is_hex(h->basis) ? host_segments(h) : 1, bs = host_groups(h), ni = (size_t)h->nx * h->ny;
+  return std::max(fs > 1 ? fs * h->np * h->nu : (ni + 1) / 2, bs > 1 ? bs * ni : 0);
 }
 
 int run_host_forward(sgdct_projector* h) {
@@ -1006,7 +1006,8 @@ int run_host_forward(sgdct_projector* h) {
   r.sym = plain_plan(h);
   r.lone = true;
   r.split = host_segments(h);
-  r.part = r.split > 1 ? h->d_host_part : nullptr;
+  if (!is_hex(h->basis)) r.cols = reinterpret_cast<float*>(h->d_host_part);  // the transposed image
+  else if (r.split > 1) r.part = h->d_host_part;
   const hipError_t e = launch_fwd2d(h, r, h->d_img, h->d_sino, nullptr);
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
 }

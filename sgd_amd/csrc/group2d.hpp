@@ -80,7 +80,7 @@ struct GroupRun {
   int g = 1;              // values per footprint, >= sym.nh * m (1, 2, 4 or 8)
   int m = 1, batch = 1;
   int split = 1;          // A: grid segments, A^T: view groups
-  bool lone = false;      // A (g = 1): one wave per workgroup
+  bool lone = false;      // A (g = 1): `split` line segments per bin, added within a workgroup
   double* part = nullptr; // FP64 partial sums (split > 1)
   float* rows = nullptr;  // A: interleaved images (null: g = 1, read in place)
   float* cols = nullptr;  // A: their transposes (null: column walks read strided)
@@ -92,8 +92,8 @@ struct GroupRun {
 // Waves of an A workgroup share one (view, 64-bin chunk): wave w walks the
 // lines m = w mod kFwdWaves of every bin's strip, and the FP64 sums of the
 // waves are added in wave order through LDS.
-// A lone run has one wave per workgroup, which walks whole segments line by
-// line.
+// In a lone run the waves walk whole segments line by line (wave w the segments
+// w mod kFwdWaves) and the segments' sums are added in segment order.
 constexpr int kFwdWaves = 8;
 
 // The chunk a workgroup takes: centre chunks (whose strips are longest) first,

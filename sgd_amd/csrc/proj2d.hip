@@ -73,6 +73,34 @@ __global__ __launch_bounds__(64 * W) void fwd_group_kernel(Proj2DArgs g, SymPlan
                         Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]), sino, gridDim.z > 1 ? part : nullptr);
 }
 
+// A of one image in nseg line segments per bin, each summed by itself in line
+// order and the segments in theirs (GroupRun::lone).  Same bounds as
+// fwd_group_kernel; a wave's set-up serves its segments, and their sums stay in
+// LDS (one segment per wave, its sums through HBM: B0 at 256 x 256, 360 views,
+// 512 bins 131 -> 112 us, B1 at 400 x 380, 500 views, 700 bins 422 -> 395 us).
+// grid (np * nchunk), nseg rows of 64 doubles of LDS.
+template <int BASIS>
+__global__ __launch_bounds__(64 * kFwdWaves) void fwd_lone_kernel(Proj2DArgs g, int nseg,
+                                                                  const float* __restrict__ img,
+                                                                  const float* __restrict__ cols_img,
+                                                                  float* __restrict__ sino) {
+  extern __shared__ double lone_red[];
+  double(*const red)[64] = reinterpret_cast<double(*)[64]>(lone_red);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rank = blockIdx.x / g.np, v = blockIdx.x - rank * g.np;
+  const int chunk = centre_out(rank, g.nchunk);
+  for (int k = wv; k < nseg; k += kFwdWaves) {
+    double acc[1] = {0.0};
+    fwd_bin_lines<BASIS, 1>(g, v, chunk, img, cols_img, 0, 1, k, nseg, acc);
+    red[k][lane] = acc[0];
+  }
+  __syncthreads();
+  const int u = chunk * 64 + lane;
+  if (u >= g.nu) return;
+  const typename Traits<BASIS>::Bin* bins = reinterpret_cast<const typename Traits<BASIS>::Bin*>(g.bins);
+  fwd_lone_store(nseg, red, g.dx, g.dy, Traits<BASIS>::scale(bins[(size_t)v * g.nu + u]), sino + (size_t)v * g.nu + u);
+}
+
 // Interleaved copies of the images of one launch: slot s = image * nh + h of
 // pixel p holds the image at h p, rows[(iy nx + ix) G + s], and transposed,
 // cols[(ix ny + iy) G + s] (either null: not wanted).  grid (tiles x, tiles y, image
@@ -232,7 +260,12 @@ template <int BASIS>
 hipError_t forward_b(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
   switch (r.g) {
     case 1:
-      return r.lone ? forward_g<BASIS, 1, 1>(g, r, img, sino, s) : forward_g<BASIS, 1, kFwdWaves>(g, r, img, sino, s);
+      if (r.lone) {
+        fwd_lone_kernel<BASIS><<<(unsigned)(g.np * g.nchunk), 64 * kFwdWaves, (size_t)r.split * 64 * sizeof(double), s>>>(
+            g, r.split, img, r.cols, sino);
+        return hipGetLastError();
+      }
+      return forward_g<BASIS, 1, kFwdWaves>(g, r, img, sino, s);
     case 2: return forward_g<BASIS, 2, kFwdWaves>(g, r, img, sino, s);
     case 4: return forward_g<BASIS, 4, kFwdWaves>(g, r, img, sino, s);
     case 8: return forward_g<BASIS, 8, kFwdWaves>(g, r, img, sino, s);
@@ -267,13 +300,14 @@ hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float
 // r.split > 1 needs r.part with split * batch * np * nu doubles.
 hipError_t launch_forward(int basis, const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino,
                           hipStream_t s) {
-  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  if (r.split < 1 || (r.split > 1 && !r.part && !r.lone)) return hipErrorInvalidValue;
   hipError_t e = r.rows || r.cols ? launch_interleave(g, r, img, s) : hipSuccess;
   if (e != hipSuccess) return e;
   if (basis == BASIS_B1) e = forward_b<BASIS_B1>(g, r, img, sino, s);
   else if (basis == BASIS_B0) e = forward_b<BASIS_B0>(g, r, img, sino, s);
   else return hipErrorInvalidValue;
-  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
+  if (e == hipSuccess && r.split > 1 && !r.lone)
+    e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
   return e;
 }
 

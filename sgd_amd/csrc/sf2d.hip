@@ -53,6 +53,25 @@ __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp
   fwd_group_store<G, W>(g, sp, rep, v, u, m, batch, red, 1.0, 1.0, 1.0, sino, gridDim.z > 1 ? part : nullptr);
 }
 
+// A of one image in nseg line segments per bin, as fwd_lone_kernel.
+__global__ __launch_bounds__(64 * kFwdWaves) void sf_lone_kernel(Proj2DArgs g, int nseg, const float* __restrict__ img,
+                                                                 const float* __restrict__ cols_img,
+                                                                 float* __restrict__ sino) {
+  extern __shared__ double lone_red[];
+  double(*const red)[64] = reinterpret_cast<double(*)[64]>(lone_red);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rank = blockIdx.x / g.np, v = blockIdx.x - rank * g.np;
+  const int chunk = centre_out(rank, g.nchunk);
+  for (int k = wv; k < nseg; k += kFwdWaves) {
+    double acc[1] = {0.0};
+    sf_fwd_lines<1>(g, v, chunk, img, cols_img, 0, 1, k, nseg, acc);
+    red[k][lane] = acc[0];
+  }
+  __syncthreads();
+  const int u = chunk * 64 + lane;
+  if (u < g.nu) fwd_lone_store(nseg, red, 1.0, 1.0, 1.0, sino + (size_t)v * g.nu + u);
+}
+
 // A^T, launched as bwd_group_kernel; same cases as above: 841 -> 151 us, 4.13
 // -> 0.64 ms, 146 -> 49 us, 869 -> 664 us.  The FP64 projection of the pixel's
 // centre and its sorted corners are formed once per view for all values, and
@@ -96,11 +115,15 @@ hipError_t sf_backward_g(const Proj2DArgs& g, const GroupRun& r, const float* si
 }  // namespace
 
 hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
-  if (r.split < 1 || (r.split > 1 && !r.part)) return hipErrorInvalidValue;
+  if (r.split < 1 || (r.split > 1 && !r.part && !r.lone)) return hipErrorInvalidValue;
   hipError_t e = r.rows || r.cols ? launch_interleave(g, r, img, s) : hipSuccess;
   if (e != hipSuccess) return e;
-  if (r.g == 1 && r.lone) e = sf_forward_g<1, 1>(g, r, img, sino, s);
-  else if (r.g == 1) e = sf_forward_g<1, kFwdWaves>(g, r, img, sino, s);
+  if (r.g == 1 && r.lone) {
+    sf_lone_kernel<<<(unsigned)(g.np * g.nchunk), 64 * kFwdWaves, (size_t)r.split * 64 * sizeof(double), s>>>(
+        g, r.split, img, r.cols, sino);
+    return hipGetLastError();
+  }
+  if (r.g == 1) e = sf_forward_g<1, kFwdWaves>(g, r, img, sino, s);
   else if (r.g == 2) e = sf_forward_g<2, kFwdWaves>(g, r, img, sino, s);
   else if (r.g == 4) e = sf_forward_g<4, kFwdWaves>(g, r, img, sino, s);
   else if (r.g == 8) e = sf_forward_g<8, kFwdWaves>(g, r, img, sino, s);
