@@ -114,13 +114,17 @@ __device__ __forceinline__ void fwd_group_store(const Proj2DArgs& g, const SymPl
 }
 
 // A lone run's sums of bin u over its segments, times the bin's factors one by
-// one, added in segment order.  All threads of the workgroup call this after
+// one (each product rounded before the addition), added in segment order.  All threads of the workgroup call this after
 // writing red and a barrier.
 __device__ __forceinline__ void fwd_lone_store(int nseg, const double (*red)[64], double f0, double f1, double f2,
                                                float* out) {
   if (threadIdx.x >= 64) return;
   double t = 0.0;
-  for (int k = 0; k < nseg; ++k) t += red[k][threadIdx.x] * f0 * f1 * f2;
+  for (int k = 0; k < nseg; ++k) {
+#pragma clang fp contract(off)
+    const double p = red[k][threadIdx.x] * f0 * f1 * f2;
+    t += p;
+  }
   *out = (float)t;
 }
 
