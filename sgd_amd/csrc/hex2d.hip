@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "footprint.hpp"
 #include "group2d_dev.hpp"
@@ -27,12 +28,28 @@ namespace sgdct {
 
 hipError_t launch_sum_parts(const double* part, float* out, size_t n, int nparts, hipStream_t s);
 
-// Rhombus (va, vb) of H0: trapezoid box_p * box_q centred at c = (va + vb)/2.
+// H0: the hexagon's vertices project to +-a, +-b, +-c (a = b + c, the lengths
+// of its edges' projections), between which its chord length is linear.
 struct H0Bin {
-  float ka, kb;
-  float c[3], hpq[3], hmq[3], ip[3], i2pq[3];
-  float pad[3];
+  float ka, kb, a, b;
+  float c, d, k1, k2;    // d = b - c, 1 / (6 b c), 1 / (3 b)
+  float k3, k4, pad[2];  // 1 / (6 a b), 2 / (3 a)
 };
+
+// Antiderivative of the projection of a hexagon of unit area, odd in t: the
+// mean of three rhombi box_b * box_c, box_a * box_b and box_a * box_c about
+// a / 2, -c / 2 and -b / 2 (layers/A_H0.cu:229-248), whose sum over the tail
+// x = |t| is one quadratic per interval between vertices:
+//   1/2 - S(x) = u^2 / (6 b c) + v / (3 b) + v^2 / (6 a b) + 2 w / (3 a)
+// with the depths u, v, w of x into [b, a], [c, b] and [0, c].
+__device__ __forceinline__ float s_h0(float t, const H0Bin& r) {
+  const float x = __builtin_fabsf(t);
+  const float u = __builtin_amdgcn_fmed3f(r.a - x, 0.0f, r.c);
+  const float v = __builtin_amdgcn_fmed3f(r.b - x, 0.0f, r.d);
+  const float w = __builtin_fmaxf(r.c - x, 0.0f);
+  const float tail = __builtin_fmaf(u, u * r.k1, __builtin_fmaf(v, __builtin_fmaf(v, r.k3, r.k2), w * r.k4));
+  return copysign_f(0.5f - tail, t);
+}
 
 // Hl: widths p >= q >= r (p = q + r) of box_p * box_q * box_r.
 struct HlBin {
@@ -62,14 +79,7 @@ template <int HB> struct HexTraits;
 template <> struct HexTraits<BASIS_H0> {
   using Bin = H0Bin;
   __device__ static __forceinline__ float conv(const Bin& r, float ta, float tb) {
-    float s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const float sa = s_b0(ta - r.c[k], r.hpq[k], r.hmq[k], r.ip[k], r.i2pq[k]);
-      const float sb = s_b0(tb - r.c[k], r.hpq[k], r.hmq[k], r.ip[k], r.i2pq[k]);
-      s += sb - sa;
-    }
-    const float cv = s * (1.0f / 3.0f) * __builtin_amdgcn_rcpf(tb - ta);
+    const float cv = (s_h0(tb, r) - s_h0(ta, r)) * __builtin_amdgcn_rcpf(tb - ta);
     return cv > 0.0f ? cv : 0.0f;  // conv > 0 (layers/A_H0.cu:248)
   }
 };
@@ -119,7 +129,7 @@ __device__ __forceinline__ void load_point(const float* p, float (&x)[G]) {
 // rows at a time, which keeps the lines they touch in the vector L1 (walking
 // the whole lattice, near-row strips needed their rows staged in LDS for
 // that).
-template <int HB, int G>
+template <int HB, int G, bool FAR>
 __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chunk, const float* __restrict__ img, int w,
                                               int wn, int seg, int nseg, double (&acc)[G]) {
   using T = HexTraits<HB>;
@@ -144,28 +154,61 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
   const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
   const double imq = mq != 0.0 ? 1.0 / mq : 0.0, imr = mr != 0.0 ? 1.0 / mr : 0.0;
 
-  // One line: points i0, i0 + step, ... <= i1, `stride` floats apart.
-  auto walk = [&](const float* p, int i0, int i1, int step, size_t stride, float ta, float tb, float dta, float dtb) {
+  // Point values by 32-bit byte offsets into a buffer resource, or by address,
+  // clamped to the last point: for a lattice of 4 GiB and more (FAR), and for 8
+  // values, whose two 16-byte loads the vector L1 serves faster so (Hl, batch
+  // 64: 7.07 ms against 7.92).
+  using Off = std::conditional_t<FAR, size_t, unsigned>;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
+  const Off last_point = 4 * (Off)G * ((Off)g.nx * g.ny - 1);
+  auto fetch = [&](Off off, float (&x)[G]) {
+    if constexpr (FAR || G == 8)
+      load_point<G>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(img) + min(off, last_point)), x);
+    else
+      buffer_load_n<G>(rsrc, off, x);
+  };
+  // One line: n points `step` bytes apart from `off`.
+  auto walk = [&](Off off, int n, Off step, float ta, float tb, float dta, float dtb) {
     float accl[G], xn[G];
 #pragma unroll
     for (int s = 0; s < G; ++s) accl[s] = 0.0f;
-    // the next point's values are requested one step ahead (the index clamped
-    // to the line's last point, so the read needs no branch), which overlaps
+    // the next point's values are requested one step ahead, which overlaps
     // their latency with the footprint evaluation
-    load_point<G>(p + (size_t)i0 * stride, xn);
-    for (int i = i0; i <= i1; i += step) {
+    fetch(off, xn);
+    const Off end = off + (Off)n * step;
+    do {
       float xc[G];
 #pragma unroll
       for (int s = 0; s < G; ++s) xc[s] = xn[s];
-      load_point<G>(p + (size_t)min(i + step, i1) * stride, xn);
+      off += step;
+      fetch(off, xn);
       const float c = T::conv(rec, ta, tb);
 #pragma unroll
       for (int s = 0; s < G; ++s) accl[s] = __builtin_fmaf(c, xc[s], accl[s]);
       ta += dta;
       tb += dtb;
-    }
+    } while (off != end);
 #pragma unroll
     for (int s = 0; s < G; ++s) acc[s] += (double)accl[s];
+  };
+  // Points n of line l in the strip, from q: N_q + R_q >= 0 and r: N_r - R_r <
+  // 0 with N = slope n + cross l + c: [ceil(lo0 + lo1 l), floor(hi0 + hi1 l)] in
+  // FP32, widened by its error bound (the footprint is zero at the boundary);
+  // every point of the line unless both slopes have one sign.
+  float lo0 = -1e30f, lo1 = 0.0f, hi0 = 1e30f, hi1 = 0.0f;
+  auto interval = [&](double sl_q, double cr_q, double sl_r, double cr_r, double iq, double ir, int nline) {
+    if (!((sl_q > 0.0 && sl_r > 0.0) || (sl_q < 0.0 && sl_r < 0.0))) return;
+    const bool up = sl_q > 0.0;
+    const float p0 = (float)((-rq - cq) * iq), p1 = (float)(-cr_q * iq);
+    const float s0 = (float)((rr - cr) * ir), s1 = (float)(-cr_r * ir);
+    lo0 = up ? p0 : s0;
+    lo1 = up ? p1 : s1;
+    hi0 = up ? s0 : p0;
+    hi1 = up ? s1 : p1;
+    const float most = (float)nline;
+    lo0 -= 4e-7f * __builtin_fmaf(fabsf(lo1), most, fabsf(lo0)) + 1e-5f;
+    hi0 += 4e-7f * __builtin_fmaf(fabsf(hi1), most, fabsf(hi0)) + 1e-5f;
   };
 
   const int umid = min(chunk * 64 + 32, g.nu - 1);
@@ -189,24 +232,22 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
       il_hi = min(il_hi, seg * len + len - 1);
     }
     if (!inside) il_hi = -1;
-    const double kas = ka * sa, kbs = kb * sb;
+    interval(sq, mq, sr, mr, isq, isr, g.ny);
+    const double kas = ka * sa, kam = ka * ma, kac = ka * ca, kbs = kb * sb, kbm = kb * mb, kbc = kb * cb;
     const float dta = (float)kas, dtb = (float)kbs;
+    const float fc_lo = (float)c_lo, fc_hi = (float)c_hi, fc_odd = (float)min(c_hi, g.nx - 2);
+    const Off step = 4 * G;
     for (int il = il_lo; il <= il_hi; ++il) {
-      const double sh = (il & 1) ? 0.5 : 0.0;
-      const double r1 = -rq - __builtin_fma(mq, (double)il, cq) - sq * sh;  // need sq * ic >= r1
-      const double r2 = rr - __builtin_fma(mr, (double)il, cr) - sr * sh;   // need sr * ic <  r2
-      double lo = (double)c_lo, hi = (double)min(c_hi, g.nx - 1 - (il & 1));
-      if (sq > 0.0) lo = fmax(lo, ceil(r1 * isq));
-      else if (sq < 0.0) hi = fmin(hi, floor(r1 * isq));
-      else if (r1 > 0.0) continue;
-      if (sr > 0.0) hi = fmin(hi, ceil(r2 * isr) - 1.0);
-      else if (sr < 0.0) lo = fmax(lo, floor(r2 * isr) + 1.0);
-      else if (r2 <= 0.0) continue;
-      if (lo > hi) continue;
-      const int n0 = (int)lo;
-      walk(img + (size_t)il * g.nx * G, n0, (int)hi, 1, G,
-           (float)__builtin_fma(kas, n0 + sh, ka * __builtin_fma(ma, (double)il, ca)),
-           (float)__builtin_fma(kbs, n0 + sh, kb * __builtin_fma(mb, (double)il, cb)), dta, dtb);
+      const bool odd = il & 1;  // points half a column to the right
+      const float sh = odd ? 0.5f : 0.0f, fl = (float)il;
+      const float flo = fmaxf(ceilf(__builtin_fmaf(fl, lo1, lo0) - sh), fc_lo);
+      const float fhi = fminf(floorf(__builtin_fmaf(fl, hi1, hi0) - sh), odd ? fc_odd : fc_hi);
+      if (!(flo <= fhi)) continue;
+      const int n0 = (int)flo;
+      const double dn = (double)(flo + sh), dl = (double)il;
+      walk(4 * G * ((Off)il * g.nx + n0), (int)fhi - n0 + 1, step,
+           (float)__builtin_fma(kas, dn, __builtin_fma(kam, dl, kac)),
+           (float)__builtin_fma(kbs, dn, __builtin_fma(kbm, dl, kbc)), dta, dtb);
     }
   } else {
     const int r_lo = g.ny * w / wn, r_hi = g.ny * (w + 1) / wn - 1;
@@ -229,28 +270,24 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
       k_hi = min(k_hi, seg * len + len - 1);
     }
     if (!inside) k_hi = -1;
-    const double kam = ka * ma, kbm = kb * mb;
+    interval(mq, 0.5 * sq, mr, 0.5 * sr, imq, imr, kmax + 1);
+    const double kam = ka * ma, kas = 0.5 * ka * sa, kac = ka * ca, kbm = kb * mb, kbs = 0.5 * kb * sb, kbc = kb * cb;
     const float dta = (float)(2.0 * kam), dtb = (float)(2.0 * kbm);
-    for (int k = k_lo; k <= k_hi; ++k) {
-      const int par = k & 1;
-      const double xh = 0.5 * k;                   // ic' of the line
-      const double r1 = -rq - cq - sq * xh;        // need mq * il >= r1
-      const double r2 = rr - cr - sr * xh;         // need mr * il <  r2
-      double lo = (double)r_lo, hi = (double)r_hi;
-      if (mq > 0.0) lo = fmax(lo, ceil(r1 * imq));
-      else if (mq < 0.0) hi = fmin(hi, floor(r1 * imq));
-      else if (r1 > 0.0) continue;
-      if (mr > 0.0) hi = fmin(hi, ceil(r2 * imr) - 1.0);
-      else if (mr < 0.0) lo = fmax(lo, floor(r2 * imr) + 1.0);
-      else if (r2 <= 0.0) continue;
-      if (lo > hi) continue;
-      int i0 = (int)lo, i1 = (int)hi;
-      i0 += (i0 ^ par) & 1;  // rows of the line's parity
-      i1 -= (i1 ^ par) & 1;
+    const float fr_lo = (float)r_lo, fr_hi = (float)r_hi;
+    const Off step = 8 * G * (Off)g.nx;
+    for (int k = k_lo; k <= k_hi; ++k) {  // ic' = k / 2
+      const float fk = (float)k;
+      const float flo = fmaxf(ceilf(__builtin_fmaf(fk, lo1, lo0)), fr_lo);
+      const float fhi = fminf(floorf(__builtin_fmaf(fk, hi1, hi0)), fr_hi);
+      if (!(flo <= fhi)) continue;
+      int i0 = (int)flo, i1 = (int)fhi;
+      i0 += (i0 ^ k) & 1;  // rows of the line's parity
+      i1 -= (i1 ^ k) & 1;
       if (i0 > i1) continue;
-      walk(img + (size_t)(k >> 1) * G, i0, i1, 2, (size_t)g.nx * G,
-           (float)__builtin_fma(kam, (double)i0, ka * (sa * xh + ca)),
-           (float)__builtin_fma(kbm, (double)i0, kb * (sb * xh + cb)), dta, dtb);
+      const double dk = (double)k, di = (double)i0;
+      walk(4 * G * ((Off)i0 * g.nx + (k >> 1)), ((i1 - i0) >> 1) + 1, step,
+           (float)__builtin_fma(kam, di, __builtin_fma(kas, dk, kac)),
+           (float)__builtin_fma(kbm, di, __builtin_fma(kbs, dk, kbc)), dta, dtb);
     }
   }
 }
@@ -259,12 +296,13 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
 // view and 64-bin chunk, and their FP64 sums are added in wave order through
 // LDS.  Chunk-major: workgroups in flight take the same bins of adjacent views,
 // so they walk nearly the same points and reach the lattice together or miss
-// it together.  Bound by VALU issue (H0: six trapezoid antiderivatives, ~75
-// instructions per footprint; Hl ~35) and, at G = 8, by the vector L1.  Per
-// call, one value per footprint and one wave per (view, chunk) -> now: H0 256
-// x 296 points, 1024 views, 1024 bins 840 -> 476 us; Hl, batch 64 30.8 -> 7.1
-// ms; Hl 40 x 46, 60 views, batch 3 76 -> 20 us.
-template <int HB, int G, int W>
+// it together.  Bound by VALU issue (~45 instructions per footprint, and about
+// as many per line and lane) and, at G = 8, by the vector L1.  Per call, one
+// value per footprint and one wave per (view, chunk) -> now: H0 256 x 296
+// points, 1024 views, 1024 bins 840 -> 318 us (476 with three rhombi's six
+// antiderivatives and FP64 intervals); Hl, batch 64 30.8 -> 7.0 ms; Hl 40 x 46,
+// 60 views, batch 3 76 -> 16 us.
+template <int HB, int G, int W, bool FAR>
 __global__ __launch_bounds__(64 * W) void hex_fwd_kernel(HexArgs ha, SymPlan sp, int m, int batch,
                                                          const float* __restrict__ img, float* __restrict__ sino,
                                                          double* __restrict__ part) {
@@ -277,7 +315,7 @@ __global__ __launch_bounds__(64 * W) void hex_fwd_kernel(HexArgs ha, SymPlan sp,
   double acc[G];
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
-  hex_fwd_lines<HB, G>(ha, v, chunk, img + (size_t)blockIdx.y * G * g.nx * g.ny, wv, W, blockIdx.z, gridDim.z, acc);
+  hex_fwd_lines<HB, G, FAR>(ha, v, chunk, img + (size_t)blockIdx.y * G * g.nx * g.ny, wv, W, blockIdx.z, gridDim.z, acc);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
@@ -391,9 +429,10 @@ template <int HB> struct HexBwd {
   }
 };
 
-// Launched as bwd_group_kernel; bound by the LDS reads of the records (80 bytes
-// per footprint for H0) and VALU issue.  Same cases as hex_fwd_kernel: 728 ->
-// 437 us, 33.2 -> 5.5 ms, 39 -> 14 us.
+// Launched as bwd_group_kernel; bound by VALU issue and the LDS reads of the
+// records (48 bytes per footprint for H0; 80 with three rhombi, 437 us in the
+// first case).  Same cases as hex_fwd_kernel: 728 -> 257 us, 33.2 -> 5.5 ms, 39
+// -> 14 us.
 template <int HB, int G>
 __global__ __launch_bounds__(256) void hex_bwd_group_kernel(HexArgs ha, SymPlan sp, int m, int batch,
                                                             const float* __restrict__ sino, float* __restrict__ img,
@@ -417,9 +456,9 @@ __global__ __launch_bounds__(256) void hex_bwd_kernel(HexArgs ha, const float* _
   using Bin = typename T::Bin;
   constexpr int BIN4 = sizeof(Bin) / 16;
   static_assert(sizeof(Bin) % 16 == 0, "bin records are whole float4s");
-  // LDS bin window per view: H0's 80-byte records at 128 bins would hold 42
-  // KB per block (3 waves per SIMD); a 16 x 16 H0 tile spans up to ~66 bins
-  // at 0.3 mm per bin, and bins past the window are read from global memory
+  // LDS bin window per view: 72 of H0's 48-byte records (14 KB a block; a 16 x
+  // 16 H0 tile spans up to ~66 bins at 0.3 mm per bin); bins past the window are
+  // read from global memory
   constexpr int kWin = HB == BASIS_H0 ? kHexH0Window : kMaxWindow;
   __shared__ float4 lds[kViewChunk][kWin][BIN4];
   __shared__ float ldsy[kViewChunk][kWin];
@@ -567,29 +606,26 @@ void hex_bin_constants(int basis, const ViewGeo& v, int nu, double dt, void* out
     const double th = (double)(float)std::atan2(cx, cy);
     double vk[3];
     for (int k = 0; k < 3; ++k) vk[k] = dt * std::sin(th + k * 2.0 * 3.14159265358979323846 / 3.0);
+    double w[3] = {std::fabs(vk[0]), std::fabs(vk[1]), std::fabs(vk[2])};
+    std::sort(w, w + 3);
     if (basis == BASIS_H0) {
       H0Bin r{};
       r.ka = (float)ka;
       r.kb = (float)kb;
-      const int pr[3][2] = {{0, 1}, {1, 2}, {2, 0}};
-      for (int k = 0; k < 3; ++k) {
-        const double a = vk[pr[k][0]], b = vk[pr[k][1]];
-        const double p = std::max(std::fabs(a), std::fabs(b));
-        double q = std::min(std::fabs(a), std::fabs(b));
-        if (!(q > 1e-7)) q = 0.0;
-        r.c[k] = (float)(0.5 * (a + b));
-        r.hpq[k] = (float)(0.5 * (p + q));
-        r.hmq[k] = (float)(0.5 * (p - q));
-        r.ip[k] = (float)(1.0 / p);
-        r.i2pq[k] = q > 0.0 ? (float)(1.0 / (2.0 * p * q)) : 0.0f;
-      }
+      const double a = w[2], b = w[1], c = w[0];
+      r.a = (float)a;
+      r.b = (float)b;
+      r.c = (float)c;
+      r.d = (float)(b - c);
+      r.k1 = c > 1e-30 ? (float)(1.0 / (6.0 * b * c)) : 0.0f;
+      r.k2 = (float)(1.0 / (3.0 * b));
+      r.k3 = (float)(1.0 / (6.0 * a * b));
+      r.k4 = (float)(2.0 / (3.0 * a));
       static_cast<H0Bin*>(out)[u] = r;
     } else {
       HlBin r{};
       r.ka = (float)ka;
       r.kb = (float)kb;
-      double w[3] = {std::fabs(vk[0]), std::fabs(vk[1]), std::fabs(vk[2])};
-      std::sort(w, w + 3);
       const double p = w[2], q = w[1], rr = w[0];
       r.p = (float)p;
       r.q = (float)q;
@@ -619,7 +655,11 @@ hipError_t hex_forward_g(const HexArgs& ha, const GroupRun& r, const float* img,
     hex_interleave_kernel<G><<<dim3((unsigned)(g.nx + 15) / 16, (unsigned)(g.ny + 15) / 16, (unsigned)r.groups()), 256,
                                0, s>>>(r.sym, g.nx, g.ny, r.m, r.batch, img, r.rows);
   const dim3 grid((unsigned)(r.sym.nrep * g.nchunk), (unsigned)r.groups(), (unsigned)r.split);
-  hex_fwd_kernel<HB, G, W><<<grid, 64 * W, 0, s>>>(ha, r.sym, r.m, r.batch, r.rows ? r.rows : img, sino, r.part);
+  const float* const p = r.rows ? r.rows : img;
+  if (G == 1 && (size_t)g.nx * g.ny >= (size_t)1 << 30)
+    hex_fwd_kernel<HB, 1, W, true><<<grid, 64 * W, 0, s>>>(ha, r.sym, r.m, r.batch, p, sino, r.part);
+  else
+    hex_fwd_kernel<HB, G, W, false><<<grid, 64 * W, 0, s>>>(ha, r.sym, r.m, r.batch, p, sino, r.part);
   return hipGetLastError();
 }
 
