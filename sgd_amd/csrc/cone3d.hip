@@ -113,7 +113,7 @@ __device__ __forceinline__ AxialTrap trap_from_corners(const Cone3DArgs& a, cons
   t.v2 = fmaxf(h1, l2);
   const float oz = zc * a.dz;
   if (M == CONE_B1) {
-    const float w = __builtin_sqrtf(__builtin_fmaf(oz * oz, 1.0f / c.r2, 1.0f));
+    const float w = __builtin_amdgcn_sqrtf(__builtin_fmaf(oz * oz, __builtin_amdgcn_rcpf(c.r2), 1.0f));
     t.cf = a.cvol * w * 2.0f * __builtin_amdgcn_rcpf((t.v3 - t.v0) + (t.v2 - t.v1));
   } else {
     if (M == CONE_SF_TR) {  // a1 == b1, a2 == b2: a rectangle
@@ -168,14 +168,29 @@ __device__ __forceinline__ float row_off() {
 // gives the overlap's ends (equal when they do not meet).  The sloped sides
 // divide by their widths through the voxel's precomputed reciprocals, zero
 // for a side of zero width, which never overlaps.
+// A walk over adjacent rows carries the last upper edge on.
+struct AxialWalk {
+  float c0, c1, c2;  // the edge clamped into the three segments
+  __device__ __forceinline__ void start(const AxialTrap& t, float s) {
+    c0 = clamp3(s, t.v0, t.v1);
+    c1 = clamp3(s, t.v1, t.v2);
+    c2 = clamp3(s, t.v2, t.v3);
+  }
+  __device__ __forceinline__ float next(const AxialTrap& t, float e) {
+    AxialWalk n;
+    n.start(t, e);
+    const float g0 = (n.c0 - c0) * (n.c0 + c0 - 2.0f * t.v0) * t.i01;
+    const float g2 = (n.c2 - c2) * (2.0f * t.v3 - c2 - n.c2) * t.i23;
+    const float g = g0 + (n.c1 - c1) + g2;
+    *this = n;
+    return g;
+  }
+};
+
 __device__ __forceinline__ float trap_gamma(float s, const AxialTrap& t) {
-  const float e = s + 1.0f;
-  const float s0 = clamp3(s, t.v0, t.v1), e0 = clamp3(e, t.v0, t.v1);
-  const float s1 = clamp3(s, t.v1, t.v2), e1 = clamp3(e, t.v1, t.v2);
-  const float s2 = clamp3(s, t.v2, t.v3), e2 = clamp3(e, t.v2, t.v3);
-  const float g0 = (e0 - s0) * (e0 + s0 - 2.0f * t.v0) * t.i01;
-  const float g2 = (e2 - s2) * (2.0f * t.v3 - s2 - e2) * t.i23;
-  return g0 + (e1 - s1) + g2;
+  AxialWalk w;
+  w.start(t, s);
+  return w.next(t, s + 1.0f);
 }
 
 template <int M>
@@ -220,7 +235,7 @@ __global__ __launch_bounds__(256) void axial_fwd_kernel(Cone3DArgs a, int p0, co
   // above vc and min(ka, kb) below; it grows with iz (ka, kb > 0: voxels in
   // front of the source), so the first voxel reaching a row follows from that
   // line up to rounding, and the staged values settle it exactly
-  const float ikhi = 1.0f / fmaxf(ca.ka, ca.kb), iklo = 1.0f / fminf(ca.ka, ca.kb);
+  const float ikhi = __builtin_amdgcn_rcpf(fmaxf(ca.ka, ca.kb)), iklo = __builtin_amdgcn_rcpf(fminf(ca.ka, ca.kb));
   const float zoff = 0.5f * (float)(a.nz - 1) - 0.5f;
   // voxels [z0, z1): stage their records, then add their share to every row
   auto chunk = [&](int z0, int z1, bool first) {
@@ -289,7 +304,7 @@ __device__ __forceinline__ int image_column(const Proj2DArgs& g, int op, int c) 
 // Dynamic LDS: per column and voxel 6 + G floats and one of padding to an odd
 // stride.  Bound by the LDS reads of the records and, at G = 4, by the stores
 // of Y.  256^3 voxels, 360 views, 512 x 384, classes of 4: A as a whole 40.0 ->
-// 20.4 ms against one view at a time.
+// 20.0 ms against one view at a time.
 template <int M, int G>
 __global__ __launch_bounds__(256) void axial_fwd_group_kernel(Cone3DArgs a, int p0, const float* __restrict__ xT,
                                                               float* __restrict__ Y) {
@@ -322,7 +337,7 @@ __global__ __launch_bounds__(256) void axial_fwd_group_kernel(Cone3DArgs a, int 
   __syncthreads();
   if (!live) return;
   // first voxel that reaches a row, as in axial_fwd_kernel
-  const float ikhi = 1.0f / fmaxf(ca.ka, ca.kb), iklo = 1.0f / fminf(ca.ka, ca.kb);
+  const float ikhi = __builtin_amdgcn_rcpf(fmaxf(ca.ka, ca.kb)), iklo = __builtin_amdgcn_rcpf(fminf(ca.ka, ca.kb));
   const float zoff = 0.5f * (float)(a.nz - 1) - 0.5f;
   for (int j = t; j < a.nv; j += 128) {
     const float fj = (float)j + row_off<M>();
@@ -716,8 +731,11 @@ __global__ __launch_bounds__(256) void axial_bwd_kernel(Cone3DArgs a, int p0, in
       }
       float sum = 0.0f;
       float sj = (float)(jlo - k0) + ro;
-      for (int j = jlo; j <= jhi; ++j, sj += 1.0f) {
-        const float gm = trap_gamma(sj, t);
+      AxialWalk walk;
+      walk.start(t, sj);
+      for (int j = jlo; j <= jhi; ++j) {
+        sj += 1.0f;
+        const float gm = walk.next(t, sj);
         if (keep_gamma<M>(gm)) sum = __builtin_fmaf(gm, yl[j - r0], sum);
       }
       acc[s] += (double)(t.cf * sum);
@@ -737,7 +755,7 @@ __global__ __launch_bounds__(256) void axial_bwd_kernel(Cone3DArgs a, int p0, in
 // Block: 256 voxels of one column; grid (ndom, ceil(nz / 256)).  The next
 // view's profiles are requested before the current view's rows are gathered.
 // nv <= kGroupRows.  Bound by the reads of the profiles (1.6 GB per 16 views of
-// the case above); A^T as a whole 34.3 -> 21.3 ms.
+// the case above); A^T as a whole 34.3 -> 20.7 ms.
 constexpr int kGroupRows = 512;
 
 template <int M, int G>
@@ -801,8 +819,11 @@ __global__ __launch_bounds__(256) void axial_bwd_group_kernel(Cone3DArgs a, int 
 #pragma unroll
       for (int h = 0; h < G; ++h) sum[h] = 0.0f;
       float sj = (float)(jlo - k0) + ro;
-      for (int j = jlo; j <= jhi; ++j, sj += 1.0f) {
-        const float gm = trap_gamma(sj, tr);
+      AxialWalk walk;
+      walk.start(tr, sj);
+      for (int j = jlo; j <= jhi; ++j) {
+        sj += 1.0f;
+        const float gm = walk.next(tr, sj);
         if (keep_gamma<M>(gm)) {
           float y[G];
           __builtin_memcpy(y, __builtin_assume_aligned(prof + j * G, G < 4 ? 4 * G : 16), sizeof(y));
