@@ -6,7 +6,8 @@
 //   H0: hexagon indicator (circumradius dt, dyh = 1.5 dt) = three rhombi; the
 //       value is the bin average of the sum of the three rhombus projections
 //       (box splines of two of va, vb, vc each, A_H0.cu:229-245), divided by 3
-//       so that it is the hexagon's projection (the reference omits the 1/3).
+//       so that it is the hexagon's projection (the reference omits the 1/3);
+//       evaluated as the hexagon's own chord length (s_h0).
 //   Hl: three-direction box spline (dyh = dt/2), bin average of
 //       box_|va| * box_|vb| * box_|vc| (A_Hl.cu:226-236).
 // va, vb, vc = dt sin(theta + 2 pi k / 3), theta the bin's central-ray angle

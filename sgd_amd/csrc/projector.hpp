@@ -100,7 +100,8 @@ struct BatchPlan {
 // selects a view group, whose bin records and sinogram rows every x-y tile of
 // that z reads, so each XCD's L2 then holds the records of its own groups
 // instead of all of them.  Any grid: XCD k takes items [k q + min(k, r), ...)
-// with q = n / 8, r = n % 8.  Used where it measured faster (SF and H0 A^T).
+// with q = n / 8, r = n % 8.  Used by H0's A^T
+// where the tiles' bin windows are too wide for the grouped frame's LDS.
 constexpr unsigned kXcds = 8;
 __device__ __forceinline__ uint3 xcd_block() {
   const unsigned tx = gridDim.x, ty = gridDim.y, n = tx * ty * gridDim.z;

@@ -6,19 +6,21 @@
 // bfloat16, gradients of activations FP32, weights bfloat16 W[cout][9 cin]
 // (tap-major: k = (3 ky + kx) cin + c) with an FP32 master copy.
 //
-//   conv3x3_kernel   3x3 zero-padded convolution as an implicit GEMM on the
-//                    matrix cores: v_mfma_f32_16x16x32_bf16, FP32 accumulate.
-//                    Block = 4 waves, each a 32-pixel x 32-channel tile
-//                    (2 x 2 MFMA tiles); operands are gathered straight from
-//                    HBM/L2 as 16-byte vectors (8 channels of one tap).
-//                    Bias + ReLU fused; stores bf16, or FP32 for the
+//   conv3x3_halo_kernel  3x3 zero-padded convolution as an implicit GEMM on the
+//                    matrix cores: v_mfma_f32_16x16x32_bf16, FP32 accumulate;
+//                    a tile's pixel halo and weights staged in LDS for all nine
+//                    taps.  Bias + ReLU fused; stores bf16, or FP32 for the
 //                    input-gradient pass (which runs the same kernel on the
 //                    output gradient with the flipped, transposed weights).
-//   wgrad_kernel     dW[co][k] = sum_m dY[m][co] X[m + tap(k)][c(k)]: the
-//                    pixel sum is the GEMM's K; tiles of dY and X are staged
-//                    in LDS and read transposed; each block reduces a
-//                    contiguous pixel range into an FP32 partial, and a
-//                    second kernel sums the partials in a fixed order.
+//                    conv3x3_lds_kernel and conv3x3_kernel (operands gathered
+//                    per K step, from LDS or straight from L2) take the channel
+//                    counts it does not.
+//   wgrad_halo_kernel  dW[co][k] = sum_m dY[m][co] X[m + tap(k)][c(k)]: the
+//                    pixel sum is the GEMM's K; a tile of dY and its halo of X
+//                    are staged in LDS and read transposed; each block reduces a
+//                    range of tiles into an FP32 partial, and a second kernel
+//                    adds the partials in a fixed order.  wgrad_kernel gathers X
+//                    per tap for other channel counts.
 //   small kernels    input padding, 2x2 average pool, nearest upsample +
 //                    concatenation and their adjoints, the 1x1 output head,
 //                    MSE gradient, ReLU-mask + bf16 conversion, weight
