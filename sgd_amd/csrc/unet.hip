@@ -294,8 +294,9 @@ __global__ __launch_bounds__(256) void conv3x3_lds_kernel(ConvArgs a) {
 }
 
 // How a block of conv3x3_halo_kernel proceeds: one item, a run of items whose
-// weights stay in LDS (one chunk, one block of output channels), any run.
-enum HaloRun { kOneItem, kWeightsStay, kAnyRun };
+// weights stay in LDS (one chunk, one block of output channels), a run of tiles
+// whose halos stay for all blocks of output channels (one chunk), any run.
+enum HaloRun { kOneItem, kWeightsStay, kHaloStays, kAnyRun };
 
 // v, with 0 where the activation is not positive
 __device__ __forceinline__ bf16x8 relu_masked(const bf16* v, const bf16* act) {
@@ -359,6 +360,7 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
   // tile * nblk + block of output channels; the blocks of an XCD (every 8th)
   // take neighbouring items
   int item = RUN != kOneItem && G % 8 == 0 ? blockIdx.x % 8 * (G / 8) + blockIdx.x / 8 : blockIdx.x;
+  if (RUN == kHaloStays) item *= nblk;
 
   bf16x8 rh[HC], rw[WC];
   auto load_halo = [&](int it, int cc) {
@@ -409,24 +411,27 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
   if (RUN == kWeightsStay) store_weights();
   for (int next; item < nitem; item = next) {
     next = RUN == kOneItem ? nitem : item + G;
+    if (RUN == kHaloStays) next = item + 1 + (item % nblk + 1 < nblk ? 0 : (G - 1) * nblk);
+    const bool new_halo = RUN != kHaloStays || item % nblk == 0;
     const int nb = item % nblk * BN;
     float bv[TN];
     if (RUN != kOneItem)
 #pragma unroll
       for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[nb + wn * CW + 16 * j + r16] : 0.0f;
-    for (int cc = 0; cc < (RUN == kWeightsStay ? 1 : nchunk); ++cc) {
+    for (int cc = 0; cc < (RUN == kWeightsStay || RUN == kHaloStays ? 1 : nchunk); ++cc) {
       __syncthreads();  // the previous chunk's reads come first
+      if (new_halo)
 #pragma unroll
-      for (int i = 0; i < HC; ++i) {
-        const int q = tid + 256 * i, p = q / GP, cg = (q % GP) * 8;
-        if (q < NG) *reinterpret_cast<bf16x8*>(&halo[p * PS + cg]) = rh[i];
-      }
+        for (int i = 0; i < HC; ++i) {
+          const int q = tid + 256 * i, p = q / GP, cg = (q % GP) * 8;
+          if (q < NG) *reinterpret_cast<bf16x8*>(&halo[p * PS + cg]) = rh[i];
+        }
       if (RUN != kWeightsStay) store_weights();
       __syncthreads();
-      const bool last = RUN == kWeightsStay || cc + 1 == nchunk;
+      const bool last = RUN == kWeightsStay || RUN == kHaloStays || cc + 1 == nchunk;
       if (!last || (RUN != kOneItem && next < nitem)) {
         const int it = RUN != kOneItem && last ? next : item, c = last ? 0 : cc + 1;
-        load_halo(it, c);
+        if (RUN != kHaloStays || it % nblk == 0) load_halo(it, c);
         if (RUN != kWeightsStay) load_weights(it, c);
       }
 #pragma unroll 1
@@ -1315,16 +1320,20 @@ static bool halo_conv(int cin, int cout) { return (cin % 32 == 0 || cin == 16 ||
 static int halo_block(int cout) { return cout % 64 == 0 ? 64 : cout % 32 == 0 ? 32 : 16; }
 
 // Blocks walk runs of items, two per CU (three with registers and LDS for it
-// were slower: 73 -> 89 us for 32 -> 32 channels at 8 x 512 x 512).  32- and 16-
-// channel blocks do so only where their weights stay; with the registers for
+// were slower: 73 -> 89 us for 32 -> 32 channels at 8 x 512 x 512).  With one
+// chunk and several blocks of output channels a run is of tiles, each halo
+// loaded once for all of them (32 -> 96 channels, split: 260 us for an item per
+// block, 181), where that leaves a tile for every block.  Otherwise 32- and 16-
+// channel blocks walk runs only where their weights stay; with the registers for
 // reloading them an item per block, three per CU, is faster (96 -> 32 channels:
 // 178 us against 186 in runs).
 template <int TH, int BN, int WM, int WN, int CC, HaloRun RUN>
 static hipError_t run_halo(const ConvArgs& a, hipStream_t s) {
   const long long nitem = (long long)((a.W + 15) / 16) * ((a.H + TH - 1) / TH) * a.B * (a.cout / BN);
   if (nitem >= 1LL << 30) return hipErrorInvalidValue;
-  const long long blocks = RUN == kOneItem ? nitem : 512;
-  conv3x3_halo_kernel<TH, BN, WM, WN, CC, RUN><<<(unsigned)(nitem < blocks ? nitem : blocks), 256, 0, s>>>(a);
+  const long long units = RUN == kHaloStays ? nitem / (a.cout / BN) : nitem;
+  const long long blocks = RUN == kOneItem || units < 512 ? units : 512;
+  conv3x3_halo_kernel<TH, BN, WM, WN, CC, RUN><<<(unsigned)blocks, 256, 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -1332,7 +1341,11 @@ template <int CC>
 static hipError_t run_halo_cc(const ConvArgs& a, hipStream_t s) {
   const int bn = halo_block(a.cout);
   const bool stay = a.cin == CC && a.cout == bn;
-  if (bn == 64) return run_halo<8, 64, 2, 2, CC, kAnyRun>(a, s);
+  const long long tiles = (long long)((a.W + 15) / 16) * ((a.H + (bn == 64 ? 7 : 15)) / (bn == 64 ? 8 : 16)) * a.B;
+  const bool halo_stays = a.cin == CC && a.cout > bn && tiles >= 512;
+  if (bn == 64) return halo_stays ? run_halo<8, 64, 2, 2, CC, kHaloStays>(a, s) : run_halo<8, 64, 2, 2, CC, kAnyRun>(a, s);
+  if (bn == 32 && halo_stays) return run_halo<16, 32, 4, 1, CC, kHaloStays>(a, s);
+  if (bn == 16 && halo_stays) return run_halo<16, 16, 4, 1, CC, kHaloStays>(a, s);
   if (bn == 32) return stay ? run_halo<16, 32, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 32, 4, 1, CC, kOneItem>(a, s);
   return stay ? run_halo<16, 16, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 16, 4, 1, CC, kOneItem>(a, s);
 }
@@ -1349,8 +1362,8 @@ bool nn_upback_fused(int cin, int cout, int c0) { return halo_conv(cin, cout) &&
 // over 2 x 2 blocks and masked, in the convolution's epilogue: the FP32
 // gradient of the concatenation, written and read again, is 1.6 GB at 8 x 512 x
 // 512 x (64 + 32), and the two passes that split it took 614 us over the three
-// levels; the step's 32-channel-block convolutions, the largest of these among
-// them, take no longer for it (910 -> 882 us together).
+// levels; the convolution itself is no slower for it (the largest 231 -> 181 us
+// with the halo kept for its three blocks of output channels).
 hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
                              int H, int W, int cin, int cout, int c0, hipStream_t s) {
   if (!nn_upback_fused(cin, cout, c0)) return hipErrorInvalidValue;

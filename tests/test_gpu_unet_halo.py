@@ -1,7 +1,8 @@
 """The halo-tiled 3x3 convolution's block shapes and runs of tiles (unet.hip)
 against torch's FP64 conv2d on the CPU: 64-, 32- and 16-channel blocks, 8, 16
 and 32 channels per chunk, one and several chunks; images of one tile, of cut
-tiles, and of more tiles than blocks (runs of 2 and more, the last one short).
+tiles, and of more tiles than blocks (runs of 2 and more, the last one short;
+halos kept for all blocks of output channels).
 FP32 output <= 1e-5 relative L2 (only the order of the FP32 sums differs), bf16
 output with bias, ReLU and mask within one bf16 rounding (2^-8 relative, 1e-6
 absolute)."""
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("B,H,W,cin,cout", [
     (1, 1, 1, 16, 16), (2, 33, 18, 8, 16), (1, 17, 40, 16, 32), (1, 9, 20, 16, 64), (2, 20, 20, 64, 16),
-    (4, 208, 336, 8, 32), (3, 330, 200, 32, 16), (2, 210, 330, 32, 64), (1, 160, 170, 64, 192)])
+    (4, 208, 336, 8, 32), (3, 330, 200, 32, 16), (2, 210, 330, 32, 64), (1, 160, 170, 64, 192),
+    (2, 210, 330, 32, 96), (4, 208, 336, 8, 128), (2, 210, 330, 16, 48), (3, 200, 200, 32, 128)])
 def test_halo_blocks(cuda, B, H, W, cin, cout):
     import torch
     from sgd_amd import _lib as m

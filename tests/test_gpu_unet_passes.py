@@ -84,7 +84,7 @@ def test_head_gradient(cuda, M, C):
 # workspace: channels off the kernel's multiples, c0 inside a block
 @pytest.mark.parametrize("B,H,W,cin,cout,c0", [(2, 18, 30, 32, 96, 64), (1, 34, 18, 64, 192, 128), (1, 2, 2, 8, 96, 32),
                                                (2, 16, 16, 32, 48, 32), (2, 14, 24, 16, 48, 32), (1, 10, 20, 32, 192, 96),
-                                               (1, 6, 10, 32, 40, 24), (1, 12, 8, 48, 96, 64)])
+                                               (4, 130, 260, 32, 96, 64), (1, 6, 10, 32, 40, 24), (1, 12, 8, 48, 96, 64)])
 def test_concatenation_gradient(cuda, B, H, W, cin, cout, c0):
     import torch
     L, m = _lib()
