@@ -293,10 +293,10 @@ __global__ __launch_bounds__(256) void conv3x3_lds_kernel(ConvArgs a) {
   }
 }
 
-// How a block of conv3x3_halo_kernel proceeds: one item, a run of items whose
-// weights stay in LDS (one chunk, one block of output channels), a run of tiles
-// whose halos stay for all blocks of output channels (one chunk), any run.
-enum HaloRun { kOneItem, kWeightsStay, kHaloStays, kAnyRun };
+// A block's run in conv3x3_halo_kernel: of items whose weights stay in LDS (one
+// chunk, one block of output channels), of tiles whose halos stay for all blocks
+// of output channels (one chunk), any.
+enum HaloRun { kWeightsStay, kHaloStays, kAnyRun };
 
 // v, with 0 where the activation is not positive
 __device__ __forceinline__ bf16x8 relu_masked(const bf16* v, const bf16* act) {
@@ -325,13 +325,15 @@ __device__ __forceinline__ bf16x8 relu_masked(const bf16* v, const bf16* act) {
 // during the MFMAs, and the weights of a single chunk stay in LDS; each wave
 // finishes its own rows through LDS of its own without a block barrier.  With
 // an item per block the first chunk's load and the epilogue were not
-// overlapped, as much as two chunks' work.  8 x 512 x 512, 32 -> 32 channels:
-// 93 -> 73 us (268 MB), 8 -> 32: 56 -> 47 us; 8 x 256 x 256, 64 -> 64: 86 -> 69
-// us (560 TF/s); 8 x 64 x 64, 256 -> 256: 62 -> 59 us.  Bound by memory at 32
+// overlapped, as much as two chunks' work.  The K steps are unrolled, so that a
+// step's fragments are read during the one before (one step at a time: the
+// second figure).  8 x 512 x 512, 32 -> 32 channels: 93 -> 73 -> 65 us (268 MB),
+// 96 -> 32: 167 -> 178 -> 163 us; 8 x 256 x 256, 64 -> 64: 86 -> 69 -> 61 us (630
+// TF/s); 8 x 64 x 64, 256 -> 256: 62 -> 59 -> 50 us.  Bound by memory at 32
 // channels, by the loads' latency and the barriers of a chunk beyond.
 // ---------------------------------------------------------------------------
 template <int TH, int BN, int WM, int WN, int CC, HaloRun RUN>
-__global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_kernel(ConvArgs a) {
+__global__ __launch_bounds__(256, 2) void conv3x3_halo_kernel(ConvArgs a) {
   static_assert(WM * WN == 4 && TH % (2 * WM) == 0, "four waves, whole pairs of tile rows per wave");
   constexpr int TW = 16, HH = TH + 2, HWD = TW + 2;
   constexpr int PS = CC == 32 ? 40 : CC;          // LDS pixel stride (bf16)
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
   const int nitem = tiles_x * tiles_y * a.B * nblk, G = (int)gridDim.x;
   // tile * nblk + block of output channels; the blocks of an XCD (every 8th)
   // take neighbouring items
-  int item = RUN != kOneItem && G % 8 == 0 ? blockIdx.x % 8 * (G / 8) + blockIdx.x / 8 : blockIdx.x;
+  int item = G % 8 == 0 ? blockIdx.x % 8 * (G / 8) + blockIdx.x / 8 : blockIdx.x;
   if (RUN == kHaloStays) item *= nblk;
 
   bf16x8 rh[HC], rw[WC];
@@ -410,14 +412,13 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
   };
   if (RUN == kWeightsStay) store_weights();
   for (int next; item < nitem; item = next) {
-    next = RUN == kOneItem ? nitem : item + G;
+    next = item + G;
     if (RUN == kHaloStays) next = item + 1 + (item % nblk + 1 < nblk ? 0 : (G - 1) * nblk);
     const bool new_halo = RUN != kHaloStays || item % nblk == 0;
     const int nb = item % nblk * BN;
     float bv[TN];
-    if (RUN != kOneItem)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[nb + wn * CW + 16 * j + r16] : 0.0f;
+    for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[nb + wn * CW + 16 * j + r16] : 0.0f;
     for (int cc = 0; cc < (RUN == kWeightsStay || RUN == kHaloStays ? 1 : nchunk); ++cc) {
       __syncthreads();  // the previous chunk's reads come first
       if (new_halo)
@@ -429,12 +430,12 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
       if (RUN != kWeightsStay) store_weights();
       __syncthreads();
       const bool last = RUN == kWeightsStay || RUN == kHaloStays || cc + 1 == nchunk;
-      if (!last || (RUN != kOneItem && next < nitem)) {
-        const int it = RUN != kOneItem && last ? next : item, c = last ? 0 : cc + 1;
+      if (!last || next < nitem) {
+        const int it = last ? next : item, c = last ? 0 : cc + 1;
         if (RUN != kHaloStays || it % nblk == 0) load_halo(it, c);
         if (RUN != kWeightsStay) load_weights(it, c);
       }
-#pragma unroll 1
+#pragma unroll NKS
       for (int ks = 0; ks < NKS; ++ks) {
         // this lane's tap in K step ks and its halo offsets (0..2)
         const int tg = ks * TPS + (8 * g) / CC;
@@ -457,9 +458,6 @@ __global__ __launch_bounds__(256, RUN == kOneItem ? 3 : 2) void conv3x3_halo_ker
     // D layout: lane holds pixels 4 g + r of tile row wm TM + i, channel r16
     const int tile = item / nblk, tx = tile % tiles_x, rest = tile / tiles_x, ty = rest % tiles_y, b = rest / tiles_y;
     const int x0 = tx * TW, y0 = ty * TH + wm * TM, co = nb + wn * CW;
-    if (RUN == kOneItem)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bv[j] = a.bias ? a.bias[co + 16 * j + r16] : 0.0f;
     if (a.low_out && nb < a.low_c) {
       // 2 x 2 sums (low_c is a multiple of BN; tiles start at even pixels)
       const int H2 = a.H >> 1, W2 = a.W >> 1;
@@ -1322,17 +1320,14 @@ static int halo_block(int cout) { return cout % 64 == 0 ? 64 : cout % 32 == 0 ? 
 // Blocks walk runs of items, two per CU (three with registers and LDS for it
 // were slower: 73 -> 89 us for 32 -> 32 channels at 8 x 512 x 512).  With one
 // chunk and several blocks of output channels a run is of tiles, each halo
-// loaded once for all of them (32 -> 96 channels, split: 260 us for an item per
-// block, 181), where that leaves a tile for every block.  Otherwise 32- and 16-
-// channel blocks walk runs only where their weights stay; with the registers for
-// reloading them an item per block, three per CU, is faster (96 -> 32 channels:
-// 178 us against 186 in runs).
+// loaded once for all of them (32 -> 96 channels, split: 260 us where every item
+// loads its own, 181), where that leaves a tile for every block.
 template <int TH, int BN, int WM, int WN, int CC, HaloRun RUN>
 static hipError_t run_halo(const ConvArgs& a, hipStream_t s) {
   const long long nitem = (long long)((a.W + 15) / 16) * ((a.H + TH - 1) / TH) * a.B * (a.cout / BN);
   if (nitem >= 1LL << 30) return hipErrorInvalidValue;
   const long long units = RUN == kHaloStays ? nitem / (a.cout / BN) : nitem;
-  const long long blocks = RUN == kOneItem || units < 512 ? units : 512;
+  const long long blocks = units < 512 ? units : 512;
   conv3x3_halo_kernel<TH, BN, WM, WN, CC, RUN><<<(unsigned)blocks, 256, 0, s>>>(a);
   return hipGetLastError();
 }
@@ -1340,14 +1335,16 @@ static hipError_t run_halo(const ConvArgs& a, hipStream_t s) {
 template <int CC>
 static hipError_t run_halo_cc(const ConvArgs& a, hipStream_t s) {
   const int bn = halo_block(a.cout);
-  const bool stay = a.cin == CC && a.cout == bn;
   const long long tiles = (long long)((a.W + 15) / 16) * ((a.H + (bn == 64 ? 7 : 15)) / (bn == 64 ? 8 : 16)) * a.B;
-  const bool halo_stays = a.cin == CC && a.cout > bn && tiles >= 512;
-  if (bn == 64) return halo_stays ? run_halo<8, 64, 2, 2, CC, kHaloStays>(a, s) : run_halo<8, 64, 2, 2, CC, kAnyRun>(a, s);
-  if (bn == 32 && halo_stays) return run_halo<16, 32, 4, 1, CC, kHaloStays>(a, s);
-  if (bn == 16 && halo_stays) return run_halo<16, 16, 4, 1, CC, kHaloStays>(a, s);
-  if (bn == 32) return stay ? run_halo<16, 32, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 32, 4, 1, CC, kOneItem>(a, s);
-  return stay ? run_halo<16, 16, 4, 1, CC, kWeightsStay>(a, s) : run_halo<16, 16, 4, 1, CC, kOneItem>(a, s);
+  const bool weights = a.cin == CC && a.cout == bn, halos = a.cin == CC && a.cout > bn && tiles >= 512;
+  if (bn == 64) return halos ? run_halo<8, 64, 2, 2, CC, kHaloStays>(a, s) : run_halo<8, 64, 2, 2, CC, kAnyRun>(a, s);
+  if (bn == 32)
+    return weights ? run_halo<16, 32, 4, 1, CC, kWeightsStay>(a, s)
+           : halos ? run_halo<16, 32, 4, 1, CC, kHaloStays>(a, s)
+                   : run_halo<16, 32, 4, 1, CC, kAnyRun>(a, s);
+  return weights ? run_halo<16, 16, 4, 1, CC, kWeightsStay>(a, s)
+         : halos ? run_halo<16, 16, 4, 1, CC, kHaloStays>(a, s)
+                 : run_halo<16, 16, 4, 1, CC, kAnyRun>(a, s);
 }
 
 static hipError_t launch_halo(const ConvArgs& a, hipStream_t s) {
