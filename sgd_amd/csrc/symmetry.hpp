@@ -48,44 +48,103 @@ inline int window_bound(const Proj2DArgs& g, const ViewGeo* views, double cx, do
   return w;
 }
 
-// Views per symmetry op: perm[v] is the view op maps v onto, empty if some
-// view has no partner.  Source, first edge ray (`edges`) and detector step have
-// to agree within tol (the FP64 rounding of the angles); every view is the
-// partner of exactly one.
-inline std::vector<int> view_permutation(const std::vector<ViewGeo>& views, int nu, int op, double tol, bool edges) {
-  const int np = (int)views.size();
-  std::vector<std::pair<double, int>> by_angle(np);
-  for (int v = 0; v < np; ++v) by_angle[v] = {std::atan2(views[v].py, views[v].px), v};
-  std::sort(by_angle.begin(), by_angle.end());
-  std::vector<char> used(np, 0);
-  std::vector<int> perm(np, -1);
-  const double kPi = 3.14159265358979323846;
-  for (int v = 0; v < np; ++v) {
-    const ViewGeo& a = views[v];
+// The op that applies a after b.
+inline int compose(int a, int b) {
+  double x, y;
+  SymOp::point(b, 1.0, 2.0, &x, &y);
+  SymOp::point(a, x, y, &x, &y);
+  const int swap = std::fabs(x) == 2.0 ? SymOp::kSwap : 0;
+  return swap | (x < 0.0 ? SymOp::kFlipX : 0) | (y < 0.0 ? SymOp::kFlipY : 0);
+}
+
+// The views of a scan by where they are: a scan of several turns holds views
+// that coincide up to the rounding of their angles.  Places are found by their
+// first view; source, first edge ray (`edges`) and detector step have to agree
+// within tol (the FP64 rounding of the angles).
+struct ViewPlaces {
+  static constexpr double kAngle = 1e-9;
+  const std::vector<ViewGeo>& views;
+  int nu;
+  double tol;
+  bool edges;
+  std::vector<std::vector<int>> at;              // views of a place, ascending
+  std::vector<std::pair<double, int>> by_angle;  // (source angle, place), sorted
+
+  ViewPlaces(const std::vector<ViewGeo>& views_, int nu_, double tol_, bool edges_)
+      : views(views_), nu(nu_), tol(tol_), edges(edges_) {
+    const int np = (int)views.size();
+    std::vector<std::pair<double, int>> all(np);
+    for (int v = 0; v < np; ++v) all[v] = {std::atan2(views[v].py, views[v].px), v};
+    std::sort(all.begin(), all.end());
+    for (const auto& a : all) {
+      // places are added by ascending angle, so by_angle is sorted throughout
+      const int k = find(0, views[a.second]);
+      if (k >= 0) {
+        at[k].push_back(a.second);
+      } else {
+        by_angle.push_back({a.first, (int)at.size()});
+        at.push_back({a.second});
+      }
+    }
+    for (auto& p : at) std::sort(p.begin(), p.end());
+  }
+
+  // The place that op maps view a onto, -1 if there is none.
+  int find(int op, const ViewGeo& a) const {
     const bool rev = SymOp::reverses(op);
+    const double kPi = 3.14159265358979323846;
     double p[2], e[2], d[2];
     SymOp::point(op, a.px, a.py, &p[0], &p[1]);
     SymOp::point(op, a.e0x + (rev ? nu * a.pux : 0.0), a.e0y + (rev ? nu * a.puy : 0.0), &e[0], &e[1]);
     SymOp::point(op, a.pux, a.puy, &d[0], &d[1]);
     if (rev) d[0] = -d[0], d[1] = -d[1];
-    const double th = std::atan2(p[1], p[0]), eps = 1e-9;
-    for (int turn = -1; turn <= 1 && perm[v] < 0; ++turn) {
+    const double th = std::atan2(p[1], p[0]);
+    for (int turn = -1; turn <= 1; ++turn) {
       const double t = th + 2 * kPi * turn;
-      auto it = std::lower_bound(by_angle.begin(), by_angle.end(), std::make_pair(t - eps, -1));
-      for (; it != by_angle.end() && it->first <= t + eps && perm[v] < 0; ++it) {
-        const ViewGeo& b = views[it->second];
+      auto it = std::lower_bound(by_angle.begin(), by_angle.end(), std::make_pair(t - kAngle, -1));
+      for (; it != by_angle.end() && it->first <= t + kAngle; ++it) {
+        const ViewGeo& b = views[at[it->second][0]];
         double err = std::max({std::fabs(b.px - p[0]), std::fabs(b.py - p[1]), nu * std::fabs(b.pux - d[0]),
                                nu * std::fabs(b.puy - d[1])});
         if (edges) err = std::max({err, std::fabs(b.e0x - e[0]), std::fabs(b.e0y - e[1])});
-        if (!used[it->second] && err <= tol) {
-          used[it->second] = 1;
-          perm[v] = it->second;
-        }
+        if (err <= tol) return it->second;
       }
     }
-    if (perm[v] < 0) return {};
+    return -1;
   }
-  return perm;
+
+  // perm[v] is the view op maps v onto, the k-th view of a place onto the k-th
+  // of its image, so that the permutations of several ops compose as the ops
+  // do; empty if a place has no image with as many views.
+  std::vector<int> permutation(int op) const {
+    std::vector<int> perm(views.size(), -1);
+    for (const auto& from : at) {
+      const int k = find(op, views[from[0]]);
+      if (k < 0 || at[k].size() != from.size()) return {};
+      for (size_t i = 0; i < from.size(); ++i) perm[from[i]] = at[k][i];
+    }
+    return perm;
+  }
+};
+
+// Whether perm[] acts on the views as the ops `found` do on the grid: closed
+// under composition, every op a permutation, and perm[a after b] = perm[a]
+// after perm[b].  The orbits that the tables are made of are then classes.
+inline bool acts_as_group(const std::vector<int>& found, const std::vector<int>* perm) {
+  for (int a : found) {
+    std::vector<char> hit(perm[a].size(), 0);
+    for (int w : perm[a]) {
+      if (w < 0 || w >= (int)hit.size() || hit[w]) return false;
+      hit[w] = 1;
+    }
+    for (int b : found) {
+      const int ab = compose(a, b);
+      if (std::find(found.begin(), found.end(), ab) == found.end()) return false;
+      for (size_t v = 0; v < hit.size(); ++v)
+        if (perm[a][perm[b][v]] != perm[ab][v]) return false;
+    }
+  }
+  return true;
 }
 
 // The symmetries of a scan of nx x ny pixels, at most `most` of them: the
@@ -98,11 +157,13 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
                                  double tol, bool hex = false, bool edges = true, int edge = kTile) {
   SymTables t;
   const int np = (int)views.size();
+  if (most <= 1) return t;
+  const ViewPlaces places(views, nu, tol, edges);
   std::vector<int> perm[kMaxSym];
   std::vector<int> found{0};
-  for (int op = 1; op < kMaxSym && most > 1; ++op) {
+  for (int op = 1; op < kMaxSym; ++op) {
     if (!((allowed >> op) & 1)) continue;
-    perm[op] = view_permutation(views, nu, op, tol, edges);
+    perm[op] = places.permutation(op);
     if (!perm[op].empty()) found.push_back(op);
   }
   if ((int)found.size() > most) {
@@ -114,9 +175,10 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
   if ((int)found.size() > most) found.resize(most >= 2 ? 2 : 1);
   const int nh = (int)found.size();
   if (nh != 2 && nh != 4 && nh != 8) return t;
-  t.op = found;
   perm[0].resize(np);
   for (int v = 0; v < np; ++v) perm[0][v] = v;
+  if (!acts_as_group(found, perm)) return t;
+  t.op = found;
   t.view.resize((size_t)np * nh);
   for (int v = 0; v < np; ++v)
     for (int h = 0; h < nh; ++h) t.view[(size_t)v * nh + h] = perm[found[h]][v];
