@@ -537,18 +537,12 @@ int setup_cone(sgdct_projector* h) {
   const SymTables t = find_symmetries(views, h->nx, h->ny, h->nu, allowed, kMaxSym, 4e-12 * (h->lsd + h->lso), false,
                                       false, 1);
   const int nh = t.nh();
-  if (nh == 1) return SGDCT_OK;
+  std::vector<int> peer;
+  if (nh == 1 || !class_peers(t, &peer)) return SGDCT_OK;
   const size_t ns = t.rep_view.size(), nd = t.tile.size();
   std::vector<int> all(ns + ns * nh + nd + (nd + 3) / 4, 0);
-  for (size_t s = 0; s < ns; ++s) {
-    all[s] = t.rep_view[s];
-    const size_t cls = s / nh * nh;
-    for (int k = 0; k < nh && t.rep_view[s] >= 0; ++k) {
-      const int w = t.view[(size_t)t.rep_view[s] * nh + k];
-      for (int q = 0; q < nh; ++q)
-        if (t.rep_view[cls + q] == w) all[ns + s * nh + k] = q;
-    }
-  }
+  std::copy(t.rep_view.begin(), t.rep_view.end(), all.begin());
+  std::copy(peer.begin(), peer.end(), all.begin() + ns);
   std::copy(t.tile.begin(), t.tile.end(), all.begin() + ns + ns * nh);
   std::memcpy(all.data() + ns + ns * nh + nd, t.owner.data(), t.owner.size());
   e = hipMalloc(&h->d_cone, all.size() * sizeof(int));

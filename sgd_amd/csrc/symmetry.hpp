@@ -228,4 +228,23 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
   return t;
 }
 
+// For every view in its class's slot s (rep_view order, -1 where a class repeats
+// a view) and every symmetry k, the slot of view k v counted from the class's
+// first: peer[s * nh + k] (0 in a repeated slot, which nothing reads).  False if
+// some class does not hold the views its members map onto.
+inline bool class_peers(const SymTables& t, std::vector<int>* peer) {
+  const int nh = t.nh(), ns = (int)t.rep_view.size();
+  peer->assign((size_t)ns * nh, 0);
+  for (int s = 0; s < ns; ++s) {
+    if (t.rep_view[s] < 0) continue;
+    const auto cls = t.rep_view.begin() + s / nh * nh;
+    for (int k = 0; k < nh; ++k) {
+      const auto q = std::find(cls, cls + nh, t.view[(size_t)t.rep_view[s] * nh + k]);
+      if (q == cls + nh) return false;
+      (*peer)[(size_t)s * nh + k] = (int)(q - cls);
+    }
+  }
+  return true;
+}
+
 }  // namespace sgdct
