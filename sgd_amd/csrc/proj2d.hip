@@ -148,11 +148,11 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const double* __restrict
 
 // Bin window that holds every tile's window over all views (host-side, on the
 // host copy of the view table): the bound from the corner tiles, or, where
-// that is above `enough`, every tile looked at.
+// that is above `enough`, every tile looked at (kNoWindow: there is none).
 int max_tile_window(const Proj2DArgs& g, const ViewGeo* views_host, int enough) {
   const double half = 0.5 * (kTile - 1), r = half + (double)g.h;
   int w = window_bound(g, views_host, half * g.dx, half * g.dy, r * g.dx, r * g.dy);
-  if (w <= enough) return w;
+  if (w <= enough || w == kNoWindow) return w;
   w = 0;
   for (int v = 0; v < g.np; ++v)
     for (int iy0 = 0; iy0 < g.ny; iy0 += kTile)

@@ -20,8 +20,13 @@ struct SymTables {
   int nh() const { return (int)op.size(); }
 };
 
+// No window holds a tile's bins (window_bound).
+constexpr int kNoWindow = 1 << 30;
+
 // Bins that hold the projection of every pixel tile's box in every view,
-// +-1 margin.  Tile (0, 0)'s box has its centre (cx, cy) from pixel (0, 0) and
+// +-1 margin; kNoWindow where some box does not lie in front of some view's
+// source: a box that the plane beta = 0 through the source cuts projects to
+// both ends of the detector, whatever its corners do.  Tile (0, 0)'s box has its centre (cx, cy) from pixel (0, 0) and
 // half extents (hx, hy), the other tiles' lie kTile pixels apart.  A point d
 // away from a box's centre projects to kc - (d . G) / (beta + d . grad beta), G
 // = grad N_0 + kc grad beta, kc the centre's projection.  Over the image, kc is
@@ -41,8 +46,9 @@ inline int window_bound(const Proj2DArgs& g, const ViewGeo* views, double cx, do
       top = std::max(top, hx * std::fabs(vg.e0y + kc * vg.puy) + hy * std::fabs(vg.e0x + kc * vg.pux));
       room = std::min(room, -be - (hx * std::fabs(vg.puy) + hy * std::fabs(vg.pux)));
     }
+    if (!(room > 0.0)) return kNoWindow;
     // floor(kc + hw) - floor(kc - hw) <= 2 hw + 1, the window's margins 2 more
-    const double n = room > 0.0 ? std::floor(2.0 * top / room) + 4.0 : 1e9;
+    const double n = std::floor(2.0 * top / room) + 4.0;
     w = n < g.nu ? std::max(w, (int)n) : g.nu;
   }
   return w;
