@@ -198,9 +198,10 @@ int sgdct_project_dev_noalloc(sgdct_projector *h, int direction, const float *in
  * hexagonal A stays unsplit); 1..32 = fixed.  The workspace (partial sums,
  * interleaved images of A; more images per launch while it stays within 64
  * MiB, larger batches take several launches) is allocated at creation and by
- * this call, never inside a projection on the handle's stream (a hexagonal
- * handle's A takes one interleaved lattice for each stream it is called on, up
- * to four, and runs without one on others and under capture).  Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
+ * this call, never inside a projection.  An unsplit hexagonal A's interleaved
+ * images are the handle's too: its calls may overlap, the device orders their
+ * uses of them across streams, and a call under capture runs without them.
+ * Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
 int sgdct_split_config(sgdct_projector *h, int fwd_split, int bwd_split);
 
 /* Shape query: out[0..3] = nx, ny, np, nu (hexagonal: nc, nl, np, nu);

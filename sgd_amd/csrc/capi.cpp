@@ -177,14 +177,17 @@ struct sgdct_projector {
   // (0: too wide, records are read from global memory)
   SymPlan sym{};
   int* d_sym = nullptr;
-  struct Lattice {
-    hipStream_t stream;
-    bool taken;
-    double* p;
-  };
-  std::vector<Lattice> lattices;
-  std::mutex lattice_mu;
   int win = 0;
+  // Interleaved images of an unsplit A, which shares no other memory, so that a
+  // handle's calls on different streams may overlap: one buffer, made with the
+  // handle, whose uses are ordered by copies_ev, recorded after each.  (A buffer
+  // per stream would have to be known by the stream's handle, which several
+  // threads share for hipStreamPerThread and a new stream may take over.)
+  double* d_copies = nullptr;
+  size_t copies_cap = 0;
+  hipEvent_t copies_ev = nullptr;
+  bool copies_used = false;
+  std::mutex copies_mu;
   // B0 / B1 / SF: A splits each bin's walk into line segments and A^T the views
   // into groups; fwd_auto / bwd_auto are chosen at creation from one image's
   // launch size, fwd_split / bwd_split (0 = automatic) override them.  The
@@ -237,7 +240,8 @@ struct sgdct_projector {
     if (d_views) (void)hipFree(d_views);
     if (d_bins) (void)hipFree(d_bins);
     if (d_sym) (void)hipFree(d_sym);
-    for (auto& l : lattices) (void)hipFree(l.p);
+    if (d_copies) (void)hipFree(d_copies);
+    if (copies_ev) (void)hipEventDestroy(copies_ev);
     if (d_img) (void)hipFree(d_img);
     if (d_sino) (void)hipFree(d_sino);
     if (d_host_part) (void)hipFree(d_host_part);
@@ -301,7 +305,7 @@ size_t record_bytes(int basis);
 // A^T's staged bins: a record (none for SF) and g values each.
 size_t bwd_lds_bytes(int basis, int win, int g) { return (size_t)win * (record_bytes(basis) + 4 * g); }
 size_t work_doubles(const sgdct_projector* h);
-double* new_lattice(sgdct_projector* h);
+int ensure_copies(sgdct_projector* h);
 SymPlan plain_plan(const sgdct_projector* h);
 int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
 int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
@@ -463,7 +467,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     // lattice rows only, before steep waves walked the vertical lines)
     h->fwd_auto = is_hex(basis) ? 1 : kAutoMaxSplit;
     h->bwd_auto = auto_bwd_split(h);
-    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || (is_hex(basis) && !new_lattice(h))) {
+    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || (is_hex(basis) && ensure_copies(h) != SGDCT_OK)) {
       delete h;
       return nullptr;
     }
@@ -788,36 +792,19 @@ size_t work_doubles(const sgdct_projector* h) {
   return std::max(fwd, bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0);
 }
 
-// Interleaved lattices of the hexagonal A, whose unsplit launches share no
-// other memory: one buffer per stream that calls it, so that a handle's calls
-// on different streams may overlap.  The first is made with the handle and
-// taken by the first stream; a stream past kLattices, and one under capture
-// (whose graph may be launched anywhere), gets none and runs without groups.
-constexpr size_t kLattices = 4;
-
-double* new_lattice(sgdct_projector* h) {
-  double* p = nullptr;
-  const hipError_t e = hipMalloc(&p, fwd_work_doubles(h, 1) * sizeof(double));
-  if (e != hipSuccess) {
-    hip_fail(e, "interleaved lattice");
-    return nullptr;
+// Room for an unsplit A's interleaved images.
+int ensure_copies(sgdct_projector* h) {
+  const size_t need = fwd_work_doubles(h, 1);
+  hipError_t e = hipSuccess;
+  if (!h->copies_ev) e = hipEventCreateWithFlags(&h->copies_ev, hipEventDisableTiming);
+  if (e == hipSuccess && need > h->copies_cap) {
+    if (h->d_copies) (void)hipFree(h->d_copies);
+    h->d_copies = nullptr;
+    h->copies_cap = 0;
+    e = hipMalloc(&h->d_copies, need * sizeof(double));
+    if (e == hipSuccess) h->copies_cap = need;
   }
-  h->lattices.push_back({nullptr, false, p});
-  return p;
-}
-
-// Called with h->lattice_mu held, which the caller keeps until its kernels are
-// enqueued.
-double* lattice_of(sgdct_projector* h, hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
-  else if (st != hipStreamCaptureStatusNone) return nullptr;
-  for (auto& l : h->lattices)
-    if (l.taken && l.stream == s) return l.p;
-  if (h->lattices.back().taken && (h->lattices.size() >= kLattices || !new_lattice(h))) return nullptr;
-  h->lattices.back().taken = true;
-  h->lattices.back().stream = s;
-  return h->lattices.back().p;
+  return e == hipSuccess ? SGDCT_OK : hip_fail(e, "interleaved images");
 }
 
 // Room for `doubles` partial sums.
@@ -946,13 +933,26 @@ int group_backward(sgdct_projector* h, const float* sino, float* img, int batch,
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "backward launch");
 }
 
+// A without partial sums.  The lock is held until the kernels and the event
+// are enqueued.  A stream under capture, whose graph may be launched anywhere,
+// reads the images in place.
+int unsplit_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+  else if (st != hipStreamCaptureStatusNone) return group_forward(h, img, sino, batch, 1, nullptr, 0, s);
+  std::lock_guard<std::mutex> lock(h->copies_mu);
+  hipError_t e = h->copies_used ? hipStreamWaitEvent(s, h->copies_ev, 0) : hipSuccess;
+  if (e != hipSuccess) return hip_fail(e, "order of the interleaved images");
+  const int rc = group_forward(h, img, sino, batch, 1, h->d_copies, h->copies_cap, s);
+  h->copies_used = true;
+  e = hipEventRecord(h->copies_ev, s);
+  if (rc != SGDCT_OK) return rc;
+  return e == hipSuccess ? SGDCT_OK : hip_fail(e, "order of the interleaved images");
+}
+
 int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s) {
   if (is_cone(h->basis)) return cone_forward(h, img, sino, batch, s);
-  if (is_hex(h->basis) && fwd_segments(h) == 1) {
-    std::lock_guard<std::mutex> lock(h->lattice_mu);
-    double* const buf = lattice_of(h, s);
-    return group_forward(h, img, sino, batch, 1, buf, buf ? fwd_work_doubles(h, 1) : 0, s);
-  }
+  if (is_hex(h->basis) && fwd_segments(h) == 1) return unsplit_forward(h, img, sino, batch, s);
   return group_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, s);
 }
 
