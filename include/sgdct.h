@@ -194,13 +194,14 @@ int sgdct_project_dev_noalloc(sgdct_projector *h, int direction, const float *in
  * `bwd_split` groups.  Grid segments and groups write FP64 partial sums that a
  * second kernel adds in a fixed order (results are deterministic, independent
  * of the batch size, and agree across splits to FP64 rounding).  0 =
- * automatic: chosen at creation from one image's launch size (24 segments;
- * hexagonal A stays unsplit); 1..32 = fixed.  The workspace (partial sums,
+ * automatic: chosen at creation from one image's launch size (24 segments, or
+ * none from 200000 pairs of a view and 64 bins on; hexagonal A stays unsplit);
+ * 1..32 = fixed.  The workspace (partial sums,
  * interleaved images of A; more images per launch while it stays within 64
  * MiB, larger batches take several launches) is allocated at creation and by
- * this call, never inside a projection.  An unsplit hexagonal A's interleaved
- * images are the handle's too: its calls may overlap, the device orders their
- * uses of them across streams, and a call under capture runs without them.
+ * this call, never inside a projection.  An unsplit A's interleaved images are
+ * the handle's too: its calls may overlap, the device orders their uses of them
+ * across streams, and a call under capture runs without them.
  * Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
 int sgdct_split_config(sgdct_projector *h, int fwd_split, int bwd_split);
 

@@ -309,6 +309,7 @@ int ensure_copies(sgdct_projector* h);
 SymPlan plain_plan(const sgdct_projector* h);
 int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
 int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
+int auto_fwd_split(const sgdct_projector* h);
 int auto_bwd_split(const sgdct_projector* h);
 int ensure_part(sgdct_projector* h, size_t doubles);
 void release_part(sgdct_projector* h);
@@ -461,13 +462,9 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     if (bwd_lds_bytes(basis, w, h->sym.nh) <= kLdsBytes) h->win = w;
   }
   if (splits(basis)) {
-    // hexagonal A runs unsplit unless asked: at 296 x 256 points, 1024 views
-    // and 1024 bins, 2..16 row segments took one image from 1.11 to 1.20..1.40
-    // ms (H0) and a batch of 64 from 59 to 64..84 ms (measured when A walked
-    // lattice rows only, before steep waves walked the vertical lines)
-    h->fwd_auto = is_hex(basis) ? 1 : kAutoMaxSplit;
+    h->fwd_auto = auto_fwd_split(h);
     h->bwd_auto = auto_bwd_split(h);
-    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || (is_hex(basis) && ensure_copies(h) != SGDCT_OK)) {
+    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || ensure_copies(h) != SGDCT_OK) {
       delete h;
       return nullptr;
     }
@@ -663,7 +660,21 @@ constexpr int kBwdMaxViews = 8;
 constexpr int kMaxSplit = 32;      // sgdct_split_config accepts 1..kMaxSplit
 
 
+// A splits unless one image has 200000 (view, 64 bins) pairs or more, a
+// workgroup of eight waves each.  Launches left whole share no partial sums and
+// may overlap on one handle (unsplit_forward).
+// Hexagonal A runs unsplit unless asked: at 296 x 256 points, 1024 views and
+// 1024 bins, 2..16 row segments took one image from 1.11 to 1.20..1.40 ms (H0)
+// and a batch of 64 from 59 to 64..84 ms (measured when A walked lattice rows
+// only, before steep waves walked the vertical lines)
+constexpr long long kFwdWaveTarget = 200000;
+
+int auto_fwd_split(const sgdct_projector* h) {
+  return is_hex(h->basis) || (long long)h->np * h->args.nchunk >= kFwdWaveTarget ? 1 : kAutoMaxSplit;
+}
+
 int auto_bwd_split(const sgdct_projector* h) {
+  if (h->np < 32) return 1;  // left whole: few views give small groups only
   const long long tiles = h->win ? h->sym.ntile : plain_plan(h).ntile;
   // groups of >= 16 views while they add blocks up to kBwdBlockTarget; a
   // small image, which leaves the GPU idle, takes groups of >= 4 views up
@@ -786,14 +797,26 @@ size_t fwd_work_doubles(const sgdct_projector* h, int nseg) {
   return need * std::max<size_t>(1, std::min<size_t>(16, kGroupBytes / sizeof(double) / need));
 }
 
+size_t bwd_work_doubles(const sgdct_projector* h) {
+  const int bs = bwd_groups(h);
+  return bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0;
+}
+
+// What the handle's split launches need (an unsplit A's images are d_copies).
 size_t work_doubles(const sgdct_projector* h) {
-  const int nseg = grid_segments(h, fwd_segments(h)), bs = bwd_groups(h);
-  const size_t fwd = is_hex(h->basis) && nseg == 1 ? 0 : fwd_work_doubles(h, nseg);
-  return std::max(fwd, bs > 1 ? part_images(h) * (size_t)bs * h->nx * h->ny : 0);
+  const int fs = fwd_segments(h);
+  return std::max(fs == 1 ? 0 : fwd_work_doubles(h, grid_segments(h, fs)), bwd_work_doubles(h));
+}
+
+// What both of its launches need in one workspace.
+size_t slice_doubles(const sgdct_projector* h) {
+  return std::max(fwd_work_doubles(h, grid_segments(h, fwd_segments(h))), bwd_work_doubles(h));
 }
 
 // Room for an unsplit A's interleaved images.
 int ensure_copies(sgdct_projector* h) {
+  if (fwd_segments(h) > 1) return SGDCT_OK;
+  std::lock_guard<std::mutex> lock(h->copies_mu);
   const size_t need = fwd_work_doubles(h, 1);
   hipError_t e = hipSuccess;
   if (!h->copies_ev) e = hipEventCreateWithFlags(&h->copies_ev, hipEventDisableTiming);
@@ -820,9 +843,11 @@ int ensure_part(sgdct_projector* h, size_t doubles) {
 }
 
 void release_part(sgdct_projector* h) {
-  if (h->d_part) (void)hipFree(h->d_part);
-  h->d_part = nullptr;
-  h->part_cap = 0;
+  for (double** b : {&h->d_part, &h->d_copies}) {
+    if (*b) (void)hipFree(*b);
+    *b = nullptr;
+  }
+  h->part_cap = h->copies_cap = 0;
   h->fwd_auto = h->bwd_auto = 1;
 }
 
@@ -952,7 +977,7 @@ int unsplit_forward(sgdct_projector* h, const float* img, float* sino, int batch
 
 int run_forward(sgdct_projector* h, const float* img, float* sino, int batch, hipStream_t s) {
   if (is_cone(h->basis)) return cone_forward(h, img, sino, batch, s);
-  if (is_hex(h->basis) && fwd_segments(h) == 1) return unsplit_forward(h, img, sino, batch, s);
+  if (fwd_segments(h) == 1) return unsplit_forward(h, img, sino, batch, s);
   return group_forward(h, img, sino, batch, fwd_segments(h), h->d_part, h->part_cap, s);
 }
 
@@ -1258,7 +1283,7 @@ int batch_upload_plan(sgdct_batch* b) {
 // Workspace that the slices' launches need one after the other.
 int batch_workspace(sgdct_batch* b) {
   size_t need = 0;
-  for (const sgdct_projector* h : b->proj) need = std::max(need, work_doubles(h));
+  for (const sgdct_projector* h : b->proj) need = std::max(need, slice_doubles(h));
   if (need == 0) return SGDCT_OK;
   const hipError_t e = hipMalloc(&b->d_part, need * sizeof(double));
   if (e != hipSuccess) return hip_fail(e, "batch workspace");
@@ -1291,7 +1316,7 @@ int batch_run(sgdct_batch* b, int dir, const float* in, float* out, hipStream_t 
       sgdct_projector* h = b->proj[i];
       // the batch's workspace, so that the slices' handles stay free for other
       // callers; a split raised since the batch was made has its room there
-      const bool own = work_doubles(h) <= b->part_cap;
+      const bool own = slice_doubles(h) <= b->part_cap;
       double* const part = own ? b->d_part : h->d_part;
       const size_t cap = own ? b->part_cap : h->part_cap;
       const int rc = dir == 0 ? group_forward(h, in + b->img_off[i], out + b->sino_off[i], 1, fwd_segments(h), part, cap, s)
@@ -1674,7 +1699,9 @@ int sgdct_split_config(sgdct_projector* h, int fwd_split, int bwd_split) {
   const int fs = h->fwd_split, bs = h->bwd_split;
   h->fwd_split = fwd_split;
   h->bwd_split = bwd_split;
-  if (int rc = ensure_part(h, work_doubles(h))) {
+  int rc = ensure_part(h, work_doubles(h));
+  if (!rc) rc = ensure_copies(h);
+  if (rc) {
     h->fwd_split = fs;
     h->bwd_split = bs;
     return rc;

@@ -14,9 +14,22 @@ PER_THREAD = 2  # hipStreamPerThread: one handle value, a stream for each thread
 
 def handles():
     from sgd_amd.torch_ops import Projector
+
+    def fan(basis, nx, ny, views, nu, split):
+        P = Projector(basis, nx, ny, 2 * np.pi * np.arange(views) / views, nu, 1.7, 1.7, 2.9, 1000.0, 500.0)
+        P.set_split(split, split)
+        return P
+
     ang = 2 * np.pi * np.arange(1024) / 1024
     return {"Hl": lambda: Projector.hexagonal("Hl", 80, 64, ang, 256, 1.0, 1.2, 1000.0, 500.0),
-            "H0": lambda: Projector.hexagonal("H0", 41, 60, ang, 200, 1.0, 1.2, 1000.0, 500.0)}
+            "H0": lambda: Projector.hexagonal("H0", 41, 60, ang, 200, 1.0, 1.2, 1000.0, 500.0),
+            "B0, split 1": lambda: fan("B0", 110, 97, 300, 150, 1),
+            "B1, split 1": lambda: fan("B1", 128, 128, 1024, 130, 1),
+            "SF, split 1": lambda: fan("SF", 60, 97, 1024, 130, 1),
+            "B1, automatic": lambda: fan("B1", 20, 16, 3200, 4100, 0)}
+
+
+NAMES = ["Hl", "H0", "B0, split 1", "B1, split 1", "SF, split 1", "B1, automatic"]
 
 
 def images(P, cuda, n):
@@ -28,7 +41,7 @@ def images(P, cuda, n):
     return xs, ref
 
 
-@pytest.mark.parametrize("name", ["Hl", "H0"])
+@pytest.mark.parametrize("name", NAMES)
 def test_unsplit_forward_on_six_streams(cuda, name):
     import torch
     P = handles()[name]()
@@ -44,7 +57,7 @@ def test_unsplit_forward_on_six_streams(cuda, name):
         assert torch.equal(a, b), float((a - b).abs().max())
 
 
-@pytest.mark.parametrize("name", ["Hl", "H0"])
+@pytest.mark.parametrize("name", NAMES)
 def test_unsplit_forward_on_per_thread_streams(cuda, name):
     import torch
     from sgd_amd import _lib
