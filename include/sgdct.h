@@ -171,15 +171,16 @@ int sgdct_backward_dev(sgdct_projector *h, const float *sino, float *img, int ba
  * hipMalloc).  sgdct_forward_dev (direction 0: in = images, out = sinograms)
  * or sgdct_backward_dev (direction 1: in = sinograms, out = images) on a
  * fan-beam handle (B0, B1, SF, H0, Hl), with the FP64 partial sums of split
- * launches in a static device array of 32 MiB per GPU (allocated when the
- * library's code is loaded on that GPU, held until the process ends) instead
- * of the handle's workspace.  The call allocates nothing; its first call on a
+ * launches and A's interleaved images in a static device array of 32 MiB per
+ * GPU (allocated when the library's code is loaded on that GPU, held until the
+ * process ends) instead of the handle's workspace; where the interleaved images
+ * of all the scan's symmetries do not fit, A takes several launches of fewer.  The call allocates nothing; its first call on a
  * GPU looks up the array's address there.  The handle's device must be
  * current.  A split chosen automatically is lowered, when one image's partial
  * sums do not fit in 32 MiB, to the largest that fits (results agree with
  * sgdct_*_dev to FP64 rounding of the partial sums; bit for bit at the same
- * split); a split fixed by sgdct_split_config that does not fit is
- * SGDCT_EINVAL.  Cone-beam handles are SGDCT_EUNSUP.  Every call on a GPU
+ * split); a split fixed by sgdct_split_config is SGDCT_EINVAL where 32 MiB hold
+ * less than one image's sums for every segment or group.  Cone-beam handles are SGDCT_EUNSUP.  Every call on a GPU
  * shares that GPU's array (each launch writes every partial sum it reads, so
  * nothing needs clearing): calls that overlap on one GPU, from several
  * streams or threads, race. */
@@ -201,7 +202,8 @@ int sgdct_project_dev_noalloc(sgdct_projector *h, int direction, const float *in
  * MiB, larger batches take several launches) is allocated at creation and by
  * this call, never inside a projection.  An unsplit A's interleaved images are
  * the handle's too: its calls may overlap, the device orders their uses of them
- * across streams, and a call under capture runs without them.
+ * across streams, and a call under capture reads the images in place (the same
+ * values, at one value per footprint).
  * Returns SGDCT_OK, SGDCT_EINVAL or SGDCT_ENOMEM. */
 int sgdct_split_config(sgdct_projector *h, int fwd_split, int bwd_split);
 

@@ -689,7 +689,7 @@ int auto_bwd_split(const sgdct_projector* h) {
 // The identity only.
 SymPlan plain_plan(const sgdct_projector* h) {
   SymPlan p{};
-  p.nh = 1;
+  p.nh = p.row = 1;
   p.nrep = h->np;
   p.ntile = ((h->nx + kTile - 1) / kTile) * ((h->ny + kTile - 1) / kTile);
   return p;
@@ -738,7 +738,7 @@ int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views) {
   if (e == hipSuccess) e = hipMemcpy(h->d_sym, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_fail(e, "symmetry tables");
   SymPlan& p = h->sym;
-  p.nh = t.nh();
+  p.nh = p.row = t.nh();
   p.lg = p.nh == 8 ? 3 : (p.nh == 4 ? 2 : 1);
   for (int k = 0; k < p.nh; ++k) p.op[k] = t.op[k];
   p.nrep = (int)nr;
@@ -884,33 +884,44 @@ hipError_t launch_bwd2d(const sgdct_projector* h, const GroupRun& r, const float
   return launch_backward(h->basis, h->args, r, sino, img, s);
 }
 
-// A: images in groups of m, as many groups per launch as the
-// workspace buf[0, cap) holds.  Every image's values are formed the same way
-// whatever the batch.  A workspace too small for one group of one image
-// runs without symmetries, reading the image in place (partial sums, which a
-// fixed split needs, must fit).
+// The nh symmetries from h0 on.
+SymPlan part_of(const SymPlan& sym, int h0, int nh) {
+  SymPlan p = sym;
+  p.nh = nh;
+  p.lg = nh == 8 ? 3 : (nh == 4 ? 2 : (nh == 2 ? 1 : 0));
+  p.h0 = h0;
+  for (int k = 0; k < nh; ++k) p.op[k] = sym.op[h0 + k];
+  return p;
+}
+
+// A: images in groups of m, as many groups per launch as the workspace
+// buf[0, cap) holds.  Where it is too small for one image at all symmetries, the
+// launches take half of them, a quarter, or one with the image read in place (a
+// fixed split's partial sums must fit).  Every value is formed from the
+// representatives' footprints in the same order whatever the batch and the
+// workspace.
 int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, int nseg, double* buf, size_t cap,
                   hipStream_t s) {
   const size_t ni = (size_t)h->nx * h->ny, ns = (size_t)h->np * h->nu;
   nseg = grid_segments(h, nseg);
   if (nseg > 1 && (!buf || cap < nseg * ns)) return fail(SGDCT_EDEVICE, "partial-sum workspace missing");
-  GroupRun r;
-  r.sym = h->sym;
-  r.split = nseg;
-  r.m = std::max(1, std::min(batch, max_group(h) / r.sym.nh));
+  if (!buf) cap = 0;
+  int nh = h->sym.nh, m = std::max(1, std::min(batch, max_group(h) / nh));
   // a small launch takes fewer images per group and more workgroups
-  while (r.m > 1 && (long long)r.sym.nrep * h->args.nchunk * ((batch + r.m - 1) / r.m) < kSymBlocks) r.m >>= 1;
-  while (r.m > 1 && fwd_group_doubles(h, r.sym.nh, nseg, r.m) > cap) --r.m;
-  const size_t per = fwd_group_doubles(h, r.sym.nh, nseg, r.m);
-  const bool interleave = buf && per <= cap && (r.sym.nh * r.m > 1 || (!is_hex(h->basis) && std::max(h->nx, h->ny) > kDirectEdge));
-  if (!interleave) r.sym = plain_plan(h), r.m = 1;
-  r.g = group_size(r.sym.nh, r.m);
+  while (m > 1 && (long long)h->sym.nrep * h->args.nchunk * ((batch + m - 1) / m) < kSymBlocks) m >>= 1;
+  while (nh * m > 1 && fwd_group_doubles(h, nh, nseg, m) > cap) m > 1 ? --m : nh >>= 1;
+  const size_t per = fwd_group_doubles(h, nh, nseg, m);
+  const bool interleave =
+      per <= cap && (nh * m > 1 || (h->sym.nh == 1 && !is_hex(h->basis) && std::max(h->nx, h->ny) > kDirectEdge));
+  GroupRun r;
+  r.split = nseg;
   const size_t groups = interleave ? cap / per : (nseg > 1 ? cap / (nseg * ns) : (size_t)batch);
-  const int step = (int)std::min<size_t>(batch, groups * r.m);
+  const int step = (int)std::min<size_t>(batch, groups * m);
   hipError_t e = hipSuccess;
   for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += step) {
     r.batch = std::min(step, batch - b0);
-    if (r.batch < r.m) r.m = r.batch, r.g = group_size(r.sym.nh, r.m);
+    r.m = std::min(m, r.batch);
+    r.g = group_size(nh, r.m);
     double* at = buf;
     if (nseg > 1) {
       r.part = at;
@@ -922,7 +933,12 @@ int group_forward(sgdct_projector* h, const float* img, float* sino, int batch, 
       r.rows = r.g > 1 ? reinterpret_cast<float*>(at) : nullptr;
       r.cols = is_hex(h->basis) ? nullptr : reinterpret_cast<float*>(at) + n;
     }
-    e = launch_fwd2d(h, r, img + b0 * ni, sino + b0 * ns, s);
+    for (int h0 = 0; h0 < h->sym.nh && e == hipSuccess; h0 += nh) {
+      r.sym = part_of(h->sym, h0, nh);
+      if (!interleave) r.sym.place = r.sym.op[0];
+      r.sum = h0 + nh == h->sym.nh;
+      e = launch_fwd2d(h, r, img + b0 * ni, sino + b0 * ns, s);
+    }
   }
   return e == hipSuccess ? SGDCT_OK : hip_fail(e, "forward launch");
 }
@@ -1734,7 +1750,9 @@ int sgdct_project_dev_noalloc(sgdct_projector* h, int direction, const float* in
   if (int rc = scratch_on(dev, &part)) return rc;
   // The handle's split, lowered (when it was chosen automatically) to the
   // largest whose partial sums of one image fit in the scratch array; a split
-  // fixed by sgdct_split_config that does not fit is an error.
+  // fixed by sgdct_split_config is an error unless a sum per segment fits (A's
+  // waves take most of them without, so this asks for more than the launch
+  // needs: what is refused does not follow the launch shape).
   int n = direction == 0 ? fwd_segments(h) : bwd_groups(h);
   const bool fixed = direction == 0 ? h->fwd_split != 0 : h->bwd_split != 0;
   const size_t unit = direction == 0 ? (size_t)h->np * h->nu : (size_t)h->nx * h->ny;
@@ -1744,7 +1762,9 @@ int sgdct_project_dev_noalloc(sgdct_projector* h, int direction, const float* in
                                     std::to_string((size_t)n * unit * sizeof(double)) +
                                     " bytes of partial sums, more than the " + std::to_string(kScratchBytes) +
                                     "-byte scratch array (lower it with sgdct_split_config)");
-    n = (int)std::max<size_t>(1, kScratchDoubles / unit);
+    if (direction == 1) n = (int)std::max<size_t>(1, kScratchDoubles / unit);
+    else
+      while (n > 1 && grid_segments(h, n) > 1 && grid_segments(h, n) * unit > kScratchDoubles) --n;
   }
   hipStream_t s = (hipStream_t)stream;
   return direction == 0 ? group_forward(h, in, out, batch, n, part, kScratchDoubles, s)

@@ -44,6 +44,15 @@ struct SymOp {
     *ox = x;
     *oy = y;
   }
+  // pixel offset (iy nx + ix) of op (ix, iy): base + ix step_x + iy step_y
+  struct Steps {
+    int base, x, y;
+  };
+  __host__ __device__ static __forceinline__ Steps steps(int op, int nx, int ny) {
+    const int sx = (op & kFlipX) ? -1 : 1, sy = (op & kFlipY) ? -nx : nx;
+    return {((op & kFlipX) ? nx - 1 : 0) + ((op & kFlipY) ? (ny - 1) * nx : 0), (op & kSwap) ? sy : sx,
+            (op & kSwap) ? sx : sy};
+  }
   // point (ic, il) of a hexagonal lattice (odd rows hold nx - 1 points, half a
   // column on; their slot nx - 1 is no point and maps to such a slot).  A
   // vertical mirror keeps a row's parity only when ny is odd.
@@ -60,14 +69,18 @@ struct SymOp {
 };
 
 // The symmetries a launch uses (device pointers; nh = 1 has the identity
-// only and may leave every table null).
+// only and may leave every table null).  A launch of A may take some of the
+// plan's symmetries only, nh of `row` from h0 on, where there is no room for
+// the copies of all: a value's footprints and sums are the same in any launch.
 struct SymPlan {
   int nh;                      // symmetries used (1, 2, 4 or 8)
   int lg;                      // log2(nh)
-  int op[kMaxSym];             // op[0] = 0
+  int op[kMaxSym];             // op[0] = 0 where h0 = 0
+  int h0, row;                 // A: first symmetry of the launch, symmetries of the plan
+  int place;                   // A, one value per footprint: the symmetry at which the image is read in place
   int nrep;                    // A: representative views
   const int* rep;              // [nrep]
-  const int* rep_view;         // [nrep][nh] view h rep, -1 where an earlier h gives the same view
+  const int* rep_view;         // [nrep][row] view h rep, -1 where an earlier h gives the same view
   const int* view;             // [np][nh] view h v (A^T)
   int ntile;                   // A^T: tiles of the fundamental domain
   const int* tile;             // [ntile] tile_y << 16 | tile_x
@@ -82,6 +95,7 @@ struct GroupRun {
   int split = 1;          // A: grid segments, A^T: view groups
   bool lone = false;      // A (g = 1): `split` line segments per bin, added within a workgroup
   double* part = nullptr; // FP64 partial sums (split > 1)
+  bool sum = true;        // A: add the partial sums (false: a later launch writes more of them)
   float* rows = nullptr;  // A: interleaved images (null: g = 1, read in place)
   float* cols = nullptr;  // A: their transposes (null: column walks read strided)
   int vpg = 0;            // A^T: views per group

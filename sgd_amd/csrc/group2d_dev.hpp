@@ -100,7 +100,7 @@ __device__ __forceinline__ void fwd_group_store(const Proj2DArgs& g, const SymPl
   const size_t nsino = (size_t)g.np * g.nu;
   for (int s = wv; s < sp.nh * nimg; s += W) {
     const int k = s >> sp.lg, h = s & (sp.nh - 1);
-    const int vh = sp.rep_view ? sp.rep_view[rep * sp.nh + h] : v;
+    const int vh = sp.rep_view ? sp.rep_view[rep * sp.row + sp.h0 + h] : v;
     if (vh < 0) continue;
     double t = 0.0;
 #pragma unroll

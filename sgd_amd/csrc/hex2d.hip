@@ -123,7 +123,8 @@ __device__ __forceinline__ void load_point(const float* p, float (&x)[G]) {
 // line's points the w-th of wn equal ranges of columns (row walk) or rows
 // (vertical walk), of the lines segment seg of nseg.  Adds sum conv * x into
 // acc[G] (FP32 along a line, FP64 across lines; without dx dy).  img holds G
-// values per point.  Lanes past the last bin add nothing.
+// values per point; at G = 1, point p's value is img's at `place` p.  Lanes past
+// the last bin add nothing.
 // The strips lie along the lines, so splitting the points keeps every lane of
 // every wave busy, where splitting the lines would leave a lane only the few
 // it crosses; and a wave's lanes stay within one narrow range of columns or
@@ -132,8 +133,10 @@ __device__ __forceinline__ void load_point(const float* p, float (&x)[G]) {
 // that).
 template <int HB, int G, bool FAR>
 __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chunk, const float* __restrict__ img, int w,
-                                              int wn, int seg, int nseg, double (&acc)[G]) {
+                                              int wn, int seg, int nseg, double (&acc)[G],
+                                              int place = 0) {
   using T = HexTraits<HB>;
+  const bool flip_x = G == 1 && (place & SymOp::kFlipX), flip_y = G == 1 && (place & SymOp::kFlipY);
   const Proj2DArgs& g = ha.g;
   const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
   const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
@@ -237,7 +240,7 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
     const double kas = ka * sa, kam = ka * ma, kac = ka * ca, kbs = kb * sb, kbm = kb * mb, kbc = kb * cb;
     const float dta = (float)kas, dtb = (float)kbs;
     const float fc_lo = (float)c_lo, fc_hi = (float)c_hi, fc_odd = (float)min(c_hi, g.nx - 2);
-    const Off step = 4 * G;
+    const Off step = flip_x ? -(Off)(4 * G) : (Off)(4 * G);
     for (int il = il_lo; il <= il_hi; ++il) {
       const bool odd = il & 1;  // points half a column to the right
       const float sh = odd ? 0.5f : 0.0f, fl = (float)il;
@@ -246,7 +249,8 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
       if (!(flo <= fhi)) continue;
       const int n0 = (int)flo;
       const double dn = (double)(flo + sh), dl = (double)il;
-      walk(4 * G * ((Off)il * g.nx + n0), (int)fhi - n0 + 1, step,
+      const int qx = flip_x ? g.nx - (il & 1) - 1 - n0 : n0, qy = flip_y ? g.ny - 1 - il : il;
+      walk(4 * G * ((Off)qy * g.nx + qx), (int)fhi - n0 + 1, step,
            (float)__builtin_fma(kas, dn, __builtin_fma(kam, dl, kac)),
            (float)__builtin_fma(kbs, dn, __builtin_fma(kbm, dl, kbc)), dta, dtb);
     }
@@ -275,7 +279,7 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
     const double kam = ka * ma, kas = 0.5 * ka * sa, kac = ka * ca, kbm = kb * mb, kbs = 0.5 * kb * sb, kbc = kb * cb;
     const float dta = (float)(2.0 * kam), dtb = (float)(2.0 * kbm);
     const float fr_lo = (float)r_lo, fr_hi = (float)r_hi;
-    const Off step = 8 * G * (Off)g.nx;
+    const Off step = flip_y ? -(8 * G * (Off)g.nx) : 8 * G * (Off)g.nx;
     for (int k = k_lo; k <= k_hi; ++k) {  // ic' = k / 2
       const float fk = (float)k;
       const float flo = fmaxf(ceilf(__builtin_fmaf(fk, lo1, lo0)), fr_lo);
@@ -286,7 +290,8 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
       i1 -= (i1 ^ k) & 1;
       if (i0 > i1) continue;
       const double dk = (double)k, di = (double)i0;
-      walk(4 * G * ((Off)i0 * g.nx + (k >> 1)), ((i1 - i0) >> 1) + 1, step,
+      const int qx = flip_x ? g.nx - (k & 1) - 1 - (k >> 1) : k >> 1, qy = flip_y ? g.ny - 1 - i0 : i0;
+      walk(4 * G * ((Off)qy * g.nx + qx), ((i1 - i0) >> 1) + 1, step,
            (float)__builtin_fma(kam, di, __builtin_fma(kas, dk, kac)),
            (float)__builtin_fma(kbm, di, __builtin_fma(kbs, dk, kbc)), dta, dtb);
     }
@@ -316,7 +321,8 @@ __global__ __launch_bounds__(64 * W) void hex_fwd_kernel(HexArgs ha, SymPlan sp,
   double acc[G];
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
-  hex_fwd_lines<HB, G, FAR>(ha, v, chunk, img + (size_t)blockIdx.y * G * g.nx * g.ny, wv, W, blockIdx.z, gridDim.z, acc);
+  hex_fwd_lines<HB, G, FAR>(ha, v, chunk, img + (size_t)blockIdx.y * G * g.nx * g.ny, wv, W, blockIdx.z, gridDim.z, acc,
+                            sp.place);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
@@ -725,7 +731,7 @@ hipError_t launch_hex_forward(int basis, const Proj2DArgs& g, double dt, const G
   const HexArgs ha{g, dt};
   const hipError_t e = basis == BASIS_H0 ? hex_forward_b<BASIS_H0>(ha, r, img, sino, s)
                                          : hex_forward_b<BASIS_HL>(ha, r, img, sino, s);
-  if (e == hipSuccess && r.split > 1)
+  if (e == hipSuccess && r.split > 1 && r.sum)
     return launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
   return e;
 }

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(64 * W) void fwd_group_kernel(Proj2DArgs g, SymPlan
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
   fwd_bin_lines<BASIS, G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr,
-                          wv, W, blockIdx.z, gridDim.z, acc);
+                          wv, W, blockIdx.z, gridDim.z, acc, sp.place);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
@@ -306,7 +306,7 @@ hipError_t launch_forward(int basis, const Proj2DArgs& g, const GroupRun& r, con
   if (basis == BASIS_B1) e = forward_b<BASIS_B1>(g, r, img, sino, s);
   else if (basis == BASIS_B0) e = forward_b<BASIS_B0>(g, r, img, sino, s);
   else return hipErrorInvalidValue;
-  if (e == hipSuccess && r.split > 1 && !r.lone)
+  if (e == hipSuccess && r.split > 1 && r.sum && !r.lone)
     e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
   return e;
 }

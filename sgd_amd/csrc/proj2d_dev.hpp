@@ -48,12 +48,12 @@ template <> struct Traits<BASIS_B0> {
 // sum_pixel conv * x into acc[G] (FP32 along a line, FP64 across lines;
 // without the factors dx dy and scale(bin)).  rows_img holds G values per
 // pixel, [iy][ix][G]; cols_img the same transposed, [ix][iy][G], which the
-// column walks read (null: they read rows_img strided).  Lanes past the last
-// bin add nothing.
+// column walks read (null: they read rows_img strided).  At G = 1, pixel p's
+// value is rows_img's at `place` p.  Lanes past the last bin add nothing.
 template <int BASIS, int G>
 __device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int chunk, const float* __restrict__ rows_img,
                                               const float* __restrict__ cols_img, int w0, int wn, int seg, int nseg,
-                                              double (&acc)[G]) {
+                                              double (&acc)[G], int place = 0) {
   using T = Traits<BASIS>;
   const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
   const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
@@ -89,7 +89,13 @@ __device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int ch
   const double sr = rows ? rcx : rcy, mr = rows ? rcy : rcx;
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
   const bool strided = !rows && !cols_img;
-  const int smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
+  int base = 0, smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
+  if (G == 1 && place) {
+    const SymOp::Steps st = SymOp::steps(place, g.nx, g.ny);
+    base = st.base;
+    smin = rows ? st.x : st.y;
+    smaj = rows ? st.y : st.x;
+  }
   const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
   const float dta = (float)(rec.ka * sa), dtb = (float)(rec.kb * sb);
 
@@ -124,7 +130,7 @@ __device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int ch
   const float* const img = (rows || strided) ? rows_img : cols_img;
   const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
-  const unsigned bstep = 4u * G * (unsigned)smin;
+  const unsigned bstep = 4u * G * (unsigned)smin;  // offsets modulo 2^32: steps may be negative
 
   // One line: pixels [flo, fhi] (flo <= fhi) of line m.
   auto walk_line = [&](int m, float flo, float fhi) {
@@ -132,7 +138,7 @@ __device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int ch
     const double dn = (double)flo, dm = (double)m;
     float ta = (float)__builtin_fma(dn, an, __builtin_fma(dm, am, a0));
     float tb = (float)__builtin_fma(dn, bn, __builtin_fma(dm, bm, b0));
-    unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
+    unsigned off = 4u * G * (unsigned)(base + m * smaj + n0 * smin);
     const unsigned end = off + (unsigned)((int)fhi - n0 + 1) * bstep;
     float accl[G];
 #pragma unroll

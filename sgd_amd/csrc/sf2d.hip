@@ -44,7 +44,7 @@ __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
   sf_fwd_lines<G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr, wv,
-                  W, blockIdx.z, gridDim.z, acc);
+                  W, blockIdx.z, gridDim.z, acc, sp.place);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
@@ -128,7 +128,7 @@ hipError_t launch_sf_forward(const Proj2DArgs& g, const GroupRun& r, const float
   else if (r.g == 4) e = sf_forward_g<4, kFwdWaves>(g, r, img, sino, s);
   else if (r.g == 8) e = sf_forward_g<8, kFwdWaves>(g, r, img, sino, s);
   else return hipErrorInvalidValue;
-  if (e == hipSuccess && r.split > 1) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
+  if (e == hipSuccess && r.split > 1 && r.sum) e = launch_sum_parts(r.part, sino, (size_t)r.batch * g.np * g.nu, r.split, s);
   return e;
 }
 

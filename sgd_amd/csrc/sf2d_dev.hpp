@@ -95,7 +95,7 @@ __device__ __forceinline__ float sf_weight(float dx, float wx, float wy) {
 template <int G>
 __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chunk, const float* __restrict__ rows_img,
                                              const float* __restrict__ cols_img, int w0, int wn, int seg, int nseg,
-                                             double (&acc)[G]) {
+                                             double (&acc)[G], int place = 0) {
   const bool inside = chunk * 64 + (int)(threadIdx.x & 63) < g.nu;
   const int u = inside ? chunk * 64 + (int)(threadIdx.x & 63) : g.nu - 1;
   const ViewGeo vg = g.views[v];
@@ -112,7 +112,13 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const double sb = rows ? bcx : bcy, mb = rows ? bcy : bcx;
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
   const bool strided = !rows && !cols_img;
-  const int smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
+  int base = 0, smin = strided ? g.nx : 1, smaj = strided ? 1 : nmin;
+  if (G == 1 && place) {
+    const SymOp::Steps st = SymOp::steps(place, g.nx, g.ny);
+    base = st.base;
+    smin = rows ? st.x : st.y;
+    smaj = rows ? st.y : st.x;
+  }
   // beta(ix, iy) = cross(pu, w): affine, steps (bcxx, bcyy) per index
   const double bcxx = -vg.puy * g.dx, bcyy = vg.pux * g.dy, bc00 = vg.pux * vg.w0y - vg.puy * vg.w0x;
   const double sB = rows ? bcxx : bcyy, mB = rows ? bcyy : bcxx;
@@ -186,7 +192,7 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
       float wm = (float)__builtin_fma(dn, dmov, w0mov);
       const float wf = (float)__builtin_fma(dm, dfix, w0fix);
       const float ifix = __builtin_amdgcn_rcpf(fabsf(wf)), wf2 = wf * wf;
-      unsigned off = 4u * G * (unsigned)(m * smaj + n0 * smin);
+      unsigned off = 4u * G * (unsigned)(base + m * smaj + n0 * smin);
       const unsigned end = off + (unsigned)((int)fhi - n0 + 1) * bstep;
       float accl[G];
 #pragma unroll
