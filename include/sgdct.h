@@ -198,9 +198,11 @@ int sgdct_project_dev_noalloc(sgdct_projector *h, int direction, const float *in
  * automatic: chosen at creation from one image's launch size (24 segments, or
  * none from 200000 pairs of a view and 64 bins on; hexagonal A stays unsplit);
  * 1..32 = fixed.  The workspace (partial sums,
- * interleaved images of A; more images per launch while it stays within 64
- * MiB, larger batches take several launches) is allocated at creation and by
- * this call, never inside a projection.  An unsplit A's interleaved images are
+ * interleaved images of A) is allocated at creation and by this call, never
+ * inside a projection: for one image (two copies of it for every symmetry of
+ * the scan, at most 2 GiB), and for more images per launch while that stays
+ * within 192 MiB.  Where it cannot be had, an automatic split stays whole and
+ * images are read in place.  An unsplit A's interleaved images are
  * the handle's too: its calls may overlap, the device orders their uses of them
  * across streams, and a call under capture reads the images in place (the same
  * values, at one value per footprint).

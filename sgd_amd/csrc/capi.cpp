@@ -7,6 +7,7 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <string>
@@ -305,13 +306,13 @@ size_t record_bytes(int basis);
 // A^T's staged bins: a record (none for SF) and g values each.
 size_t bwd_lds_bytes(int basis, int win, int g) { return (size_t)win * (record_bytes(basis) + 4 * g); }
 size_t work_doubles(const sgdct_projector* h);
-int ensure_copies(sgdct_projector* h);
+void ensure_copies(sgdct_projector* h);
 SymPlan plain_plan(const sgdct_projector* h);
 int fwd_segments(const sgdct_projector* h) { return h->fwd_split ? h->fwd_split : h->fwd_auto; }
 int bwd_groups(const sgdct_projector* h) { return h->bwd_split ? h->bwd_split : h->bwd_auto; }
 int auto_fwd_split(const sgdct_projector* h);
 int auto_bwd_split(const sgdct_projector* h);
-int ensure_part(sgdct_projector* h, size_t doubles);
+int ensure_part(sgdct_projector* h);
 void release_part(sgdct_projector* h);
 size_t part_need(const sgdct_projector* h);
 size_t host_part_doubles(const sgdct_projector* h);
@@ -464,10 +465,8 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
   if (splits(basis)) {
     h->fwd_auto = auto_fwd_split(h);
     h->bwd_auto = auto_bwd_split(h);
-    if (ensure_part(h, work_doubles(h)) != SGDCT_OK || ensure_copies(h) != SGDCT_OK) {
-      delete h;
-      return nullptr;
-    }
+    if (ensure_part(h) != SGDCT_OK) h->fwd_auto = h->bwd_auto = 1;  // whole launches share no memory
+    ensure_copies(h);
   }
   return h;
 }
@@ -786,15 +785,32 @@ size_t fwd_group_doubles(const sgdct_projector* h, int nh, int nseg, int m) {
 // transpose is a launch that the column walks do not earn back.
 constexpr int kDirectEdge = 96;
 
-constexpr size_t kGroupBytes = (size_t)64 << 20;  // several image groups per launch up to this much workspace
+// Workspace bounds.  A handle is made for one image's launch, fewer symmetries
+// at a time where all take more than kOneBytes (as much as the cone beam's row
+// profiles; 8 symmetries from 5793 x 5793 pixels on); for several images per
+// footprint while that stays within kGroupBytes, and several such groups per
+// launch within kMoreBytes.
+constexpr size_t kOneBytes = (size_t)2 << 30, kGroupBytes = (size_t)192 << 20, kMoreBytes = (size_t)64 << 20;
 
-// Workspace of a handle: one image group of A with as many images
-// as fit kMaxGroup values, more while it stays within kGroupBytes; the FP64
-// partial images of A^T.
+// Partial sums of one image, without which a split launch cannot run.
+size_t fwd_sums(const sgdct_projector* h, int nseg) { return nseg > 1 ? (size_t)nseg * h->np * h->nu : 0; }
+size_t bwd_sums(const sgdct_projector* h) { return bwd_groups(h) > 1 ? (size_t)bwd_groups(h) * h->nx * h->ny : 0; }
+
+// A's launch of one image (in place past kOneBytes: the sums alone).
+size_t fwd_one_doubles(const sgdct_projector* h, int nseg) {
+  for (int nh = h->sym.nh; nh > 1 || nh == h->sym.nh; nh >>= 1) {
+    const size_t n = fwd_group_doubles(h, nh, nseg, 1);
+    if (n <= kOneBytes / sizeof(double)) return n;
+  }
+  return fwd_sums(h, nseg);
+}
+
 size_t fwd_work_doubles(const sgdct_projector* h, int nseg) {
-  const int m = std::max(1, max_group(h) / h->sym.nh);
-  const size_t need = fwd_group_doubles(h, h->sym.nh, nseg, m);
-  return need * std::max<size_t>(1, std::min<size_t>(16, kGroupBytes / sizeof(double) / need));
+  int m = std::max(1, max_group(h) / h->sym.nh);
+  while (m > 1 && fwd_group_doubles(h, h->sym.nh, nseg, m) > kGroupBytes / sizeof(double)) --m;
+  const size_t need = m > 1 ? fwd_group_doubles(h, h->sym.nh, nseg, m) : fwd_one_doubles(h, nseg);
+  if (need == 0) return 0;
+  return need * std::max<size_t>(1, std::min<size_t>(16, kMoreBytes / sizeof(double) / need));
 }
 
 size_t bwd_work_doubles(const sgdct_projector* h) {
@@ -808,38 +824,53 @@ size_t work_doubles(const sgdct_projector* h) {
   return std::max(fs == 1 ? 0 : fwd_work_doubles(h, grid_segments(h, fs)), bwd_work_doubles(h));
 }
 
+// The least that its split launches run with.
+size_t least_doubles(const sgdct_projector* h) {
+  return std::max(fwd_sums(h, grid_segments(h, fwd_segments(h))), bwd_sums(h));
+}
+
 // What both of its launches need in one workspace.
 size_t slice_doubles(const sgdct_projector* h) {
   return std::max(fwd_work_doubles(h, grid_segments(h, fwd_segments(h))), bwd_work_doubles(h));
 }
 
-// Room for an unsplit A's interleaved images.
-int ensure_copies(sgdct_projector* h) {
-  if (fwd_segments(h) > 1) return SGDCT_OK;
-  std::lock_guard<std::mutex> lock(h->copies_mu);
-  const size_t need = fwd_work_doubles(h, 1);
-  hipError_t e = hipSuccess;
-  if (!h->copies_ev) e = hipEventCreateWithFlags(&h->copies_ev, hipEventDisableTiming);
-  if (e == hipSuccess && need > h->copies_cap) {
-    if (h->d_copies) (void)hipFree(h->d_copies);
-    h->d_copies = nullptr;
-    h->copies_cap = 0;
-    e = hipMalloc(&h->d_copies, need * sizeof(double));
-    if (e == hipSuccess) h->copies_cap = need;
+// Grows buf to the first of `want` (descending) that can be allocated, if it
+// is smaller; true if it then holds the last of them at least.
+bool grow(double** buf, size_t* cap, std::initializer_list<size_t> want) {
+  for (size_t n : want) {
+    if (n <= *cap) return true;
+    double* p = nullptr;
+    if (hipMalloc(&p, n * sizeof(double)) == hipSuccess) {
+      if (*buf) (void)hipFree(*buf);
+      *buf = p;
+      *cap = n;
+      return true;
+    }
+    (void)hipGetLastError();
   }
-  return e == hipSuccess ? SGDCT_OK : hip_fail(e, "interleaved images");
+  return false;
 }
 
-// Room for `doubles` partial sums.
-int ensure_part(sgdct_projector* h, size_t doubles) {
-  if (doubles <= h->part_cap) return SGDCT_OK;
-  if (h->d_part) (void)hipFree(h->d_part);
-  h->d_part = nullptr;
-  h->part_cap = 0;
-  hipError_t e = hipMalloc(&h->d_part, doubles * sizeof(double));
-  if (e != hipSuccess) return hip_fail(e, "partial-sum workspace");
-  h->part_cap = doubles;
-  return SGDCT_OK;
+// Room for an unsplit A's interleaved images; without it they are read in place.
+void ensure_copies(sgdct_projector* h) {
+  if (fwd_segments(h) > 1) return;
+  std::lock_guard<std::mutex> lock(h->copies_mu);
+  if (!h->copies_ev && hipEventCreateWithFlags(&h->copies_ev, hipEventDisableTiming) != hipSuccess) {
+    (void)hipGetLastError();
+    h->copies_ev = nullptr;
+    return;
+  }
+  (void)grow(&h->d_copies, &h->copies_cap, {fwd_work_doubles(h, 1), fwd_one_doubles(h, 1), 0});
+}
+
+// Room for the split launches: for images in groups, one image at all
+// symmetries, or its partial sums alone.
+int ensure_part(sgdct_projector* h) {
+  const int fs = fwd_segments(h);
+  const size_t least = least_doubles(h);
+  const size_t one = std::max(fs > 1 ? fwd_one_doubles(h, grid_segments(h, fs)) : 0, least);
+  if (grow(&h->d_part, &h->part_cap, {work_doubles(h), one, least})) return SGDCT_OK;
+  return fail(SGDCT_ENOMEM, "partial-sum workspace: " + std::to_string(least * sizeof(double)) + " bytes");
 }
 
 void release_part(sgdct_projector* h) {
@@ -982,6 +1013,7 @@ int unsplit_forward(sgdct_projector* h, const float* img, float* sino, int batch
   if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
   else if (st != hipStreamCaptureStatusNone) return group_forward(h, img, sino, batch, 1, nullptr, 0, s);
   std::lock_guard<std::mutex> lock(h->copies_mu);
+  if (!h->d_copies) return group_forward(h, img, sino, batch, 1, nullptr, 0, s);
   hipError_t e = h->copies_used ? hipStreamWaitEvent(s, h->copies_ev, 0) : hipSuccess;
   if (e != hipSuccess) return hip_fail(e, "order of the interleaved images");
   const int rc = group_forward(h, img, sino, batch, 1, h->d_copies, h->copies_cap, s);
@@ -1296,15 +1328,15 @@ int batch_upload_plan(sgdct_batch* b) {
   return SGDCT_OK;
 }
 
-// Workspace that the slices' launches need one after the other.
-int batch_workspace(sgdct_batch* b) {
-  size_t need = 0;
-  for (const sgdct_projector* h : b->proj) need = std::max(need, slice_doubles(h));
-  if (need == 0) return SGDCT_OK;
-  const hipError_t e = hipMalloc(&b->d_part, need * sizeof(double));
-  if (e != hipSuccess) return hip_fail(e, "batch workspace");
-  b->part_cap = need;
-  return SGDCT_OK;
+// Workspace that the slices' launches need one after the other.  Without it a
+// batch that nobody has configured takes the persistent queue, which needs none.
+void batch_workspace(sgdct_batch* b) {
+  size_t most = 0, least = 0;
+  for (const sgdct_projector* h : b->proj) {
+    most = std::max(most, slice_doubles(h));
+    least = std::max(least, least_doubles(h));
+  }
+  if (!grow(&b->d_part, &b->part_cap, {most, least})) b->fwd_bpc = b->bwd_bpc = 8;
 }
 
 // Launches of a batch that nobody has configured: one per slice, which splits
@@ -1332,7 +1364,7 @@ int batch_run(sgdct_batch* b, int dir, const float* in, float* out, hipStream_t 
       sgdct_projector* h = b->proj[i];
       // the batch's workspace, so that the slices' handles stay free for other
       // callers; a split raised since the batch was made has its room there
-      const bool own = slice_doubles(h) <= b->part_cap;
+      const bool own = least_doubles(h) <= b->part_cap;
       double* const part = own ? b->d_part : h->d_part;
       const size_t cap = own ? b->part_cap : h->part_cap;
       const int rc = dir == 0 ? group_forward(h, in + b->img_off[i], out + b->sino_off[i], 1, fwd_segments(h), part, cap, s)
@@ -1628,10 +1660,7 @@ sgdct_batch* sgdct_batch_create(sgdct_projector* const* slices, int nslice) {
   }
   b->fwd_bpc = auto_blocks(b, 0);
   b->bwd_bpc = auto_blocks(b, 1);
-  if (batch_workspace(b) != SGDCT_OK) {
-    delete b;
-    return nullptr;
-  }
+  batch_workspace(b);
   if (b->plan.nfwd >= (1LL << 32) || b->plan.nbwd >= (1LL << 32)) {
     fail(SGDCT_EUNSUP, "batch has more than 2^32 work items");
     delete b;
@@ -1715,9 +1744,9 @@ int sgdct_split_config(sgdct_projector* h, int fwd_split, int bwd_split) {
   const int fs = h->fwd_split, bs = h->bwd_split;
   h->fwd_split = fwd_split;
   h->bwd_split = bwd_split;
-  int rc = ensure_part(h, work_doubles(h));
-  if (!rc) rc = ensure_copies(h);
-  if (rc) {
+  const int rc = ensure_part(h);
+  if (!rc) ensure_copies(h);
+  else {
     h->fwd_split = fs;
     h->bwd_split = bs;
     return rc;
