@@ -456,7 +456,10 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     const int w = (is_hex(basis) ? hex_tile_window(a, dt, views.data())
                                  : max_tile_window(a, views.data(), kMaxWindow - 2)) + 2;
     h->bwd_lds = w <= kMaxWindow;
-    if (setup_symmetry(h, views) != SGDCT_OK) {
+    // next to a source footprints have no bound, and their rounding none either:
+    // every view by itself where the image reaches behind one
+    h->sym = plain_plan(h);
+    if (w < kNoWindow && setup_symmetry(h, views) != SGDCT_OK) {
       delete h;
       return nullptr;
     }
@@ -709,7 +712,6 @@ int max_group(const sgdct_projector* h) {
 constexpr long long kSymBlocks = 256;
 
 int setup_symmetry(sgdct_projector* h, const std::vector<ViewGeo>& views) {
-  h->sym = plain_plan(h);
   // B0's footprint is cut off at the corner range where it is not small, so
   // that a pixel corner that falls on a bin edge (every axis-aligned view of
   // an even image has such) belongs to either bin by rounding alone; a

@@ -57,3 +57,25 @@ def test_hex_backward_behind_the_source(cuda, oracle_exact, basis):
     m = off_planes(px, py, ang, lso, 6 * np.sqrt(3) * dt)
     m[1::2, -1] = False
     check(Projector.hexagonal(basis, *geo), cuda, HexGeometry(oracle_exact, *geo).backward(basis, y.astype(float)), m, y)
+
+
+@pytest.mark.parametrize("basis", ["B1", "SF", "H0"])
+def test_views_by_themselves_behind_the_source(cuda, basis):
+    """A of one view is bit for bit the scan's (no other view's footprints)."""
+    import torch
+    from sgd_amd.torch_ops import Projector
+    n = 250 if basis == "H0" else 1024  # hexagons: as many waves per launch as one view takes
+    ang = 2 * np.pi * np.arange(n) / n
+
+    def make(a):
+        P = (Projector.hexagonal("H0", 301, 300, a, 512, 2.2, 1.7, 1000.0, 500.0) if basis == "H0" else
+             Projector(basis, 400, 400, a, 512, 3.2, 3.2, 1.7, 1000.0, 500.0))
+        P.set_split(1, 1)
+        return P
+
+    P = make(ang)
+    x = torch.randn(P.img_shape, device=cuda, generator=torch.Generator(device=cuda).manual_seed(1))
+    y = torch.nan_to_num(P.forward(x))
+    for k in (0, 5, n // 4 - 1, n // 4, n // 2 + 3, n - 1):
+        print(basis, "view", k, flush=True)
+        assert torch.equal(torch.nan_to_num(make(ang[k:k + 1]).forward(x))[0], y[k])
