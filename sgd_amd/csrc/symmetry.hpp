@@ -164,6 +164,8 @@ inline SymTables find_symmetries(const std::vector<ViewGeo>& views, int nx, int 
   SymTables t;
   const int np = (int)views.size();
   if (most <= 1) return t;
+  for (const ViewGeo& v : views)  // angles that are no numbers have no order
+    if (!std::isfinite(v.px + v.py + v.e0x + v.e0y + v.pux + v.puy)) return t;
   const ViewPlaces places(views, nu, tol, edges);
   std::vector<int> perm[kMaxSym];
   std::vector<int> found{0};

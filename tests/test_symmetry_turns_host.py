@@ -51,3 +51,13 @@ def test_symmetry_tables_of_coincident_views(tables, name):  # noqa: F811
             ab = [k for k, c in enumerate(op) if np.allclose(apply(c, *probe), apply(a, *apply(b, *probe)))]
             assert len(ab) == 1
             assert np.array_equal(view[view[:, j], i], view[:, ab[0]]), (a, b)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_views_that_are_no_numbers_have_no_symmetries(tables, bad):  # noqa: F811
+    ang = turn(60)
+    views = np.array(scan(ang, 64))
+    views[17] = bad
+    views[40, 0] = bad
+    op, *_ = tables(32, 32, 64, views, 0xff)
+    assert list(op) == [0]
