@@ -8,8 +8,10 @@
 #include <cmath>
 #include <cstring>
 #include <initializer_list>
+#include <memory>
 #include <mutex>
 #include <new>
+#include <stdexcept>
 #include <string>
 #include <vector>
 
@@ -385,6 +387,24 @@ size_t record_bytes(int basis) {
 // fan-beam handles split both A (line or row segments) and A^T (view groups)
 bool splits(int basis) { return basis == BASIS_B0 || basis == BASIS_B1 || basis == BASIS_SF || is_hex(basis); }
 
+// f's result, or `failed` where it throws: no exception leaves a C entry point.
+template <class F, class R>
+R no_throw(F&& f, R failed) {
+  try {
+    return f();
+  } catch (const std::bad_alloc&) {
+    fail(SGDCT_ENOMEM, "host allocation failed");
+  } catch (const std::length_error&) {
+    fail(SGDCT_ENOMEM, "host allocation failed");
+  } catch (...) {
+    fail(SGDCT_EDEVICE, "unexpected exception");
+  }
+  return failed;
+}
+
+int fill(sgdct_projector* h, int basis, int nx, int ny, int np, int nu, double dx, double dy, double du, double lsd,
+         double lso, const double* angles, const double* drho, double dt, double ushift);
+
 // ushift moves the bin edges by ushift bins: 0.5 gives cells centred on
 // integer detector coordinates (layers/SF_projector.cu:209-216).
 sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, double dy, double du,
@@ -395,11 +415,15 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     fail(SGDCT_EINVAL, "invalid geometry arguments");
     return nullptr;
   }
-  auto* h = new (std::nothrow) sgdct_projector();
-  if (!h) {
-    fail(SGDCT_ENOMEM, "host allocation failed");
-    return nullptr;
-  }
+  return no_throw([&]() -> sgdct_projector* {
+    auto h = std::make_unique<sgdct_projector>();
+    return fill(h.get(), basis, nx, ny, np, nu, dx, dy, du, lsd, lso, angles, drho, dt, ushift) == SGDCT_OK ? h.release()
+                                                                                                            : nullptr;
+  }, (sgdct_projector*)nullptr);
+}
+
+int fill(sgdct_projector* h, int basis, int nx, int ny, int np, int nu, double dx, double dy, double du, double lsd,
+         double lso, const double* angles, const double* drho, double dt, double ushift) {
   h->basis = basis;
   h->nx = nx; h->ny = ny; h->np = np; h->nu = nu;
   h->dx = dx; h->dy = dy; h->du = du; h->lsd = lsd; h->lso = lso;
@@ -439,11 +463,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
   if (e == hipSuccess) e = hipMemcpy(h->d_views, views.data(), sizeof(ViewGeo) * np, hipMemcpyHostToDevice);
   if (e == hipSuccess && rec) e = hipMalloc(&h->d_bins, bins.size());
   if (e == hipSuccess && rec) e = hipMemcpy(h->d_bins, bins.data(), bins.size(), hipMemcpyHostToDevice);
-  if (e != hipSuccess) {
-    hip_fail(e, "projector init");
-    delete h;
-    return nullptr;
-  }
+  if (e != hipSuccess) return hip_fail(e, "projector init");
   Proj2DArgs& a = h->args;
   a.views = h->d_views;
   a.bins = h->d_bins;
@@ -459,10 +479,8 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     // next to a source footprints have no bound, and their rounding none either:
     // every view by itself where the image reaches behind one
     h->sym = plain_plan(h);
-    if (w < kNoWindow && setup_symmetry(h, views) != SGDCT_OK) {
-      delete h;
-      return nullptr;
-    }
+    if (w < kNoWindow)
+      if (int rc = setup_symmetry(h, views)) return rc;
     if (bwd_lds_bytes(basis, w, h->sym.nh) <= kLdsBytes) h->win = w;
   }
   if (splits(basis)) {
@@ -471,7 +489,7 @@ sgdct_projector* create(int basis, int nx, int ny, int np, int nu, double dx, do
     if (ensure_part(h) != SGDCT_OK) h->fwd_auto = h->bwd_auto = 1;  // whole launches share no memory
     ensure_copies(h);
   }
-  return h;
+  return SGDCT_OK;
 }
 
 size_t img_elems(const sgdct_projector* h) { return (size_t)h->nx * h->ny * h->nz; }
@@ -1385,8 +1403,8 @@ int batch_run(sgdct_batch* b, int dir, const float* in, float* out, hipStream_t 
 // 2 pi (np-1)/np) (utils/geo.cu:209-230), COO triplets in the reference's
 // order.  Returns the triplet count or a negative code; a buffer smaller than
 // the count is an error (the reference asserts, A_B1.cu:578-579).
-int matrix_generation(int basis, int np, int nu, int nx, int ny, double dx, double dy, double du, double lsd,
-                      double lso, double* spmat, int buffer_size, double dt = 0.0) {
+int generate_matrix(int basis, int np, int nu, int nx, int ny, double dx, double dy, double du, double lsd, double lso,
+                    double* spmat, int buffer_size, double dt) {
   const bool query = !spmat && buffer_size == 0;  // count only
   if ((!spmat && !query) || buffer_size < 0) return fail(SGDCT_EINVAL, "null or negative matrix buffer");
   if (np <= 0) return fail(SGDCT_EINVAL, "np must be positive");
@@ -1437,6 +1455,12 @@ int matrix_generation(int basis, int np, int nu, int nx, int ny, double dx, doub
   if (d_out) (void)hipFree(d_out);
   delete h;
   return rc != SGDCT_OK ? rc : (int)total;
+}
+
+int matrix_generation(int basis, int np, int nu, int nx, int ny, double dx, double dy, double du, double lsd,
+                      double lso, double* spmat, int buffer_size, double dt = 0.0) {
+  return no_throw([&] { return generate_matrix(basis, np, nu, nx, ny, dx, dy, du, lsd, lso, spmat, buffer_size, dt); },
+                  (int)SGDCT_ENOMEM);
 }
 
 }  // namespace
@@ -1547,7 +1571,7 @@ sgdct_projector* b1_3d_init(int nx, int ny, int nz, int np, int nu, int nv, doub
   h->nv = nv;
   h->dz = dz;
   h->dv = dv;
-  if (setup_cone(h) != SGDCT_OK) {
+  if (no_throw([&] { return setup_cone(h); }, (int)SGDCT_ENOMEM) != SGDCT_OK) {
     delete h;
     return nullptr;
   }
@@ -1579,7 +1603,7 @@ sgdct_projector* sf3d_init(int nx, int ny, int nz, int np, int nu, int nv, doubl
   h->nv = nv;
   h->dz = dz;
   h->dv = dv;
-  if (setup_cone(h) != SGDCT_OK) {
+  if (no_throw([&] { return setup_cone(h); }, (int)SGDCT_ENOMEM) != SGDCT_OK) {
     delete h;
     return nullptr;
   }
@@ -1602,31 +1626,16 @@ int sgdct_shape3(const sgdct_projector* h, int* out) {
 
 void sgdct_destroy(sgdct_projector* h) { delete h; }
 
-sgdct_batch* sgdct_batch_create(sgdct_projector* const* slices, int nslice) {
-  if (!slices || nslice <= 0) {
-    fail(SGDCT_EINVAL, "empty slice list");
-    return nullptr;
-  }
-  auto* b = new (std::nothrow) sgdct_batch();
-  if (!b) {
-    fail(SGDCT_ENOMEM, "host allocation failed");
-    return nullptr;
-  }
+namespace {
+int fill_batch(sgdct_batch* b, sgdct_projector* const* slices, int nslice) {
   b->n = nslice;
   b->img_off.assign(nslice + 1, 0);
   b->sino_off.assign(nslice + 1, 0);
   for (int i = 0; i < nslice; ++i) {
     const sgdct_projector* h = slices[i];
-    if (!h || (h->basis != BASIS_B0 && h->basis != BASIS_B1 && h->basis != BASIS_SF)) {
-      fail(SGDCT_EUNSUP, "batched slices must be B0, B1 or SF projectors");
-      delete b;
-      return nullptr;
-    }
-    if (i > 0 && h->device != slices[0]->device) {
-      fail(SGDCT_EINVAL, "batched slices must live on one device");
-      delete b;
-      return nullptr;
-    }
+    if (!h || (h->basis != BASIS_B0 && h->basis != BASIS_B1 && h->basis != BASIS_SF))
+      return fail(SGDCT_EUNSUP, "batched slices must be B0, B1 or SF projectors");
+    if (i > 0 && h->device != slices[0]->device) return fail(SGDCT_EINVAL, "batched slices must live on one device");
     b->proj.push_back(slices[i]);
     SliceDesc d;
     d.g = h->args;
@@ -1651,24 +1660,26 @@ sgdct_batch* sgdct_batch_create(sgdct_projector* const* slices, int nslice) {
   if (e == hipSuccess) e = hipMalloc(&b->d_order, sizeof(int) * 2 * nslice);
   if (e == hipSuccess) e = hipMalloc(&b->d_prefix, sizeof(long long) * 2 * (nslice + 1));
   if (e == hipSuccess) e = hipMalloc(&b->d_counters, sizeof(unsigned int) * 2);
-  if (e != hipSuccess) {
-    hip_fail(e, "batch allocation");
-    delete b;
-    return nullptr;
-  }
-  if (batch_upload_plan(b) != SGDCT_OK) {
-    delete b;
-    return nullptr;
-  }
+  if (e != hipSuccess) return hip_fail(e, "batch allocation");
+  if (int rc = batch_upload_plan(b)) return rc;
   b->fwd_bpc = auto_blocks(b, 0);
   b->bwd_bpc = auto_blocks(b, 1);
   batch_workspace(b);
-  if (b->plan.nfwd >= (1LL << 32) || b->plan.nbwd >= (1LL << 32)) {
-    fail(SGDCT_EUNSUP, "batch has more than 2^32 work items");
-    delete b;
+  if (b->plan.nfwd >= (1LL << 32) || b->plan.nbwd >= (1LL << 32))
+    return fail(SGDCT_EUNSUP, "batch has more than 2^32 work items");
+  return SGDCT_OK;
+}
+}  // namespace
+
+sgdct_batch* sgdct_batch_create(sgdct_projector* const* slices, int nslice) {
+  if (!slices || nslice <= 0) {
+    fail(SGDCT_EINVAL, "empty slice list");
     return nullptr;
   }
-  return b;
+  return no_throw([&]() -> sgdct_batch* {
+    auto b = std::make_unique<sgdct_batch>();
+    return fill_batch(b.get(), slices, nslice) == SGDCT_OK ? b.release() : nullptr;
+  }, (sgdct_batch*)nullptr);
 }
 
 void sgdct_batch_destroy(sgdct_batch* b) { delete b; }
@@ -1693,7 +1704,7 @@ int sgdct_batch_config(sgdct_batch* b, int fwd_blocks_per_cu, int bwd_blocks_per
     b->order = order;
     hipError_t e = hipSetDevice(b->device);
     if (e != hipSuccess) return hip_fail(e, "set device");
-    return batch_upload_plan(b);
+    return no_throw([&] { return batch_upload_plan(b); }, (int)SGDCT_ENOMEM);
   }
   return SGDCT_OK;
 }
