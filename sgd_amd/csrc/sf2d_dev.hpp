@@ -152,25 +152,10 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
   const unsigned bstep = 4u * G * (unsigned)smin;
-  // Pixel interval of line m, from N_u + R_u >= 0 and N_{u+1} - R_{u+1} < 0:
-  // [ceil(lo(m)), floor(hi(m))], affine in m, in FP32 and widened by its error
-  // bound: the trapezoid's own area decides at the boundary, where it is zero.
-  // sa and sb share a sign where the strip is within ~45 degrees of the walk
-  // direction, as the wave's orientation has it; otherwise the lane walks whole
-  // lines.
+  // Pixel interval of line m, from N_u + R_u >= 0 and N_{u+1} - R_{u+1} < 0.
   const float lastn = (float)(nmin - 1);
-  float lo0 = 0.0f, lo1 = 0.0f, hi0 = lastn, hi1 = 0.0f;
-  if ((sa > 0.0 && sb > 0.0) || (sa < 0.0 && sb < 0.0)) {
-    const float p0 = (float)((-ra - ac0) / sa), p1 = (float)(-ma / sa);
-    const float r0 = (float)((rb - bc0) / sb), r1 = (float)(-mb / sb);
-    lo0 = sa > 0.0 ? p0 : r0;
-    lo1 = sa > 0.0 ? p1 : r1;
-    hi0 = sa > 0.0 ? r0 : p0;
-    hi1 = sa > 0.0 ? r1 : p1;
-    const float most = (float)nmaj;
-    lo0 -= 4e-7f * __builtin_fmaf(fabsf(lo1), most, fabsf(lo0)) + 1e-5f;
-    hi0 += 4e-7f * __builtin_fmaf(fabsf(hi1), most, fabsf(hi0)) + 1e-5f;
-  }
+  StripLines lines;
+  lines.set(sa, ma, -ra - ac0, sb, mb, rb - bc0, (float)nmaj);
   // The weight's larger coordinate is the fixed one (reciprocal once per line)
   // if every lane's strip stays inside 45 degrees: at a line's end pixels the
   // moving coordinate exceeds the ray's by at most the strip's half width and a
@@ -181,9 +166,11 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
                                                              2.0 * (fabs(dmov) + fabs(dfix)))) == 0;
   auto walk = [&](auto own_c) {
     for (int m = m_lo + ((w0 - m_lo) & (wn - 1)); m <= m_hi; m += wn) {
-      const float fm = (float)m;
-      const float flo = fmaxf(ceilf(__builtin_fmaf(fm, lo1, lo0)), 0.0f);
-      const float fhi = fminf(floorf(__builtin_fmaf(fm, hi1, hi0)), lastn);
+      float flo, fhi;
+      if (!lines.ends((float)m, 0.0f, &flo, &fhi))
+        strip_exact(sa, -ra - ma * m - ac0, sb, rb - mb * m - bc0, 0.0, (double)lastn, &flo, &fhi);
+      flo = fmaxf(flo, 0.0f);
+      fhi = fminf(fhi, lastn);
       if (!(flo <= fhi)) continue;
       const int n0 = (int)flo;
       const double dm = (double)m, dn = (double)flo;
