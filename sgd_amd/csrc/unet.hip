@@ -1410,13 +1410,19 @@ static int halo_wgrad_cc(int cin, int cout) {
 static int halo_wgrad_co(int cc, int cout) { return cc == 32 && cout % 64 == 0 ? 64 : cout % 32 == 0 ? 32 : 16; }
 
 // Pixel-range splits of wgrad_halo_kernel: as many as give the launch its two
-// workgroups per CU at once, with at least 4 tiles each.
+// workgroups per CU at once, with at least 4 tiles each; and twice, three times
+// as many, so that no FP32 accumulator holds more than kWgTiles tiles (8192
+// pixels, as the gathered form's ranges) however large the batch is.
+constexpr int kWgTiles = 8192 / (kWgTH * kWgTW);
+
 static int halo_wgrad_splits(int B, int H, int W, int cin, int cout, int cc) {
   const long long ntile = (long long)B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH);
   const long long blocks = (long long)(cout / halo_wgrad_co(cc, cout)) * (cin / cc);
-  long long n = 512 / blocks;
-  if (n > ntile / 4) n = ntile / 4;
-  return (int)(n < 1 ? 1 : n);
+  const long long once = 512 / blocks < 1 ? 1 : 512 / blocks;
+  long long n = once;
+  if (n > ntile / 4) n = ntile / 4 < 1 ? 1 : ntile / 4;
+  if ((ntile + n - 1) / n > kWgTiles) n = ((ntile + kWgTiles - 1) / kWgTiles + once - 1) / once * once;
+  return (int)n;
 }
 
 // Rows of partial sums a weight gradient may need: each holds cout * (9 cin +
