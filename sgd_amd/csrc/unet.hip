@@ -735,13 +735,16 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
 // dY = 0.  CC = 8 (the network's first layer, bound by reading dY): 32 co x 9
 // taps x 8 channels per wave as five tiles of two taps each (the tenth is
 // dropped), one tile row per wave.
+// EDGE (images that are no whole tiles): beyond the image a cut tile's dY is 0,
+// and so is X but for the pixel on the edge, which the first pixel beyond meets
+// at kx = 0 (ky = 0).  An infinite X must not meet it, and is left out there.
 // At 8 x 512 x 512: 32 -> 32 channels 211 -> 77 us (268 MB; 500 TF/s), 96 -> 32
 // 476 -> 200 us, 8 -> 32 180 -> 48 us; at 8 x 256 x 256 64 -> 64 167 -> 57 us
 // (680 TF/s), 192 -> 64 339 -> 143 us.
 // ---------------------------------------------------------------------------
 constexpr int kWgTH = 4, kWgTW = 32;
 
-template <int CO_T, int CC>
+template <int CO_T, int CC, bool EDGE>
 __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int tiles_per_split) {
   static_assert(CC == 32 ? CO_T == 64 || CO_T == 32 : (CC == 8 || CC == 16) && CO_T <= 32, "tile");
   constexpr int PW = CC < 32 ? 4 : CO_T == 32 ? 2 : 1, TR = kWgTH / PW;  // waves along the rows; rows per wave
@@ -816,13 +819,26 @@ __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int til
     if (t + 1 < t_end) load(t + 1);
     const int row = 8 * g + (r16 >> 2), col = 4 * (r16 & 3);
     bf16x8 fa[TR][NI];
+    // EDGE: a fragment (this lane's pixels 8 g .. 8 g + 7) without pixel edge_x
+    const int edge_x = a.W - t % tiles_x * kWgTW, rows_in = a.H - t / tiles_x % tiles_y * kWgTH - wr;
+    auto off_edge = [&](bf16x8 fb) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (8 * g + e == edge_x) fb[e] = (bf16)0.0f;
+      return fb;
+    };
     if constexpr (CC == 8) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) fa[0][i] = tr_fragment(sd, wr * kWgTW + row, 16 * i + col, SD);
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const int tap = min(2 * j + ((r16 & 3) >> 1), 8);
-        const bf16x8 fb = tr_fragment(sx, (wr + tap / 3) * HW + row + tap % 3, 4 * (r16 & 1), SX);
+        bf16x8 fb = tr_fragment(sx, (wr + tap / 3) * HW + row + tap % 3, 4 * (r16 & 1), SX);
+        if constexpr (EDGE) {
+          const int mine = min(2 * j + (r16 >> 3), 8);  // the tap of this lane's column
+          if (mine % 3 == 0) fb = off_edge(fb);
+          if (mine < 3 && rows_in <= 0) fb = zero8();
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0][i], fb, acc[i][j], 0, 0, 0);
@@ -837,14 +853,16 @@ __global__ __launch_bounds__(256, 2) void wgrad_halo_kernel(WgradArgs a, int til
           fa[hr][i] = tr_fragment(sd, (wr + hr) * kWgTW + row, wco + 16 * i + col, SD);
 #pragma unroll
       for (int kx = 0; kx < 3; ++kx) {
-        const bf16x8 fb = tr_fragment(sx, (wr + hr) * HW + row + kx, wch + col, SX);
+        bf16x8 fb = tr_fragment(sx, (wr + hr) * HW + row + kx, wch + col, SX);
+        if (EDGE && kx == 0) fb = off_edge(fb);
 #pragma unroll
         for (int ky = 0; ky < 3; ++ky) {
           const int r = hr - ky, j = (3 * ky + kx) % NB;
           if (r < 0 || r >= TR) continue;
+          const bf16x8 fk = EDGE && ky == 0 && r >= rows_in ? zero8() : fb;
 #pragma unroll
           for (int i = 0; i < NI; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][i], fb, acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[r][i], fk, acc[i][j], 0, 0, 0);
         }
       }
     }
@@ -1435,6 +1453,12 @@ long long nn_wgrad_parts(int B, int H, int W, int cin, int cout) {
   return h > n ? h : n;
 }
 
+template <int CO_T, int CC>
+static void run_wgrad_halo(const WgradArgs& a, dim3 grid, int tiles_per_split, hipStream_t s) {
+  if (a.W % kWgTW || a.H % kWgTH) wgrad_halo_kernel<CO_T, CC, true><<<grid, 256, 0, s>>>(a, tiles_per_split);
+  else wgrad_halo_kernel<CO_T, CC, false><<<grid, 256, 0, s>>>(a, tiles_per_split);
+}
+
 hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float* dw, float* db, float* partial, int B,
                     int H, int W, int cin, int cout, hipStream_t s) {
   const long long M = (long long)B * H * W;
@@ -1452,12 +1476,12 @@ hipError_t nn_wgrad(const void* x, const void* x2, int c0, const void* dy, float
     const int ntile = B * ((W + kWgTW - 1) / kWgTW) * ((H + kWgTH - 1) / kWgTH), tps = (ntile + ns - 1) / ns;
     parts = ns;
     a.bias_partial = db ? partial + parts * cout * K : nullptr;
-    if (cc == 32 && co == 64) wgrad_halo_kernel<64, 32><<<grid, 256, 0, s>>>(a, tps);
-    else if (cc == 32) wgrad_halo_kernel<32, 32><<<grid, 256, 0, s>>>(a, tps);
-    else if (cc == 16 && co == 32) wgrad_halo_kernel<32, 16><<<grid, 256, 0, s>>>(a, tps);
-    else if (cc == 16) wgrad_halo_kernel<16, 16><<<grid, 256, 0, s>>>(a, tps);
-    else if (co == 32) wgrad_halo_kernel<32, 8><<<grid, 256, 0, s>>>(a, tps);
-    else wgrad_halo_kernel<16, 8><<<grid, 256, 0, s>>>(a, tps);
+    if (cc == 32 && co == 64) run_wgrad_halo<64, 32>(a, grid, tps, s);
+    else if (cc == 32) run_wgrad_halo<32, 32>(a, grid, tps, s);
+    else if (cc == 16 && co == 32) run_wgrad_halo<32, 16>(a, grid, tps, s);
+    else if (cc == 16) run_wgrad_halo<16, 16>(a, grid, tps, s);
+    else if (co == 32) run_wgrad_halo<32, 8>(a, grid, tps, s);
+    else run_wgrad_halo<16, 8>(a, grid, tps, s);
   } else {
     a.bias_partial = db ? partial + parts * cout * K : nullptr;
     if (cout <= 32) wgrad_kernel<32><<<dim3(1, (K + 127) / 128, (unsigned)parts), 256, 0, s>>>(a);
