@@ -17,12 +17,13 @@ __device__ __forceinline__ float min2f(float a, float b) { return __builtin_amdg
 __device__ __forceinline__ float max2f(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
 __device__ __forceinline__ float clamp3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
 
-// 1 / d for a normal double d of float range: the float reciprocal (relative
-// error ~6e-8) refined by one Newton step (error ~4e-15), in place of the
-// double division's longer sequence
+// 1 / d for a normal double d: the approximation of v_rcp_f64 (relative error
+// below 2^-23) refined by two Newton steps to an ulp, in place of the double
+// division's longer sequence (scaling, three steps, fix-up)
 __device__ __forceinline__ double recip(double d) {
-  const double r0 = (double)__builtin_amdgcn_rcpf((float)d);
-  return __builtin_fma(r0, __builtin_fma(-d, r0, 1.0), r0);
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
 // Unit-height trapezoid over sorted corners, 1 / (q1 - q0) and 1 / (q3 - q2)
