@@ -275,6 +275,7 @@ struct sgdct_batch {
   // persistent choice on 256 uneven slices (A^T at 8 blocks per CU: 165.5 ms
   // against 200.8 ms at 4).
   int fwd_bpc = 8, bwd_bpc = 8, order = 0;
+  bool far = false;  // a slice of 4 GiB: one launch per slice in any configuration
   double* d_part = nullptr;
   size_t part_cap = 0;
   struct Graph {
@@ -1378,7 +1379,7 @@ int auto_blocks(const sgdct_batch* b, int dir) {
 }
 
 int batch_run(sgdct_batch* b, int dir, const float* in, float* out, hipStream_t s) {
-  if ((dir == 0 ? b->fwd_bpc : b->bwd_bpc) == 0) {
+  if (b->far || (dir == 0 ? b->fwd_bpc : b->bwd_bpc) == 0) {
     // one launch per slice, in slice order, the slices' own splits
     for (int i = 0; i < b->n; ++i) {
       sgdct_projector* h = b->proj[i];
@@ -1644,6 +1645,7 @@ int fill_batch(sgdct_batch* b, sgdct_projector* const* slices, int nslice) {
     d.img_off = b->img_off[i];
     d.sino_off = b->sino_off[i];
     b->desc.push_back(d);
+    b->far |= (size_t)h->nx * h->ny >= (size_t)1 << 30;
     b->img_off[i + 1] = b->img_off[i] + (long long)h->nx * h->ny;
     b->sino_off[i + 1] = b->sino_off[i] + (long long)h->np * h->nu;
     const double w = basis_weight(h->basis);

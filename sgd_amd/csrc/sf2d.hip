@@ -29,7 +29,7 @@ hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float
 // views, batch 5 266 -> 72 us; one value, 721 views from another start angle
 // 1455 -> 1133 us.  (FP64 line intervals, a four-value sort, compared ramps and
 // the weight's reciprocal per pixel: 260, 1130, 84, 1418 us.)
-template <int G, int W>
+template <int G, int W, bool FAR>
 __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
                                                         const float* __restrict__ rows_img,
                                                         const float* __restrict__ cols_img, float* __restrict__ sino,
@@ -43,8 +43,8 @@ __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp
   double acc[G];
 #pragma unroll
   for (int s = 0; s < G; ++s) acc[s] = 0.0;
-  sf_fwd_lines<G>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr, wv,
-                  W, blockIdx.z, gridDim.z, acc, sp.place);
+  sf_fwd_lines<G, FAR>(g, v, chunk, rows_img + blockIdx.y * gpix, cols_img ? cols_img + blockIdx.y * gpix : nullptr,
+                       wv, W, blockIdx.z, gridDim.z, acc, sp.place);
 #pragma unroll
   for (int s = 0; s < G; ++s) red[wv][s][lane] = acc[s];
   __syncthreads();
@@ -101,7 +101,11 @@ namespace {
 template <int G, int W>
 hipError_t sf_forward_g(const Proj2DArgs& g, const GroupRun& r, const float* img, float* sino, hipStream_t s) {
   const dim3 grid((unsigned)(r.sym.nrep * g.nchunk), (unsigned)r.groups(), (unsigned)r.split);
-  sf_fwd_kernel<G, W><<<grid, 64 * W, 0, s>>>(g, r.sym, r.m, r.batch, r.rows ? r.rows : img, r.cols, sino, r.part);
+  const float* const rows = r.rows ? r.rows : img;
+  if (G == 1 && (size_t)g.nx * g.ny >= (size_t)1 << 30)
+    sf_fwd_kernel<1, W, true><<<grid, 64 * W, 0, s>>>(g, r.sym, r.m, r.batch, rows, r.cols, sino, r.part);
+  else
+    sf_fwd_kernel<G, W, false><<<grid, 64 * W, 0, s>>>(g, r.sym, r.m, r.batch, rows, r.cols, sino, r.part);
   return hipGetLastError();
 }
 

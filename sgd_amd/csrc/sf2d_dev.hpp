@@ -92,8 +92,9 @@ __device__ __forceinline__ float sf_weight(float dx, float wx, float wy) {
 
 // A: bin-driven gather (the strip walk of fwd_bin_lines, corner rule h = 1/2).
 // One wave: bins [64 chunk, 64 chunk + 64) of view v, lines m = w0 mod wn of
-// segment seg of nseg, sums into acc[G]; images as in fwd_bin_lines.
-template <int G>
+// segment seg of nseg, sums into acc[G]; images as in fwd_bin_lines, by address
+// where they hold 4 GiB or more (FAR).
+template <int G, bool FAR = false>
 __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chunk, const float* __restrict__ rows_img,
                                              const float* __restrict__ cols_img, int w0, int wn, int seg, int nseg,
                                              double (&acc)[G], int place = 0) {
@@ -152,7 +153,8 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const float* const img = (rows || strided) ? rows_img : cols_img;
   const __amdgpu_buffer_rsrc_t img_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(img), (short)0, (int)(4u * G * (unsigned)g.nx * (unsigned)g.ny), 0x00020000);
-  const unsigned bstep = 4u * G * (unsigned)smin;
+  using Off = std::conditional_t<FAR, size_t, unsigned>;  // modulo its range: steps may be negative
+  const Off bstep = 4 * G * (Off)smin;
   // Pixel interval of line m, from N_u + R_u >= 0 and N_{u+1} - R_{u+1} < 0.
   const float lastn = (float)(nmin - 1);
   StripLines lines;
@@ -180,8 +182,8 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
       float wm = (float)__builtin_fma(dn, dmov, w0mov);
       const float wf = (float)__builtin_fma(dm, dfix, w0fix);
       const float ifix = __builtin_amdgcn_rcpf(fabsf(wf)), wf2 = wf * wf;
-      unsigned off = 4u * G * (unsigned)(base + m * smaj + n0 * smin);
-      const unsigned end = off + (unsigned)((int)fhi - n0 + 1) * bstep;
+      Off off = 4 * G * ((Off)base + (Off)m * (Off)smaj + (Off)n0 * (Off)smin);
+      const Off end = off + (Off)((int)fhi - n0 + 1) * bstep;
       float accl[G];
 #pragma unroll
       for (int k = 0; k < G; ++k) accl[k] = 0.0f;
@@ -191,7 +193,8 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
       sort2((nl2 - nu_) * __builtin_amdgcn_rcpf(be - bl2), (nl1 - nu_) * __builtin_amdgcn_rcpf(be - bl1), t1, t2);
       do {
         float x[G];
-        buffer_load_n<G>(img_rsrc, off, x);
+        if constexpr (FAR) __builtin_memcpy(x, reinterpret_cast<const char*>(img) + off, sizeof(x));
+        else buffer_load_n<G>(img_rsrc, off, x);
         float l1, l2;
         sort2(-(nu_ + nl1) * __builtin_amdgcn_rcpf(be + bl1), -(nu_ + nl2) * __builtin_amdgcn_rcpf(be + bl2), l1, l2);
         const Trap t = make_trap(t1, t2, l1, l2);
