@@ -270,6 +270,9 @@ int sgdct_batch_layout(const sgdct_batch *b, long long *img_off, long long *sino
  * one launch per slice, or, for more than 16 small slices, the persistent
  * queue at 8 blocks per CU, order 0. */
 int sgdct_batch_config(sgdct_batch *b, int fwd_blocks_per_cu, int bwd_blocks_per_cu, int order);
+/* The launch shape in use: out[0..2] = blocks per CU of A and A^T (0: one
+ * launch per slice), slice order. */
+int sgdct_batch_shape(const sgdct_batch *b, int *out);
 int sgdct_batch_forward(sgdct_batch *b, const float *img, float *sino, void *stream);
 int sgdct_batch_backward(sgdct_batch *b, const float *sino, float *img, void *stream);
 /* Same as forward (direction 0) / backward (1), through a hipGraph captured on

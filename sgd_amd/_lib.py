@@ -130,6 +130,8 @@ def lib():
     L.sgdct_batch_layout.restype = ctypes.c_int
     L.sgdct_batch_config.argtypes = [_h, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     L.sgdct_batch_config.restype = ctypes.c_int
+    L.sgdct_batch_shape.argtypes = [_h, ctypes.POINTER(ctypes.c_int)]
+    L.sgdct_batch_shape.restype = ctypes.c_int
     for name in ("sgdct_batch_forward", "sgdct_batch_backward"):
         f = getattr(L, name)
         f.argtypes = [_h, _fp, _fp, _fp]

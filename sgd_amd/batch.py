@@ -87,9 +87,14 @@ class SliceBatch:
         _lib.check(L.sgdct_batch_layout(h, io, so), "batch layout")
         self.img_off, self.sino_off = list(io), list(so)
         self.device = self.projectors[0].device
-        # the persistent shape, used where the batch's own choice (one launch
-        # per slice, or the persistent queue) is the queue
-        self.config = (8, 8, 0)
+        self.config = self._shape()
+
+    def _shape(self):
+        """Launch shape in use: persistent blocks per CU of A and A^T (0: one
+        launch per slice), slice order."""
+        out = (ctypes.c_int * 3)()
+        _lib.check(_lib.lib().sgdct_batch_shape(self.handle, out), "batch shape")
+        return tuple(out)
 
     def close(self):
         if getattr(self, "handle", None):
@@ -127,7 +132,7 @@ class SliceBatch:
     def set_config(self, fwd_blocks_per_cu, bwd_blocks_per_cu, order):
         _lib.check(_lib.lib().sgdct_batch_config(self.handle, int(fwd_blocks_per_cu), int(bwd_blocks_per_cu),
                                                  int(order)), "batch config")
-        self.config = (int(fwd_blocks_per_cu), int(bwd_blocks_per_cu), int(order))
+        self.config = self._shape()
 
     def _stream(self):
         return ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)

@@ -1711,6 +1711,14 @@ int sgdct_batch_config(sgdct_batch* b, int fwd_blocks_per_cu, int bwd_blocks_per
   return SGDCT_OK;
 }
 
+int sgdct_batch_shape(const sgdct_batch* b, int* out) {
+  if (!b || !out) return fail(SGDCT_EINVAL, "null argument");
+  out[0] = b->far ? 0 : b->fwd_bpc;
+  out[1] = b->far ? 0 : b->bwd_bpc;
+  out[2] = b->order;
+  return SGDCT_OK;
+}
+
 int sgdct_batch_forward(sgdct_batch* b, const float* img, float* sino, void* stream) {
   if (!b || !img || !sino) return fail(SGDCT_EINVAL, "null argument");
   return batch_run(b, 0, img, sino, (hipStream_t)stream);
