@@ -181,7 +181,6 @@ struct sgdct_projector {
   SymPlan sym{};
   int* d_sym = nullptr;
   int win = 0;
-  bool in_front = true;  // of every view's source, all pixels
   // Interleaved images of an unsplit A, which shares no other memory, so that a
   // handle's calls on different streams may overlap: one buffer, made with the
   // handle, whose uses are ordered by copies_ev, recorded after each.  (A buffer
@@ -481,8 +480,7 @@ int fill(sgdct_projector* h, int basis, int nx, int ny, int np, int nu, double d
     // next to a source footprints have no bound, and their rounding none either:
     // every view by itself where the image reaches behind one
     h->sym = plain_plan(h);
-    h->in_front = w < kNoWindow;
-    if (h->in_front)
+    if (w < kNoWindow)
       if (int rc = setup_symmetry(h, views)) return rc;
     if (bwd_lds_bytes(basis, w, h->sym.nh) <= kLdsBytes) h->win = w;
   }
@@ -552,7 +550,7 @@ Cone3DArgs cone_args(const sgdct_projector* h) {
 int setup_cone(sgdct_projector* h) {
   h->nslot = h->np;
   h->cone.nh = 1;
-  if (!h->in_front || !cone_groups_fit(h->nz, h->nv) || h->nx > 0xffff || h->ny > 0x7fff) return SGDCT_OK;
+  if (!cone_groups_fit(h->nz, h->nv) || h->nx > 0xffff || h->ny > 0x7fff) return SGDCT_OK;
   std::vector<ViewGeo> views(h->np);
   hipError_t e = hipMemcpy(views.data(), h->d_views, sizeof(ViewGeo) * h->np, hipMemcpyDeviceToHost);
   if (e != hipSuccess) return hip_fail(e, "cone-beam symmetries");

@@ -79,17 +79,3 @@ def test_views_by_themselves_behind_the_source(cuda, basis):
     for k in (0, 5, n // 4 - 1, n // 4, n // 2 + 3, n - 1):
         print(basis, "view", k, flush=True)
         assert torch.equal(torch.nan_to_num(make(ang[k:k + 1]).forward(x))[0], y[k])
-
-
-@pytest.mark.parametrize("model", ["B1", "SF-TR"])
-def test_cone_views_by_themselves_behind_the_source(cuda, model):
-    import torch
-    from sgd_amd.torch_ops import Projector
-    ang = 2 * np.pi * np.arange(12) / 12
-    make = lambda a: Projector.cone_beam(60, 60, 8, a, 50, 30, 2.0, 2.0, 0.4, 2.0, 1.5, 100.0, 50.0, model=model)
-    P = make(ang)
-    x = torch.randn(P.img_shape, device=cuda, generator=torch.Generator(device=cuda).manual_seed(1))
-    y = torch.nan_to_num(P.forward(x))
-    for k in range(12):
-        print(model, "view", k, flush=True)
-        assert torch.equal(torch.nan_to_num(make(ang[k:k + 1]).forward(x))[0], y[k])
