@@ -129,15 +129,14 @@ __device__ __forceinline__ void fwd_lone_store(int nseg, const double (*red)[64]
 }
 
 // Points [flo, fhi] of line l of a strip, from the tests
-//   q:  s_q n + m_q l >= q0     and     r:  s_r n + m_r l < r0
+//   q:  s_q n >= r1     and     r:  s_r n < r2,      r1 = q0 - m_q l, r2 = r0 - m_r l,
 // on whole n.  Their ends are affine in l and formed in FP32; where one comes
-// within its error of a whole number, or the slopes s are not of one sign, the
-// caller takes them from strip_exact, so that a line holds the points of the
-// FP64 tests and no other (a point outside has no weight, but an infinite one
-// would still turn the bin's sum into NaN).
+// within its error of a whole number, `settle` tests that number in FP64, so that
+// a line holds the points of the FP64 tests and no other (a point outside has
+// no weight, but an infinite one would still turn the bin's sum into NaN).
 struct StripLines {
   float lo0 = 0.0f, lo1 = 0.0f, hi0 = 0.0f, hi1 = 0.0f, tlo = -1.0f, thi = -1.0f;
-  // lines |l| <= most
+  // lines |l| <= most; slopes that are not of one sign leave every line unsettled
   __device__ __forceinline__ void set(double s_q, double m_q, double q0, double s_r, double m_r, double r0, float most) {
     if (!((s_q > 0.0 && s_r > 0.0) || (s_q < 0.0 && s_r < 0.0))) return;
     const bool up = s_q > 0.0;
@@ -146,31 +145,37 @@ struct StripLines {
     lo1 = up ? a1 : b1;
     hi0 = up ? b0 : a0;
     hi1 = up ? b1 : a1;
-    // three roundings of at most 2^-24 of each term (ends(): one more), and some
+    // three roundings of at most 2^-24 of each term (at(): one more), and some
     tlo = 0.5f - 1e-6f - 2.4e-7f * __builtin_fmaf(fabsf(lo1), most, fabsf(lo0) + 1.0f);
     thi = 0.5f - 1e-6f - 2.4e-7f * __builtin_fmaf(fabsf(hi1), most, fabsf(hi0) + 1.0f);
   }
-  // points n + shift; false: strip_exact's ends are needed
-  __device__ __forceinline__ bool ends(float l, float shift, float* flo, float* fhi) const {
-    const float a = __builtin_fmaf(l, lo1, lo0) - shift, b = __builtin_fmaf(l, hi1, hi0) - shift;
-    *flo = ceilf(a);
-    *fhi = floorf(b);
-    return fabsf(__builtin_amdgcn_fractf(a) - 0.5f) <= tlo && fabsf(__builtin_amdgcn_fractf(b) - 0.5f) <= thi;
+  // points n + shift; false: not settled
+  __device__ __forceinline__ bool at(float l, float shift, float* lo, float* hi) const {
+    *lo = __builtin_fmaf(l, lo1, lo0) - shift;
+    *hi = __builtin_fmaf(l, hi1, hi0) - shift;
+    return fabsf(__builtin_amdgcn_fractf(*lo) - 0.5f) <= tlo && fabsf(__builtin_amdgcn_fractf(*hi) - 0.5f) <= thi;
+  }
+  // at()'s ends, moved to the first and last point, within [0, last]
+  __device__ __forceinline__ void settle(double s_q, double r1, double s_r, double r2, double last, float* lo,
+                                         float* hi) const {
+    if (tlo > 0.0f && thi > 0.0f) {  // off by less than a half: one of two whole numbers
+      const double a = rint((double)*lo), b = rint((double)*hi);
+      const bool up = s_q > 0.0;
+      *lo = (float)((up ? s_q * a >= r1 : s_r * a < r2) ? a : a + 1.0);
+      *hi = (float)((up ? s_r * b < r2 : s_q * b >= r1) ? b : b - 1.0);
+      return;
+    }
+    double x = 0.0, y = last;
+    if (s_q > 0.0) x = fmax(x, ceil(r1 / s_q));
+    else if (s_q < 0.0) y = fmin(y, floor(r1 / s_q));
+    else if (r1 > 0.0) y = -1.0;
+    if (s_r > 0.0) y = fmin(y, ceil(r2 / s_r) - 1.0);
+    else if (s_r < 0.0) x = fmax(x, floor(r2 / s_r) + 1.0);
+    else if (r2 <= 0.0) y = -1.0;
+    *lo = (float)x;
+    *hi = (float)y;
   }
 };
-
-// The ends for s_q n >= r1 and s_r n < r2, within [lo, hi].
-__device__ __forceinline__ void strip_exact(double s_q, double r1, double s_r, double r2, double lo, double hi,
-                                            float* flo, float* fhi) {
-  if (s_q > 0.0) lo = fmax(lo, ceil(r1 * (1.0 / s_q)));
-  else if (s_q < 0.0) hi = fmin(hi, floor(r1 * (1.0 / s_q)));
-  else if (r1 > 0.0) hi = -1.0;
-  if (s_r > 0.0) hi = fmin(hi, ceil(r2 * (1.0 / s_r)) - 1.0);
-  else if (s_r < 0.0) lo = fmax(lo, floor(r2 * (1.0 / s_r)) + 1.0);
-  else if (r2 <= 0.0) hi = -1.0;
-  *flo = (float)lo;
-  *fhi = (float)hi;
-}
 
 // A tile's staged bins in LDS: the records as REC float4 planes, then the G
 // sinogram values of each bin as planes of up to 4, so that 16-byte reads of

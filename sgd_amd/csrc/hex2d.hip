@@ -236,11 +236,11 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
       const bool odd = il & 1;  // points half a column to the right
       const float sh = odd ? 0.5f : 0.0f;
       float flo, fhi;
-      if (!lines.ends((float)il, sh, &flo, &fhi))
-        strip_exact(sq, -rq - __builtin_fma(mq, (double)il, cq) - sq * sh, sr,
-                    rr - __builtin_fma(mr, (double)il, cr) - sr * sh, 0.0, (double)(g.nx - 1), &flo, &fhi);
-      flo = fmaxf(flo, fc_lo);
-      fhi = fminf(fhi, odd ? fc_odd : fc_hi);
+      if (!lines.at((float)il, sh, &flo, &fhi))
+        lines.settle(sq, -rq - __builtin_fma(mq, (double)il, cq) - sq * sh, sr,
+                     rr - __builtin_fma(mr, (double)il, cr) - sr * sh, (double)(g.nx - 1), &flo, &fhi);
+      flo = fmaxf(ceilf(flo), fc_lo);
+      fhi = fminf(floorf(fhi), odd ? fc_odd : fc_hi);
       if (!(flo <= fhi)) continue;
       const int n0 = (int)flo;
       const double dn = (double)(flo + sh), dl = (double)il;
@@ -277,10 +277,10 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
     const Off step = flip_y ? -(8 * G * (Off)g.nx) : 8 * G * (Off)g.nx;
     for (int k = k_lo; k <= k_hi; ++k) {  // ic' = k / 2
       float flo, fhi;
-      if (!lines.ends((float)k, 0.0f, &flo, &fhi))
-        strip_exact(mq, -rq - cq - sq * (0.5 * k), mr, rr - cr - sr * (0.5 * k), 0.0, (double)(g.ny - 1), &flo, &fhi);
-      flo = fmaxf(flo, fr_lo);
-      fhi = fminf(fhi, fr_hi);
+      if (!lines.at((float)k, 0.0f, &flo, &fhi))
+        lines.settle(mq, -rq - cq - sq * (0.5 * k), mr, rr - cr - sr * (0.5 * k), (double)(g.ny - 1), &flo, &fhi);
+      flo = fmaxf(ceilf(flo), fr_lo);
+      fhi = fminf(floorf(fhi), fr_hi);
       if (!(flo <= fhi)) continue;
       int i0 = (int)flo, i1 = (int)fhi;
       i0 += (i0 ^ k) & 1;  // rows of the line's parity

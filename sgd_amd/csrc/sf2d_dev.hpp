@@ -170,10 +170,10 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   auto walk = [&](auto own_c) {
     for (int m = m_lo + ((w0 - m_lo) & (wn - 1)); m <= m_hi; m += wn) {
       float flo, fhi;
-      if (!lines.ends((float)m, 0.0f, &flo, &fhi))
-        strip_exact(sa, -ra - ma * m - ac0, sb, rb - mb * m - bc0, 0.0, (double)lastn, &flo, &fhi);
-      flo = fmaxf(flo, 0.0f);
-      fhi = fminf(fhi, lastn);
+      if (!lines.at((float)m, 0.0f, &flo, &fhi))
+        lines.settle(sa, -ra - ma * m - ac0, sb, rb - mb * m - bc0, (double)lastn, &flo, &fhi);
+      flo = fmaxf(ceilf(flo), 0.0f);
+      fhi = fminf(floorf(fhi), lastn);
       if (!(flo <= fhi)) continue;
       const int n0 = (int)flo;
       const double dm = (double)m, dn = (double)flo;
