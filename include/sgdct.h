@@ -304,7 +304,8 @@ int sgdct_nn_conv3x3_ex(const void *in, const void *in2, int c0, const void *w, 
  * the first c0 of the cout gradient channels summed over 2x2 blocks and masked
  * by low_mask > 0, gskip (B, H, W, cout - c0) the others (sgdct_nn_conv3x3 with
  * out_f32 followed by sgdct_nn_upcat_back; the workspace holds the gradient in
- * between where the two do not run as one, and is empty where they do). */
+ * between where the two do not run as one, and is empty where they do).
+ * low_out, low_mask and gskip are 16-byte aligned. */
 long long sgdct_nn_conv3x3_upback_workspace(int B, int H, int W, int cin, int cout, int c0);
 int sgdct_nn_conv3x3_upback(const void *in, const void *w, void *low_out, const void *low_mask, float *gskip,
                             float *workspace, long long workspace_floats, int B, int H, int W, int cin, int cout,

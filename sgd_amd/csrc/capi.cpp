@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <initializer_list>
 #include <memory>
@@ -1875,6 +1876,8 @@ int sgdct_nn_conv3x3_upback(const void* in, const void* w, void* low_out, const 
   if (!in || !w || !low_out || !low_mask || !gskip || !dims_ok(B, H, W) || H % 2 || W % 2 || cin <= 0 || cin % 8 ||
       cout <= 0 || c0 <= 0 || c0 >= cout)
     return fail(SGDCT_EINVAL, "bad conv3x3_upback arguments");
+  if (((uintptr_t)low_out | (uintptr_t)low_mask | (uintptr_t)gskip) & 15)
+    return fail(SGDCT_EINVAL, "conv3x3_upback outputs must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   if (nn_upback_fused(cin, cout, c0))
     return nn_ret(nn_conv3x3_upback(in, w, low_out, low_mask, gskip, B, H, W, cin, cout, c0, s), "conv3x3_upback");

@@ -1328,6 +1328,10 @@ __global__ void to_bf16_kernel(const float* __restrict__ src, bf16* __restrict__
 // ---------------------------------------------------------------------------
 static inline unsigned blocks_for(long long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
+static bool aligned16(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
+}
+
 // 3x3 convolutions with cin % 32 == 0 (or cin 16 or 8) and cout % 16 == 0 run
 // the halo-tiled kernel; the others the K-step-staged ones.
 static bool halo_conv(int cin, int cout) { return (cin % 32 == 0 || cin == 16 || cin == 8) && cout % 16 == 0; }
@@ -1381,7 +1385,7 @@ bool nn_upback_fused(int cin, int cout, int c0) { return halo_conv(cin, cout) &&
 // with the halo kept for its three blocks of output channels).
 hipError_t nn_conv3x3_upback(const void* in, const void* w, void* low_out, const void* low_mask, float* skip_out, int B,
                              int H, int W, int cin, int cout, int c0, hipStream_t s) {
-  if (!nn_upback_fused(cin, cout, c0)) return hipErrorInvalidValue;
+  if (!nn_upback_fused(cin, cout, c0) || !aligned16(low_out, low_mask, skip_out)) return hipErrorInvalidValue;
   ConvArgs a{static_cast<const bf16*>(in), static_cast<const bf16*>(w), nullptr, nullptr, B, H, W, cin, cout, 0, 1,
              nullptr, nullptr, 0, static_cast<bf16*>(low_out), static_cast<const bf16*>(low_mask), skip_out, c0};
   return launch_halo(a, s);
@@ -1393,7 +1397,9 @@ hipError_t nn_conv3x3(const void* in, const void* in2, int c0, const void* w, co
              static_cast<const bf16*>(mask), static_cast<const bf16*>(in2), c0, nullptr, nullptr, nullptr, 0};
   const long long M = (long long)B * H * W;
   if (cin % 8 != 0) return hipErrorInvalidValue;
-  if (halo_conv(cin, cout)) return launch_halo(a, s);
+  // the halo kernel stores (and reads the mask) 16 bytes at a time, the others
+  // element by element
+  if (halo_conv(cin, cout) && aligned16(out, mask)) return launch_halo(a, s);
   if (cout % 128 == 0) {
     conv3x3_lds_kernel<128, 128, 2, 2><<<dim3(blocks_for(M, 128), cout / 128), 256, 0, s>>>(a);
   } else if (cout % 64 == 0) {
@@ -1503,9 +1509,6 @@ hipError_t nn_pad_input(const float* x, void* out8, long long n, hipStream_t s) 
 
 // The vector kernels take 8 channels as aligned vectors, index one image in 32
 // bits and the image by grid.y.
-static bool aligned16(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
-  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
-}
 static bool vec8(long long per_image, int B, int C) { return C % 8 == 0 && per_image < (1LL << 31) && B < 65536; }
 
 hipError_t nn_pool2(const void* src, void* dst, int B, int H, int W, int C, hipStream_t s) {
