@@ -6,6 +6,10 @@
  * and host layouts:
  *   image     x[ix*ny + iy]  (FP64, host)       layers/A_B1.cu:621-623
  *   sinogram  b[p*nu + u]    (FP64, host)       layers/A_B1.cu:639-641
+ *     (a 2-D call of fewer than 1.5e8 (pixel, view) pairs evaluates every view
+ *     by itself, so that a view's values do not depend on the handle's other
+ *     views; larger calls share footprints between symmetric views as the
+ *     device entry points do, which agrees to FP32 rounding)
  *   A overwrites b, A^T overwrites x.
  * Differences from the reference, all additive:
  *   - dz / drho are explicit nullable pointers (the reference relies on C++

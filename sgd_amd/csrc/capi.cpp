@@ -1060,11 +1060,12 @@ int run_backward(sgdct_projector* h, const float* sino, float* img, int batch, h
 // lines and views in an order of their own (contiguous line segments, whole
 // groups of views), which neither the scan's symmetries nor the launch shape
 // of the device entry points change: what they return for a view is the same
-// to the last bit whichever other views the handle holds.  That costs little
-// while the conversions and copies of their arrays are most of a call (256 x
-// 256, 360 views: the kernels are 0.2 of 0.46 ms per pair).  From kHostPairs
-// (pixel, view) pairs on the kernels are most of it, and the call takes the
-// device entry points' launches.
+// to the last bit whichever other views the handle holds.  It costs small
+// arrays up to half of a call (256 x 256, 360 views: 0.22 of 0.42 ms a pair are
+// kernels).  From kHostPairs (pixel, view) pairs on, where the kernels are most
+// of it, the call takes the device entry points' launches (include/sgdct.h
+// says so): 512 x 512, 720 views, B1: A 0.55, A^T 0.56 ms a call, 1.51 and 1.28
+// before.
 constexpr double kHostPairs = 1.5e8;
 bool host_alone(const sgdct_projector* h) {
   return !is_cone(h->basis) && (double)h->nx * h->ny * h->np < kHostPairs;
