@@ -305,7 +305,7 @@ __device__ __forceinline__ int image_column(const Proj2DArgs& g, int op, int c) 
 // Dynamic LDS: per column and voxel 6 + G floats and one of padding to an odd
 // stride.  Bound by the LDS reads of the records and, at G = 4, by the stores
 // of Y.  256^3 voxels, 360 views, 512 x 384, classes of 4: A as a whole 40.0 ->
-// 20.0 ms against one view at a time.
+// 20.5 ms against one view at a time.
 template <int M, int G>
 __global__ __launch_bounds__(256) void axial_fwd_group_kernel(Cone3DArgs a, int p0, const float* __restrict__ xT,
                                                               float* __restrict__ Y) {
@@ -756,7 +756,7 @@ __global__ __launch_bounds__(256) void axial_bwd_kernel(Cone3DArgs a, int p0, in
 // Block: 256 voxels of one column; grid (ndom, ceil(nz / 256)).  The next
 // view's profiles are requested before the current view's rows are gathered.
 // nv <= kGroupRows.  Bound by the reads of the profiles (1.6 GB per 16 views of
-// the case above); A^T as a whole 34.3 -> 20.7 ms.
+// the case above); A^T as a whole 34.3 -> 21.2 ms.
 constexpr int kGroupRows = 512;
 
 template <int M, int G>

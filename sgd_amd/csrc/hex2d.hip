@@ -302,9 +302,10 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
 // it together.  Bound by VALU issue (~45 instructions per footprint, and about
 // as many per line and lane) and, at G = 8, by the vector L1.  Per call, one
 // value per footprint and one wave per (view, chunk) -> now: H0 256 x 296
-// points, 1024 views, 1024 bins 840 -> 318 us (476 with three rhombi's six
-// antiderivatives and FP64 intervals); Hl, batch 64 30.8 -> 7.0 ms; Hl 40 x 46,
-// 60 views, batch 3 76 -> 16 us.
+// points, 1024 views, 1024 bins 840 -> 315 us (476 with three rhombi's six
+// antiderivatives and FP64 divisions for every line); Hl, batch 64 30.8 -> 7.0
+// ms; Hl 40 x 46, 60 views, batch 3 76 -> 18 us, 3 of them the events that order
+// the interleaved points' uses.
 template <int HB, int G, int W, bool FAR>
 __global__ __launch_bounds__(64 * W) void hex_fwd_kernel(HexArgs ha, SymPlan sp, int m, int batch,
                                                          const float* __restrict__ img, float* __restrict__ sino,
@@ -436,7 +437,7 @@ template <int HB> struct HexBwd {
 // Launched as bwd_group_kernel; bound by VALU issue and the LDS reads of the
 // records (48 bytes per footprint for H0; 80 with three rhombi, 437 us in the
 // first case).  Same cases as hex_fwd_kernel: 728 -> 257 us, 33.2 -> 5.5 ms, 39
-// -> 14 us.
+// -> 13 us.
 template <int HB, int G>
 __global__ __launch_bounds__(256) void hex_bwd_group_kernel(HexArgs ha, SymPlan sp, int m, int batch,
                                                             const float* __restrict__ sino, float* __restrict__ img,

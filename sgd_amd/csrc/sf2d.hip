@@ -25,10 +25,11 @@ hipError_t launch_interleave(const Proj2DArgs& g, const GroupRun& r, const float
 // new corner projections, the merge of two sorted pairs, the trapezoid's area),
 // and about as many per line, beside one multiply-add per value.  512 x 512,
 // 720 views, 768 bins, per call: one value per footprint 1456 us, the scan's 8
-// symmetries 212 us; 1024 x 1024, 900 views 7.04 -> 0.90 ms; 256 x 256, 90
-// views, batch 5 266 -> 72 us; one value, 721 views from another start angle
-// 1455 -> 1133 us.  (FP64 line intervals, a four-value sort, compared ramps and
-// the weight's reciprocal per pixel: 260, 1130, 84, 1418 us.)
+// symmetries 215 us; 1024 x 1024, 900 views 7.04 -> 0.91 ms; 256 x 256, 90
+// views, batch 5 266 -> 74 us; one value, 721 views from another start angle
+// 1455 -> 1170 us.  (Line ends by FP64 divisions throughout, a four-value sort,
+// compared ramps and the weight's reciprocal per pixel: 260, 1130, 84, 1418 us.)
+// FAR: an image of 4 GiB and more (G = 1).
 template <int G, int W, bool FAR>
 __global__ __launch_bounds__(64 * W) void sf_fwd_kernel(Proj2DArgs g, SymPlan sp, int m, int batch,
                                                         const float* __restrict__ rows_img,
@@ -72,8 +73,8 @@ __global__ __launch_bounds__(64 * kFwdWaves) void sf_lone_kernel(Proj2DArgs g, i
   if (u < g.nu) fwd_lone_store(nseg, red, 1.0, 1.0, 1.0, sino + (size_t)v * g.nu + u);
 }
 
-// A^T, launched as bwd_group_kernel; same cases as above: 841 -> 151 us, 4.13
-// -> 0.64 ms, 146 -> 49 us, 869 -> 664 us.  The FP64 projection of the pixel's
+// A^T, launched as bwd_group_kernel; same cases as above: 841 -> 154 us, 4.13
+// -> 0.65 ms, 146 -> 50 us, 869 -> 683 us.  The FP64 projection of the pixel's
 // centre and its sorted corners are formed once per view for all values, and
 // each bin's area from one new edge (both edges per bin, and a double division
 // per view: 174 us in the first case).

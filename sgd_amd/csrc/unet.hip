@@ -739,7 +739,7 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
 // and so is X but for the pixel on the edge, which the first pixel beyond meets
 // at kx = 0 (ky = 0).  An infinite X must not meet it, and is left out there.
 // At 8 x 512 x 512: 32 -> 32 channels 211 -> 77 us (268 MB; 500 TF/s), 96 -> 32
-// 476 -> 200 us, 8 -> 32 180 -> 48 us; at 8 x 256 x 256 64 -> 64 167 -> 57 us
+// 476 -> 204 us, 8 -> 32 180 -> 48 us; at 8 x 256 x 256 64 -> 64 167 -> 57 us
 // (680 TF/s), 192 -> 64 339 -> 143 us.
 // ---------------------------------------------------------------------------
 constexpr int kWgTH = 4, kWgTW = 32;
