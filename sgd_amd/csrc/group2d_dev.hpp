@@ -177,6 +177,23 @@ struct StripLines {
   }
 };
 
+// Lines l of [0, n) on which some point x of [x0, x1] can pass both tests, s_q x
+// + m_q l >= q0 and s_r x + m_r l < r0: each bounds l from one side at most,
+// one line of margin.  (The rows at which the strip's two edges meet x0 and x1
+// bound it only if the strip is narrower than they are far apart: a slab inside
+// a wide bin's strip may lie to one side of all four.)
+__device__ __forceinline__ void strip_lines(double s_q, double m_q, double q0, double s_r, double m_r, double r0,
+                                            double x0, double x1, int n, int* lo, int* hi) {
+  const double a = q0 - fmax(s_q * x0, s_q * x1), b = r0 - fmin(s_r * x0, s_r * x1);
+  double l = 0.0, h = (double)(n - 1);
+  if (m_q > 0.0) l = fmax(l, floor(a / m_q) - 1.0);
+  else if (m_q < 0.0) h = fmin(h, ceil(a / m_q) + 1.0);
+  if (m_r > 0.0) h = fmin(h, ceil(b / m_r) + 1.0);
+  else if (m_r < 0.0) l = fmax(l, floor(b / m_r) - 1.0);
+  *lo = (int)fmin(l, (double)n);
+  *hi = (int)fmax(h, -1.0);
+}
+
 // A tile's staged bins in LDS: the records as REC float4 planes, then the G
 // sinogram values of each bin as planes of up to 4, so that 16-byte reads of
 // consecutive bins touch all banks.

@@ -161,8 +161,6 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
   constexpr double kTouch = 1.0 + 1e-10;
   const double rq = kTouch * hex_reach(-lay, lax, ha.dt), rr = kTouch * hex_reach(-lby, lbx, ha.dt);
   const double ka = rec.ka, kb = rec.kb;
-  const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
-  const double imq = mq != 0.0 ? 1.0 / mq : 0.0, imr = mr != 0.0 ? 1.0 / mr : 0.0;
 
   // Point values by 32-bit byte offsets into a buffer resource, or by address,
   // clamped to the last point: for a lattice of 4 GiB and more (FAR), and for 8
@@ -210,17 +208,9 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
   const double rmx = vg.e0x + (umid + 0.5) * vg.pux, rmy = vg.e0y + (umid + 0.5) * vg.puy;
   if (fabs(rmy) * g.dx <= 2.0 * g.dy * fabs(rmx)) {
     const int c_lo = g.nx * w / wn, c_hi = g.nx * (w + 1) / wn - 1;
-    // rows the strip can reach within the columns: between the crossings of
-    // its two boundary lines with ic' = c_lo and c_hi + 1, one row of margin
-    int il_lo = 0, il_hi = g.ny - 1;
-    if (mq != 0.0 && mr != 0.0) {
-      const double x0 = (double)c_lo, x1 = (double)(c_hi + 1);
-      const double c1 = (-rq - cq - sq * x0) * imq, c2 = (-rq - cq - sq * x1) * imq;
-      const double c3 = (rr - cr - sr * x0) * imr, c4 = (rr - cr - sr * x1) * imr;
-      const double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-      il_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)g.ny);
-      il_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(g.ny - 1)), -1.0);
-    }
+    // rows the strip can reach within the columns (ic' = ic + 1/2 on odd rows)
+    int il_lo, il_hi;
+    strip_lines(sq, mq, -rq - cq, sr, mr, rr - cr, (double)c_lo, (double)(c_hi + 1), g.ny, &il_lo, &il_hi);
     if (nseg > 1) {
       const int len = (g.ny + nseg - 1) / nseg;
       il_lo = max(il_lo, seg * len);
@@ -251,19 +241,10 @@ __device__ __forceinline__ void hex_fwd_lines(const HexArgs& ha, int v, int chun
     }
   } else {
     const int r_lo = g.ny * w / wn, r_hi = g.ny * (w + 1) / wn - 1;
-    // vertical lines the strip can reach within the rows: between the
-    // crossings of its two boundary lines with rows r_lo and r_hi, one line of
-    // margin
+    // vertical lines the strip can reach within the rows
     const int kmax = 2 * g.nx - 2;
-    int k_lo = 0, k_hi = kmax;
-    if (sq != 0.0 && sr != 0.0) {
-      const double y0 = (double)r_lo, y1 = (double)r_hi;
-      const double c1 = (-rq - cq - mq * y0) * isq, c2 = (-rq - cq - mq * y1) * isq;
-      const double c3 = (rr - cr - mr * y0) * isr, c4 = (rr - cr - mr * y1) * isr;
-      const double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-      k_lo = (int)fmin(fmax(floor(2.0 * lo) - 2.0, 0.0), (double)(kmax + 1));
-      k_hi = (int)fmax(fmin(ceil(2.0 * hi) + 2.0, (double)kmax), -1.0);
-    }
+    int k_lo, k_hi;
+    strip_lines(mq, 0.5 * sq, -rq - cq, mr, 0.5 * sr, rr - cr, (double)r_lo, (double)r_hi, kmax + 1, &k_lo, &k_hi);
     if (nseg > 1) {
       const int len = (kmax + nseg) / nseg;
       k_lo = max(k_lo, seg * len);
