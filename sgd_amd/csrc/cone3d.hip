@@ -469,15 +469,8 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(Cone3DArgs a, int p0, int
   const int nmin = rows ? g.nx : g.ny, nmaj = rows ? g.ny : g.nx;
   const int smin = rows ? 1 : g.nx, smaj = rows ? g.nx : 1;
 
-  int m_lo = 0, m_hi = nmaj - 1;
-  if (mq != 0.0 && mr != 0.0) {
-    const double last = nmin - 1;
-    double c1 = (-ra - qc0) / mq, c2 = (-ra - qc0 - sq * last) / mq;
-    double c3 = (rb - rc0) / mr, c4 = (rb - rc0 - sr * last) / mr;
-    double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    m_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
-    m_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
-  }
+  int m_lo, m_hi;
+  strip_lines(sq, mq, -ra - qc0, sr, mr, rb - rc0, 0.0, (double)(nmin - 1), nmaj, &m_lo, &m_hi);
   if (!live) m_lo = nmaj, m_hi = -1;
   double lo0 = 0.0, lo1 = 0.0, hi0 = nmin - 1, hi1 = 0.0;
   if (sq > 0.0 && sr > 0.0) {

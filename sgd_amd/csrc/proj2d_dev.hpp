@@ -99,19 +99,8 @@ __device__ __forceinline__ void fwd_bin_lines(const Proj2DArgs& g, int v, int ch
   const double isq = sq != 0.0 ? 1.0 / sq : 0.0, isr = sr != 0.0 ? 1.0 / sr : 0.0;
   const float dta = (float)(rec.ka * sa), dtb = (float)(rec.kb * sb);
 
-  // Lines crossed by the strip: between the extreme crossings of its two
-  // boundary lines with the first and last pixel of a line.
-  int m_lo = 0, m_hi = nmaj - 1;
-  if (mq != 0.0 && mr != 0.0) {
-    const double last = nmin - 1;
-    double c1 = (-ra - qc0) / mq, c2 = (-ra - qc0 - sq * last) / mq;
-    double c3 = (rb - rc0) / mr, c4 = (rb - rc0 - sr * last) / mr;
-    double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    lo = fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
-    hi = fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
-    m_lo = (int)lo;
-    m_hi = (int)hi;
-  }
+  int m_lo, m_hi;
+  strip_lines(sq, mq, -ra - qc0, sr, mr, rb - rc0, 0.0, (double)(nmin - 1), nmaj, &m_lo, &m_hi);
   if (nseg > 1) {
     const int len = (nmaj + nseg - 1) / nseg;
     m_lo = max(m_lo, seg * len);

@@ -135,15 +135,8 @@ __device__ __forceinline__ void sf_fwd_lines(const Proj2DArgs& g, int v, int chu
   const float w_n = 0.5f * (float)sa, c_n = 0.5f * (float)ma, w_b = 0.5f * (float)sB, c_b = 0.5f * (float)mB;
   const float nl1 = w_n - c_n, nl2 = w_n + c_n, bl1 = w_b - c_b, bl2 = w_b + c_b;
 
-  int m_lo = 0, m_hi = nmaj - 1;
-  if (ma != 0.0 && mb != 0.0) {
-    const double last = nmin - 1;
-    double c1 = (-ra - ac0) / ma, c2 = (-ra - ac0 - sa * last) / ma;
-    double c3 = (rb - bc0) / mb, c4 = (rb - bc0 - sb * last) / mb;
-    double lo = fmin(fmin(c1, c2), fmin(c3, c4)), hi = fmax(fmax(c1, c2), fmax(c3, c4));
-    m_lo = (int)fmin(fmax(floor(lo) - 1.0, 0.0), (double)nmaj);
-    m_hi = (int)fmax(fmin(ceil(hi) + 1.0, (double)(nmaj - 1)), -1.0);
-  }
+  int m_lo, m_hi;
+  strip_lines(sa, ma, -ra - ac0, sb, mb, rb - bc0, 0.0, (double)(nmin - 1), nmaj, &m_lo, &m_hi);
   if (nseg > 1) {
     const int len = (nmaj + nseg - 1) / nseg;
     m_lo = max(m_lo, seg * len);

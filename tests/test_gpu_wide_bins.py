@@ -44,3 +44,51 @@ def test_hex_wide_bins(cuda, oracle_exact, basis, case, split):
     P = Projector.hexagonal(basis, *geo)
     P.set_split(split, split)
     check(P, HexGeometry(oracle_exact, *geo), cuda, basis, case)
+
+
+# nx, ny, dx, dy, views, start, bins, bin width, lso
+FAN = [(1, 12, 16.7, 16.7, 74, 0.31, 3, 179.3, 500.3), (12, 1, 16.7, 16.7, 74, 0.31, 3, 179.3, 500.3),
+       (2, 2, 100.0, 93.0, 9, 0.37, 2, 253.7, 500.3), (3, 3, 66.7, 50.0, 51, 0.11, 2, 246.1, 500.3),
+       (109, 109, 1.83, 1.83, 105, 0.37, 2, 220.3, 400.0), (60, 7, 3.3, 3.9, 33, 0.23, 5, 61.1, 500.3),
+       (41, 12, 4.88, 6.72, 13, 0.4, 2, 237.0, 500.3), (64, 64, 3.1, 3.1, 40, 0.0, 1, 431.0, 500.0)]
+
+
+@pytest.mark.parametrize("basis", ["B0", "B1", "SF"])
+@pytest.mark.parametrize("case", range(len(FAN)))
+@pytest.mark.parametrize("split", [0, 24])
+def test_fan_wide_bins(cuda, oracle_exact, basis, case, split):
+    from pyoracle import Geometry
+    from sgd_amd.torch_ops import Projector
+    nx, ny, dx, dy, n, start, nu, du, lso = FAN[case]
+    geo = (nx, ny, start + 2 * np.pi * np.arange(n) / n, nu, dx, dy, du, 2 * lso, lso)
+    print(basis, FAN[case], split, flush=True)
+    if (basis, case) in (("B0", 2), ("B1", 3)):
+        # Points whose range ends within a bin's margin of the detector: the
+        # model is not zero there and the oracle leaves them out (B0 2.5e-3 in
+        # both directions, B1 2.2e-5 in A; no line is lost).
+        pytest.xfail("pixels of 50 and more at the detector's end bins")
+    P = Projector(basis, *geo)
+    P.set_split(split, split)
+    check(P, Geometry(oracle_exact, *geo), cuda, basis, case)
+
+
+@pytest.mark.parametrize("model", ["B1", "SF-TR", "SF-TT"])
+@pytest.mark.parametrize("case", range(len(FAN)))
+def test_cone_wide_bins(cuda, oracle_exact, model, case):
+    from pyoracle import Geometry3
+    from sgd_amd.torch_ops import Projector
+    nx, ny, dx, dy, n, start, nu, du, lso = FAN[case]
+    n = min(n, 21)
+    geo = (nx, ny, 5, start + 2 * np.pi * np.arange(n) / n, nu, 9, dx, dy, 1.0, du, 2.0, 2 * lso, lso)
+    print(model, FAN[case], flush=True)
+
+    class Oracle:
+        g = Geometry3(oracle_exact, *geo)
+
+        def forward(self, _, x):
+            return self.g.forward(x) if model == "B1" else self.g.sf_forward(x, trap_v=model == "SF-TT")
+
+        def backward(self, _, y):
+            return self.g.backward(y) if model == "B1" else self.g.sf_backward(y, trap_v=model == "SF-TT")
+
+    check(Projector.cone_beam(*geo, model=model), Oracle(), cuda, model, case)
